@@ -89,7 +89,7 @@ __global__ __launch_bounds__(256) void q8_im2col_kernel(const uint8_t *in, uint8
 // together from single LDS bytes (k in (kh, kw, channel) order: the k_w * cin bytes of one kh lie
 // side by side in a staged row; bytes past the depth are 0x80, zero after the shift).  The filter
 // stays in registers as MFMA fragments for the whole kernel; the epilogue is the streaming GEMM
-// kernel's (threshold requantization, 16-byte stores).
+// kernel's (requantization by multiply-add, 16-byte stores).
 struct ConvShortParams {
   const uint8_t *in, *filter;
   const int32_t *bias;
@@ -106,16 +106,14 @@ struct ConvShortParams {
   int32_t xcoef, ycoef, yadd;
   RequantFixed rq;
 };
-static_assert(sizeof(ConvShortParams) % alignof(RequantTable) == 0, "argument layout");
 
 // (Occupancy 3 in the launch bounds: with at most 170 registers the compiler keeps the MFMA results
 // in ordinary registers, which spares the epilogue a move per output.)
 template <int FX>
-__global__ __launch_bounds__(256, 3) void q8_conv_short_kernel(ConvShortParams p, RequantTable) {
+__global__ __launch_bounds__(256, 3) void q8_conv_short_kernel(ConvShortParams p) {
   extern __shared__ __align__(16) uint8_t lds[];
   int32_t *s_cx = (int32_t *)lds;                                 // [32 FX]
-  int32_t *s_tab = s_cx + 32 * FX;                                // the comparison table's pairs
-  uint8_t *rows = lds + 128 * FX + MH_REQUANT_PAIRS_BYTES;        // staged input rows
+  uint8_t *rows = lds + 128 * FX;                                 // staged input rows
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, r32 = lane & 31;
@@ -128,7 +126,7 @@ __global__ __launch_bounds__(256, 3) void q8_conv_short_kernel(ConvShortParams p
 
   // The strip's input rows go to LDS BATCH dwords per thread at a time: all loads of a turn are
   // requested before the first is stored, and the first turn's before anything else of the
-  // prologue, so that the filter's and the table's loads travel with them (one load per turn of a
+  // prologue, so that the filter's loads travel with them (one load per turn of a
   // loop would put a dozen memory round trips in front of every workgroup's first block).  No
   // load sits under a condition: padding and rows outside the image load from a clamped address
   // and are replaced; a row's last, partial dword is taken from the dword that ends at the row's
@@ -190,10 +188,6 @@ __global__ __launch_bounds__(256, 3) void q8_conv_short_kernel(ConvShortParams p
     bias_v[i] = 0;
     if (p.bias) bias_v[i] = p.bias[c];
   }
-  // (the comparison table's load travels with them)
-  stage_requant_pairs_from((const int32_t *)((const char *)__builtin_amdgcn_kernarg_segment_ptr() +
-                                             sizeof(ConvShortParams)),
-                           s_tab, p.rq, tid, 256);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = 0; i < FX; ++i) {
@@ -236,7 +230,7 @@ __global__ __launch_bounds__(256, 3) void q8_conv_short_kernel(ConvShortParams p
       if (++off == p.run) { off = 0; kh_off += p.pitch; }
     }
   }
-  const RequantLds rql = requant_lds(p.rq, s_tab);
+  const RequantMad rqm = requant_mad(p.rq);
   __syncthreads();
 
   const int nblk = (npix + 31) >> 5;
@@ -287,7 +281,7 @@ __global__ __launch_bounds__(256, 3) void q8_conv_short_kernel(ConvShortParams p
         for (int e = 0; e < 4; ++e) v[g * 4 + e] = (int32_t)((uint32_t)acc[g * 4 + e] + (uint32_t)cx[e] + cy);
       }
       uint32_t packed[4];
-      requant_16_by_table(v, rql, packed);
+      requant_16_by_mad(v, rqm, packed);
       const v2u s02 = __builtin_amdgcn_permlane32_swap(packed[0], packed[2], false, false);
       const v2u s13 = __builtin_amdgcn_permlane32_swap(packed[1], packed[3], false, false);
       const v4i o = {(int)s02.x, (int)s02.y, (int)s13.x, (int)s13.y};
@@ -314,11 +308,10 @@ __global__ __launch_bounds__(256, 3) void q8_conv_short_kernel(ConvShortParams p
 // filter tap, such layers went through the one-launch kernel (3 x 3, 112 x 112 x 32 -> 64 at batch
 // 64: 78 us).
 template <int FX, int KS>
-__global__ __launch_bounds__(256, 2) void q8_conv_rows_kernel(ConvShortParams p, RequantTable) {
+__global__ __launch_bounds__(256, 2) void q8_conv_rows_kernel(ConvShortParams p) {
   extern __shared__ __align__(16) uint8_t lds[];
   int32_t *s_cx = (int32_t *)lds;                                 // [32 FX]
-  int32_t *s_tab = s_cx + 32 * FX;                                // the comparison table's pairs
-  uint8_t *rows = lds + ((128 * FX + MH_REQUANT_PAIRS_BYTES + 15) & ~15);   // staged input rows
+  uint8_t *rows = lds + 128 * FX;                                 // staged input rows
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, r32 = lane & 31;
@@ -395,10 +388,6 @@ __global__ __launch_bounds__(256, 2) void q8_conv_rows_kernel(ConvShortParams p,
     bias_v[i] = 0;
     if (p.bias) bias_v[i] = p.bias[c];
   }
-  // (the comparison table's load travels with them)
-  stage_requant_pairs_from((const int32_t *)((const char *)__builtin_amdgcn_kernarg_segment_ptr() +
-                                             sizeof(ConvShortParams)),
-                           s_tab, p.rq, tid, 256);
   __builtin_amdgcn_sched_barrier(0);
   // where piece 2 ks + h of a patch lies relative to the patch's first byte: pieces follow one
   // another along a filter row and step by the pitch from row to row (the same in every lane but
@@ -444,7 +433,7 @@ __global__ __launch_bounds__(256, 2) void q8_conv_rows_kernel(ConvShortParams p,
     stage_issue(base0);
     stage_commit();
   }
-  const RequantLds rql = requant_lds(p.rq, s_tab);
+  const RequantMad rqm = requant_mad(p.rq);
   __syncthreads();
 
   const int nblk = (npix + 31) >> 5;
@@ -505,7 +494,7 @@ __global__ __launch_bounds__(256, 2) void q8_conv_rows_kernel(ConvShortParams p,
         for (int e = 0; e < 4; ++e) v[g * 4 + e] = (int32_t)((uint32_t)acc[i][g * 4 + e] + (uint32_t)cx[e] + cy);
       }
       uint32_t packed[4];
-      requant_16_by_table(v, rql, packed);
+      requant_16_by_mad(v, rqm, packed);
       const v2u s02 = __builtin_amdgcn_permlane32_swap(packed[0], packed[2], false, false);
       const v2u s13 = __builtin_amdgcn_permlane32_swap(packed[1], packed[3], false, false);
       const v4i o = {(int)s02.x, (int)s02.y, (int)s13.x, (int)s13.y};
@@ -851,7 +840,7 @@ int conv_short(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, c
   if (shift < 0 || shift > 31 || clamp_min < 0 || clamp_max > 255 || clamp_min > clamp_max)
     return MACE_HIP_SUCCESS;   // (the general path reports these)
   RequantFixed rq;
-  if (!mh_make_requant(mult, shift, out_zp, clamp_min, clamp_max, &rq) || !rq.table)
+  if (!mh_make_requant(mult, shift, out_zp, clamp_min, clamp_max, &rq) || !requant_by_mad(rq))
     return MACE_HIP_SUCCESS;
   // staged rows: pixel positions -pad_left ... up to the last one any patch or the image reaches
   const int64_t reach = std::max<int64_t>(in_w + pad_left, (out_w - 1) * stride_w + k_w);
@@ -859,7 +848,7 @@ int conv_short(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, c
   const int gbase = lead - (int)(pad_left * cin);
   const int64_t pitch = (int64_t)mh_align_up((size_t)(gbase + reach * cin), 4);
   const int fx = cout <= 32 ? 1 : (cout <= 64 ? 2 : 4);
-  const int64_t fixed = 128 * fx + MH_REQUANT_PAIRS_BYTES;
+  const int64_t fixed = 128 * fx;
   auto lds_of = [&](int64_t r) { return fixed + ((r - 1) * stride_h + k_h) * pitch; };
   if (lds_of(1) > 64 * 1024 || n * in_h >= (1ll << 31) || in_w * cin >= (1ll << 30)) return MACE_HIP_SUCCESS;
   // Rows per strip: about columns / (2 CUs) pixels per workgroup, between 128 and 1024, and what
@@ -886,8 +875,6 @@ int conv_short(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, c
   ArenaScope scope(ctx);
   const int32_t *bias_used = nullptr;
   MH_RETURN_IF_ERROR(conv_bias(ctx, bias, cout, input_scale, filter_scale, bias_scale, &bias_used));
-  RequantTable tab;
-  mh_requant_table_cached(ctx, rq, tab.t);
   const uint32_t zl = (uint32_t)filter_zp - 128u, zr = (uint32_t)input_zp - 128u;
   ConvShortParams p{};
   p.in = input; p.filter = filter; p.bias = bias_used; p.out = out;
@@ -904,9 +891,9 @@ int conv_short(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, c
   dim3 grid((unsigned)(n * strips)), block(256);
   mh_plan_main(ctx, MACE_HIP_KF_Q8_CONV_SHORT, mhv::conv_short(fx), grid, block, (int)lds);
   MH_PROF_BEGIN(ctx);
-  if (fx == 1) MH_KLAUNCH(ctx, q8_conv_short_kernel<1>, grid, block, lds, ctx->stream, p, tab);
-  else if (fx == 2) MH_KLAUNCH(ctx, q8_conv_short_kernel<2>, grid, block, lds, ctx->stream, p, tab);
-  else MH_KLAUNCH(ctx, q8_conv_short_kernel<4>, grid, block, lds, ctx->stream, p, tab);
+  if (fx == 1) MH_KLAUNCH(ctx, q8_conv_short_kernel<1>, grid, block, lds, ctx->stream, p);
+  else if (fx == 2) MH_KLAUNCH(ctx, q8_conv_short_kernel<2>, grid, block, lds, ctx->stream, p);
+  else MH_KLAUNCH(ctx, q8_conv_short_kernel<4>, grid, block, lds, ctx->stream, p);
   MH_PROF_END(ctx);
   MH_LAUNCH_CHECK(ctx);
   return MACE_HIP_SUCCESS;
@@ -934,7 +921,7 @@ int conv_rows(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, co
   if (shift < 0 || shift > 31 || clamp_min < 0 || clamp_max > 255 || clamp_min > clamp_max)
     return MACE_HIP_SUCCESS;   // (the general path reports these)
   RequantFixed rq;
-  if (!mh_make_requant(mult, shift, out_zp, clamp_min, clamp_max, &rq) || !rq.table)
+  if (!mh_make_requant(mult, shift, out_zp, clamp_min, clamp_max, &rq) || !requant_by_mad(rq))
     return MACE_HIP_SUCCESS;
   // staged rows: pixel positions -pad_left ... up to the last one any patch or the image reaches
   // (cin is a multiple of 16, so every position starts a 16-byte piece)
@@ -942,7 +929,7 @@ int conv_rows(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, co
   const int lead = (int)(pad_left * cin);
   const int64_t pitch = reach * cin;
   const int fx = cout <= 32 ? 1 : (cout <= 64 ? 2 : 4);
-  const int64_t fixed = (128 * fx + MH_REQUANT_PAIRS_BYTES + 15) & ~(int64_t)15;
+  const int64_t fixed = 128 * fx;
   auto lds_of = [&](int64_t r) { return fixed + ((r - 1) * stride_h + k_h) * pitch; };
   // (the kernel multiplies row numbers by row lengths with 24-bit factors and keeps offsets inside
   // an image and inside the filter in 32 bits)
@@ -968,8 +955,6 @@ int conv_rows(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, co
   ArenaScope scope(ctx);
   const int32_t *bias_used = nullptr;
   MH_RETURN_IF_ERROR(conv_bias(ctx, bias, cout, input_scale, filter_scale, bias_scale, &bias_used));
-  RequantTable tab;
-  mh_requant_table_cached(ctx, rq, tab.t);
   const uint32_t zl = (uint32_t)filter_zp - 128u, zr = (uint32_t)input_zp - 128u;
   ConvShortParams p{};
   p.in = input; p.filter = filter; p.bias = bias_used; p.out = out;
@@ -986,7 +971,7 @@ int conv_rows(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, co
   dim3 grid((unsigned)(n * strips)), block(256);
   mh_plan_main(ctx, MACE_HIP_KF_Q8_CONV_ROWS, mhv::conv_rows(fx, (int)ks), grid, block, (int)lds);
   MH_PROF_BEGIN(ctx);
-#define MH_ROWS(FX_, KS_) MH_KLAUNCH(ctx, (q8_conv_rows_kernel<FX_, KS_>), grid, block, lds, ctx->stream, p, tab)
+#define MH_ROWS(FX_, KS_) MH_KLAUNCH(ctx, (q8_conv_rows_kernel<FX_, KS_>), grid, block, lds, ctx->stream, p)
   if (ks == 5) {
     if (fx == 1) MH_ROWS(1, 5); else if (fx == 2) MH_ROWS(2, 5); else MH_ROWS(4, 5);
   } else {

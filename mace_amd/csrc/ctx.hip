@@ -7,6 +7,7 @@
 #include <new>
 
 #include "common.h"
+#include "q8_requant.h"
 
 int mh_fail(mace_hip_ctx *ctx, int code, const char *fmt, ...) {
   if (ctx) {
@@ -556,6 +557,10 @@ int mace_hip_requant_table_u8(int32_t acc, int32_t multiplier, int right_shift,
   if (!out || clamp_min < 0 || clamp_max > 255 || clamp_min > clamp_max ||
       !mh_make_requant(multiplier, right_shift, offset_after_shift, clamp_min, clamp_max, &q))
     return -1;
+  if (requant_by_mad(q)) {
+    *out = (uint8_t)requant_mad_one(acc, requant_mad(q));
+    return 1;
+  }
   if (!q.table) {
     *out = (uint8_t)mh_requant_fixed(acc, q);
     return 0;

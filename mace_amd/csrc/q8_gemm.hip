@@ -134,10 +134,12 @@ __device__ inline int sum16_i8(const v4i &f, int acc) {
 }
 
 // The comparison table's first halves follow GemmParams in the argument segment (indexing a
-// by-value copy with a lane-dependent index would spill it).
+// by-value copy with a lane-dependent index would spill it).  Needed only by calls outside the
+// multiply-add form.
 __device__ inline void stage_requant_pairs(int32_t *pairs, const RequantFixed &rq, int tid,
                                            int nthreads) {
   static_assert(sizeof(GemmParams) % alignof(RequantTable) == 0, "argument layout");
+  if (!rq.table || requant_by_mad(rq)) return;   // (the same for every thread)
   stage_requant_pairs_from((const int32_t *)((const char *)__builtin_amdgcn_kernarg_segment_ptr() +
                                              sizeof(GemmParams)),
                            pairs, rq, tid, nthreads);
@@ -182,7 +184,7 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
       sc[TX + i] = (int32_t)c;
     }
   if constexpr (sizeof(OutT) == 1) {
-    if (rq.table) stage_requant_pairs(tab, rq, tid, NT);
+    stage_requant_pairs(tab, rq, tid, NT);
   }
   __syncthreads();
   }
@@ -197,10 +199,14 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
   const bool wide16 = (p.ldo % 16 == 0) && (((uintptr_t)outb) % 16 == 0) && (p.XN % 16 == 0);
 
   const RequantLds rql = requant_lds(rq, tab);
-  // One fully unrolled copy of the store loop per combination that occurs: TABLE = threshold
-  // requantization, WIDE = whole tile inside the matrix and 16-byte aligned rows.
-  auto store_tile = [&](auto table_tag, auto wide_tag) __attribute__((always_inline)) {
-    constexpr bool TABLE = decltype(table_tag)::value;
+  const bool by_mad = requant_by_mad(rq);
+  RequantMad rqm{};
+  if (by_mad) rqm = requant_mad(rq);
+  // One fully unrolled copy of the store loop per combination that occurs: MAD = requantization by
+  // multiply-add, WIDE = whole tile inside the matrix and 16-byte aligned rows.  Parameters outside
+  // the multiply-add form share one copy, by table or by the plain arithmetic.
+  auto store_tile = [&](auto mad_tag, auto wide_tag) __attribute__((always_inline)) {
+    constexpr bool MAD = decltype(mad_tag)::value;
     constexpr bool WIDE = decltype(wide_tag)::value;
 #pragma unroll
     for (int j = 0; j < FY; ++j) {
@@ -246,7 +252,9 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
           }
         } else {
           uint32_t packed[4] = {0, 0, 0, 0};
-          if constexpr (TABLE) {
+          if constexpr (MAD) {
+            requant_16_by_mad(v, rqm, packed);
+          } else if (rq.table) {
             requant_16_by_table(v, rql, packed);
           } else {
 #pragma unroll
@@ -294,8 +302,8 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
   if constexpr (sizeof(OutT) == 4) {
     store_tile(std::false_type{}, std::false_type{});
   } else {
-    if (rq.table && interior16) store_tile(std::true_type{}, std::true_type{});
-    else if (rq.table) store_tile(std::true_type{}, std::false_type{});
+    if (by_mad && interior16) store_tile(std::true_type{}, std::true_type{});
+    else if (by_mad) store_tile(std::true_type{}, std::false_type{});
     else store_tile(std::false_type{}, std::false_type{});
   }
 }
@@ -647,7 +655,7 @@ __global__ __launch_bounds__(256, BW ? 5 : 1) void q8_gemm_fused_small_kernel(Ge
   // Everything the epilogue needs from memory is asked for now, so that it arrives under the
   // operand loads: the comparison table (into LDS) and this lane's bias.
   if constexpr (sizeof(OutT) == 1) {
-    if (p.rq.table) stage_requant_pairs(sc + 2 * T, p.rq, tid, 256);
+    stage_requant_pairs(sc + 2 * T, p.rq, tid, 256);
   }
   const int32_t xbias = p.xbias ? p.xbias[min(x0 + wx * 32 + (lane & 31), p.XN - 1)] : 0;
 
@@ -1108,7 +1116,7 @@ __global__ __launch_bounds__(WX *WY * 64, OCC) void q8_gemm_dma_kernel(GemmParam
       }
     }
     if constexpr (sizeof(OutT) == 1) {
-      if (p.rq.table) stage_requant_pairs(sc + TX + TY, p.rq, tid, NW * 64);
+      stage_requant_pairs(sc + TX + TY, p.rq, tid, NW * 64);
     }
     __syncthreads();
     gemm_epilogue<WX, WY, FX, FY, OutT, SUMY, true>(acc, ysum, p, lds, b, x0, y0, wx, wy, tid);
@@ -1387,7 +1395,7 @@ __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p, Requa
         for (int r = 0; r < 16; ++r) mine[(j * 16 + r) * 64] = acc[0][j][r];
     }
     if constexpr (sizeof(OutT) == 1) {
-      if (p.rq.table) stage_requant_pairs(sc + 2 * T, p.rq, tid, 512);
+      stage_requant_pairs(sc + 2 * T, p.rq, tid, 512);
     }
     __syncthreads();
 #pragma unroll
@@ -1610,7 +1618,7 @@ __global__ __launch_bounds__(256, OCC) void q8_gemm_xres_kernel(GemmParams p, Re
       sc[i] = (int32_t)c;
     }
     if constexpr (sizeof(OutT) == 1) {
-      if (rq.table) stage_requant_pairs(sc + TX + TYW, rq, tid, 256);
+      stage_requant_pairs(sc + TX + TYW, rq, tid, 256);
     }
     __syncthreads();
   } else {
@@ -1674,7 +1682,7 @@ __global__ __launch_bounds__(256, OCC) void q8_gemm_xres_kernel(GemmParams p, Re
       sc[row] = (int32_t)c;
     }
     if constexpr (sizeof(OutT) == 1) {
-      if (rq.table) stage_requant_pairs(sc + TX + TYW, rq, tid, 256);
+      stage_requant_pairs(sc + TX + TYW, rq, tid, 256);
     }
     __syncthreads();
   }
@@ -1768,17 +1776,16 @@ __global__ __launch_bounds__(256, OCC) void q8_gemm_xres_kernel(GemmParams p, Re
 // per workgroup, into LDS; Y per block from the fragments), so the call is this one launch.
 //
 // XN a multiple of 16 in (32 (FX XW - 1), 32 FX XW], K = 32 KS or 32 KS - 16, uint8 output by
-// threshold look-up only, result rows (ldo = XN bytes) and base 16-byte aligned: the host checks
+// multiply-add only, result rows (ldo = XN bytes) and base 16-byte aligned: the host checks
 // all of that.
 // (The occupancy in the launch bounds is what the host launches, see launch_gemm_stream; with at
 // most 256 registers per wavefront the compiler also keeps the MFMA results in ordinary VGPRs,
 // which spares the epilogue one register move per output.)
 template <int FX, int KS, int XW, int D>
 __global__ __launch_bounds__(256, (FX * KS <= 2 ? 4 : (FX * KS <= 4 ? 3 : (FX * KS <= 16 ? 2 : 1))))
-void q8_gemm_stream_kernel(GemmParams p, RequantTable) {
+void q8_gemm_stream_kernel(GemmParams p) {
   constexpr int YW = 4 / XW;   // wavefronts of the workgroup along Y
-  __shared__ int32_t s_cx[32 * FX * XW];
-  __shared__ __align__(8) int32_t s_tab[MH_REQUANT_PAIRS_BYTES / 4];
+  __shared__ __align__(16) int32_t s_cx[32 * FX * XW];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1817,8 +1824,7 @@ void q8_gemm_stream_kernel(GemmParams p, RequantTable) {
       s_cx[xi] = (int32_t)c;
     }
   }
-  stage_requant_pairs(s_tab, rq, tid, 256);
-  const RequantLds rql = requant_lds(rq, s_tab);
+  const RequantMad rqm = requant_mad(rq);
   __syncthreads();
 
   const int nblk = (p.YN + 31) / 32;
@@ -1876,7 +1882,7 @@ void q8_gemm_stream_kernel(GemmParams p, RequantTable) {
               v[q * 4 + e] = (int32_t)((uint32_t)acc[q * 4 + e] + (uint32_t)cx[e] + cy);
           }
           uint32_t packed[4];
-          requant_16_by_table(v, rql, packed);
+          requant_16_by_mad(v, rqm, packed);
           const v2u s02 = __builtin_amdgcn_permlane32_swap(packed[0], packed[2], false, false);
           const v2u s13 = __builtin_amdgcn_permlane32_swap(packed[1], packed[3], false, false);
           const v4i w = {(int)s02.x, (int)s02.y, (int)s13.x, (int)s13.y};
@@ -2486,7 +2492,7 @@ int launch_gemm_xres_any(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &t
 
 // the streaming kernel; the caller has checked its preconditions (see the kernel)
 template <int FX, int XW>
-int launch_gemm_stream(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, int batch) {
+int launch_gemm_stream(mace_hip_ctx *ctx, GemmParams &p, int batch) {
   constexpr int YW = 4 / XW;
   const int nblk = (p.YN + 31) / 32;
   const int ks = (p.K + 31) / 32;
@@ -2499,8 +2505,8 @@ int launch_gemm_stream(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab
   mh_plan_main(ctx, MACE_HIP_KF_Q8_GEMM_STREAM, mhv::stream(FX, ks), grid, block, 0);
   MH_PROF_BEGIN(ctx);
   switch (ks) {
-    case 1: MH_KLAUNCH(ctx, (q8_gemm_stream_kernel<FX, 1, XW, 4>), grid, block, 0, ctx->stream, p, tab); break;
-    case 2: MH_KLAUNCH(ctx, (q8_gemm_stream_kernel<FX, 2, XW, 4>), grid, block, 0, ctx->stream, p, tab); break;
+    case 1: MH_KLAUNCH(ctx, (q8_gemm_stream_kernel<FX, 1, XW, 4>), grid, block, 0, ctx->stream, p); break;
+    case 2: MH_KLAUNCH(ctx, (q8_gemm_stream_kernel<FX, 2, XW, 4>), grid, block, 0, ctx->stream, p); break;
     default: return mh_fail(ctx, MACE_HIP_RUNTIME_ERROR, "streaming kernel: unsupported depth");
   }
   MH_PROF_END(ctx);
@@ -2736,7 +2742,7 @@ int Q8Call::prepare(bool *done) {
           (ctx->lds_bytes > 0 ? (size_t)ctx->lds_bytes : 65536) &&
       !mh_q8_small_problem(ctx, batch, rows, cols, depth, true, false) &&
       // (depths of 16 to 48 against at most 128 X rows are the streaming kernel's, see `stream`)
-      !(out_u8 && rq.table && mh_q8_stream_shape(depth, mid_xn, mid_yn) && (uintptr_t)out % 16 == 0) &&
+      !(out_u8 && requant_by_mad(rq) && mh_q8_stream_shape(depth, mid_xn, mid_yn) && (uintptr_t)out % 16 == 0) &&
       !(ctx->kernel_mask & MH_MASK_NO_XRES);
   return MACE_HIP_SUCCESS;
 }
@@ -2760,7 +2766,7 @@ int Q8Call::small_problem(bool *done) {
     // kernel to go to: the one-launch kernel takes them at any size -- except the shapes of the
     // streaming kernel for a small X panel (see `stream` below), which is faster there.
     const int64_t xn_s = xl ? rows : cols, yn_s = xl ? cols : rows;
-    const bool stream_shape = out_u8 && rq.table && mh_q8_stream_shape(depth, xn_s, yn_s) &&
+    const bool stream_shape = out_u8 && requant_by_mad(rq) && mh_q8_stream_shape(depth, xn_s, yn_s) &&
                               ((uintptr_t)out % 16 == 0);
     const bool in_place = !lhs_t && !rhs_t && lhs_direct && rhs_direct && rhs_ld == 0;
     const bool any_size = in_place && depth % 64 != 0 && !stream_shape && !tail_xres;
@@ -2790,7 +2796,7 @@ int Q8Call::small_problem(bool *done) {
       p.y_dword = p.y_bytewise && (cv ? (uintptr_t)p.Y % 4 == 0 && cv->cin % 4 == 0
                                       : by_dwords(p.Y, p.ldy, p.ybs, yt, p.YN));
       RequantTable tab;
-      if (out_u8 && rq.table) mh_requant_table_cached(ctx, rq, tab.t);
+      if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
       *done = true;
       return launch_gemm_fused_small(ctx, p, tab, out_u8, xt, yt, (int)batch);
     }
@@ -2853,7 +2859,7 @@ int Q8Call::kmajor_in_place(bool *done) {
       GemmParams p = kmajor_params();
       p.sum_y = true;
       RequantTable tab;
-      if (out_u8 && rq.table) mh_requant_table_cached(ctx, rq, tab.t);
+      if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
       *done = true;
       return launch_gemm_xres_any(ctx, p, tab, out_u8, (int)batch, tx, true);
     }
@@ -2868,7 +2874,7 @@ int Q8Call::kmajor_in_place(bool *done) {
     if (mid_xt) {
       GemmParams p = kmajor_params();
       RequantTable tab;
-      if (out_u8 && rq.table) mh_requant_table_cached(ctx, rq, tab.t);
+      if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
       *done = true;
       return launch_gemm_mid(ctx, p, tab, out_u8, (int)batch, true);
     }
@@ -2889,7 +2895,7 @@ int Q8Call::kmajor_in_place(bool *done) {
                                  rhs_offset, ep.bias);
         p.sum_y = true;
         RequantTable tab;
-        if (out_u8 && rq.table) mh_requant_table_cached(ctx, rq, tab.t);
+        if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
         *done = true;
         return launch_gemm_xres_any(ctx, p, tab, out_u8, (int)batch, tx8, false);
       }
@@ -2915,7 +2921,7 @@ int Q8Call::kmajor_in_place(bool *done) {
         GemmParams p = q8_params(xl, xl ? Xo : Yo, xl ? Yo : Xo, rows, cols, depth, (int)depth, out,
                                  out_u8, rq, lhs_offset, rhs_offset, ep.bias);
         RequantTable tab;
-        if (out_u8 && rq.table) mh_requant_table_cached(ctx, rq, tab.t);
+        if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
         *done = true;
         return launch_gemm_mid(ctx, p, tab, out_u8, (int)batch, x_kmajor, true);
       }
@@ -2948,7 +2954,7 @@ int Q8Call::kmajor_in_place(bool *done) {
       if (!p.sum_y)
         MH_RETURN_IF_ERROR(launch_panel_sums(ctx, yp, depth, p.ybs, yn, (int)depth, y_nb, sum_y_buf));
       RequantTable tab;
-      if (out_u8 && rq.table) mh_requant_table_cached(ctx, rq, tab.t);
+      if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
       *done = true;
       return launch_gemm_big_xt(ctx, p, tab, out_u8, (int)batch, sum_x_in_kernel);
     }
@@ -3150,7 +3156,7 @@ int Q8Call::general() {
   // long Y panel goes to the streaming kernel, which also sums both panels itself.
   const int64_t xn = x_is_lhs ? rows : cols, yn = x_is_lhs ? cols : rows;
   // (Measured: it wins for K <= 64; from K = 128 on the tiled kernels are as fast.)
-  const bool stream = !cv && out_u8 && rq.table && lhs_direct && rhs_direct && rhs_ld == 0 &&
+  const bool stream = !cv && out_u8 && requant_by_mad(rq) && lhs_direct && rhs_direct && rhs_ld == 0 &&
                       mh_q8_stream_shape(depth, xn, yn) && ((uintptr_t)out % 16 == 0);
   const int32_t *sumL = L.sums ? L.sums : corrL, *sumR = R.sums ? R.sums : corrR;
   // An X panel whose tile (64 or 128 rows, all of k) fits in LDS twice per CU goes to the kernel
@@ -3220,7 +3226,7 @@ int Q8Call::general() {
   p.cxbs = (x_is_lhs ? lhs_nb : rhs_nb) > 1 ? p.XN : 0;
   p.cybs = (x_is_lhs ? rhs_nb : lhs_nb) > 1 ? p.YN : 0;
   RequantTable tab;
-  if (out_u8 && rq.table) mh_requant_table_cached(ctx, rq, tab.t);
+  if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
   p.sum_y = sum_y;
   if (cv) {
     q8_params_conv(&p, *cv);
@@ -3236,10 +3242,10 @@ int Q8Call::general() {
   if (mid) return launch_gemm_mid(ctx, p, tab, out_u8, (int)batch);
   if (stream) {
     switch ((p.XN + 31) / 32) {
-      case 1: return launch_gemm_stream<1, 1>(ctx, p, tab, (int)batch);
-      case 2: return launch_gemm_stream<2, 1>(ctx, p, tab, (int)batch);
-      case 3: return launch_gemm_stream<3, 1>(ctx, p, tab, (int)batch);
-      default: return launch_gemm_stream<4, 1>(ctx, p, tab, (int)batch);
+      case 1: return launch_gemm_stream<1, 1>(ctx, p, (int)batch);
+      case 2: return launch_gemm_stream<2, 1>(ctx, p, (int)batch);
+      case 3: return launch_gemm_stream<3, 1>(ctx, p, (int)batch);
+      default: return launch_gemm_stream<4, 1>(ctx, p, (int)batch);
     }
   }
 
