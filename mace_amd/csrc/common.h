@@ -586,10 +586,11 @@ inline int mh_f32_ksplit(const mace_hip_ctx *ctx, int64_t batch, int64_t rows, i
   if (parts > 16) parts = 16;
   return parts < 2 ? 1 : (int)parts;
 }
-// scratch of that split (0 without one)
+// scratch of that split (0 without one); a batch may also be run as one long row of columns
 inline size_t mh_f32_ksplit_bytes(const mace_hip_ctx *ctx, int64_t batch, int64_t rows, int64_t cols,
                                   int64_t depth) {
-  const int parts = mh_f32_ksplit(ctx, batch, rows, cols, depth);
+  const int parts = std::max(mh_f32_ksplit(ctx, batch, rows, cols, depth),
+                             mh_f32_ksplit(ctx, 1, rows, batch * cols, depth));
   return parts > 1 ? sizeof(float) * (size_t)parts * batch * rows * cols + 256 : 0;
 }
 

@@ -4,21 +4,21 @@
 // semantics mace/ops/ref/gemm.cc:58-146; the NEON implementation it stands in for is
 // mace/ops/arm/base/gemm.cc:520-683): out[b] = lhs[b or 0] * rhs[b or 0] with each of the
 // three matrices RowMajor or ColMajor.  The NEON kernel packs both operands into cache
-// panels; here the panels are LDS tiles ([k][m] and [k][n], so a wavefront's fragment read
-// is one conflict-free row segment) feeding v_mfma_f32_32x32x2_f32.  Products and sums are
-// binary32; the summation order differs from the reference's serial k loop, which the
-// reference's own tolerance (1e-4 relative + 1e-2 absolute) covers.
+// panels; here the panels are LDS tiles of the operands' three bf16 parts (below).  Products are
+// good to binary32 and sums are binary32; the summation order differs from the reference's serial k
+// loop, which the reference's own tolerance (1e-4 relative + 1e-2 absolute) covers.
 //
 // Gemv replaces delegator::Gemv for float (mace/ops/delegator/gemv.h:35-44,
 // mace/ops/ref/gemv.cc:46-81): one wavefront per output row, lane-strided loads.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-constexpr int TM = 128, TN = 128, TK = 16;
-constexpr int LDT = TM + 4;   // padded LDS row (floats)
+constexpr int TM = 128, TN = 128, TK = 16;   // (TK: the unit a k split deals out)
 
 struct F32GemmParams {
   const float *lhs, *rhs;
@@ -28,16 +28,18 @@ struct F32GemmParams {
   int64_t ors, ocs;   // out element strides for (row, col)
   int64_t lbs, rbs, obs;
   int M, N, K;
+  int flat;   // columns per batch where the columns of all batches are one long row of N (0: not so)
   const float *bias_row;   // added per result row (a convolution's output channel), or nullptr
   const float *bias_col;   // added per result column (MatMul's bias), or nullptr
   int act;
   float limit;
   int tiles_m;
   // k split: blockIdx.y takes k tiles [y kt_split, (y + 1) kt_split) and
-  // stores its raw sums into part[(y batches + b) obs + ...] with the result's own strides;
+  // stores its raw sums into part[y part_stride + ...] with the result's own strides;
   // f32_ksplit_reduce_kernel adds the parts in the order of y and applies bias and activation.
   // kt_split = 0: no split.
   float *part;
+  int64_t part_stride;   // elements of one part: the whole result
   int kt_split;
 };
 
@@ -63,112 +65,327 @@ __device__ inline float apply_act(float v, int act, float limit) {
   return v;
 }
 
-// LK / RK: the operand is contiguous along depth (true) or along its outer index (false);
-// it only selects which thread reads which element so that global loads coalesce.
-template <bool LK, bool RK>
-__global__ __launch_bounds__(256) void f32_gemm_kernel(F32GemmParams p) {
-  __shared__ float sA[2][TK][LDT];
-  __shared__ float sB[2][TK][LDT];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
+// ---- the tile kernels: binary32 products out of bf16 matrix instructions --------------------------
+//
+// v_mfma_f32_32x32x2_f32 multiplies 64 binary32 pairs per cycle and SIMD, v_mfma_f32_32x32x16_bf16
+// sixteen times as many bf16 pairs into the same binary32 accumulators.  A binary32 number is the
+// sum of three bf16 numbers, EXACTLY: hi = bf16(x) (to nearest), mid = bf16(x - hi),
+// lo = x - hi - mid; x - hi has at most 16 significant bits, what mid leaves of it at most 7.  Of the
+// nine products of two such sums the kernels form the six largest and leave out mid lo, lo mid and
+// lo lo: with |mid| <= 2^-8 |x| and |lo| <= 2^-17 |x| (to nearest, so of either sign) that is at most
+// 2^-24 |a b| and half a unit in the last place of the product, less than the rounding a binary32
+// multiply-add makes anyway.  The six go into one binary32 accumulator, sixteen depths per
+// instruction, so the running sum is rounded less often than with two depths per instruction: the
+// 2-norm error against binary64 measures 1.9e-7 where the binary32 instruction's was 4.1e-7 (4 x
+// 1024^3, normal operands; a 512-channel convolution, four wavefronts: 2.4e-7 and 2.9e-7).  In time, 4 x
+// 1024^3 against transposed weights 86.0 -> 51.3 us, MobileNet's five pointwise layers at batch 64
+// 688 -> 318 us; the matrix cores are busy 35 - 45 % of it, the rest is each k tile's chain of LDS
+// reads, MFMAs, LDS writes and barrier (one to three workgroups per CU overlap).
+//
+// Where that does not hold, the workgroup computes its tile again with the binary32 instruction
+// (f32_tile_again): an operand so small (below 2^-110) that lo has no exact bf16 form, which the
+// split sees in the bits lo would lose, or so large (from 2^127 (2 - 2^-8) on, infinite, not a
+// number) that hi is not finite, which leaves a result that is not finite.
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+typedef __bf16 b8v __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ uint32_t bf16_pair(float x, float y) {   // to nearest even; x in the low half
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t d;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(d) : "v"(x), "v"(y));
+  return d;
+#else
+  return 0;
+#endif
+}
+__device__ __forceinline__ float bf16_low(uint32_t pair) { return __uint_as_float(pair << 16); }
+__device__ __forceinline__ float bf16_high(uint32_t pair) { return __uint_as_float(pair & 0xffff0000u); }
+
+// Eight consecutive depths of one row (or column) as three 16-byte pieces: an MFMA fragment each.
+// Bits that `lo` cannot hold are left in the low half of `lost`.
+__device__ __forceinline__ void split_8(const float (&x)[8], u4v (&part)[3], uint32_t &lost) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float x0 = x[2 * e], x1 = x[2 * e + 1];
+    const uint32_t hi = bf16_pair(x0, x1);
+    const float r0 = x0 - bf16_low(hi), r1 = x1 - bf16_high(hi);
+    const uint32_t mid = bf16_pair(r0, r1);
+    const float s0 = r0 - bf16_low(mid), s1 = r1 - bf16_high(mid);
+    part[0][e] = hi;
+    part[1][e] = mid;
+    part[2][e] = bf16_pair(s0, s1);
+    lost |= __float_as_uint(s0) | __float_as_uint(s1);
+  }
+}
+
+// One wavefront's FM x FN blocks of 32 x 32 by the binary32 instruction, operands straight from memory.
+template <int FM, int FN>
+__device__ __forceinline__ void f32_tile_again(const F32GemmParams &p, const float *A, const float *B, int m0,
+                                               const int64_t (&cols)[FN], int k0, int kend,
+                                               v16f (&acc)[FM * FN]) {
+  const int lane = threadIdx.x & 63;
+  const float *a[FM], *b[FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i) a[i] = A + (int64_t)min(m0 + i * 32 + (lane & 31), p.M - 1) * p.lrs;
+#pragma unroll
+  for (int j = 0; j < FN; ++j) b[j] = B + cols[j];
+#pragma unroll
+  for (int t = 0; t < FM * FN; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+  for (int k = k0; k < kend; k += 2) {
+    const int kk = k + (lane >> 5);
+    float av[FM], bv[FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) av[i] = kk < kend ? a[i][(int64_t)kk * p.lcs] : 0.f;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) bv[j] = kk < kend ? b[j][(int64_t)kk * p.rrs] : 0.f;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+        acc[i * FN + j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i * FN + j], 0, 0, 0);
+  }
+}
+
+// A TMT x 128 tile of the result per workgroup.  LK / RK: the operand is contiguous along depth (true)
+// or along its outer index (false).  SPLIT = 1: four wavefronts of 64 x 64 (TMT = 64: of 64 x 32), k
+// tiles of 16, up to three workgroups per CU; SPLIT = 2: eight wavefronts of 64 x 32, k tiles of 32,
+// for launches of at most one tile per CU, where one wavefront per SIMD would leave every LDS wait
+// exposed.
+// GUARD: depths that are not whole k tiles of 16, or an operand that is contiguous along depth in
+// rows that are not aligned 16-byte pieces: single loads, each checked against the depth.
+//
+// A thread's unit is eight consecutive depths of one row: two 16-byte loads where depth is
+// contiguous, else eight 4-byte loads, each coalesced over the wavefront's 64 rows (so rows of any
+// length and alignment).  It splits them (about 6 vector instructions per element, once per tile that
+// reads the element) and stores three 16-byte pieces, [part][8-depth piece][row] in LDS: lanes write
+// and read consecutive 16-byte pieces.  Two LDS stages and two register sets: k tile t + 3 is
+// requested, and k tile t + 1 split and stored, while k tile t is multiplied (a load has two k tiles
+// of time to arrive), the split's instructions dealt out between the MFMAs.
+template <bool LK, bool RK, int SPLIT, bool GUARD, int TMT>
+__device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
+  constexpr int NT = 256 * SPLIT;
+  constexpr int BKT = 16 * SPLIT;          // depths per k tile
+  constexpr int KC = BKT / 8;              // 8-depth pieces per row
+  constexpr int WM = TMT / 64, WN = NT / 64 / WM;   // wavefronts along m and n
+  constexpr int FM = 2, FN = TN / 32 / WN;
+  static_assert(TN * KC == NT && TMT * KC <= NT, "at most one unit of either operand per thread");
+  // (PAD: where depth is contiguous 16 lanes write 16 / KC rows of all KC pieces, which a pitch of a
+  // whole 256 bytes would put into the same banks: 27 % of the cycles of 4 x 1024^3)
+  constexpr int PAD = 16 / KC, PA_ = TMT + PAD, PB_ = TN + PAD;
+  __shared__ __align__(16) u4v sA[2][3][KC][PA_];
+  __shared__ __align__(16) u4v sB[2][3][KC][PB_];
+  __shared__ __align__(16) float s_bias[TMT];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, wn = wave / WM;
   int bid, b;
   span_of_block(&bid, &b);
-  const int m0 = (bid % p.tiles_m) * TM, n0 = (bid / p.tiles_m) * TN;
+  const int m0 = (bid % p.tiles_m) * TMT, n0 = (bid / p.tiles_m) * TN;
   const float *A = p.lhs + (int64_t)b * p.lbs;
   const float *B = p.rhs + (int64_t)b * p.rbs;
 
-  constexpr int PER = TM * TK / 256;   // elements per thread per operand tile
-  float ra[PER], rb[PER];
-  int am[PER], ak[PER], bn[PER], bk[PER];
+  // Element offset of column n of an operand or of the result: columns of all batches side by side
+  // where the launch is flat (p.flat: columns per batch).
+  auto col_at = [&](int n, int64_t step, int64_t batch_step) -> int64_t {
+    if (!p.flat) return (int64_t)n * step;
+    const int img = n / p.flat;
+    return img * batch_step + (int64_t)(n - img * p.flat) * step;
+  };
+  // this thread's unit of either operand (rows past the end repeat the last one; not stored)
+  const bool has_a = TMT * KC == NT || tid < TMT * KC;
+  const int am = LK ? tid / KC : tid % TMT, ac = LK ? tid % KC : tid / TMT;
+  const int bn = RK ? tid / KC : tid % TN, bc = RK ? tid % KC : tid / TN;
+  const float *pa = A + (int64_t)min(m0 + am, p.M - 1) * p.lrs;
+  const float *pb = B + col_at(min(n0 + bn, p.N - 1), p.rcs, p.rbs);
+  u4v *const da = &sA[0][0][has_a ? ac : 0][has_a ? am : 0], *const db = &sB[0][0][bc][bn];
+
+  const int kt0 = p.kt_split * (int)blockIdx.y * TK;
+  const int kend = p.kt_split ? min(kt0 + p.kt_split * TK, p.K) : p.K;
+  const int nk = (kend - kt0 + BKT - 1) / BKT;
+  // No load sits under a condition (the waits in front of their use then leave younger requests in
+  // flight): units past the depth re-read its last eight, single elements past it the last one.
+  auto load_unit = [&](auto contig, const float *at, int64_t step, int kk, float (&x)[8]) __attribute__((always_inline)) {
+    if constexpr (GUARD) {
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int e = tid + i * 256;
-    if (LK) { ak[i] = e % TK; am[i] = e / TK; } else { am[i] = e % TM; ak[i] = e / TM; }
-    if (RK) { bk[i] = e % TK; bn[i] = e / TK; } else { bn[i] = e % TN; bk[i] = e / TN; }
-  }
-  auto load_global = [&](int k0) {
+      for (int e = 0; e < 8; ++e) x[e] = at[(int64_t)min(kk + e, kend - 1) * step];
+    } else {
+      kk = min(kk, kend - 8);
+      if constexpr (decltype(contig)::value) {
+        const f4v v0 = *(const f4v *)(at + kk), v1 = *(const f4v *)(at + kk + 4);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int m = m0 + am[i], k = k0 + ak[i];
-      ra[i] = (m < p.M && k < p.K) ? A[(int64_t)m * p.lrs + (int64_t)k * p.lcs] : 0.f;
-      const int n = n0 + bn[i], k2 = k0 + bk[i];
-      rb[i] = (n < p.N && k2 < p.K) ? B[(int64_t)k2 * p.rrs + (int64_t)n * p.rcs] : 0.f;
+        for (int e = 0; e < 4; ++e) { x[e] = v0[e]; x[4 + e] = v1[e]; }
+      } else {
+        const float *q = at + (int64_t)kk * step;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { x[e] = *q; q += step; }
+      }
     }
   };
-  auto store_lds = [&](int buf) {
+  float xa[2][8], xb[2][8];
+  auto load_tile = [&](auto set, int kt) __attribute__((always_inline)) {
+    constexpr int S = decltype(set)::value;
+    load_unit(std::integral_constant<bool, LK>{}, pa, p.lcs, kt0 + kt * BKT + ac * 8, xa[S]);
+    load_unit(std::integral_constant<bool, RK>{}, pb, p.rrs, kt0 + kt * BKT + bc * 8, xb[S]);
+  };
+  uint32_t lost = 0;
+  auto store_tile = [&](auto set, int kt, int buf) __attribute__((always_inline)) {
+    constexpr int S = decltype(set)::value;
+    if constexpr (GUARD) {   // what lies past the depth counts as zero
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      sA[buf][ak[i]][am[i]] = ra[i];
-      sB[buf][bk[i]][bn[i]] = rb[i];
+      for (int e = 0; e < 8; ++e) {
+        if (kt0 + kt * BKT + ac * 8 + e >= kend) xa[S][e] = 0.f;
+        if (kt0 + kt * BKT + bc * 8 + e >= kend) xb[S][e] = 0.f;
+      }
+    }
+    u4v part[3];
+    split_8(xa[S], part, lost);
+    if (has_a) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) da[(buf * 3 + q) * KC * PA_] = part[q];
+    }
+    split_8(xb[S], part, lost);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) db[(buf * 3 + q) * KC * PB_] = part[q];
+  };
+
+  // the running sum of hi hi; with eight wavefronts, whose registers allow it, the five smaller
+  // products have one of their own, so that they do not each round the large one
+  constexpr int NACC = SPLIT == 2 ? 2 : 1;
+  v16f acc[NACC][FM * FN];
+#pragma unroll
+  for (int s = 0; s < NACC; ++s)
+#pragma unroll
+    for (int t = 0; t < FM * FN; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[s][t][r] = 0.f;
+  auto multiply = [&](auto steps, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < decltype(steps)::value; ++ks) {
+      const int kc = 2 * ks + (lane >> 5);
+      b8v a[FM][3], bb[FN][3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i) a[i][q] = __builtin_bit_cast(b8v, sA[buf][q][kc][wm * 64 + i * 32 + (lane & 31)]);
+#pragma unroll
+        for (int j = 0; j < FN; ++j) bb[j][q] = __builtin_bit_cast(b8v, sB[buf][q][kc][(wn * FN + j) * 32 + (lane & 31)]);
+      }
+      // smallest products first
+      constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+      for (int t = 0; t < 6; ++t)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            v16f &c = acc[t < 5 ? NACC - 1 : 0][i * FN + j];
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][PA[t]], bb[j][PB[t]], c, 0, 0, 0);
+          }
     }
   };
 
-  v16f acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  // (k split: this workgroup's k tiles are [kt0, nk), see F32GemmParams)
-  const int kt0 = p.kt_split * (int)blockIdx.y;
-  const int nk_all = (p.K + TK - 1) / TK;
-  const int nk = p.kt_split ? min(kt0 + p.kt_split, nk_all) : nk_all;
-  load_global(kt0 * TK);
-  store_lds(0);
+  constexpr std::integral_constant<int, 0> set0{};
+  constexpr std::integral_constant<int, 1> set1{};
+  const float bias_m = p.bias_row ? p.bias_row[min(m0 + tid % TMT, p.M - 1)] : 0.f;
+  load_tile(set0, 0);
+  load_tile(set1, 1);
+  if (tid < TMT) s_bias[tid] = bias_m;
+  store_tile(set0, 0, 0);
+  load_tile(set0, 2);
   __syncthreads();
-  for (int kt = kt0; kt < nk; ++kt) {
-    const int buf = (kt - kt0) & 1;
-    if (kt + 1 < nk) load_global((kt + 1) * TK);
-    // v_mfma_f32_32x32x2: lane l supplies A[row l % 32][k = l / 32], B[k = l / 32][col l % 32].
-    // The fragments of step ks + 1 are read while the MFMAs of step ks run (one wavefront per
-    // SIMD has nobody else to hide the LDS latency behind).
-    float a[2][2], bb[2][2];
-    auto read_frags = [&](int ks, int slot) {
-      const int kk = ks * 2 + (lane >> 5);
+  // k tile t: its fragments read, the MFMAs with the split of tile t + 1 between them, then the request
+  // for tile t + 3 into the registers that the split has freed
+  auto step = [&](auto set, int kt) __attribute__((always_inline)) {
+    constexpr int S = decltype(set)::value;   // tile kt + 1's registers
+    multiply(std::integral_constant<int, BKT / 16>{}, S ^ 1);
+    store_tile(set, kt + 1, S);
+    constexpr int MFMAS = BKT / 16 * 6 * FM * FN;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) a[slot][i] = sA[buf][kk][wm * 64 + i * 32 + (lane & 31)];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) bb[slot][j] = sB[buf][kk][wn * 64 + j * 32 + (lane & 31)];
-    };
-    read_frags(0, 0);
-#pragma unroll
-    for (int ks = 0; ks < TK / 2; ++ks) {
-      if (ks + 1 < TK / 2) read_frags(ks + 1, (ks + 1) & 1);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[ks & 1][i], bb[ks & 1][j], acc[i][j],
-                                                           0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < MFMAS; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // an MFMA
+      __builtin_amdgcn_sched_group_barrier(0x002, 120 / MFMAS, 0);   // vector instructions
     }
-    if (kt + 1 < nk) store_lds(buf ^ 1);
+    load_tile(set, kt + 3);
     __syncthreads();
+  };
+  // (eight wavefronts: half a k tile at the end of a depth that has one; a guarded one is filled up
+  // with zeros instead)
+  const int nfull = GUARD ? nk : (kend - kt0) / BKT;
+  for (int kt = 0; kt + 1 < nfull; kt += 2) {
+    step(set1, kt);
+    step(set0, kt + 1);
+  }
+  if (nfull & 1) step(set1, nfull - 1);
+  if (BKT == 32 && nfull < nk) multiply(std::integral_constant<int, 1>{}, nfull & 1);
+
+  if constexpr (NACC == 2) {
+#pragma unroll
+    for (int t = 0; t < FM * FN; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][t][r] = acc[0][t][r] + acc[1][t][r];
+  }
+  // anything the split could not represent: this tile once more, see above
+  float worst = 0.f;   // not finite if one of the sums is not
+#pragma unroll
+  for (int t = 0; t < FM * FN; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) worst = __fmaf_rn(acc[0][t][r], 0.f, worst);
+  if (__syncthreads_or((lost & 0xffffu) != 0 || worst != 0.f)) {
+    int64_t cols[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+      cols[j] = col_at(min(n0 + (wn * FN + j) * 32 + (lane & 31), p.N - 1), p.rcs, p.rbs);
+    f32_tile_again<FM, FN>(p, A, B, m0 + wm * 64, cols, kt0, kend, acc[0]);
   }
 
   const bool raw = p.kt_split != 0;   // a part of the k range: bias and activation come with the sum of the parts
-  float *O = raw ? p.part + ((int64_t)blockIdx.y * gridDim.z + b) * p.obs : p.out + (int64_t)b * p.obs;
+  float *O = (raw ? p.part + (int64_t)blockIdx.y * p.part_stride : p.out) + (int64_t)b * p.obs;
+  const bool whole = m0 + TMT <= p.M && n0 + TN <= p.N;
+  // (one copy per activation, none of its tests per element)
+  auto store = [&](auto act_tag) __attribute__((always_inline)) {
+    constexpr int ACT = decltype(act_tag)::value;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < FN; ++j) {
+      const int n = n0 + (wn * FN + j) * 32 + (lane & 31);
+      const float bias_n = !raw && p.bias_col ? p.bias_col[min(n, p.N - 1)] : 0.f;
+      float *oc = O + col_at(min(n, p.N - 1), p.ocs, p.obs);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + wn * 64 + j * 32 + (lane & 31);
+      for (int i = 0; i < FM; ++i) {
+        const int ml = wm * 64 + i * 32 + 4 * (lane >> 5);
+        float *orow = oc + (int64_t)(m0 + ml) * p.ors;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (m < p.M && n < p.N) {
-          float v = acc[i][j][r];
-          if (!raw) {
-            if (p.bias_row) v = v + p.bias_row[m];
-            if (p.bias_col) v = v + p.bias_col[n];
-            v = apply_act(v, p.act, p.limit);
+        for (int q = 0; q < 4; ++q) {
+          const f4v bias = *(const f4v *)&s_bias[ml + 8 * q];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float v = acc[0][i * FN + j][4 * q + e];
+            if (!raw) {
+              if (p.bias_row) v = v + bias[e];
+              if (p.bias_col) v = v + bias_n;
+            }
+            v = apply_act(v, ACT, p.limit);
+            if (whole || (m0 + ml + 8 * q + e < p.M && n < p.N)) *orow = v;
+            orow += p.ors;
           }
-          O[(int64_t)m * p.ors + (int64_t)n * p.ocs] = v;
+          orow += 4 * p.ors;
         }
       }
     }
+  };
+  if (!raw && p.act == MACE_HIP_ACT_RELU) store(std::integral_constant<int, MACE_HIP_ACT_RELU>{});
+  else if (!raw && p.act == MACE_HIP_ACT_RELUX) store(std::integral_constant<int, MACE_HIP_ACT_RELUX>{});
+  else store(std::integral_constant<int, MACE_HIP_ACT_NOOP>{});
+}
+
+template <bool LK, bool RK, int SPLIT, int TMT>
+__global__ __launch_bounds__(256 * SPLIT, SPLIT == 1 ? 3 : 1) void f32_gemm_vec_kernel(F32GemmParams p) {
+  f32_tile<LK, RK, SPLIT, false, TMT>(p);
+}
+template <bool LK, bool RK, int SPLIT, int TMT, bool GUARD>
+__global__ __launch_bounds__(256 * SPLIT, SPLIT == 2 ? 1 : (GUARD && TMT == 128 ? 2 : 3)) void f32_gemm_kernel(F32GemmParams p) {
+  f32_tile<LK, RK, SPLIT, GUARD, TMT>(p);
 }
 
 // depth == 0: the reference's loop leaves sum = 0
@@ -184,207 +401,6 @@ __global__ void f32_fill_kernel(F32GemmParams p, int64_t total) {
     if (p.bias_col) v = v + p.bias_col[n];
     p.out[bb * p.obs + (int64_t)m * p.ors + (int64_t)n * p.ocs] = apply_act(v, p.act, p.limit);
   }
-}
-
-// The same tile for matrices whose sizes are multiples of the tile (M, N % 128 == 0, K % 16 == 0)
-// and whose rows are 16-byte aligned: no bounds checks, 16-byte global loads through pointers
-// advanced once per k tile (the general kernel spends about 85 vector instructions per k tile on
-// guarded 4-byte loads and their addresses, in front of 32 MFMAs).
-typedef float f4v __attribute__((ext_vector_type(4)));
-
-//
-// SPLIT = 2: eight wavefronts per tile instead of four.  Wavefronts 4..7 cover the same four
-// 64 x 64 quarters as 0..3 but take the second half of every k tile's k steps; their sums are
-// added to the first half's through LDS at the end (a fixed order).  Used when the launch has
-// no more tiles than CUs: one wavefront per SIMD leaves every LDS wait and barrier exposed
-// (matrix core busy 69 % of the time on 4 x 1024^3), two hide each other's.
-template <bool LK, bool RK, int SPLIT>
-__global__ __launch_bounds__(256 * SPLIT) void f32_gemm_vec_kernel(F32GemmParams p) {
-  constexpr int NT = 256 * SPLIT;
-  __shared__ __align__(16) float sA[3][TK][LDT];
-  __shared__ __align__(16) float sB[3][TK][LDT];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int khalf = wave >> 2;           // which part of the k steps (0 when SPLIT == 1)
-  const int wm = wave & 1, wn = (wave >> 1) & 1;
-  int bid, b;
-  span_of_block(&bid, &b);
-  const int m0 = (bid % p.tiles_m) * TM, n0 = (bid / p.tiles_m) * TN;
-  const float *A = p.lhs + (int64_t)b * p.lbs;
-  const float *B = p.rhs + (int64_t)b * p.rbs;
-
-  // NP 16-byte pieces per operand per thread and k tile; KQ pieces along k per row
-  constexpr int NP = TM * TK / 4 / NT, KQ = TK / 4;
-  const float *pa[NP], *pb[NP];
-  int sa_off[NP], sb_off[NP];   // float offset of the piece inside one LDS buffer
-#pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const int f = tid + i * NT;
-    // Rows / columns past the end of a ragged last tile re-read the last valid ones (the host
-    // checks that those come in whole pieces of four); their results are not stored.
-    if (LK) {   // 4 consecutive k of row m
-      const int m = f / KQ, k4 = f % KQ;
-      pa[i] = A + (int64_t)min(m0 + m, p.M - 1) * p.lrs + 4 * k4;
-      sa_off[i] = (4 * k4) * LDT + m;
-    } else {    // 4 consecutive m of depth k
-      const int k = f >> 5, m4 = f & 31;
-      pa[i] = A + (int64_t)k * p.lcs + min(m0 + 4 * m4, p.M - 4);
-      sa_off[i] = k * LDT + 4 * m4;
-    }
-    if (RK) {
-      const int n = f / KQ, k4 = f % KQ;
-      pb[i] = B + (int64_t)min(n0 + n, p.N - 1) * p.rcs + 4 * k4;
-      sb_off[i] = (4 * k4) * LDT + n;
-    } else {
-      const int k = f >> 5, n4 = f & 31;
-      pb[i] = B + (int64_t)k * p.rrs + min(n0 + 4 * n4, p.N - 4);
-      sb_off[i] = k * LDT + 4 * n4;
-    }
-  }
-  const int64_t a_step = LK ? TK : (int64_t)TK * p.lcs;
-  const int64_t b_step = RK ? TK : (int64_t)TK * p.rrs;
-  const int kt0 = p.kt_split * (int)blockIdx.y;   // this workgroup's first k tile
-  if (p.kt_split) {
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      pa[i] += kt0 * a_step;
-      pb[i] += kt0 * b_step;
-    }
-  }
-  f4v ra[NP], rb[NP];
-  auto load_global = [&]() {
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      ra[i] = *(const f4v *)pa[i];
-      rb[i] = *(const f4v *)pb[i];
-      pa[i] += a_step;
-      pb[i] += b_step;
-    }
-  };
-  auto store_lds = [&](int buf) {
-    float *a = &sA[buf][0][0], *bq = &sB[buf][0][0];
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      if (LK) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) a[sa_off[i] + e * LDT] = ra[i][e];
-      } else {
-        *(f4v *)(a + sa_off[i]) = ra[i];
-      }
-      if (RK) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bq[sb_off[i] + e * LDT] = rb[i][e];
-      } else {
-        *(f4v *)(bq + sb_off[i]) = rb[i];
-      }
-    }
-  };
-
-  v16f acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  // Three LDS buffers.  While tile kt is multiplied, tile kt + 1 is already in LDS (stored during
-  // tile kt - 1, visible since the barrier that ended it), tile kt + 2 sits in registers (requested
-  // a whole iteration earlier) and goes to LDS in the middle of the MFMA sequence, where the
-  // request for tile kt + 3 goes out too.  The first fragments of tile kt + 1 can therefore be
-  // read during the last k step of tile kt, in front of the barrier, and no LDS latency is
-  // exposed behind it.  The buffer written (tile kt + 2's = tile kt - 1's) is free: everybody
-  // passed the barrier that ended tile kt - 1.
-  const int nk = p.kt_split ? min(p.kt_split, p.K / TK - kt0) : p.K / TK;
-  load_global();
-  store_lds(0);
-  if (nk > 1) {
-    load_global();
-    store_lds(1);
-  }
-  if (nk > 2) load_global();
-  __syncthreads();
-  constexpr int KS = TK / 2 / SPLIT;   // k steps of this wavefront per k tile
-  const int ks0 = khalf * KS;
-  float a[2][2], bb[2][2];
-  auto read_frags = [&](int buf, int ks, int slot) {
-    const int kk = ks * 2 + (lane >> 5);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) a[slot][i] = sA[buf][kk][wm * 64 + i * 32 + (lane & 31)];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) bb[slot][j] = sB[buf][kk][wn * 64 + j * 32 + (lane & 31)];
-  };
-  static_assert(KS % 2 == 0, "fragment slots alternate; a tile must end on slot 1");
-  read_frags(0, ks0, 0);
-  int buf = 0;
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf1 = buf == 2 ? 0 : buf + 1;    // tile kt + 1
-    const int buf2 = buf1 == 2 ? 0 : buf1 + 1;  // tile kt + 2 (= where tile kt - 1 was)
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      if (ks + 1 < KS) read_frags(buf, ks0 + ks + 1, (ks + 1) & 1);
-      else read_frags(buf1, ks0, 0);   // past the last tile: stale data, never used
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[ks & 1][i], bb[ks & 1][j], acc[i][j],
-                                                           0, 0, 0);
-      if (ks == KS / 2 - 1 && kt + 2 < nk) {
-        store_lds(buf2);
-        if (kt + 3 < nk) load_global();
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    __syncthreads();
-    buf = buf1;
-  }
-
-  if constexpr (SPLIT == 2) {
-    // second half's sums -> first half, one accumulator block (16 values per lane) at a time
-    // through the A buffers (every wavefront is past the last barrier of the loop)
-    float *ex = &sA[0][0][0];
-    static_assert(sizeof(sA) >= 4 * 64 * 16 * sizeof(float), "exchange area");
-    __syncthreads();   // the fragment reads in front of the last barrier are done with
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        if (khalf == 1) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) ex[((wave & 3) * 16 + r) * 64 + lane] = acc[i][j][r];
-        }
-        __syncthreads();
-        if (khalf == 0) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] += ex[((wave & 3) * 16 + r) * 64 + lane];
-        }
-        __syncthreads();
-      }
-    if (khalf == 1) return;
-  }
-
-  const bool raw = p.kt_split != 0;   // a part of the k range: bias and activation come with the sum of the parts
-  float *O = raw ? p.part + ((int64_t)blockIdx.y * gridDim.z + b) * p.obs : p.out + (int64_t)b * p.obs;
-  const bool whole = m0 + TM <= p.M && n0 + TN <= p.N;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + wn * 64 + j * 32 + (lane & 31);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (whole || (m < p.M && n < p.N)) {
-          float v = acc[i][j][r];
-          if (!raw) {
-            if (p.bias_row) v = v + p.bias_row[m];
-            if (p.bias_col) v = v + p.bias_col[n];
-            v = apply_act(v, p.act, p.limit);
-          }
-          O[(int64_t)m * p.ors + (int64_t)n * p.ocs] = v;
-        }
-      }
-    }
 }
 
 // The sum of a k split's parts, in the order of the parts, with the bias and the activation of the
@@ -525,19 +541,32 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
   p.obs = rows * cols;
   p.M = (int)rows; p.N = (int)cols; p.K = (int)depth;
   p.bias_row = ep.bias_row; p.bias_col = ep.bias_col; p.act = ep.act; p.limit = ep.limit;
+  const int64_t total = batch * rows * cols;
   if (depth == 0) {
-    const int64_t total = batch * rows * cols;
     mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_FILL, 0, dim3(1), dim3(256), 0);
     MH_KLAUNCH(ctx, f32_fill_kernel, dim3((unsigned)((total + 255) / 256 > 65535 ? 65535 : (total + 255) / 256)),
                        dim3(256), 0, ctx->stream, p, total);
     MH_LAUNCH_CHECK(ctx);
     return MACE_HIP_SUCCESS;
   }
-  p.tiles_m = (p.M + TM - 1) / TM;
+  // A shared left-hand matrix (a convolution's filter) against a batch: the columns of all batches
+  // are one long row, so that tiles do not end at an image (7 x 7 pixels fill 49 of a tile's 128
+  // columns: 1024 -> 1024 channels at batch 64 190 -> 55 us, the split above included).
+  if (batch > 1 && !lhs_batched && rhs_batched && out_major == MACE_HIP_ROW_MAJOR &&
+      rhs_major == MACE_HIP_ROW_MAJOR && batch * cols < (1ll << 31)) {
+    p.flat = (int)cols;
+    p.N = (int)(batch * cols);
+    batch = 1;
+  }
+  // Rows that leave the last 128-row tile at most half full: tiles of 64 rows (while there is at least
+  // one for every CU; below, the eight-wavefront form with 128 rows).
+  const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  const bool half = (p.M - 1) % TM < TM / 2 && ((p.M + 63) / 64) * ((p.N + TN - 1) / TN) * batch > cus;
+  const int tm = half ? TM / 2 : TM;
+  p.tiles_m = (p.M + tm - 1) / tm;
   const int64_t tiles = (int64_t)p.tiles_m * ((p.N + TN - 1) / TN);
   MH_CHECK(ctx, tiles < (1ll << 31), "too many tiles");
   dim3 grid((unsigned)tiles, 1, (unsigned)batch), block(256), block2(512);
-  const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
   const bool split = tiles * batch <= cus;   // at most one tile per CU
   const bool lk = lhs_major == MACE_HIP_ROW_MAJOR;   // depth contiguous
   const bool rk = rhs_major == MACE_HIP_COL_MAJOR;
@@ -550,9 +579,9 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
   // second launch adds up in a fixed order.  (A tile's time is its k tiles at about 1 us each
   // whatever else runs: 512^3, 16 tiles, took 43.7 us with 240 CUs idle.)
   ArenaScope scope(ctx);
-  const int parts = mh_f32_ksplit(ctx, batch, rows, cols, depth);
+  const int parts = mh_f32_ksplit(ctx, batch, rows, p.N, depth);
   if (parts > 1) {
-    const size_t bytes = mh_f32_ksplit_bytes(ctx, batch, rows, cols, depth);
+    const size_t bytes = sizeof(float) * (size_t)parts * total + 256;
     const bool room = ctx->arena_used + bytes + 16 * 256 <= ctx->arena_bytes;
     // (scratch that does not fit while other slices of the arena are in use: no split)
     if (room || ctx->arena_used == 0) {
@@ -561,29 +590,40 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
       if (!p.part) return mh_fail(ctx, MACE_HIP_RUNTIME_ERROR, "arena slice unavailable");
       const int64_t nk = (depth + TK - 1) / TK;
       p.kt_split = (int)((nk + parts - 1) / parts);
+      p.part_stride = total;
       grid.y = (unsigned)((nk + p.kt_split - 1) / p.kt_split);
       mh_plan_aux(ctx, MACE_HIP_AUX_F32_KSPLIT);
     }
   }
   if (vec) mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_VEC, mhv::f32_gemm_vec(split, lk, rk), grid,
                         split ? block2 : block, 0);
-  else mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_GENERAL, mhv::f32_gemm_general(lk, rk), grid, block, 0);
+  else mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_GENERAL, mhv::f32_gemm_general(lk, rk), grid,
+                    split ? block2 : block, 0);
   MH_PROF_BEGIN(ctx);
-  if (vec && split && lk && rk) MH_KLAUNCH(ctx, (f32_gemm_vec_kernel<true, true, 2>), grid, block2, 0, ctx->stream, p);
-  else if (vec && split && lk) MH_KLAUNCH(ctx, (f32_gemm_vec_kernel<true, false, 2>), grid, block2, 0, ctx->stream, p);
-  else if (vec && split && rk) MH_KLAUNCH(ctx, (f32_gemm_vec_kernel<false, true, 2>), grid, block2, 0, ctx->stream, p);
-  else if (vec && split) MH_KLAUNCH(ctx, (f32_gemm_vec_kernel<false, false, 2>), grid, block2, 0, ctx->stream, p);
-  else if (vec && lk && rk) MH_KLAUNCH(ctx, (f32_gemm_vec_kernel<true, true, 1>), grid, block, 0, ctx->stream, p);
-  else if (vec && lk) MH_KLAUNCH(ctx, (f32_gemm_vec_kernel<true, false, 1>), grid, block, 0, ctx->stream, p);
-  else if (vec && rk) MH_KLAUNCH(ctx, (f32_gemm_vec_kernel<false, true, 1>), grid, block, 0, ctx->stream, p);
-  else if (vec) MH_KLAUNCH(ctx, (f32_gemm_vec_kernel<false, false, 1>), grid, block, 0, ctx->stream, p);
-  else if (lk && rk) MH_KLAUNCH(ctx, (f32_gemm_kernel<true, true>), grid, block, 0, ctx->stream, p);
-  else if (lk) MH_KLAUNCH(ctx, (f32_gemm_kernel<true, false>), grid, block, 0, ctx->stream, p);
-  else if (rk) MH_KLAUNCH(ctx, (f32_gemm_kernel<false, true>), grid, block, 0, ctx->stream, p);
-  else MH_KLAUNCH(ctx, (f32_gemm_kernel<false, false>), grid, block, 0, ctx->stream, p);
+  // depths in whole k tiles, and rows along depth in aligned 16-byte pieces
+  const bool whole = depth % TK == 0 && (!lk || (uintptr_t)lhs % 16 == 0) && (!rk || (uintptr_t)rhs % 16 == 0);
+#define MH_F32(KERNEL, ...) MH_KLAUNCH(ctx, (KERNEL<__VA_ARGS__>), grid, split ? block2 : block, 0, ctx->stream, p)
+#define MH_F32_LR(KERNEL, ...)                                                                  \
+  do {                                                                                          \
+    if (lk && rk) MH_F32(KERNEL, true, true, __VA_ARGS__);                                      \
+    else if (lk) MH_F32(KERNEL, true, false, __VA_ARGS__);                                      \
+    else if (rk) MH_F32(KERNEL, false, true, __VA_ARGS__);                                      \
+    else MH_F32(KERNEL, false, false, __VA_ARGS__);                                             \
+  } while (0)
+  if (vec && split) MH_F32_LR(f32_gemm_vec_kernel, 2, 128);
+  else if (vec && half) MH_F32_LR(f32_gemm_vec_kernel, 1, 64);
+  else if (vec) MH_F32_LR(f32_gemm_vec_kernel, 1, 128);
+  else if (whole && split) MH_F32_LR(f32_gemm_kernel, 2, 128, false);
+  else if (whole && half) MH_F32_LR(f32_gemm_kernel, 1, 64, false);
+  else if (whole) MH_F32_LR(f32_gemm_kernel, 1, 128, false);
+  else if (split) MH_F32_LR(f32_gemm_kernel, 2, 128, true);
+  else if (half) MH_F32_LR(f32_gemm_kernel, 1, 64, true);
+  else MH_F32_LR(f32_gemm_kernel, 1, 128, true);
+#undef MH_F32_LR
+#undef MH_F32
   MH_PROF_END(ctx);
   if (p.kt_split) {
-    const int64_t total = batch * rows * cols;
+    p.N = (int)cols;   // (the parts and the result hold batch after batch, whatever the tiles were)
     const int64_t blocks = (total + 255) / 256;
     MH_KLAUNCH(ctx, f32_ksplit_reduce_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0,
                ctx->stream, p, (int)grid.y, total);

@@ -1,0 +1,87 @@
+"""The fp32 GEMM kernels at the edges of their forms: k tiles of 16 and 32 with half a tile at the end,
+guarded depths, 64- and 128-row tiles, columns of a batch run as one long row, parts of the depth; and
+operands that the split into bf16 parts cannot represent, which a tile is computed again for.
+
+Bound: six MFMAs per 16 depths, each rounding the running sum twice (2^-24 of at most sum |a||b|), eight
+products at a time aligned to the largest of them (8 2^-24), left-out products 2^-24 and the split's
+own last bit: (0.75 K + 16) 2^-24 sum |a||b|, element by element."""
+import numpy as np
+import pytest
+
+from mace_amd import lib as mh
+from gpu_util import Dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = mh.Context(0)
+    yield c
+    c.close()
+
+
+def run(ctx, a, b, lb=True, rb=True, ta=False, tb=False):
+    """a [batch, m, k], b [batch, k, n] -> result and the sums of |a||b|, binary64 on the CPU"""
+    batch = max(a.shape[0], b.shape[0])
+    m, k, n = a.shape[1], a.shape[2], b.shape[2]
+    d = Dev()
+    pa = d.put(a.transpose(0, 2, 1) if ta else a)
+    pb = d.put(b.transpose(0, 2, 1) if tb else b)
+    t, po = d.empty(batch * m * n, np.float32)
+    d.sync()
+    ctx.call("mace_hip_matmul_f32", pa, pb, None, batch, *((k, m) if ta else (m, k)), *((n, k) if tb else (k, n)),
+             int(ta), int(tb), int(lb), int(rb), po)
+    ctx.sync()
+    with np.errstate(all="ignore"):
+        want = np.matmul(a.astype(np.float64), b.astype(np.float64))
+        size = np.matmul(np.abs(a).astype(np.float64), np.abs(b).astype(np.float64))
+    return t.cpu().numpy().reshape(batch, m, n), want, size
+
+
+def close(got, want, size, k):
+    assert np.all(np.abs(got - want) <= (0.75 * k + 16) * 2.0 ** -24 * size)
+
+
+@pytest.mark.parametrize("m,k,n", [(128, 16, 128), (64, 48, 129), (130, 80, 49), (65, 33, 127), (1, 7, 1), (200, 100, 260)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+def test_tile_edges(ctx, m, k, n, ta, tb):
+    rng = np.random.default_rng(m + k + n)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((1, m, k), (1, k, n)))
+    close(*run(ctx, a, b, False, False, ta, tb), k)
+
+
+@pytest.mark.parametrize("batch,m,k,n", [(3, 70, 64, 49), (200, 48, 32, 196), (5, 128, 96, 1), (90, 160, 40, 400)])
+def test_shared_left_matrix_over_a_batch(ctx, batch, m, k, n):
+    rng = np.random.default_rng(batch)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((1, m, k), (batch, k, n)))
+    close(*run(ctx, a, b, lb=False), k)
+
+
+def test_few_tiles_and_a_long_depth(ctx):
+    rng = np.random.default_rng(9)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((1, 100, 2064), (4, 2064, 30)))
+    close(*run(ctx, a, b, lb=False), 2064)
+
+
+@pytest.mark.parametrize("m,k,n", [(140, 64, 133), (40, 50, 300)])
+def test_operands_outside_the_split(ctx, m, k, n):
+    rng = np.random.default_rng(k)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((1, m, k), (1, k, n)))
+    close(*run(ctx, a * np.float32(2.0 ** -120), b * np.float32(2.0 ** 120), False, False), k)   # lo below bf16's smallest
+    tiny = a.copy()
+    tiny[0, 3] *= np.float32(2.0 ** -140)                  # a row of subnormal numbers
+    close(*run(ctx, tiny, b * np.float32(2.0 ** 90), False, False), k)
+    huge = a.copy()
+    huge[0, 5] = 0
+    huge[0, 5, 1] = np.finfo(np.float32).max               # hi would round to infinity
+    close(*run(ctx, huge, np.clip(b, -0.9, 0.9), False, False), k)
+    inf = a.copy()
+    inf[0, 7, 2] = np.inf
+    inf[0, 8, 0] = np.nan
+    bb = b.copy()
+    bb[0, 2] = 1.0                                         # exact in bf16: its smaller parts are zeros
+    got, want, _ = run(ctx, inf, bb, False, False)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    got, want, size = run(ctx, np.zeros_like(a), b, False, False)
+    assert not got.any()
