@@ -349,7 +349,8 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
       const int n = n0 + (wn * FN + j) * 32 + (lane & 31);
-      const float bias_n = !raw && p.bias_col ? p.bias_col[min(n, p.N - 1)] : 0.f;
+      const int col = min(n, p.N - 1);   // (of the long row of all batches, whose bias repeats)
+      const float bias_n = !raw && p.bias_col ? p.bias_col[p.flat ? col % p.flat : col] : 0.f;
       float *oc = O + col_at(min(n, p.N - 1), p.ocs, p.obs);
 #pragma unroll
       for (int i = 0; i < FM; ++i) {

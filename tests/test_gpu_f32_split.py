@@ -21,21 +21,24 @@ def ctx():
     c.close()
 
 
-def run(ctx, a, b, lb=True, rb=True, ta=False, tb=False):
-    """a [batch, m, k], b [batch, k, n] -> result and the sums of |a||b|, binary64 on the CPU"""
+def run(ctx, a, b, lb=True, rb=True, ta=False, tb=False, bias=None):
+    """a [batch, m, k], b [batch, k, n], bias [n] -> result and the sums of |a||b|, binary64 on the CPU"""
     batch = max(a.shape[0], b.shape[0])
     m, k, n = a.shape[1], a.shape[2], b.shape[2]
     d = Dev()
     pa = d.put(a.transpose(0, 2, 1) if ta else a)
     pb = d.put(b.transpose(0, 2, 1) if tb else b)
+    pbias = None if bias is None else d.put(bias)
     t, po = d.empty(batch * m * n, np.float32)
     d.sync()
-    ctx.call("mace_hip_matmul_f32", pa, pb, None, batch, *((k, m) if ta else (m, k)), *((n, k) if tb else (k, n)),
+    ctx.call("mace_hip_matmul_f32", pa, pb, pbias, batch, *((k, m) if ta else (m, k)), *((n, k) if tb else (k, n)),
              int(ta), int(tb), int(lb), int(rb), po)
     ctx.sync()
     with np.errstate(all="ignore"):
         want = np.matmul(a.astype(np.float64), b.astype(np.float64))
         size = np.matmul(np.abs(a).astype(np.float64), np.abs(b).astype(np.float64))
+        if bias is not None:
+            want, size = want + bias, size + np.abs(bias)
     return t.cpu().numpy().reshape(batch, m, n), want, size
 
 
@@ -56,6 +59,14 @@ def test_shared_left_matrix_over_a_batch(ctx, batch, m, k, n):
     rng = np.random.default_rng(batch)
     a, b = (rng.standard_normal(s).astype(np.float32) for s in ((1, m, k), (batch, k, n)))
     close(*run(ctx, a, b, lb=False), k)
+
+
+@pytest.mark.parametrize("batch,m,k,n", [(3, 70, 64, 49), (40, 48, 33, 100), (300, 130, 64, 132)])
+def test_shared_left_matrix_with_a_bias_per_column(ctx, batch, m, k, n):
+    """every batch's columns take the same n biases"""
+    rng = np.random.default_rng(n)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((1, m, k), (batch, k, n)))
+    close(*run(ctx, a, b, lb=False, bias=rng.standard_normal(n).astype(np.float32)), k)
 
 
 def test_few_tiles_and_a_long_depth(ctx):
