@@ -1899,102 +1899,50 @@ void q8_gemm_stream_kernel(GemmParams p) {
 
 // ---- repacking ---------------------------------------------------------------------------
 
-// src is k-contiguous already ([n][k], row stride = k) but k is not a multiple of 16 or the
-// base is misaligned: copy into [n][kp] rows padded with 0x80.  One thread per 16 bytes of the
-// padded row: a piece that lies wholly inside the source row is one unaligned 16-byte load (the
-// hardware reads those from global memory at any address), the piece at the row end is put
-// together from single bytes.
-__global__ void q8_pack_rows_kernel(const uint8_t *src, int64_t src_bs, uint8_t *dst,
-                                    int64_t dst_bs, int n, int k, int kp) {
-  const int cpr = kp >> 4;   // 16-byte pieces per padded row
-  const int64_t total = (int64_t)n * cpr;
-  const uint8_t *s = src + (int64_t)blockIdx.z * src_bs;
-  uint8_t *d = dst + (int64_t)blockIdx.z * dst_bs;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = i / cpr;
-    const int c = (int)(i - r * cpr) * 16;   // first byte of the piece inside the row
-    const uint8_t *from = s + r * k + c;
-    const int left = k - c;
-    v4i v;
-    if (left >= 16) {
-      __builtin_memcpy(&v, from, 16);
-    } else {
-      uint32_t w[4] = {0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
-      for (int e = 0; e < left; ++e)
-        w[e >> 2] = (w[e >> 2] & ~(0xffu << (8 * (e & 3)))) | ((uint32_t)from[e] << (8 * (e & 3)));
-      v = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-    }
-    *(v4i *)(d + i * 16) = v;
+// One operand to copy into padded panels [n][kp] (kp a multiple of 64, bytes past k are 0x80): k-contiguous
+// rows ([n][k]; tiles_n = 0) or k-major ([k][n], to be transposed).  Rows may have any length and
+// start at any address.
+struct RepackJob {
+  const uint8_t *src;
+  uint8_t *dst;
+  int64_t rows;           // k-contiguous: rows of all batches, which follow each other on both sides
+  int64_t blocks;         // workgroups
+  int32_t *sums;          // k-major: where the shifted bytes of every output row are added up, or nullptr
+  uint32_t flip;          // k-major: 0x80808080 writes the panel already shifted to int8, 0: as read
+  int n, k, kp;
+  int tiles_n, tiles_k;   // k-major: 128 x 128 tiles of a batch
+};
+
+// Bytes [at, at + 16) of a row of `len` bytes (at < len), 0x80 past its end, in two steps so that several
+// loads can be in flight.  The hardware loads 16 bytes from global memory at any address; the piece
+// that holds the row's end is loaded as the row's last 16 bytes and then moved down, so nothing
+// outside the row is read.
+__device__ inline uint4 repack_load(const uint8_t *row, int at, int len) {
+  uint4 v = {0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+  if (len >= 16) {
+    __builtin_memcpy(&v, row + min(at, len - 16), 16);
+  } else {
+    uint32_t w[4] = {0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+#pragma unroll
+    for (int e = 0; e < 15; ++e)
+      if (at + e < len) w[e >> 2] = (w[e >> 2] & ~(0xffu << (8 * (e & 3)))) | ((uint32_t)row[at + e] << (8 * (e & 3)));
+    v = uint4{w[0], w[1], w[2], w[3]};
   }
+  return v;
+}
+__device__ inline void repack_align(uint4 &v, int at, int len) {
+  const int past = at - (len - 16);   // bytes loaded that precede the piece
+  if (len < 16 || past <= 0) return;
+  uint32_t w[8] = {v.x, v.y, v.z, v.w, 0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+#pragma unroll
+  for (int e = 0; e < 6; ++e) w[e] = (past & 8) ? w[e + 2] : w[e];
+#pragma unroll
+  for (int e = 0; e < 5; ++e) w[e] = (past & 4) ? w[e + 1] : w[e];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w[e] = (uint32_t)((((uint64_t)w[e + 1] << 32) | w[e]) >> (8 * (past & 3)));
+  v = uint4{w[0], w[1], w[2], w[3]};
 }
 
-// The same for k % 4 == 0 and a 4-byte aligned base: one thread per 16 bytes of the padded row,
-// read as four dwords (a 24-channel activation tensor: rows of six dwords become rows of 64 bytes).
-__global__ void q8_pack_rows4_kernel(const uint8_t *src, int64_t src_bs, uint8_t *dst,
-                                     int64_t dst_bs, int n, int k, int kp) {
-  const int cpr = kp >> 4;   // 16-byte pieces per padded row
-  const int64_t total = (int64_t)n * cpr;
-  const uint32_t *s = (const uint32_t *)(src + (int64_t)blockIdx.z * src_bs);
-  uint8_t *d = dst + (int64_t)blockIdx.z * dst_bs;
-  const int k4 = k >> 2;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = i / cpr;
-    const int c4 = (int)(i - r * cpr) * 4;   // first dword of the piece inside the row
-    v4i v;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = c4 + e < k4 ? (int)s[r * k4 + c4 + e] : (int)0x80808080;
-    *(v4i *)(d + i * 16) = v;
-  }
-}
-
-// src is [k][n] with n contiguous (row stride = n): write dst [n][kp], padding k..kp with
-// 0x80.  64x64-byte tiles through LDS; 16-byte global accesses when n % 16 == 0 and the
-// base is aligned, byte accesses otherwise.
-__global__ __launch_bounds__(256) void q8_pack_transpose_kernel(const uint8_t *src,
-                                                                int64_t src_bs, uint8_t *dst,
-                                                                int64_t dst_bs, int n, int k,
-                                                                int kp, int vec_ok) {
-  __shared__ uint8_t tile[64][64 + 4];
-  const uint8_t *s = src + (int64_t)blockIdx.z * src_bs;
-  uint8_t *d = dst + (int64_t)blockIdx.z * dst_bs;
-  const int n0 = blockIdx.x * 64, k0 = blockIdx.y * 64;
-  const int tid = threadIdx.x;
-  {
-    const int kk = tid >> 2, nc = (tid & 3) * 16;   // row kk of the tile, 16 bytes of n
-    const int gk = k0 + kk, gn = n0 + nc;
-    uint8_t v[16];
-    if (gk < k && vec_ok && gn + 15 < n) {
-      *(uint4 *)v = *(const uint4 *)(s + (int64_t)gk * n + gn);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        v[e] = (gk < k && gn + e < n) ? s[(int64_t)gk * n + gn + e] : (uint8_t)0x80;
-    }
-#pragma unroll
-    for (int e = 0; e < 16; ++e) tile[kk][nc + e] = v[e];
-  }
-  __syncthreads();
-  {
-    const int nn = tid >> 2, kc = (tid & 3) * 16;   // output row nn, 16 bytes of k
-    const int gn = n0 + nn, gk = k0 + kc;
-    if (gn < n && gk < kp) {
-      uint8_t v[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) v[e] = tile[kc + e][nn];
-      // kp is a multiple of 64, so the 16-byte store stays inside the padded row
-      *(uint4 *)(d + (int64_t)gn * kp + gk) = *(uint4 *)v;
-    }
-  }
-}
-
-// The same repack for n % 16 == 0 and a 16-byte aligned source: 128 x 128-byte tiles, whole
-// 128-byte lines on both sides.  A thread loads 16 bytes of one k row (four times) and parks
-// them in LDS as dwords of 4 n each, laid out [n / 4][k]; then it picks up 16 consecutive k of
-// one n group (4 n x 16 k), transposes the four 4 x 4 byte blocks in registers (8 v_perm each)
-// and stores 16 bytes of k for each of its 4 n.  Row pitch 130 dwords: the 8 x 8 (n group, k)
-// pattern of a wavefront's LDS stores falls into 64 distinct banks.
 __device__ inline void transpose4x4_bytes(const uint32_t (&d)[4], uint32_t (&o)[4]) {
   const uint32_t t0 = __builtin_amdgcn_perm(d[1], d[0], 0x05010400);   // d0.b0 d1.b0 d0.b1 d1.b1
   const uint32_t t1 = __builtin_amdgcn_perm(d[1], d[0], 0x07030602);   // d0.b2 d1.b2 d0.b3 d1.b3
@@ -2006,38 +1954,67 @@ __device__ inline void transpose4x4_bytes(const uint32_t (&d)[4], uint32_t (&o)[
   o[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302);
 }
 
-// With `sums` (zeroed beforehand, n entries per batch) the kernel also adds up what the panel
-// sums pass would: the shifted bytes of every output row, one atomic per row and tile.
-__global__ __launch_bounds__(256) void q8_pack_transpose128_kernel(const uint8_t *src,
-                                                                   int64_t src_bs, uint8_t *dst,
-                                                                   int64_t dst_bs, int n, int k,
-                                                                   int kp, int32_t *sums,
-                                                                   uint32_t flip) {
-  // flip = 0x80808080: the panel is written already shifted to int8 (for the kernel variant that
-  // then leaves this operand's fragments alone); 0: as read
-  constexpr int PITCH = 130;
-  __shared__ uint32_t tile[32 * PITCH];   // [n / 4][k]
-  const uint8_t *s = src + (int64_t)blockIdx.z * src_bs;
-  uint8_t *d = dst + (int64_t)blockIdx.z * dst_bs;
-  const int n0 = blockIdx.x * 128, k0 = blockIdx.y * 128;
+// Workgroup `id` of a job with k-contiguous rows: REPACK_PIECES consecutive 16-byte pieces of the panel.
+constexpr int REPACK_PIECES = 512;
+__device__ inline void repack_rows(const RepackJob &j, int64_t id) {
+  const uint32_t cpr = (uint32_t)j.kp >> 4;   // pieces per row
+  const int64_t p0 = id * REPACK_PIECES;
+  const int64_t r0 = p0 < ((int64_t)1 << 32) ? (int64_t)((uint32_t)p0 / cpr) : p0 / cpr;
+  const uint32_t first = (uint32_t)(p0 - r0 * cpr) + threadIdx.x;
+  uint4 v[REPACK_PIECES / 256];
+#pragma unroll
+  for (int u = 0; u < REPACK_PIECES / 256; ++u) {
+    const uint32_t o = first + 256 * u, r = o / cpr;
+    const int at = (int)(o - r * cpr) * 16;
+    v[u] = uint4{0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+    if (r0 + r < j.rows && at < j.k) v[u] = repack_load(j.src + (r0 + r) * j.k, at, j.k);
+  }
+#pragma unroll
+  for (int u = 0; u < REPACK_PIECES / 256; ++u) {
+    const uint32_t o = first + 256 * u, r = o / cpr;
+    const int at = (int)(o - r * cpr) * 16;
+    if (at < j.k) repack_align(v[u], at, j.k);
+    if (r0 + r < j.rows) *(uint4 *)(j.dst + (p0 + 256 * u + threadIdx.x) * 16) = v[u];
+  }
+}
+
+// Workgroup `id` of a job that transposes: a 128 x 128-byte tile, whole 128-byte runs on both sides.  A
+// thread loads 16 bytes of one k row (four times) and parks them in LDS as dwords of 4 n each,
+// laid out [n / 4][k]; then it picks up 16 consecutive k of one n group (4 n x 16 k), transposes the
+// four 4 x 4 byte blocks in registers (8 v_perm each) and stores 16 bytes of k for each of its 4 n.
+// Row pitch 130 dwords: the 8 x 8 (n group, k) pattern of a wavefront's LDS stores falls into 64
+// distinct banks.
+constexpr int REPACK_PITCH = 130;
+__device__ inline void repack_transpose(const RepackJob &j, uint32_t id, uint32_t *tile) {
+  const uint32_t nt = (uint32_t)j.tiles_n, kt = (uint32_t)j.tiles_k, q = id / nt;
+  const int n = j.n, n0 = (int)(id - q * nt) * 128, k0 = (int)(q % kt) * 128, batch = (int)(q / kt);
+  const uint8_t *s = j.src + (int64_t)batch * n * j.k;
+  uint8_t *d = j.dst + (int64_t)batch * n * j.kp;
   const int tid = threadIdx.x;
   {
-    const int nc = (tid & 7) * 16;   // 16 bytes of n, rows kk = tid / 8 + 32 j
+    const int nc = (tid & 7) * 16;   // 16 bytes of n, rows kk = tid / 8 + 32 i
     const int gn = n0 + nc;
+    uint4 v[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int kk = (tid >> 3) + 32 * j;
-      const int gk = k0 + kk;
-      uint4 v = {0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
-      if (gk < k && gn < n) v = *(const uint4 *)(s + (int64_t)gk * n + gn);   // n % 16 == 0
-      uint32_t *t = tile + (nc >> 2) * PITCH + kk;
-      t[0] = v.x; t[PITCH] = v.y; t[2 * PITCH] = v.z; t[3 * PITCH] = v.w;
+    for (int i = 0; i < 4; ++i) {
+      const int gk = k0 + (tid >> 3) + 32 * i;
+      v[i] = uint4{0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+      if (gk < j.k && gn < n) v[i] = repack_load(s + (int64_t)gk * n, gn, n);
+    }
+    if (n0 + 128 > n && gn < n) {   // (a row past the depth is 0x80 throughout and moves 0x80 down)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) repack_align(v[i], gn, n);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t *t = tile + (nc >> 2) * REPACK_PITCH + (tid >> 3) + 32 * i;
+      t[0] = v[i].x; t[REPACK_PITCH] = v[i].y; t[2 * REPACK_PITCH] = v[i].z; t[3 * REPACK_PITCH] = v[i].w;
     }
   }
   __syncthreads();
   {
     const int kc = tid & 7, g = tid >> 3;   // 16 k starting at 16 kc, n = 4 g .. 4 g + 3
-    const uint32_t *t = tile + g * PITCH + 16 * kc;
+    const uint32_t *t = tile + g * REPACK_PITCH + 16 * kc;
     uint32_t o[4][4];                       // [k block][n]
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
@@ -2045,33 +2022,47 @@ __global__ __launch_bounds__(256) void q8_pack_transpose128_kernel(const uint8_t
       transpose4x4_bytes(din, o[b]);
     }
     const int gk = k0 + 16 * kc;
-    if (gk < kp) {   // kp is a multiple of 64: a 16-byte piece is inside the row or outside
+    if (gk < j.kp) {   // kp is a multiple of 64: a 16-byte piece is inside the row or outside
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int gn = n0 + 4 * g + j;
+      for (int e = 0; e < 4; ++e) {
+        const int gn = n0 + 4 * g + e;
         if (gn < n)
-          *(uint4 *)(d + (int64_t)gn * kp + gk) =
-              uint4{o[0][j] ^ flip, o[1][j] ^ flip, o[2][j] ^ flip, o[3][j] ^ flip};
+          *(uint4 *)(d + (int64_t)gn * j.kp + gk) =
+              uint4{o[0][e] ^ j.flip, o[1][e] ^ j.flip, o[2][e] ^ j.flip, o[3][e] ^ j.flip};
       }
     }
-    if (sums) {
+    if (j.sums) {
       // bytes beyond k were loaded as 0x80 and count as zero; the 8 threads that share a row
       // group are neighbouring lanes
-      int32_t *sb = sums + (int64_t)blockIdx.z * n;
+      int32_t *sb = j.sums + (int64_t)batch * n;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int e = 0; e < 4; ++e) {
         int v = 0;
 #pragma unroll
         for (int b = 0; b < 4; ++b)
-          v = __builtin_amdgcn_sdot4((int)(o[b][j] ^ 0x80808080u), 0x01010101, v, false);
+          v = __builtin_amdgcn_sdot4((int)(o[b][e] ^ 0x80808080u), 0x01010101, v, false);
         v += __shfl_xor(v, 1, 64);
         v += __shfl_xor(v, 2, 64);
         v += __shfl_xor(v, 4, 64);
-        const int gn = n0 + 4 * g + j;
+        const int gn = n0 + 4 * g + e;
         if (kc == 0 && gn < n) atomicAdd(sb + gn, v);
       }
     }
   }
+}
+
+// Both operands of a call in one launch: a copy is bound by its launch, drain and HBM.
+__global__ __launch_bounds__(256) void q8_repack_kernel(RepackJob a, RepackJob b) {
+  __shared__ uint32_t tile[32 * REPACK_PITCH];   // [n / 4][k]
+  int64_t id = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+  if (id >= a.blocks + b.blocks) return;
+  RepackJob j = a;
+  if (id >= a.blocks) {
+    id -= a.blocks;
+    j = b;
+  }
+  if (j.tiles_n == 0) repack_rows(j, id);   // uniform over the workgroup
+  else repack_transpose(j, (uint32_t)id, tile);
 }
 
 __global__ __launch_bounds__(256) void q8_zero_i32_kernel(int32_t *p, int64_t n) {
@@ -2963,9 +2954,29 @@ int Q8Call::kmajor_in_place(bool *done) {
 }
 
 int Q8Call::general() {
-  size_t need = sizeof(int32_t) * ((size_t)lhs_nb * rows + (size_t)rhs_nb * cols) + 4096 + 512;
-  if (!lhs_direct && !lhs_w) need += (size_t)lhs_nb * rows * kp + 256;
-  if (!rhs_direct && !rhs_w) need += (size_t)rhs_nb * cols * kp + 256;
+  auto need_of = [&](int64_t pitch, bool l_direct, bool r_direct) {
+    return sizeof(int32_t) * ((size_t)lhs_nb * rows + (size_t)rhs_nb * cols) + 4096 + 512 +
+           (!l_direct && !lhs_w ? (size_t)lhs_nb * rows * pitch + 256 : 0) +
+           (!r_direct && !rhs_w ? (size_t)rhs_nb * cols * pitch + 256 : 0);
+  };
+  // Operands that are copied anyway get rows of whole 128-byte slabs where the depth is long: the
+  // eight-wavefront kernel and the 256 x 256 tiles take those and sum the panels themselves.  An operand that
+  // could be read in place is copied as well where its depth is not made of whole 64-byte slabs,
+  // which no ring kernel takes (999 x 1488 x 1001 24.1 -> 21.8 us; 4 x 1001 x 1500 x 777, no sums
+  // launches, 37.7 -> 33.6).  Not below a quarter of a round of 128 x 128 tiles (333 x 4097 x 555: 28.0
+  // against 29.4 us), nor where scratch is limited to what the plain panels need.
+  const bool repack_both = (!lhs_direct && !rhs_direct) ||
+                           (depth % 64 != 0 && lhs_direct != rhs_direct && !(lhs_direct ? lhs_w : rhs_w));
+  const int64_t tiles_128 = ((rows + 127) / 128) * ((cols + 127) / 128) * batch;
+  if (repack_both && !cv && rhs_ld == 0 && depth > 512 && 4 * tiles_128 >= (ctx->cu_count > 0 ? ctx->cu_count : 256)) {
+    const int64_t pitch = (kp + 127) & ~(int64_t)127;
+    const size_t most = ctx->arena_used + need_of(pitch, false, false) + 16 * 256;   // (as mh_arena_reserve counts)
+    if (most <= ctx->arena_bytes || !(ctx->no_alloc || ctx->capturing || ctx->arena_used != 0)) {
+      kp = pitch;
+      lhs_direct = rhs_direct = false;
+    }
+  }
+  const size_t need = need_of(kp, lhs_direct, rhs_direct);
   MH_RETURN_IF_ERROR(mh_arena_reserve(ctx, need));
   ArenaScope scope(ctx);
 
@@ -2977,8 +2988,22 @@ int Q8Call::general() {
     bool flipped = false;   // repacked already shifted to int8 (X operand of the 256 x 256 kernel)
   } L, R;
 
+  // The repacks wait in `jobs` until launch_repacks(): those of both operands go in one launch.
+  RepackJob jobs[2] = {};
+  int njobs = 0;
+  auto launch_repacks = [&]() -> int {
+    if (njobs == 0) return MACE_HIP_SUCCESS;
+    const int64_t blocks = jobs[0].blocks + jobs[1].blocks;
+    const int64_t gx = std::min<int64_t>(blocks, 1 << 22);
+    MH_KLAUNCH(ctx, q8_repack_kernel, dim3((unsigned)gx, (unsigned)((blocks + gx - 1) / gx)), dim3(256), 0,
+                       ctx->stream, jobs[0], jobs[1]);
+    MH_LAUNCH_CHECK(ctx);
+    njobs = 0;
+    jobs[0] = jobs[1] = RepackJob{};
+    return MACE_HIP_SUCCESS;
+  };
   // fused_sums: where the repack may leave the panel's row sums as well (or nullptr); *fused
-  // tells whether it did
+  // tells whether it will
   // sums_cleared: an earlier launch of this call has zeroed fused_sums already
   bool sums_cleared = false;
   auto pack = [&](const uint8_t *src, int order_is_kcontig, int nb, int64_t n, uint8_t *dst,
@@ -2986,46 +3011,36 @@ int Q8Call::general() {
                   bool *flipped = nullptr) -> int {
     if (fused) *fused = false;
     if (flipped) *flipped = false;
+    RepackJob j{};
+    j.src = src;
+    j.dst = dst;
+    j.n = (int)n; j.k = (int)depth; j.kp = (int)kp;
     if (order_is_kcontig) {
       mh_plan_aux(ctx, MACE_HIP_AUX_PACK_ROWS);
-      if (depth % 4 == 0 && (uintptr_t)src % 4 == 0) {
-        const int64_t total = n * (kp / 16);
-        dim3 grid((unsigned)std::min<int64_t>((total + 255) / 256, 1 << 20), 1, nb);
-        MH_KLAUNCH(ctx, q8_pack_rows4_kernel, grid, dim3(256), 0, ctx->stream, src,
-                           n * depth, dst, n * kp, (int)n, (int)depth, (int)kp);
-      } else {
-        const int64_t total = n * (kp / 16);
-        dim3 grid((unsigned)std::min<int64_t>((total + 255) / 256, 1 << 20), 1, nb);
-        MH_KLAUNCH(ctx, q8_pack_rows_kernel, grid, dim3(256), 0, ctx->stream, src,
-                           n * depth, dst, n * kp, (int)n, (int)depth, (int)kp);
-      }
+      j.rows = nb * n;
+      j.blocks = (j.rows * (kp / 16) + REPACK_PIECES - 1) / REPACK_PIECES;
     } else {
       MH_CHECK(ctx, (kp / 64) <= 65535, "depth too large to repack");
-      const int vec_ok = (n % 16 == 0) && ((uintptr_t)src % 16 == 0);
       mh_plan_aux(ctx, MACE_HIP_AUX_PACK_TRANSPOSE);
-      if (vec_ok) {
-        dim3 grid((unsigned)((n + 127) / 128), (unsigned)((kp + 127) / 128), nb);
-        if (fused_sums) {
-          const int64_t cnt = (int64_t)nb * n;
-          if (!sums_cleared) mh_plan_aux(ctx, MACE_HIP_AUX_ZERO);
-          if (!sums_cleared)
-            MH_KLAUNCH(ctx, q8_zero_i32_kernel, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0,
-                               ctx->stream, fused_sums, cnt);
-          *fused = true;
-        }
-        const bool fl = want_flipped && flipped;
-        MH_KLAUNCH(ctx, q8_pack_transpose128_kernel, grid, dim3(256), 0, ctx->stream, src,
-                           n * depth, dst, n * kp, (int)n, (int)depth, (int)kp, fused_sums,
-                           fl ? 0x80808080u : 0u);
-        if (fl) mh_plan_aux(ctx, MACE_HIP_AUX_PACK_SHIFTED);
-        if (fl) *flipped = true;
-      } else {
-        dim3 grid((unsigned)((n + 63) / 64), (unsigned)(kp / 64), nb);
-        MH_KLAUNCH(ctx, q8_pack_transpose_kernel, grid, dim3(256), 0, ctx->stream, src,
-                           n * depth, dst, n * kp, (int)n, (int)depth, (int)kp, 0);
+      j.tiles_n = (int)((n + 127) / 128);
+      j.tiles_k = (int)((kp + 127) / 128);
+      j.blocks = (int64_t)j.tiles_n * j.tiles_k * nb;
+      if (fused_sums) {
+        const int64_t cnt = (int64_t)nb * n;
+        if (!sums_cleared) mh_plan_aux(ctx, MACE_HIP_AUX_ZERO);
+        if (!sums_cleared)
+          MH_KLAUNCH(ctx, q8_zero_i32_kernel, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0,
+                             ctx->stream, fused_sums, cnt);
+        j.sums = fused_sums;
+        *fused = true;
+      }
+      if (want_flipped && flipped) {
+        j.flip = 0x80808080u;
+        mh_plan_aux(ctx, MACE_HIP_AUX_PACK_SHIFTED);
+        *flipped = true;
       }
     }
-    MH_LAUNCH_CHECK(ctx);
+    jobs[njobs++] = j;
     return MACE_HIP_SUCCESS;
   };
 
@@ -3061,8 +3076,9 @@ int Q8Call::general() {
       hipError_t e = dev_alloc((void **)&c.panel, (size_t)nb * n * kp);
       if (e != hipSuccess) { dev_free(c.sums); MH_HIP(ctx, e); }
       // the sums come from the repack where it can take them (always where it shifts the bytes)
-      const int rc = pack(src, order_is_kcontig, nb, n, c.panel, want_flipped ? c.sums : nullptr, &fused,
-                          want_flipped, &c.flipped);
+      int rc = pack(src, order_is_kcontig, nb, n, c.panel, want_flipped ? c.sums : nullptr, &fused,
+                    want_flipped, &c.flipped);
+      if (rc == MACE_HIP_SUCCESS) rc = launch_repacks();
       if (rc != MACE_HIP_SUCCESS) { dev_free(c.panel); dev_free(c.sums); return rc; }
     }
     if (!fused) {
@@ -3108,6 +3124,61 @@ int Q8Call::general() {
   int32_t *corrR = (int32_t *)mh_arena_take(ctx, sizeof(int32_t) * rhs_nb * cols);
   if (!corrL || !corrR) return mh_fail(ctx, MACE_HIP_RUNTIME_ERROR, "arena slice unavailable");
   const bool x_is_lhs = out_order == MACE_HIP_COL_MAJOR;
+  // A small X panel (at most 128 rows of at most 64 bytes: an early 1x1 convolution's filter) against a
+  // long Y panel goes to the streaming kernel, which also sums both panels itself.
+  const int64_t xn = x_is_lhs ? rows : cols, yn = x_is_lhs ? cols : rows;
+  // (Measured: it wins for K <= 64; from K = 128 on the tiled kernels are as fast.)
+  const bool stream = !cv && out_u8 && requant_by_mad(rq) && lhs_direct && rhs_direct && rhs_ld == 0 &&
+                      mh_q8_stream_shape(depth, xn, yn) && ((uintptr_t)out % 16 == 0);
+  const int64_t cu_n = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  // Which of the kernels that sum both panels themselves takes the call, for panels with kk readable
+  // bytes of depth in rows of ldl and ldr bytes.
+  struct Route { bool xres, mid; int tx; };
+  auto route_of = [&](int kk, int64_t ldl, int64_t ldr) -> Route {
+    // An X panel whose tile (64 or 128 rows, all of k) fits in LDS twice per CU goes to the kernel
+    // that keeps it there and sums both panels itself.  Measured against the tiled kernels (k from
+    // 64 to 1024, 64 to 1024 X rows, 4 Ki to 256 Ki Y rows): with the block height chosen as in
+    // launch_gemm_xres_any it wins or ties throughout (where the tile only fits once, k >= 640 at
+    // 128 rows, the tiled kernels win by 10 - 35 % and keep the shape).  A convolution whose
+    // patches the kernel gathers (cin % 64 == 0) takes it whenever the tile fits: 25 % faster
+    // than the gathering tiled kernel on 3x3, 56x56x64 -> 64 at batch 64 (splitting a 128-row tile
+    // that does not fit into two of 64 rows was slower than the tiled kernel).
+    // (Bit MH_MASK_NO_XRES of the kernel mask: test hook that keeps the tiled kernels in use.)
+    const size_t lds_cu = ctx->lds_bytes > 0 ? (size_t)ctx->lds_bytes : 65536;
+    auto xres_fits = [&](int tx) {
+      return 2 * (XRES_SC_BYTES + (size_t)tx * ((kk + 63) & ~63)) <= lds_cu;
+    };
+    // Where 128 rows of a long k do not fit, 64-row tiles (Y is then read once per 64 X rows) still
+    // win between one and two 64 x 64 blocks per CU, where the tiled kernels leave most of the chip
+    // idle (k = 1024, 512 X rows, 3136 Y rows: 16.0 -> 9.4 us); beyond that they lose.
+    const int64_t blocks_tx64 = ((xn + 63) / 64) * ((yn + 63) / 64) * batch;
+    const bool xres_narrow = !cv && !xres_fits(128) && blocks_tx64 > cu_n && blocks_tx64 <= 2 * cu_n;
+    const int xres_tx = (xn <= 64 || xres_narrow) ? 64 : 128;
+    const bool xres_cv = cv && !cv_small && out_u8 && cv->cin % 64 == 0 && depth % 64 == 0;
+    const int64_t tiles128 = ((xn + 127) / 128) * ((yn + 127) / 128) * batch;
+    // (one round of 128 x 128 tiles at k >= 512 is faster on the eight-wavefront kernel, see above;
+    // from k = 2048 on also below a quarter of a round, where the 64 x 64 tiles and their sums pass took
+    // the shape: 6 - 11 % faster with k-contiguous operands at 1 to 63 tiles)
+    const bool mid_shape = !cv && !stream && kk % 128 == 0 && kk >= 512 && xn > 64 && yn > 64 &&
+                           (4 * tiles128 >= cu_n || kk >= 2048) && ldl < (1 << 24) && ldr < (1 << 24) &&
+                           (size_t)4 * 256 * 128 <= lds_cu && !(ctx->kernel_mask & MH_MASK_NO_MID);
+    const bool xres = (!cv || xres_cv) && !stream && depth > 0 && (kk % 64 == 0 || tail_xres) && yn >= 256 &&
+                      xres_fits(xres_tx) && !(mid_shape && tiles128 <= cu_n) &&
+                      !(ctx->kernel_mask & MH_MASK_NO_XRES);
+    // From a quarter of a round to one round of 128 x 128 tiles, and up to two and a half rounds where
+    // k is long (with short k and several rounds the two-workgroups-per-CU kernel, which overlaps one
+    // tile's epilogue with another's loop, wins: 32 x 512 x 1024 x 512 29.8 against 33.7 us): the
+    // kernel with eight wavefronts per tile that sums both panels itself, so no pass over either
+    // operand is launched.  Measured against the other tiled kernels (k-contiguous operands): 1024 x 4096 x 1024
+    // (64 tiles) 19.2 -> 18.7 us, 1280 x 2048 x 1280 (100) 16.3 -> 12.2, 2048^3 (256) 19.3 -> 14.8,
+    // 2560 x 2048 x 2560 (400) 25.8 -> 23.8, 3072 x 1024 x 3072 (576) 26.6 -> 24.9; at 1024 tiles
+    // (4096 x 1024 x 4096, 4096^3) the 256 x 256 tiles win by 8 - 13 %.
+    const bool mid = mid_shape && !xres &&
+                     (tiles128 <= cu_n || (kk >= 2048 && 2 * tiles128 <= 5 * cu_n));
+    return Route{xres, mid, xres_tx};
+  };
+  const Route planned = route_of((int)std::min(lhs_direct ? depth : kp, rhs_direct ? (rhs_ld ? rhs_ld : depth) : kp),
+                                 lhs_direct ? depth : kp, rhs_direct ? (rhs_ld ? rhs_ld : depth) : kp);
   // The Y operand's row sums can be taken inside the GEMM kernel from the fragments it already
   // holds, which saves one pass over that operand.  The pass costs YN * K bytes of HBM traffic,
   // the in-kernel sums about 3.6 % of the GEMM's own time (measured at 8192^3: +17 us against an
@@ -3115,30 +3186,22 @@ int Q8Call::general() {
   const bool sum_y_shape = cv || (depth > 0 && (depth <= 1024 || (x_is_lhs ? rows : cols) <= 4096));
   // A transposing repack can add up its rows on the way; worth its extra (zeroing) launch only
   // where it replaces a pass, i.e. not for a Y operand whose sums the GEMM kernel takes anyway.
-  // ... nor where the call will go to the kernel that sums both panels itself (the shape test of
-  // the dispatch below, with a depth too long for the kernel that keeps a panel in LDS)
-  const int64_t tiles128_pre = (((x_is_lhs ? rows : cols) + 127) / 128) * (((x_is_lhs ? cols : rows) + 127) / 128) * batch;
-  const int64_t cu_pre = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  const bool sums_in_kernel = !cv && depth % 128 == 0 && depth >= 1280 && rows > 64 && cols > 64 &&
-                              4 * tiles128_pre >= cu_pre &&
-                              (tiles128_pre <= cu_pre || (depth >= 2048 && 2 * tiles128_pre <= 5 * cu_pre)) &&
-                              !(ctx->kernel_mask & MH_MASK_NO_MID);
+  // ... nor where the call will go to a kernel that sums both panels itself.
+  const bool sums_in_kernel = !cv && (stream || planned.xres || planned.mid);
   // An X operand that is repacked for the 256 x 256 kernel with 128-byte slabs is written already
   // shifted to int8, which spares that kernel half of its sign flips (8192^3, same box: 505.3 ->
   // 498.5 us per call).  The test
   // repeats the dispatch below: a depth too long for the kernel that keeps a panel in LDS, not the
   // eight-wavefront kernel's range, 256 x 256 tiles chosen, rows within the ring's 32-bit offsets.
   const bool x_flip = !(ctx->kernel_mask & MH_MASK_NO_XFLIP) && !cv && depth % 128 == 0 && depth >= 1280 && depth < (1 << 24) && !sums_in_kernel &&
-                      mh_q8_tile_choice(x_is_lhs ? rows : cols, x_is_lhs ? cols : rows, batch, cu_pre) ==
-                          MH_TILE_BIG;
+                      mh_q8_tile_choice(xn, yn, batch, cu_n) == MH_TILE_BIG;
   // Where the left-hand matrix is read in place and needs a pass for its sums (the Y operand of the
   // 256 x 256 kernel on a shape too large for in-kernel sums) while the right-hand one is repacked
   // with fused sums, the pass goes first and clears the repack's sums buffer on the way: one launch
   // less in front of the GEMM kernel (8192^3, same process: 502.3 -> 500.3 us per call).
   // x_flip repeats the dispatch's shape test: none of the kernels that sum their own panels applies.
   const bool l_sums_first = x_flip && !x_is_lhs && !sum_y_shape && lhs_direct && !lhs_w && !rhs_w &&
-                            !rhs_direct && rhs_order == MACE_HIP_ROW_MAJOR && cols % 16 == 0 &&
-                            (uintptr_t)rhs % 16 == 0;
+                            !rhs_direct && rhs_order == MACE_HIP_ROW_MAJOR;
   if (l_sums_first) {
     MH_RETURN_IF_ERROR(launch_panel_sums(ctx, lhs, depth, lhs_nb > 1 ? rows * depth : 0, rows, (int)depth,
                                          lhs_nb, corrL, corrR, (int64_t)rhs_nb * cols));
@@ -3151,56 +3214,12 @@ int Q8Call::general() {
                              rhs_ld != 0 ? rhs_ld : depth, rhs_w,
                              ((x_is_lhs && sum_y_shape) || sums_in_kernel) ? nullptr : corrR, &R,
                              x_flip && !x_is_lhs));
+  MH_RETURN_IF_ERROR(launch_repacks());
   const bool sum_y = cv || (sum_y_shape && !(x_is_lhs ? R.sums : L.sums));   // cached sums cost nothing
-  // A small X panel (at most 128 rows of at most 64 bytes: an early 1x1 convolution's filter) against a
-  // long Y panel goes to the streaming kernel, which also sums both panels itself.
-  const int64_t xn = x_is_lhs ? rows : cols, yn = x_is_lhs ? cols : rows;
-  // (Measured: it wins for K <= 64; from K = 128 on the tiled kernels are as fast.)
-  const bool stream = !cv && out_u8 && requant_by_mad(rq) && lhs_direct && rhs_direct && rhs_ld == 0 &&
-                      mh_q8_stream_shape(depth, xn, yn) && ((uintptr_t)out % 16 == 0);
   const int32_t *sumL = L.sums ? L.sums : corrL, *sumR = R.sums ? R.sums : corrR;
-  // An X panel whose tile (64 or 128 rows, all of k) fits in LDS twice per CU goes to the kernel
-  // that keeps it there and sums both panels itself.  Measured against the tiled kernels (k from
-  // 64 to 1024, 64 to 1024 X rows, 4 Ki to 256 Ki Y rows): with the block height chosen as in
-  // launch_gemm_xres_any it wins or ties throughout (where the tile only fits once, k >= 640 at
-  // 128 rows, the tiled kernels win by 10 - 35 % and keep the shape).  A convolution whose
-  // patches the kernel gathers (cin % 64 == 0) takes it whenever the tile fits: 25 % faster
-  // than the gathering tiled kernel on 3x3, 56x56x64 -> 64 at batch 64 (splitting a 128-row tile
-  // that does not fit into two of 64 rows was slower than the tiled kernel).
-  // (Bit MH_MASK_NO_XRES of the kernel mask: test hook that keeps the tiled kernels in use.)
-  const int kk = L.k < R.k ? L.k : R.k;
-  const size_t lds_cu = ctx->lds_bytes > 0 ? (size_t)ctx->lds_bytes : 65536;
-  auto xres_fits = [&](int tx) {
-    return 2 * (XRES_SC_BYTES + (size_t)tx * ((kk + 63) & ~63)) <= lds_cu;
-  };
-  // Where 128 rows of a long k do not fit, 64-row tiles (Y is then read once per 64 X rows) still
-  // win between one and two 64 x 64 blocks per CU, where the tiled kernels leave most of the chip
-  // idle (k = 1024, 512 X rows, 3136 Y rows: 16.0 -> 9.4 us); beyond that they lose.
-  const int64_t blocks_tx64 = ((xn + 63) / 64) * ((yn + 63) / 64) * batch;
-  const int64_t cu_n = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  const bool xres_narrow = !cv && !xres_fits(128) && blocks_tx64 > cu_n && blocks_tx64 <= 2 * cu_n;
-  const int xres_tx = (xn <= 64 || xres_narrow) ? 64 : 128;
-  const bool xres_cv = cv && !cv_small && out_u8 && cv->cin % 64 == 0 && depth % 64 == 0;
-  const int64_t tiles128 = ((xn + 127) / 128) * ((yn + 127) / 128) * batch;
-  // (one round of 128 x 128 tiles at k >= 512 is faster on the eight-wavefront kernel, see above;
-  // from k = 2048 on also below a quarter of a round, where the 64 x 64 tiles and their sums pass took
-  // the shape: 6 - 11 % faster with k-contiguous operands at 1 to 63 tiles)
-  const bool mid_shape = !cv && !stream && kk % 128 == 0 && kk >= 512 && xn > 64 && yn > 64 &&
-                         (4 * tiles128 >= cu_n || kk >= 2048) && L.ld < (1 << 24) && R.ld < (1 << 24) &&
-                         (size_t)4 * 256 * 128 <= lds_cu && !(ctx->kernel_mask & MH_MASK_NO_MID);
-  const bool xres = (!cv || xres_cv) && !stream && depth > 0 && (kk % 64 == 0 || tail_xres) && yn >= 256 &&
-                    xres_fits(xres_tx) && !(mid_shape && tiles128 <= cu_n) &&
-                    !(ctx->kernel_mask & MH_MASK_NO_XRES);
-  // From a quarter of a round to one round of 128 x 128 tiles, and up to two and a half rounds where
-  // k is long (with short k and several rounds the two-workgroups-per-CU kernel, which overlaps one
-  // tile's epilogue with another's loop, wins: 32 x 512 x 1024 x 512 29.8 against 33.7 us): the
-  // kernel with eight wavefronts per tile that sums both panels itself, so no pass over either
-  // operand is launched.  Measured against the other tiled kernels (k-contiguous operands): 1024 x 4096 x 1024
-  // (64 tiles) 19.2 -> 18.7 us, 1280 x 2048 x 1280 (100) 16.3 -> 12.2, 2048^3 (256) 19.3 -> 14.8,
-  // 2560 x 2048 x 2560 (400) 25.8 -> 23.8, 3072 x 1024 x 3072 (576) 26.6 -> 24.9; at 1024 tiles
-  // (4096 x 1024 x 4096, 4096^3) the 256 x 256 tiles win by 8 - 13 %.
-  const bool mid = mid_shape && !xres &&
-                   (tiles128 <= cu_n || (kk >= 2048 && 2 * tiles128 <= 5 * cu_n));
+  // (a registered weight's panel may be padded otherwise than one made for this call)
+  const Route route = route_of(std::min(L.k, R.k), L.ld, R.ld);
+  const bool xres = route.xres, mid = route.mid;
   MH_CHECK(ctx, !tail_xres || xres, "internal: depth tail outside the resident-tile kernel");
   MH_CHECK(ctx, !l_sums_first || (!stream && !xres && !mid && !L.sums && !sum_y),
            "internal: early sums pass on a shape whose kernel takes its own");
@@ -3237,7 +3256,7 @@ int Q8Call::general() {
   }
   if (xres) {
     p.sum_y = true;
-    return launch_gemm_xres_any(ctx, p, tab, out_u8, (int)batch, xres_tx, false);
+    return launch_gemm_xres_any(ctx, p, tab, out_u8, (int)batch, route.tx, false);
   }
   if (mid) return launch_gemm_mid(ctx, p, tab, out_u8, (int)batch);
   if (stream) {

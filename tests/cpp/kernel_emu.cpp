@@ -537,22 +537,47 @@ static void small_conv_case(int n, int hw, int cin, int cout, int k, int stride,
   small_case<false, false>(cout, n * out * out, k * k * cin, &cv);
 }
 
-static void pack_case(int n, int k, bool by_dwords) {
+// both operands of a call copied into padded panels by one launch: nb batches of n rows of k bytes
+// next to nb batches of a k-major [k][nt] operand, with its row sums, as read or shifted
+static void pack_case(int nb, int n, int nt, int k, bool flip) {
   ++g_cases;
   const int kp = (k + 63) & ~63;
-  uint8_t *src = new uint8_t[(int64_t)n * k], *dst = new uint8_t[(int64_t)n * kp];
-  for (int64_t i = 0; i < (int64_t)n * k; ++i) src[i] = rnd();
-  memset(dst, 0xEE, (int64_t)n * kp);
-  const int64_t total = (int64_t)n * (kp / 16);
-  const dim3 grid((unsigned)((total + 255) / 256), 1, 1);
-  if (by_dwords) run_grid(grid, [&] { q8_pack_rows4_kernel(src, (int64_t)n * k, dst, (int64_t)n * kp, n, k, kp); });
-  else run_grid(grid, [&] { q8_pack_rows_kernel(src, (int64_t)n * k, dst, (int64_t)n * kp, n, k, kp); });
+  const int64_t rows = (int64_t)nb * n, cols = (int64_t)nb * nt;
+  uint8_t *src = new uint8_t[rows * k], *dst = new uint8_t[rows * kp];
+  uint8_t *tsrc = new uint8_t[cols * k], *tdst = new uint8_t[cols * kp];
+  int32_t *sums = new int32_t[cols]();
+  for (int64_t i = 0; i < rows * k; ++i) src[i] = rnd();
+  for (int64_t i = 0; i < cols * k; ++i) tsrc[i] = rnd();
+  memset(dst, 0xEE, rows * kp);
+  memset(tdst, 0xEE, cols * kp);
+  RepackJob a{}, b{};
+  a.src = src; a.dst = dst; a.rows = rows; a.n = n; a.k = k; a.kp = kp;
+  a.blocks = (rows * (kp / 16) + REPACK_PIECES - 1) / REPACK_PIECES;
+  b.src = tsrc; b.dst = tdst; b.n = nt; b.k = k; b.kp = kp; b.sums = sums;
+  b.flip = flip ? 0x80808080u : 0u;
+  b.tiles_n = (nt + 127) / 128; b.tiles_k = (kp + 127) / 128;
+  b.blocks = (int64_t)b.tiles_n * b.tiles_k * nb;
+  // (a grid with more workgroups than there is work, in two rows)
+  const dim3 grid((unsigned)((a.blocks + b.blocks) / 2 + 1), 2, 1);
+  run_grid(grid, [&] { q8_repack_kernel(a, b); });
   int64_t bad = 0;
-  for (int r = 0; r < n; ++r)
-    for (int c = 0; c < kp; ++c) bad += dst[(int64_t)r * kp + c] != (c < k ? src[(int64_t)r * k + c] : 0x80);
-  EXPECT(bad == 0, "pack_rows%s n %d k %d: %lld bytes differ", by_dwords ? "4" : "", n, k, (long long)bad);
+  for (int64_t r = 0; r < rows; ++r)
+    for (int c = 0; c < kp; ++c) bad += dst[r * kp + c] != (c < k ? src[r * k + c] : 0x80);
+  for (int64_t r = 0; r < cols; ++r) {
+    int s = 0;
+    for (int c = 0; c < kp; ++c) {
+      const int v = c < k ? tsrc[(r / nt * k + c) * nt + r % nt] : 0x80;
+      s += v - 128;
+      bad += tdst[r * kp + c] != (uint8_t)(flip ? v ^ 0x80 : v);
+    }
+    bad += s != sums[r];
+  }
+  EXPECT(bad == 0, "repack nb %d n %d nt %d k %d: %lld bytes differ", nb, n, nt, k, (long long)bad);
   delete[] src;
   delete[] dst;
+  delete[] tsrc;
+  delete[] tdst;
+  delete[] sums;
 }
 
 template <int LPR>
@@ -582,9 +607,11 @@ static void sums_case(int n, int k) {
 #endif
 int main() {
 #if PART != 2
-  // the repacks of k-contiguous rows (any k; k % 4 == 0 by dwords)
-  for (int k : {1, 3, 15, 16, 17, 24, 63, 64, 65, 100, 127}) pack_case(37, k, false);
-  for (int k : {4, 8, 24, 40, 60, 64, 68, 120}) pack_case(301, k, true);
+  // the repacks of k-contiguous rows and of k-major operands: any row length
+  for (int k : {1, 3, 15, 16, 17, 24, 63, 64, 65, 100, 127}) pack_case(1, 37, k, k, false);
+  for (int k : {4, 8, 24, 40, 60, 64, 68, 120}) pack_case(1, 301, 130 + k, k, true);
+  pack_case(3, 41, 157, 131, false);
+  pack_case(2, 17, 7, 300, true);
   // row sums: rows of 16 .. 1024 bytes, row counts that leave part of a wavefront without a row
   sums_case<1>(70, 16);
   sums_case<2>(33, 32);

@@ -20,7 +20,7 @@ PIECES = [
      "// ---- the kernel for an X panel that fits in LDS"),
     ("template <int FX, int FY, int G, typename OutT, int OCC, bool CONV = false, bool XT = false,",
      "// ---- the streaming kernel for a small X panel"),
-    ("__global__ void q8_pack_rows_kernel", "// src is [k][n] with n contiguous"),
+    ("struct RepackJob {", "__global__ __launch_bounds__(256) void q8_zero_i32_kernel"),
     ("template <int LPR>\n__global__ __launch_bounds__(256) void q8_panel_sums_kernel",
      "int launch_panel_sums("),
 ]

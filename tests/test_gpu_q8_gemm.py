@@ -320,6 +320,27 @@ def test_q8_gemm_depth_tail_of_half_a_piece(ctx, batch, rows, depth, cols, lb, r
     assert check_gemm(ctx, batch, rows, depth, cols, lb, rb, lo, ro, oo) == ("xres/TAIL", "xres/TAIL")
 
 
+# Operands copied into padded panels, both by one launch: rows of any length (odd, shorter than 16 bytes,
+# one more and one less than whole pieces), one operand shared or both per batch, every pair of
+# layouts; depths whose padded row is an odd number of 64-byte slabs (rounded up to 128 from 513 on),
+# and depths in whole 16-byte pieces where only the other operand cannot be read in place.
+REPACK_SHAPES = [
+    (1, 300, 513, 129, True, True), (2, 131, 575, 127, True, True), (3, 97, 1100, 113, False, True),
+    (2, 200, 1488, 333, True, False), (1, 129, 1040, 77, True, True), (2, 513, 64, 15, True, True),
+    (1, 9, 640, 517, True, True), (1, 257, 2111, 255, True, True), (5, 70, 200, 301, True, True),
+]
+
+
+@pytest.mark.parametrize("batch,rows,depth,cols,lb,rb", REPACK_SHAPES)
+@pytest.mark.parametrize("lo,ro,oo", [(R, R, R), (R, Cm, R), (Cm, R, R), (Cm, Cm, Cm), (R, R, Cm)])
+def test_q8_gemm_repacked_operands(ctx, batch, rows, depth, cols, lb, rb, lo, ro, oo):
+    ctx.call("mace_hip_ctx_set_kernel_mask", mh.MASK_NO_SMALL)
+    try:
+        check_gemm(ctx, batch, rows, depth, cols, lb, rb, lo, ro, oo)
+    finally:
+        ctx.call("mace_hip_ctx_set_kernel_mask", 0)
+
+
 def test_q8_gemm_config1_matmul(ctx):
     """benchmark configuration 1: A [128x256], B [256x128], zero points 128/128/128, scales
     0.02/0.015/0.05 -> (1649267328, shift 7)."""

@@ -470,3 +470,17 @@ def test_recipes_cover_every_launchable_variant_and_still_plan_to_it(ctx):
         assert kernel_recipes.plan_call(ctx, r["call"]) == mh.SUCCESS, r
         p = ctx.last_plan()
         assert (p.family, p.variant, p.kernel) == (r["family"], r["variant"], r["kernel"]), (p, r)
+
+
+def test_repacked_operands(ctx):
+    both = mh.AUX_PACK_ROWS | mh.AUX_PACK_TRANSPOSE
+    # both operands into panels of whole 128-byte slabs by one launch, sums in the kernel
+    for depth in (1500, 1400):            # 24 and 22 slabs of 64 bytes
+        p = gemm(ctx, 4, 1001, depth, 777, u8=False)
+        assert p.family == mh.KF_Q8_GEMM_MID and p.aux == both and p.launches == 2
+    # 1488 = 93 pieces of 16 bytes: readable in place, but not in whole slabs
+    p = gemm(ctx, 1, 999, 1488, 1001)
+    assert p.family == mh.KF_Q8_GEMM_MID and p.aux == both and p.launches == 2
+    # whole slabs on the left: only the right-hand matrix is copied
+    p = gemm(ctx, 1, 2048, 1024, 2047)
+    assert p.aux == mh.AUX_PACK_TRANSPOSE and p.launches == 2
