@@ -149,8 +149,13 @@ __device__ inline void stage_requant_pairs(int32_t *pairs, const RequantFixed &r
 // stores int32 results or requantized bytes.  Accumulator register r of a 32x32 tile holds
 //   x (MFMA row)    = 8 * (r / 4) + 4 * (lane / 32) + r % 4
 //   y (MFMA column) = lane % 32
-// so every lane owns runs of four consecutive x, stored as one 16-byte (int32) or 4-byte
-// (uint8) access.  The correction vectors of the tile are staged through LDS first (the
+// so every lane owns runs of four consecutive x, stored as one 16-byte access (uint8: 16 bytes put
+// together from two lanes).  Rows of any length are stored that way, at whatever address their
+// pieces start (the hardware takes 16-byte stores at any address): only the piece that holds the end
+// of a row goes element by element.  Element-wise stores of rows that are not whole aligned pieces
+// touch 64 rows per instruction and took two thirds of such calls: 5001 x 211 x 6003 106 -> 34 us, 4 x 1001
+// x 1500 x 777 33.6 -> 25.4 (int32) and 32.4 -> 24.1 (uint8); rows of whole dwords, 2044 columns, 11.7 ->
+// 11.2.  The correction vectors of the tile are staged through LDS first (the
 // operand buffers are dead by then), so the stores do not wait on scattered global loads.
 // PRESTAGED: the caller has already put the tile's x correction terms and the comparison table
 // into `lds` (same layout) and synchronised the workgroup.
@@ -190,13 +195,7 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
   }
 
   OutT *outb = (OutT *)p.out + (int64_t)b * p.obs;
-  const bool vec_ok = (p.ldo % 4 == 0) && (((uintptr_t)outb) % (4 * sizeof(OutT)) == 0);
-  const bool interior = vec_ok && x0 + TX <= p.XN && y0 + TY <= p.YN;
-  const bool interior16 = interior && (p.ldo % 16 == 0) && (((uintptr_t)outb) % 16 == 0);
-  // uint8 rows made of whole 16-byte pieces (XN % 16 == 0, aligned): a ragged tile still stores 16
-  // bytes per lane, each lane deciding for its own piece (XN = 48 against 64 columns at 200704 x 128:
-  // 25.6 -> 13 us; before, every tile that was not wholly inside stored byte by byte)
-  const bool wide16 = (p.ldo % 16 == 0) && (((uintptr_t)outb) % 16 == 0) && (p.XN % 16 == 0);
+  const bool interior16 = x0 + TX <= p.XN && y0 + TY <= p.YN && p.ldo % 16 == 0 && (uintptr_t)outb % 16 == 0;
 
   const RequantLds rql = requant_lds(rq, tab);
   const bool by_mad = requant_by_mad(rq);
@@ -241,10 +240,11 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const int xl = xb + 8 * q;
-            // (rows of whole, aligned 16-byte pieces: a ragged tile stores them whole as well)
-            if (interior || (vec_ok && p.XN % 4 == 0 && y < p.YN && x0 + xl < p.XN)) {
-              *(v4i *)(orow + xl) = v4i{v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
-            } else if (y < p.YN) {
+            if (y >= p.YN) continue;
+            if (x0 + xl + 4 <= p.XN) {
+              const v4i w = {v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
+              __builtin_memcpy(orow + xl, &w, 16);
+            } else {
 #pragma unroll
               for (int e = 0; e < 4; ++e)
                 if (x0 + xl + e < p.XN) orow[xl + e] = (OutT)v[q * 4 + e];
@@ -261,35 +261,22 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
             for (int r = 0; r < 16; ++r)
               packed[r / 4] |= (uint32_t)mh_requant_fixed(v[r], rq) << (8 * (r % 4));
           }
+          // Lane (y, h = lane / 32) holds bytes x = 8 q + 4 h + 0..3 of this 32-wide block
+          // in packed[q].  Swapping the upper half of one register with the lower half of
+          // another gives lane (y, 0) bytes 0..15 and lane (y, 1) bytes 16..31.
+          const v2u s02 = __builtin_amdgcn_permlane32_swap(packed[0], packed[2], false, false);
+          const v2u s13 = __builtin_amdgcn_permlane32_swap(packed[1], packed[3], false, false);
+          const v4i w = {(int)s02.x, (int)s02.y, (int)s13.x, (int)s13.y};
+          const int xh = (wx * FX + i) * 32 + 16 * (lane >> 5);
           if constexpr (WIDE) {
-            // Lane (y, h = lane / 32) holds bytes x = 8 q + 4 h + 0..3 of this 32-wide block
-            // in packed[q].  Swapping the upper half of one register with the lower half of
-            // another gives lane (y, 0) bytes 0..15 and lane (y, 1) bytes 16..31.
-            const v2u s02 = __builtin_amdgcn_permlane32_swap(packed[0], packed[2], false, false);
-            const v2u s13 = __builtin_amdgcn_permlane32_swap(packed[1], packed[3], false, false);
-            const v4i w = {(int)s02.x, (int)s02.y, (int)s13.x, (int)s13.y};
-            *(v4i *)(orow + (wx * FX + i) * 32 + 16 * (lane >> 5)) = w;
-          } else if (wide16) {
-            // the same 16-byte pieces in a tile that is not wholly inside the matrix: every lane
-            // checks its own piece (uniform branch; the requantization above is shared with the
-            // dword / byte stores below, so no further unrolled copy of it exists)
-            const v2u s02 = __builtin_amdgcn_permlane32_swap(packed[0], packed[2], false, false);
-            const v2u s13 = __builtin_amdgcn_permlane32_swap(packed[1], packed[3], false, false);
-            const v4i w = {(int)s02.x, (int)s02.y, (int)s13.x, (int)s13.y};
-            const int xh = (wx * FX + i) * 32 + 16 * (lane >> 5);
-            if (y < p.YN && x0 + xh < p.XN) *(v4i *)(orow + xh) = w;
-          } else {
+            *(v4i *)(orow + xh) = w;
+          } else if (y < p.YN) {   // every lane checks its own piece
+            if (x0 + xh + 16 <= p.XN) {
+              __builtin_memcpy(orow + xh, &w, 16);
+            } else {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int xl = xb + 8 * q;
-              // (rows of whole, aligned dwords: a ragged tile stores them whole as well)
-              if (interior || (vec_ok && p.XN % 4 == 0 && y < p.YN && x0 + xl < p.XN)) {
-                *(uint32_t *)(orow + xl) = packed[q];
-              } else if (y < p.YN) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                  if (x0 + xl + e < p.XN) orow[xl + e] = (OutT)((packed[q] >> (8 * e)) & 0xff);
-              }
+              for (int e = 0; e < 16; ++e)
+                if (x0 + xh + e < p.XN) orow[xh + e] = (OutT)(((uint32_t)w[e / 4] >> (8 * (e % 4))) & 0xff);
             }
           }
         }
