@@ -88,14 +88,23 @@ __device__ __forceinline__ void requant_16_by_mad(const int32_t (&v)[16], const 
         asm("v_med3_i32 %0, %1, %2, %3" : "=v"(h[r]) : "v"(h[r]), "s"(m.lo), "v"(m.hi));
     }
   }
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    // the two lower bytes, then the two upper ones (op_sel: the result goes to the upper half and
-    // the lower half is kept)
-    asm("v_ashr_pk_u8_i32 %0, %1, %2, %3" : "=v"(packed[q]) : "v"(h[4 * q]), "v"(h[4 * q + 1]), "s"(m.sh));
-    asm("v_ashr_pk_u8_i32 %0, %1, %2, %3 op_sel:[0,0,0,1]"
-        : "+v"(packed[q]) : "v"(h[4 * q + 2]), "v"(h[4 * q + 3]), "s"(m.sh));
-  }
+  // Lower halves first, then the upper ones (op_sel: the result goes to the upper half and the lower
+  // half is kept).  Every caller swaps halves of the packed dwords next: a v_permlane32_swap must come
+  // at least two wait states after the vector instruction that writes an operand of it, and what the
+  // upper-half form writes may be read one after.  The compiler keeps those distances for instructions
+  // of its own but not for assembly, so the wait stands in the block, behind all eight.
+  asm("v_ashr_pk_u8_i32 %0, %4, %5, %20\n\t"
+      "v_ashr_pk_u8_i32 %1, %8, %9, %20\n\t"
+      "v_ashr_pk_u8_i32 %2, %12, %13, %20\n\t"
+      "v_ashr_pk_u8_i32 %3, %16, %17, %20\n\t"
+      "v_ashr_pk_u8_i32 %0, %6, %7, %20 op_sel:[0,0,0,1]\n\t"
+      "v_ashr_pk_u8_i32 %1, %10, %11, %20 op_sel:[0,0,0,1]\n\t"
+      "v_ashr_pk_u8_i32 %2, %14, %15, %20 op_sel:[0,0,0,1]\n\t"
+      "v_ashr_pk_u8_i32 %3, %18, %19, %20 op_sel:[0,0,0,1]\n\t"
+      "s_nop 1"
+      : "=&v"(packed[0]), "=&v"(packed[1]), "=&v"(packed[2]), "=&v"(packed[3])
+      : "v"(h[0]), "v"(h[1]), "v"(h[2]), "v"(h[3]), "v"(h[4]), "v"(h[5]), "v"(h[6]), "v"(h[7]), "v"(h[8]),
+        "v"(h[9]), "v"(h[10]), "v"(h[11]), "v"(h[12]), "v"(h[13]), "v"(h[14]), "v"(h[15]), "s"(m.sh));
 #else
   for (int q = 0; q < 4; ++q) packed[q] = 0;
 #endif
