@@ -256,6 +256,11 @@ inline int f32_gemv_vec(int nb) { return log2i(nb); }
 // must be taken before any kernel of the call is launched: mh_arena_reserve() first.
 int mh_arena_reserve(mace_hip_ctx *ctx, size_t bytes);
 void *mh_arena_take(mace_hip_ctx *ctx, size_t bytes);   // 256-byte aligned, after reserve
+// whether mh_arena_reserve(bytes) would find the room or may allocate it
+inline bool mh_arena_can_hold(const mace_hip_ctx *ctx, size_t bytes) {
+  return ctx->arena_used + bytes + 16 * 256 <= ctx->arena_bytes ||
+         !(ctx->no_alloc || ctx->capturing || ctx->arena_used != 0);
+}
 inline size_t mh_align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 struct ArenaScope {
   mace_hip_ctx *ctx;
@@ -586,11 +591,11 @@ inline int mh_f32_ksplit(const mace_hip_ctx *ctx, int64_t batch, int64_t rows, i
   if (parts > 16) parts = 16;
   return parts < 2 ? 1 : (int)parts;
 }
-// scratch of that split (0 without one); a batch may also be run as one long row of columns
+// scratch of that split (0 without one); joined: a batch may also be run as one long row of columns
 inline size_t mh_f32_ksplit_bytes(const mace_hip_ctx *ctx, int64_t batch, int64_t rows, int64_t cols,
-                                  int64_t depth) {
+                                  int64_t depth, bool joined = true) {
   const int parts = std::max(mh_f32_ksplit(ctx, batch, rows, cols, depth),
-                             mh_f32_ksplit(ctx, 1, rows, batch * cols, depth));
+                             joined ? mh_f32_ksplit(ctx, 1, rows, batch * cols, depth) : 1);
   return parts > 1 ? sizeof(float) * (size_t)parts * batch * rows * cols + 256 : 0;
 }
 

@@ -553,6 +553,7 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
   // A shared left-hand matrix (a convolution's filter) against a batch: the columns of all batches
   // are one long row, so that tiles do not end at an image (7 x 7 pixels fill 49 of a tile's 128
   // columns: 1024 -> 1024 channels at batch 64 190 -> 55 us, the split above included).
+  const int64_t images = batch;
   if (batch > 1 && !lhs_batched && rhs_batched && out_major == MACE_HIP_ROW_MAJOR &&
       rhs_major == MACE_HIP_ROW_MAJOR && batch * cols < (1ll << 31)) {
     p.flat = (int)cols;
@@ -580,12 +581,17 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
   // second launch adds up in a fixed order.  (A tile's time is its k tiles at about 1 us each
   // whatever else runs: 512^3, 16 tiles, took 43.7 us with 240 CUs idle.)
   ArenaScope scope(ctx);
-  const int parts = mh_f32_ksplit(ctx, batch, rows, p.N, depth);
+  auto bytes_of = [&](int n) { return sizeof(float) * (size_t)n * total + 256; };
+  int parts = mh_f32_ksplit(ctx, batch, rows, p.N, depth);
+  // The long row has fewer tiles than the images have one by one, so it is split where they are not.
+  // That needs scratch; where none can be had (in a capture, or beside other slices of the arena) the
+  // images' own tiles decide, so that no call is refused for joining them.
+  if (parts > 1 && p.flat && !mh_arena_can_hold(ctx, bytes_of(parts)))
+    parts = mh_f32_ksplit(ctx, images, rows, cols, depth);
   if (parts > 1) {
-    const size_t bytes = sizeof(float) * (size_t)parts * total + 256;
-    const bool room = ctx->arena_used + bytes + 16 * 256 <= ctx->arena_bytes;
+    const size_t bytes = bytes_of(parts);
     // (scratch that does not fit while other slices of the arena are in use: no split)
-    if (room || ctx->arena_used == 0) {
+    if (mh_arena_can_hold(ctx, bytes) || ctx->arena_used == 0) {
       MH_RETURN_IF_ERROR(mh_arena_reserve(ctx, bytes));
       p.part = (float *)mh_arena_take(ctx, bytes);
       if (!p.part) return mh_fail(ctx, MACE_HIP_RUNTIME_ERROR, "arena slice unavailable");
@@ -775,8 +781,11 @@ int mace_hip_conv2d_f32_nchw(mace_hip_ctx *ctx, const float *input, const float 
   MH_CHECK(ctx, total < (1ll << 40), "dimension too large");
   if (total == 0 || cout == 0) return MACE_HIP_SUCCESS;
   MH_CHECK(ctx, input && out, "null operand");
-  MH_RETURN_IF_ERROR(mh_arena_reserve(ctx, sizeof(float) * (size_t)total +
-                                           mh_f32_ksplit_bytes(ctx, n, cout, ph * pw, cin) + 4096));
+  // (the scratch of a split that only the joined images take is asked for, not insisted on)
+  const size_t scratch = sizeof(float) * (size_t)total + 4096;
+  const size_t joined = scratch + mh_f32_ksplit_bytes(ctx, n, cout, ph * pw, cin);
+  MH_RETURN_IF_ERROR(mh_arena_reserve(ctx, mh_arena_can_hold(ctx, joined) ? joined
+                                           : scratch + mh_f32_ksplit_bytes(ctx, n, cout, ph * pw, cin, false)));
   ArenaScope scope(ctx);
   float *padded = (float *)mh_arena_take(ctx, sizeof(float) * (size_t)total);
   if (!padded) return mh_fail(ctx, MACE_HIP_RUNTIME_ERROR, "arena slice unavailable");

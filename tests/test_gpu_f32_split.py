@@ -96,3 +96,44 @@ def test_operands_outside_the_split(ctx, m, k, n):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
     got, want, size = run(ctx, np.zeros_like(a), b, False, False)
     assert not got.any()
+
+
+def test_joined_images_captured_without_scratch():
+    """32 images of 7 x 7: joined they are few enough tiles to split the depth, one by one they are not.
+    A context without scratch records the call unsplit; one that had to split before still refuses."""
+    import ctypes as C
+    n, cin, hw, cout = 32, 1024, 49, 1024
+    rng = np.random.default_rng(1)
+    x = rng.standard_normal((n, cin, hw)).astype(np.float32)
+    f = (rng.standard_normal((cout, cin)) / 32).astype(np.float32)
+    c = mh.Context(0)
+    try:
+        d = Dev()
+        px, pf = d.put(x), d.put(f)
+        t, po = d.empty(n * cout * hw, np.float32)
+        d.sync()
+        args = (px, pf, None, n, cin, hw, cout, mh.ACT_RELU, 0.0, po)
+        g = C.c_void_p()
+        c.call("mace_hip_graph_capture_begin")
+        status = c.status("mace_hip_conv1x1_f32_nchw", *args)
+        plan = c.last_plan()
+        refused = c.status("mace_hip_gemm_f32", px, pf, 1, 512, 512, 512, 0, 0, 0, 1, 1, po)
+        c.call("mace_hip_graph_capture_end", C.byref(g))
+        assert status == mh.SUCCESS and plan.launches == 1 and refused == mh.INVALID_ARGS
+        want = np.maximum(np.matmul(f.astype(np.float64), x.astype(np.float64)), 0)
+        size = np.matmul(np.abs(f).astype(np.float64), np.abs(x).astype(np.float64))
+        for _ in range(3):
+            t.zero_()
+            d.sync()
+            c.call("mace_hip_graph_launch", g)
+            c.sync()
+            close(t.cpu().numpy().reshape(want.shape), want, size, cin)
+            t.zero_()
+            d.sync()
+            c.call("mace_hip_conv1x1_f32_nchw", *args)      # outside the capture: split, with scratch
+            assert c.last_plan().aux & mh.AUX_F32_KSPLIT
+            c.sync()
+            close(t.cpu().numpy().reshape(want.shape), want, size, cin)
+        c.call("mace_hip_graph_destroy", g)
+    finally:
+        c.close()
