@@ -82,10 +82,15 @@ __device__ inline float apply_act(float v, int act, float limit) {
 // 688 -> 318 us; the matrix cores are busy 35 - 45 % of it, the rest is each k tile's chain of LDS
 // reads, MFMAs, LDS writes and barrier (one to three workgroups per CU overlap).
 //
-// Where that does not hold, the workgroup computes its tile again with the binary32 instruction
-// (f32_tile_again): an operand so small (below 2^-110) that lo has no exact bf16 form, which the
-// split sees in the bits lo would lose, or so large (from 2^127 (2 - 2^-8) on, infinite, not a
-// number) that hi is not finite, which leaves a result that is not finite.
+// Both operands are multiplied by 2^23 before the split and the sums by 2^-46 behind it, all exact: the
+// last bit of the smallest subnormal number then lies at 2^-126, so every part of every number is a
+// normal bf16 number or zero, and values of any smallness (the tails of a softmax) go at one speed.
+// That replaces a test for bits the split would lose: the loop takes as long as with it (4 x 1024^3 50.4
+// and 50.1 us, 2304 x 512 x 2304 45.7 and 44.4).
+//
+// What the scaled split cannot take are operands from about 2^105 on, sums from 2^82 on, and numbers that
+// are not finite.  They leave a sum that is not finite, and the workgroup computes its tile again with
+// the binary32 instruction (`again` in f32_tile): with an infinity in every tile 4 x 1024^3 takes 140 us.
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 typedef __bf16 b8v __attribute__((ext_vector_type(8)));
@@ -102,12 +107,13 @@ __device__ __forceinline__ uint32_t bf16_pair(float x, float y) {   // to neares
 __device__ __forceinline__ float bf16_low(uint32_t pair) { return __uint_as_float(pair << 16); }
 __device__ __forceinline__ float bf16_high(uint32_t pair) { return __uint_as_float(pair & 0xffff0000u); }
 
+constexpr float SPLIT_SCALE = 0x1p23f, SUM_SCALE = 0x1p-46f;
+
 // Eight consecutive depths of one row (or column) as three 16-byte pieces: an MFMA fragment each.
-// Bits that `lo` cannot hold are left in the low half of `lost`.
-__device__ __forceinline__ void split_8(const float (&x)[8], u4v (&part)[3], uint32_t &lost) {
+__device__ __forceinline__ void split_8(const float (&x)[8], u4v (&part)[3]) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const float x0 = x[2 * e], x1 = x[2 * e + 1];
+    const float x0 = x[2 * e] * SPLIT_SCALE, x1 = x[2 * e + 1] * SPLIT_SCALE;
     const uint32_t hi = bf16_pair(x0, x1);
     const float r0 = x0 - bf16_low(hi), r1 = x1 - bf16_high(hi);
     const uint32_t mid = bf16_pair(r0, r1);
@@ -115,37 +121,6 @@ __device__ __forceinline__ void split_8(const float (&x)[8], u4v (&part)[3], uin
     part[0][e] = hi;
     part[1][e] = mid;
     part[2][e] = bf16_pair(s0, s1);
-    lost |= __float_as_uint(s0) | __float_as_uint(s1);
-  }
-}
-
-// One wavefront's FM x FN blocks of 32 x 32 by the binary32 instruction, operands straight from memory.
-template <int FM, int FN>
-__device__ __forceinline__ void f32_tile_again(const F32GemmParams &p, const float *A, const float *B, int m0,
-                                               const int64_t (&cols)[FN], int k0, int kend,
-                                               v16f (&acc)[FM * FN]) {
-  const int lane = threadIdx.x & 63;
-  const float *a[FM], *b[FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i) a[i] = A + (int64_t)min(m0 + i * 32 + (lane & 31), p.M - 1) * p.lrs;
-#pragma unroll
-  for (int j = 0; j < FN; ++j) b[j] = B + cols[j];
-#pragma unroll
-  for (int t = 0; t < FM * FN; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
-  for (int k = k0; k < kend; k += 2) {
-    const int kk = k + (lane >> 5);
-    float av[FM], bv[FN];
-#pragma unroll
-    for (int i = 0; i < FM; ++i) av[i] = kk < kend ? a[i][(int64_t)kk * p.lcs] : 0.f;
-#pragma unroll
-    for (int j = 0; j < FN; ++j) bv[j] = kk < kend ? b[j][(int64_t)kk * p.rrs] : 0.f;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-        acc[i * FN + j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i * FN + j], 0, 0, 0);
   }
 }
 
@@ -229,23 +204,26 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
     load_unit(std::integral_constant<bool, LK>{}, pa, p.lcs, kt0 + kt * BKT + ac * 8, xa[S]);
     load_unit(std::integral_constant<bool, RK>{}, pb, p.rrs, kt0 + kt * BKT + bc * 8, xb[S]);
   };
-  uint32_t lost = 0;
-  auto store_tile = [&](auto set, int kt, int buf) __attribute__((always_inline)) {
-    constexpr int S = decltype(set)::value;
+  auto clear_past_depth = [&](auto set, int kt) __attribute__((always_inline)) {
     if constexpr (GUARD) {   // what lies past the depth counts as zero
+      constexpr int S = decltype(set)::value;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         if (kt0 + kt * BKT + ac * 8 + e >= kend) xa[S][e] = 0.f;
         if (kt0 + kt * BKT + bc * 8 + e >= kend) xb[S][e] = 0.f;
       }
     }
+  };
+  auto store_tile = [&](auto set, int kt, int buf) __attribute__((always_inline)) {
+    constexpr int S = decltype(set)::value;
+    clear_past_depth(set, kt);
     u4v part[3];
-    split_8(xa[S], part, lost);
+    split_8(xa[S], part);
     if (has_a) {
 #pragma unroll
       for (int q = 0; q < 3; ++q) da[(buf * 3 + q) * KC * PA_] = part[q];
     }
-    split_8(xb[S], part, lost);
+    split_8(xb[S], part);
 #pragma unroll
     for (int q = 0; q < 3; ++q) db[(buf * 3 + q) * KC * PB_] = part[q];
   };
@@ -305,7 +283,7 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
 #pragma unroll
     for (int i = 0; i < MFMAS; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // an MFMA
-      __builtin_amdgcn_sched_group_barrier(0x002, 120 / MFMAS, 0);   // vector instructions
+      __builtin_amdgcn_sched_group_barrier(0x002, 144 / MFMAS, 0);   // vector instructions
     }
     load_tile(set, kt + 3);
     __syncthreads();
@@ -326,19 +304,56 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[0][t][r] = acc[0][t][r] + acc[1][t][r];
   }
-  // anything the split could not represent: this tile once more, see above
+  // The tile by the binary32 instruction: k tiles of the operands as they are in LDS, depth by depth,
+  // the next k tile requested while one is multiplied.
+  auto again = [&]() __attribute__((always_inline)) {
+    // (opaque, so that nothing made up for this rare pass is kept in registers through the main loop)
+    int t = tid, first = 0;
+    asm("" : "+v"(t), "+s"(first));
+    const int am = LK ? t / KC : t % TMT, ac = LK ? t % KC : t / TMT;
+    const int bn = RK ? t / KC : t % TN, bc = RK ? t % KC : t / TN;
+    const bool has_a = TMT * KC == NT || t < TMT * KC;
+    float *const fa = (float *)sA + ac * 8 * PA_ + am, *const fb = (float *)sB + bc * 8 * PB_ + bn;
+    static_assert(sizeof(sA) >= sizeof(float) * BKT * PA_ && sizeof(sB) >= sizeof(float) * BKT * PB_, "a k tile of binary32");
+#pragma unroll
+    for (int t = 0; t < FM * FN; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][t][r] = 0.f;
+    load_tile(set0, first);
+    for (int kt = first; kt < nk; ++kt) {
+      clear_past_depth(set0, kt);
+      __syncthreads();   // (nobody reads the k tile before any more)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (has_a) fa[e * PA_] = xa[0][e];
+        fb[e * PB_] = xb[0][e];
+      }
+      load_tile(set0, kt + 1);
+      __syncthreads();
+      const int depth = min(BKT, kend - kt0 - kt * BKT);
+      for (int k = lane >> 5; k < depth + (lane >> 5); k += 2) {
+        float a[FM], bb[FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i) a[i] = ((const float *)sA)[k * PA_ + wm * 64 + i * 32 + (lane & 31)];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) bb[j] = ((const float *)sB)[k * PB_ + (wn * FN + j) * 32 + (lane & 31)];
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            acc[0][i * FN + j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], bb[j], acc[0][i * FN + j], 0, 0, 0);
+      }
+    }
+  };
   float worst = 0.f;   // not finite if one of the sums is not
 #pragma unroll
   for (int t = 0; t < FM * FN; ++t)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) worst = __fmaf_rn(acc[0][t][r], 0.f, worst);
-  if (__syncthreads_or((lost & 0xffffu) != 0 || worst != 0.f)) {
-    int64_t cols[FN];
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-      cols[j] = col_at(min(n0 + (wn * FN + j) * 32 + (lane & 31), p.N - 1), p.rcs, p.rbs);
-    f32_tile_again<FM, FN>(p, A, B, m0 + wm * 64, cols, kt0, kend, acc[0]);
-  }
+    for (int r = 0; r < 16; ++r) {
+      worst = __fmaf_rn(acc[0][t][r], 0.f, worst);
+      acc[0][t][r] = acc[0][t][r] * SUM_SCALE;
+    }
+  if (__syncthreads_or(worst != 0.f)) again();
 
   const bool raw = p.kt_split != 0;   // a part of the k range: bias and activation come with the sum of the parts
   float *O = (raw ? p.part + (int64_t)blockIdx.y * p.part_stride : p.out) + (int64_t)b * p.obs;

@@ -1,6 +1,7 @@
 """The fp32 GEMM kernels at the edges of their forms: k tiles of 16 and 32 with half a tile at the end,
 guarded depths, 64- and 128-row tiles, columns of a batch run as one long row, parts of the depth; and
-operands that the split into bf16 parts cannot represent, which a tile is computed again for.
+operands that the split into bf16 parts cannot represent, which a tile is computed again for; and operands
+so small that unscaled parts would be subnormal.
 
 Bound: six MFMAs per 16 depths, each rounding the running sum twice (2^-24 of at most sum |a||b|), eight
 products at a time aligned to the largest of them (8 2^-24), left-out products 2^-24 and the split's
@@ -75,27 +76,81 @@ def test_few_tiles_and_a_long_depth(ctx):
     close(*run(ctx, a, b, lb=False), 2064)
 
 
-@pytest.mark.parametrize("m,k,n", [(140, 64, 133), (40, 50, 300)])
-def test_operands_outside_the_split(ctx, m, k, n):
+# (at most one tile per CU; more: 128-row tiles, 64-row tiles with idle loader threads; depths that are not
+# whole k tiles)
+OUTSIDE = [(140, 64, 133), (40, 50, 300), (2304, 32, 2200), (2304, 33, 2200), (2241, 48, 2050), (2241, 19, 2050)]
+
+
+@pytest.mark.parametrize("m,k,n", OUTSIDE)
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_operands_outside_the_split(ctx, m, k, n, ta, tb):
     rng = np.random.default_rng(k)
     a, b = (rng.standard_normal(s).astype(np.float32) for s in ((1, m, k), (1, k, n)))
-    close(*run(ctx, a * np.float32(2.0 ** -120), b * np.float32(2.0 ** 120), False, False), k)   # lo below bf16's smallest
+    form = dict(lb=False, rb=False, ta=ta, tb=tb)
+    close(*run(ctx, a * np.float32(2.0 ** -120), b * np.float32(2.0 ** 120), **form), k)   # scaled past bf16's range
     tiny = a.copy()
     tiny[0, 3] *= np.float32(2.0 ** -140)                  # a row of subnormal numbers
-    close(*run(ctx, tiny, b * np.float32(2.0 ** 90), False, False), k)
+    close(*run(ctx, tiny, b * np.float32(2.0 ** 90), **form), k)
     huge = a.copy()
     huge[0, 5] = 0
     huge[0, 5, 1] = np.finfo(np.float32).max               # hi would round to infinity
-    close(*run(ctx, huge, np.clip(b, -0.9, 0.9), False, False), k)
+    close(*run(ctx, huge, np.clip(b, -0.9, 0.9), **form), k)
     inf = a.copy()
     inf[0, 7, 2] = np.inf
     inf[0, 8, 0] = np.nan
+    inf[0, m - 1, 1] = -np.inf
     bb = b.copy()
     bb[0, 2] = 1.0                                         # exact in bf16: its smaller parts are zeros
-    got, want, _ = run(ctx, inf, bb, False, False)
-    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
-    got, want, size = run(ctx, np.zeros_like(a), b, False, False)
+    got, want, _ = run(ctx, inf, bb, **form)
+    for kind in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(kind(got), kind(want))
+    keep = np.isfinite(want).all(axis=2)[0]
+    close(got[:, keep], want[:, keep], np.matmul(np.abs(a[:, keep]).astype(np.float64), np.abs(bb)), k)
+    got, want, size = run(ctx, np.zeros_like(a), b, **form)
     assert not got.any()
+
+
+@pytest.mark.parametrize("batch,m,k,n", [(40, 48, 33, 100), (300, 130, 64, 132)])
+def test_images_outside_the_split(ctx, batch, m, k, n):
+    """tiles that straddle images are computed again as well"""
+    rng = np.random.default_rng(batch)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((1, m, k), (batch, k, n)))
+    b[:, 1, ::37] = 1e38
+    close(*run(ctx, np.clip(a, -0.9, 0.9), b, lb=False), k)
+
+
+# Relative 2-norm error: a part that the matrix instruction took for zero would show as 2^-18 = 4e-6
+# (lo) or 2^-9 (mid); binary32 sums of these depths measure 1e-7 to 2e-7.
+@pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -105, 2.0 ** -110, 2.0 ** -118, 2.0 ** -126])
+@pytest.mark.parametrize("m,k,n", [(140, 64, 133), (2304, 33, 2200)])
+def test_small_operands_keep_all_their_parts(ctx, scale, m, k, n):
+    rng = np.random.default_rng(k)
+    a = (rng.standard_normal((1, m, k)) * scale).astype(np.float32)
+    b = (rng.standard_normal((1, k, n)) * 2.0 ** 80).astype(np.float32)
+    got, want, _ = run(ctx, a, b, False, False)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
+def test_small_operands_go_at_full_speed(ctx):
+    """the tails of a softmax (down to 1e-45 here) once took seven times as long"""
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((4, 1024, 1024)) * 25
+    soft = np.exp(x - x.max(axis=2, keepdims=True))
+    soft = (soft / soft.sum(axis=2, keepdims=True)).astype(np.float32)
+    assert ((soft > 0) & (soft < 2.0 ** -112)).any(axis=2).mean() > 0.01
+    b = rng.standard_normal((4, 1024, 1024)).astype(np.float32)
+    times = []
+    for a in (x.astype(np.float32), soft):
+        d = Dev()
+        pa, pb = d.put(a), d.put(b)
+        _, po = d.empty(4 * 1024 * 1024, np.float32)
+        d.sync()
+        ctx.profile(True)
+        for _ in range(20):
+            ctx.call("mace_hip_gemm_f32", pa, pb, 4, 1024, 1024, 1024, 0, 0, 0, 1, 1, po)
+        times.append(min(ctx.kernel_ms_list()))
+        ctx.profile(False)
+    assert times[1] < 2 * times[0], times
 
 
 def test_joined_images_captured_without_scratch():
