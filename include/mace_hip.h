@@ -128,7 +128,7 @@ enum {
   MACE_HIP_KF_Q8_GEMV_GENERAL,       /* q8_gemv_kernel: any width and alignment                   */
   MACE_HIP_KF_F32_GEMM_VEC,          /* f32_gemm_vec_kernel: 16-byte loads, fp32 MFMA             */
   MACE_HIP_KF_F32_GEMM_GENERAL,      /* f32_gemm_kernel: bounds-checked                           */
-  MACE_HIP_KF_F32_GEMM_FILL,         /* depth 0: the epilogue alone                               */
+  MACE_HIP_KF_F32_GEMM_FILL,         /* depths 0 to 2: multiply-adds, element by element          */
   MACE_HIP_KF_F32_GEMV_VEC,          /* f32_gemv_vec_kernel                                       */
   MACE_HIP_KF_F32_GEMV_GENERAL,      /* f32_gemv_kernel                                           */
   MACE_HIP_KF_Q8_CONV_SHORT,         /* q8_conv_short_kernel: patches of at most 32 bytes        */

@@ -73,14 +73,16 @@ __device__ inline float apply_act(float v, int act, float limit) {
 // lo = x - hi - mid; x - hi has at most 16 significant bits, what mid leaves of it at most 7.  Of the
 // nine products of two such sums the kernels form the six largest and leave out mid lo, lo mid and
 // lo lo: with |mid| <= 2^-8 |x| and |lo| <= 2^-17 |x| (to nearest, so of either sign) that is at most
-// 2^-24 |a b| and half a unit in the last place of the product, less than the rounding a binary32
-// multiply-add makes anyway.  The six go into one binary32 accumulator, sixteen depths per
-// instruction, so the running sum is rounded less often than with two depths per instruction: the
-// 2-norm error against binary64 measures 1.9e-7 where the binary32 instruction's was 4.1e-7 (4 x
-// 1024^3, normal operands; a 512-channel convolution, four wavefronts: 2.4e-7 and 2.9e-7).  In time, 4 x
-// 1024^3 against transposed weights 86.0 -> 51.3 us, MobileNet's five pointwise layers at batch 64
-// 688 -> 318 us; the matrix cores are busy 35 - 45 % of it, the rest is each k tile's chain of LDS
-// reads, MFMAs, LDS writes and barrier (one to three workgroups per CU overlap).
+// 2^-24 |a b|.  The six go into one binary32 accumulator, sixteen depths per instruction, so the running
+// sum is rounded less often than with two depths per instruction.  2-norm error against binary64, the
+// binary32 instruction's first: 4 x 1024^3, normal operands, 4.1e-7 and 1.9e-7; 2304 x 2200 outputs (four
+// wavefronts) 1.0e-7 and 6.9e-8 at depth 32, 7.4e-8 and 3.4e-8 at 16, 3.6e-8 and 3.3e-8 at 3, 3.1e-8 and
+// 3.4e-8 at 2.  One product alone is off by up to 0.9 units in the last place with eight wavefronts and 1.4
+// with four, where the binary32 instruction rounds it to nearest: depths 1 and 2 go to f32_fill_kernel
+// for that.  (Rows with one entry other than zero keep it; where that entry is a power of two the product
+// is exact.)  In time, 4 x 1024^3 against transposed weights 86.0 -> 51.3 us, MobileNet's five pointwise layers
+// at batch 64 688 -> 318 us; the matrix cores are busy 35 - 45 % of it, the rest is each k tile's chain of
+// LDS reads, MFMAs, LDS writes and barrier (one to three workgroups per CU overlap).
 //
 // Both operands are multiplied by 2^23 before the split and the sums by 2^-46 behind it, all exact: the
 // last bit of the smallest subnormal number then lies at 2^-126, so every part of every number is a
@@ -404,18 +406,75 @@ __global__ __launch_bounds__(256 * SPLIT, SPLIT == 2 ? 1 : (GUARD && TMT == 128 
   f32_tile<LK, RK, SPLIT, GUARD, TMT>(p);
 }
 
-// depth == 0: the reference's loop leaves sum = 0
-__global__ void f32_fill_kernel(F32GemmParams p, int64_t total) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t bm = i / p.N;
-    const int m = (int)(bm % p.M);
-    float v = 0.f;
-    if (p.bias_row) v = v + p.bias_row[m];
-    const int64_t bb = bm / p.M;
-    const int n = (int)(i - bm * p.N);
-    if (p.bias_col) v = v + p.bias_col[n];
-    p.out[bb * p.obs + (int64_t)m * p.ors + (int64_t)n * p.ocs] = apply_act(v, p.act, p.limit);
+// Depths of at most two: 0 (the reference's loop leaves sum = 0), and 1 and 2 by binary32 multiply-adds,
+// because the tile kernels' products are not rounded to nearest (see there).  Bound by the stores: four
+// neighbouring outputs per thread, so that divisions and loads are shared.  Against the tile kernels:
+// 4096 x 1 x 4096 28.0 -> 16.6 us (column-major result 46.8 -> 16.6), two depths 28.1 -> 17.2.
+template <typename Index>
+__global__ __launch_bounds__(256) void f32_fill_kernel(F32GemmParams p, Index total) {
+  // outputs in memory order: `in` runs fastest (columns of a row-major result, rows of a column-major one)
+  const bool along_n = p.ocs == 1;
+  const Index inner = (Index)(along_n ? p.N : p.M), outer = (Index)(along_n ? p.M : p.N);
+  const float *const x = along_n ? p.rhs : p.lhs, *const y = along_n ? p.lhs : p.rhs;
+  const int64_t xs = along_n ? p.rcs : p.lrs, ys = along_n ? p.lrs : p.rcs;
+  const int64_t xk = along_n ? p.rrs : p.lcs, yk = along_n ? p.lcs : p.rrs;
+  const int64_t xb = along_n ? p.rbs : p.lbs, yb = along_n ? p.lbs : p.rbs;
+  const float *const bias_in = along_n ? p.bias_col : p.bias_row, *const bias_out = along_n ? p.bias_row : p.bias_col;
+  const Index units = (total + 3) / 4;
+  for (Index u = (Index)blockIdx.x * 256 + threadIdx.x; u < units; u += (Index)gridDim.x * 256) {
+    const Index i = u * 4, line = i / inner;
+    Index in = i - line * inner, b = line / outer, out = line - b * outer;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    if (in + 4 <= inner) {   // four of one line: one factor of each product is the same, the others lie side by side
+      const float *const px = x + (int64_t)b * xb + (int64_t)in * xs, *const py = y + (int64_t)b * yb + (int64_t)out * ys;
+      if (p.K > 0) {
+        float f[2][4] = {};
+        if (xs == 1) {
+          __builtin_memcpy(f[0], px, 16);
+          if (p.K > 1) __builtin_memcpy(f[1], px + xk, 16);
+        } else {               // (two depths side by side)
+          float pair[8];
+          __builtin_memcpy(pair, px, 32);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { f[0][e] = pair[2 * e]; f[1][e] = pair[2 * e + 1]; }
+        }
+        const float y0 = py[0], y1 = p.K > 1 ? py[yk] : 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = __fmaf_rn(f[0][e], y0, v[e]);
+          if (p.K > 1) v[e] = __fmaf_rn(f[1][e], y1, v[e]);
+        }
+      }
+      const float bo = bias_out ? bias_out[out] : 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {   // (a call has one bias or none)
+        if (bias_in) v[e] = v[e] + bias_in[in + e];
+        if (bias_out) v[e] = v[e] + bo;
+        v[e] = apply_act(v[e], p.act, p.limit);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (i + e >= total) break;
+        const float *const px = x + (int64_t)b * xb + (int64_t)in * xs, *const py = y + (int64_t)b * yb + (int64_t)out * ys;
+        if (p.K > 0) v[e] = __fmaf_rn(px[0], py[0], v[e]);
+        if (p.K > 1) v[e] = __fmaf_rn(px[xk], py[yk], v[e]);
+        if (bias_in) v[e] = v[e] + bias_in[in];
+        if (bias_out) v[e] = v[e] + bias_out[out];
+        v[e] = apply_act(v[e], p.act, p.limit);
+        if (++in == inner) {
+          in = 0;
+          if (++out == outer) { out = 0; ++b; }
+        }
+      }
+    }
+    if (i + 4 <= total) {
+      __builtin_memcpy(p.out + i, v, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (i + e < total) p.out[i + e] = v[e];
+    }
   }
 }
 
@@ -558,10 +617,12 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
   p.M = (int)rows; p.N = (int)cols; p.K = (int)depth;
   p.bias_row = ep.bias_row; p.bias_col = ep.bias_col; p.act = ep.act; p.limit = ep.limit;
   const int64_t total = batch * rows * cols;
-  if (depth == 0) {
-    mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_FILL, 0, dim3(1), dim3(256), 0);
-    MH_KLAUNCH(ctx, f32_fill_kernel, dim3((unsigned)((total + 255) / 256 > 65535 ? 65535 : (total + 255) / 256)),
-                       dim3(256), 0, ctx->stream, p, total);
+  if (depth <= 2) {
+    dim3 grid((unsigned)std::min<int64_t>((total + 1023) / 1024, 65535));
+    mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_FILL, 0, grid, dim3(256), 0);
+    // (32-bit divisions where they do; the last stride past the end must not wrap either)
+    if (total < (1ll << 31)) MH_KLAUNCH(ctx, f32_fill_kernel<uint32_t>, grid, dim3(256), 0, ctx->stream, p, (uint32_t)total);
+    else MH_KLAUNCH(ctx, f32_fill_kernel<int64_t>, grid, dim3(256), 0, ctx->stream, p, total);
     MH_LAUNCH_CHECK(ctx);
     return MACE_HIP_SUCCESS;
   }

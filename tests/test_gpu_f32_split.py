@@ -192,3 +192,43 @@ def test_joined_images_captured_without_scratch():
         c.call("mace_hip_graph_destroy", g)
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("lm,rm,om", [(0, 0, 0), (0, 1, 1), (1, 0, 1), (1, 1, 0)])
+@pytest.mark.parametrize("k", [1, 2])
+@pytest.mark.parametrize("batch,m,n,lb", [(1, 300, 257, 1), (3, 70, 129, 1), (70, 1, 1001, 0), (3, 1001, 1, 1), (5, 1, 1, 1), (2, 64, 128, 1)])
+def test_one_or_two_products_per_output(ctx, batch, m, n, lb, k, lm, rm, om):
+    """as binary32 multiply-adds round them: one product once, two products twice"""
+    rng = np.random.default_rng(m + n)
+
+    def some(*shape):
+        return (rng.standard_normal(shape) * 2.0 ** rng.integers(-60, 60, shape)).astype(np.float32)
+    a, b = some(batch if lb else 1, m, k), some(batch, k, n)
+    d = Dev()
+    pa = d.put(a.transpose(0, 2, 1) if lm else a)
+    pb = d.put(b.transpose(0, 2, 1) if rm else b)
+    t, po = d.empty(batch * m * n, np.float32)
+    d.sync()
+    ctx.call("mace_hip_gemm_f32", pa, pb, batch, m, n, k, lm, rm, om, lb, 1, po)
+    ctx.sync()
+    got = t.cpu().numpy()
+    got = got.reshape(batch, n, m).transpose(0, 2, 1) if om else got.reshape(batch, m, n)
+    first = a[:, :, :1] * b[:, :1]
+    if k == 1:
+        assert np.array_equal(got, first)
+    else:      # (binary64 holds the second product exactly; its sum with the first is rounded twice)
+        want = first.astype(np.float64) + a[:, :, 1:].astype(np.float64) * b[:, 1:]
+        assert np.all(np.abs(got - want) <= 0.5001 * np.spacing(np.abs(want).astype(np.float32)))
+
+
+def test_one_product_per_output_with_bias_and_activation(ctx):
+    rng = np.random.default_rng(2)
+    x, f, bias = (rng.standard_normal(s).astype(np.float32) for s in ((3, 1, 50), (40, 1), (40,)))
+    d = Dev()
+    px, pf, pb = d.put(x), d.put(f), d.put(bias)
+    t, po = d.empty(3 * 40 * 50, np.float32)
+    d.sync()
+    ctx.call("mace_hip_conv1x1_f32_nchw", px, pf, pb, 3, 1, 50, 40, mh.ACT_RELUX, 1.5, po)
+    ctx.sync()
+    want = np.clip(f[None] * x + bias[None, :, None], 0, np.float32(1.5))
+    assert np.array_equal(t.cpu().numpy().reshape(3, 40, 50), want)
