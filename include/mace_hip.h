@@ -126,8 +126,8 @@ enum {
   MACE_HIP_KF_Q8_GEMV_MFMA,          /* q8_gemv_mfma_kernel: rows too wide for LDS                */
   MACE_HIP_KF_Q8_GEMV_ROWS,          /* q8_gemv_rows_kernel: vectors of one pass in LDS           */
   MACE_HIP_KF_Q8_GEMV_GENERAL,       /* q8_gemv_kernel: any width and alignment                   */
-  MACE_HIP_KF_F32_GEMM_VEC,          /* f32_gemm_vec_kernel: 16-byte loads, fp32 MFMA             */
-  MACE_HIP_KF_F32_GEMM_GENERAL,      /* f32_gemm_kernel: bounds-checked                           */
+  MACE_HIP_KF_F32_GEMM_VEC,          /* f32_gemm_vec_kernel: fp32 by bf16 MFMAs, see f32_gemm.hip */
+  MACE_HIP_KF_F32_GEMM_GENERAL,      /* f32_gemm_kernel: the same for any length and alignment    */
   MACE_HIP_KF_F32_GEMM_FILL,         /* depths 0 to 2: multiply-adds, element by element          */
   MACE_HIP_KF_F32_GEMV_VEC,          /* f32_gemv_vec_kernel                                       */
   MACE_HIP_KF_F32_GEMV_GENERAL,      /* f32_gemv_kernel                                           */
@@ -234,13 +234,12 @@ uint8_t mace_hip_quantize_u8(float value, float scale, int32_t zero_point);
  * gemmlowp quantize-down-by-fixed-point + saturating cast (see mace_hip_gemm_q8_u8). */
 uint8_t mace_hip_requant_fixed_u8(int32_t acc, int32_t multiplier, int right_shift,
                                   int32_t offset_after_shift, int clamp_min, int clamp_max);
-/* The same pipeline in the form the GEMM kernels use for their uint8 stores, evaluated on the
- * host for CPU-side tests: the pipeline is a non-decreasing step function of the accumulator,
- * so the kernels locate the step with one float multiply-add and one comparison against a
- * table of exact thresholds.  Returns 1 when that form applies to the parameters, 0 when the
- * kernels fall back to the arithmetic of mace_hip_requant_fixed_u8 (non-positive multiplier,
- * clamp window further than 2^15 from the offset), -1 on invalid arguments; *out is the
- * requantized value in the first two cases. */
+/* The same pipeline in the form the GEMM and convolution kernels use for their uint8 stores, evaluated
+ * on the host for CPU-side tests: one 64-bit multiply-add and a shift per accumulator.  Returns 1 when
+ * that form applies to the parameters, 0 when the kernels take the arithmetic of
+ * mace_hip_requant_fixed_u8 (multiplier below 1, clamp window further than 2^15 from the offset), -1 on
+ * invalid arguments; *out is the requantized value in the first two cases.  (The name is that of an
+ * earlier form, a table of thresholds.) */
 int mace_hip_requant_table_u8(int32_t acc, int32_t multiplier, int right_shift,
                               int32_t offset_after_shift, int clamp_min, int clamp_max,
                               uint8_t *out);

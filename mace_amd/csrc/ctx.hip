@@ -561,14 +561,8 @@ int mace_hip_requant_table_u8(int32_t acc, int32_t multiplier, int right_shift,
     *out = (uint8_t)requant_mad_one(acc, requant_mad(q));
     return 1;
   }
-  if (!q.table) {
-    *out = (uint8_t)mh_requant_fixed(acc, q);
-    return 0;
-  }
-  int32_t tab[MH_REQUANT_TABLE_MAX];
-  for (int j = 0; j <= q.n + 1; ++j) tab[j] = mh_requant_table_entry(q, j);
-  *out = (uint8_t)(q.lo + mh_requant_step(acc, q, tab));
-  return 1;
+  *out = (uint8_t)mh_requant_fixed(acc, q);
+  return 0;
 }
 
 uint8_t mace_hip_requant_float_u8(int32_t acc, float multiplier, int32_t out_zp, int mode) {

@@ -133,18 +133,6 @@ __device__ inline int sum16_i8(const v4i &f, int acc) {
   return acc;
 }
 
-// The comparison table's first halves follow GemmParams in the argument segment (indexing a
-// by-value copy with a lane-dependent index would spill it).  Needed only by calls outside the
-// multiply-add form.
-__device__ inline void stage_requant_pairs(int32_t *pairs, const RequantFixed &rq, int tid,
-                                           int nthreads) {
-  static_assert(sizeof(GemmParams) % alignof(RequantTable) == 0, "argument layout");
-  if (!rq.table || requant_by_mad(rq)) return;   // (the same for every thread)
-  stage_requant_pairs_from((const int32_t *)((const char *)__builtin_amdgcn_kernarg_segment_ptr() +
-                                             sizeof(GemmParams)),
-                           pairs, rq, tid, nthreads);
-}
-
 // Epilogue shared by the GEMM kernels: adds the correction vectors to the accumulators and
 // stores int32 results or requantized bytes.  Accumulator register r of a 32x32 tile holds
 //   x (MFMA row)    = 8 * (r / 4) + 4 * (lane / 32) + r % 4
@@ -157,8 +145,8 @@ __device__ inline void stage_requant_pairs(int32_t *pairs, const RequantFixed &r
 // x 1500 x 777 33.6 -> 25.4 (int32) and 32.4 -> 24.1 (uint8); rows of whole dwords, 2044 columns, 11.7 ->
 // 11.2.  The correction vectors of the tile are staged through LDS first (the
 // operand buffers are dead by then), so the stores do not wait on scattered global loads.
-// PRESTAGED: the caller has already put the tile's x correction terms and the comparison table
-// into `lds` (same layout) and synchronised the workgroup.
+// PRESTAGED: the caller has already put the tile's x correction terms into `lds` (same layout) and
+// synchronised the workgroup.
 template <int WX, int WY, int FX, int FY, typename OutT, bool SUMY, bool PRESTAGED = false>
 __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&ysum)[FY],
                                      const GemmParams &p, uint8_t *lds, int b, int x0, int y0,
@@ -170,8 +158,6 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
   const int32_t *cY = p.corrY + (int64_t)b * p.cybs;
   int32_t *sc = (int32_t *)lds;   // [TX] corrections along x, then [TY] along y
   const RequantFixed rq = p.rq;
-  static_assert((TX + TY) % 2 == 0, "the table entries are read as 8-byte pairs");
-  int32_t *tab = sc + TX + TY;    // [n + 1] 8-byte entries of the threshold requantization
   if constexpr (!PRESTAGED) {
   __syncthreads();                // every wavefront is done reading operand tiles
   // panel sums -> correction terms: coef * sum + add (+ bias on the side the result rows are on)
@@ -188,22 +174,18 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
       if (p.ybias) c += (uint32_t)p.ybias[y];
       sc[TX + i] = (int32_t)c;
     }
-  if constexpr (sizeof(OutT) == 1) {
-    stage_requant_pairs(tab, rq, tid, NT);
-  }
   __syncthreads();
   }
 
   OutT *outb = (OutT *)p.out + (int64_t)b * p.obs;
   const bool interior16 = x0 + TX <= p.XN && y0 + TY <= p.YN && p.ldo % 16 == 0 && (uintptr_t)outb % 16 == 0;
 
-  const RequantLds rql = requant_lds(rq, tab);
   const bool by_mad = requant_by_mad(rq);
   RequantMad rqm{};
   if (by_mad) rqm = requant_mad(rq);
   // One fully unrolled copy of the store loop per combination that occurs: MAD = requantization by
   // multiply-add, WIDE = whole tile inside the matrix and 16-byte aligned rows.  Parameters outside
-  // the multiply-add form share one copy, by table or by the plain arithmetic.
+  // the multiply-add form take the plain arithmetic.
   auto store_tile = [&](auto mad_tag, auto wide_tag) __attribute__((always_inline)) {
     constexpr bool MAD = decltype(mad_tag)::value;
     constexpr bool WIDE = decltype(wide_tag)::value;
@@ -254,8 +236,6 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
           uint32_t packed[4] = {0, 0, 0, 0};
           if constexpr (MAD) {
             requant_16_by_mad(v, rqm, packed);
-          } else if (rq.table) {
-            requant_16_by_table(v, rql, packed);
           } else {
 #pragma unroll
             for (int r = 0; r < 16; ++r)
@@ -296,7 +276,7 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[FX][FY], const int (&y
 }
 
 template <int WX, int WY, int FX, int FY, typename OutT, bool SUMY = false>
-__global__ __launch_bounds__(WX *WY * 64) void q8_gemm_kernel(GemmParams p, RequantTable) {
+__global__ __launch_bounds__(WX *WY * 64) void q8_gemm_kernel(GemmParams p) {
   constexpr int NT = WX * WY * 64;
   constexpr int TX = WX * FX * 32;
   constexpr int TY = WY * FY * 32;
@@ -463,10 +443,10 @@ __global__ __launch_bounds__(WX *WY * 64) void q8_gemm_kernel(GemmParams p, Requ
 // (MobileNet's first convolution at batch 64: 79 us at five wavefronts, 92 at four).  The same bound
 // on the other instantiations makes the k-major ones spill.
 template <typename OutT, bool XT, bool YT, bool BW>
-__global__ __launch_bounds__(256, BW ? 5 : 1) void q8_gemm_fused_small_kernel(GemmParams p, RequantTable) {
+__global__ __launch_bounds__(256, BW ? 5 : 1) void q8_gemm_fused_small_kernel(GemmParams p) {
   constexpr int T = 64;
   __shared__ __align__(16) uint8_t tile[2][T * LDS_ROW];   // X rows, Y rows: [row][k], sign-flipped
-  __shared__ __align__(16) int32_t sc[2 * T + MH_REQUANT_PAIRS_BYTES / 4];
+  __shared__ __align__(16) int32_t sc[2 * T];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -639,11 +619,8 @@ __global__ __launch_bounds__(256, BW ? 5 : 1) void q8_gemm_fused_small_kernel(Ge
   const uint8_t *fx = tile[0] + wx * 32 * LDS_ROW + frag;
   const uint8_t *fy = tile[1] + wy * 32 * LDS_ROW + frag;
 
-  // Everything the epilogue needs from memory is asked for now, so that it arrives under the
-  // operand loads: the comparison table (into LDS) and this lane's bias.
-  if constexpr (sizeof(OutT) == 1) {
-    stage_requant_pairs(sc + 2 * T, p.rq, tid, 256);
-  }
+  // This lane's bias, all that the epilogue needs from memory, is asked for now, so that it arrives
+  // under the operand loads.
   const int32_t xbias = p.xbias ? p.xbias[min(x0 + wx * 32 + (lane & 31), p.XN - 1)] : 0;
 
   // NPRE k tiles of both operands are in flight at a time: with only a few tiles in all, what a
@@ -679,7 +656,7 @@ __global__ __launch_bounds__(256, BW ? 5 : 1) void q8_gemm_fused_small_kernel(Ge
     }
   }
 
-  // x corrections of the tile and the comparison table -> LDS; y corrections come from ys
+  // x corrections of the tile -> LDS; y corrections come from ys
   xs += __shfl_xor(xs, 32, 64);
   if (wy == 0 && lane < 32) {
     const int xl = wx * 32 + lane;
@@ -777,7 +754,7 @@ __device__ inline void wait_vmcnt() {
 template <int WX, int WY, int FX, int FY, int STAGES, typename OutT, int OCC = 1,
           bool SUMY = false, bool CONV = false, int KB = SLAB, bool XT = false, bool XF = false,
           bool SUMX = false>
-__global__ __launch_bounds__(WX *WY * 64, OCC) void q8_gemm_dma_kernel(GemmParams p, RequantTable) {
+__global__ __launch_bounds__(WX *WY * 64, OCC) void q8_gemm_dma_kernel(GemmParams p) {
   static_assert(!SUMX || !XF, "a panel written already shifted comes with its sums");
   constexpr int NW = WX * WY;
   constexpr int TX = WX * FX * 32;
@@ -1077,8 +1054,8 @@ __global__ __launch_bounds__(WX *WY * 64, OCC) void q8_gemm_dma_kernel(GemmParam
   }
 
   if constexpr (SUMX) {
-    // x terms from the sums taken here (both wavefront rows hold them; wy == 0 writes), y terms and
-    // the comparison table staged as the epilogue would, then the epilogue on what is in LDS
+    // x terms from the sums taken here (both wavefront rows hold them; wy == 0 writes) and y terms
+    // staged as the epilogue would, then the epilogue on what is in LDS
 #pragma unroll
     for (int i = 0; i < FX; ++i) xsum[i] -= sum16_u8(a0[i] ^ flip, 0) + 64 * p.K;
     __syncthreads();   // every wavefront is done reading operand tiles, every transfer has landed
@@ -1101,9 +1078,6 @@ __global__ __launch_bounds__(WX *WY * 64, OCC) void q8_gemm_dma_kernel(GemmParam
         if (p.ybias) c += (uint32_t)p.ybias[y];
         sc[TX + i] = (int32_t)c;
       }
-    }
-    if constexpr (sizeof(OutT) == 1) {
-      stage_requant_pairs(sc + TX + TY, p.rq, tid, NW * 64);
     }
     __syncthreads();
     gemm_epilogue<WX, WY, FX, FY, OutT, SUMY, true>(acc, ysum, p, lds, b, x0, y0, wx, wy, tid);
@@ -1151,7 +1125,7 @@ __global__ __launch_bounds__(WX *WY * 64, OCC) void q8_gemm_dma_kernel(GemmParam
 // Requirements (checked by the host): K % 128 == 0, rows addressable with 32-bit offsets; XT / YT:
 // XN / YN a multiple of 16, 16-byte aligned base, the whole operand within 32-bit offsets.
 template <typename OutT, int STAGES, bool XT, bool YT = false>
-__global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p, RequantTable) {
+__global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p) {
   constexpr int KB = 128, T = 128, NW = 8;
   constexpr int RPI = 1024 / KB, CPR = KB / 16;
   constexpr int NL = 2 * T / RPI / NW;            // transfers per wavefront per slab
@@ -1354,7 +1328,7 @@ __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p, Requa
   // the other half to the wavefront of the other group on the same SIMD.
   wait_vmcnt<0>();
   __syncthreads();
-  int32_t *sc = (int32_t *)lds;                       // [T] x terms, [T] y terms, then the table
+  int32_t *sc = (int32_t *)lds;                       // [T] x terms, [T] y terms
   int32_t *part = (int32_t *)(lds + 16384);           // [4][T] partial X sums, [4][T] partial Y sums
   int32_t *ex = (int32_t *)(lds + 32768);             // [8 wavefronts][32 registers][64 lanes]
 #pragma unroll
@@ -1380,9 +1354,6 @@ __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p, Requa
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mine[(j * 16 + r) * 64] = acc[0][j][r];
-    }
-    if constexpr (sizeof(OutT) == 1) {
-      stage_requant_pairs(sc + 2 * T, p.rq, tid, 512);
     }
     __syncthreads();
 #pragma unroll
@@ -1433,9 +1404,9 @@ __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p, Requa
 // share of the group from the tap's pixel, or from a buffer of zero-point bytes where the tap
 // falls into the padding.
 //
-// LDS: [0, 3072): x correction terms [TX], unused [32 FY], comparison table (the layout
-// gemm_epilogue expects); then K/64 slabs of TX rows x 64 bytes, 16-byte chunk c of row r in
-// slot c ^ ((r >> 2) & 3) as in q8_gemm_dma_kernel.
+// LDS: [0, 3072): x correction terms [TX], unused [32 FY] (the layout gemm_epilogue expects) and room
+// to spare, with which the bounds on the depth were measured (the tile twice per CU); then K/64 slabs of
+// TX rows x 64 bytes, 16-byte chunk c of row r in slot c ^ ((r >> 2) & 3) as in q8_gemm_dma_kernel.
 // Requirements (checked by the host): K % G == 0, 2048 + TX K bytes of LDS available.
 constexpr int XRES_SC_BYTES = 3072;
 // 16 x 16 bytes held as 16 rows of 16 bytes, transposed in place (v_perm_b32: 4 x 4 byte blocks
@@ -1467,13 +1438,13 @@ __device__ __forceinline__ void transpose_16x16_bytes(v4i (&r)[16]) {
 // aligned.
 template <int FX, int FY, int G, typename OutT, int OCC, bool CONV = false, bool XT = false,
           bool TAIL = false>
-__global__ __launch_bounds__(256, OCC) void q8_gemm_xres_kernel(GemmParams p, RequantTable) {
+__global__ __launch_bounds__(256, OCC) void q8_gemm_xres_kernel(GemmParams p) {
   static_assert(!TAIL || (!CONV && !XT && G == 64), "the depth tail: plain operands, 64-byte groups");
   constexpr int TX = FX * 32, TYW = FY * 32;
   constexpr int KPG = G / 32;   // k steps per group
   static_assert(G == 64 || G == 128, "group width");
   static_assert(TX == 64 || TX == 128, "X tile rows");
-  static_assert((TX + TYW) * 4 + MH_REQUANT_PAIRS_BYTES <= XRES_SC_BYTES, "correction area");
+  static_assert((TX + TYW) * 4 <= XRES_SC_BYTES, "correction area");
   extern __shared__ __align__(16) uint8_t lds[];
   int32_t *sc = (int32_t *)lds;
   uint8_t *xt = lds + XRES_SC_BYTES;
@@ -1496,7 +1467,6 @@ __global__ __launch_bounds__(256, OCC) void q8_gemm_xres_kernel(GemmParams p, Re
   const int b = wg / (gridDim.y * gridDim.x);
   const uint8_t *Xb = p.X + (int64_t)b * p.xbs;
   const uint8_t *Yb = p.Y + (int64_t)b * p.ybs;
-  const RequantFixed rq = p.rq;
   const v4i flip = {(int)0x80808080, (int)0x80808080, (int)0x80808080, (int)0x80808080};
 
   const int nblk = (p.YN + TYW - 1) / TYW;
@@ -1604,9 +1574,6 @@ __global__ __launch_bounds__(256, OCC) void q8_gemm_xres_kernel(GemmParams p, Re
       if (p.xbias) c += (uint32_t)p.xbias[x];
       sc[i] = (int32_t)c;
     }
-    if constexpr (sizeof(OutT) == 1) {
-      stage_requant_pairs(sc + TX + TYW, rq, tid, 256);
-    }
     __syncthreads();
   } else {
     // X tile -> LDS: one transfer instruction moves 16 rows x 64 bytes
@@ -1667,9 +1634,6 @@ __global__ __launch_bounds__(256, OCC) void q8_gemm_xres_kernel(GemmParams p, Re
       uint32_t c = (uint32_t)p.xcoef * (uint32_t)xs + (uint32_t)p.xadd;
       if (p.xbias) c += (uint32_t)p.xbias[x];
       sc[row] = (int32_t)c;
-    }
-    if constexpr (sizeof(OutT) == 1) {
-      stage_requant_pairs(sc + TX + TYW, rq, tid, 256);
     }
     __syncthreads();
   }
@@ -2189,7 +2153,7 @@ int launch_kmajor_sums(mace_hip_ctx *ctx, const uint8_t *P, int64_t ld, int64_t 
 }
 
 template <int WX, int WY, int FX, int FY>
-int launch_gemm(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, bool out_u8,
+int launch_gemm(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
                 int batch) {
   constexpr int TX = WX * FX * 32, TY = WY * FY * 32;
   p.tiles_x = (p.XN + TX - 1) / TX;
@@ -2202,7 +2166,7 @@ int launch_gemm(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, bool 
   auto launch = [&](auto k) -> int {
     if (lds > 64 * 1024) MH_HIP(ctx, mh_allow_big_lds(ctx, (const void *)k, lds));
     MH_PROF_BEGIN(ctx);
-    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p, tab);
+    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p);
     return MACE_HIP_SUCCESS;
   };
   if (out_u8 && p.sum_y) {
@@ -2221,7 +2185,7 @@ int launch_gemm(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, bool 
 
 // the streaming kernel; the caller has checked K % 64 == 0 and K >= 64 * (STAGES - 1)
 template <int WX, int WY, int FX, int FY, int STAGES, int OCC, int KB = SLAB>
-int launch_gemm_dma(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, bool out_u8,
+int launch_gemm_dma(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
                     int batch) {
   constexpr int TX = WX * FX * 32, TY = WY * FY * 32;
   p.tiles_x = (p.XN + TX - 1) / TX;
@@ -2235,7 +2199,7 @@ int launch_gemm_dma(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, b
   auto launch = [&](auto k) -> int {
     if (lds > 64 * 1024) MH_HIP(ctx, mh_allow_big_lds(ctx, (const void *)k, lds));
     MH_PROF_BEGIN(ctx);
-    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p, tab);
+    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p);
     return MACE_HIP_SUCCESS;
   };
   if constexpr (KB == SLAB) {
@@ -2262,7 +2226,7 @@ int launch_gemm_dma(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, b
 }
 
 // one round of 128 x 128 tiles; the caller has checked K % 128 == 0 and the 32-bit row offsets
-int launch_gemm_mid(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, bool out_u8, int batch,
+int launch_gemm_mid(mace_hip_ctx *ctx, GemmParams &p, bool out_u8, int batch,
                     bool xt = false, bool yt = false) {
   constexpr int STAGES = 4;
   p.tiles_x = (p.XN + 127) / 128;
@@ -2273,7 +2237,7 @@ int launch_gemm_mid(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, b
   auto launch = [&](auto k) -> int {
     MH_HIP(ctx, mh_allow_big_lds(ctx, (const void *)k, lds));
     MH_PROF_BEGIN(ctx);
-    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p, tab);
+    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p);
     return MACE_HIP_SUCCESS;
   };
   if (yt) {
@@ -2297,7 +2261,7 @@ int launch_gemm_mid(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, b
 }
 
 // 256 x 256 tiles, X operand k-major in memory; the caller has checked the preconditions
-int launch_gemm_big_xt(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, bool out_u8,
+int launch_gemm_big_xt(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
                        int batch, bool sum_x) {
   p.tiles_x = (p.XN + 255) / 256;
   p.tiles_y = (p.YN + 255) / 256;
@@ -2307,7 +2271,7 @@ int launch_gemm_big_xt(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab
   auto launch = [&](auto k) -> int {
     MH_HIP(ctx, mh_allow_big_lds(ctx, (const void *)k, lds));
     MH_PROF_BEGIN(ctx);
-    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p, tab);
+    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p);
     return MACE_HIP_SUCCESS;
   };
 #define MH_XT(OUT_, SY_, SX_) \
@@ -2330,7 +2294,7 @@ int launch_gemm_big_xt(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab
 }
 
 // 256 x 256 tiles, X panel repacked already shifted to int8; the caller has checked the preconditions
-int launch_gemm_big_xf(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, bool out_u8,
+int launch_gemm_big_xf(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
                        int batch) {
   p.tiles_x = (p.XN + 255) / 256;
   p.tiles_y = (p.YN + 255) / 256;
@@ -2340,7 +2304,7 @@ int launch_gemm_big_xf(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab
   auto launch = [&](auto k) -> int {
     MH_HIP(ctx, mh_allow_big_lds(ctx, (const void *)k, lds));
     MH_PROF_BEGIN(ctx);
-    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p, tab);
+    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p);
     return MACE_HIP_SUCCESS;
   };
   if (out_u8 && p.sum_y) {
@@ -2358,7 +2322,7 @@ int launch_gemm_big_xf(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab
 }
 
 // the one-launch kernel for small problems; the caller has checked its preconditions
-int launch_gemm_fused_small(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, bool out_u8,
+int launch_gemm_fused_small(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
                             bool xt, bool yt, int batch) {
   p.tiles_x = (p.XN + 63) / 64;
   p.tiles_y = (p.YN + 63) / 64;
@@ -2369,10 +2333,10 @@ int launch_gemm_fused_small(mace_hip_ctx *ctx, GemmParams &p, const RequantTable
 #define MH_FUSED(OutT_, XT_, YT_)                                                                 \
   if (bw)                                                                                         \
     MH_KLAUNCH(ctx, (q8_gemm_fused_small_kernel<OutT_, XT_, YT_, true>), grid, block, 0,       \
-                       ctx->stream, p, tab);                                                      \
+                       ctx->stream, p);                                                      \
   else                                                                                            \
     MH_KLAUNCH(ctx, (q8_gemm_fused_small_kernel<OutT_, XT_, YT_, false>), grid, block, 0,      \
-                       ctx->stream, p, tab)
+                       ctx->stream, p)
   switch ((out_u8 ? 4 : 0) | (xt ? 2 : 0) | (yt ? 1 : 0)) {
     case 0: MH_FUSED(int32_t, false, false); break;
     case 1: MH_FUSED(int32_t, false, true); break;
@@ -2391,7 +2355,7 @@ int launch_gemm_fused_small(mace_hip_ctx *ctx, GemmParams &p, const RequantTable
 
 // X panel resident in LDS; the caller has checked the preconditions (see the kernel)
 template <int FX, int FY>
-int launch_gemm_xres(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, bool out_u8,
+int launch_gemm_xres(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
                      int batch, bool xt = false) {
   constexpr int TX = FX * 32, TYW = FY * 32;
   const bool tail = p.K % 64 != 0;   // (a multiple of 16: checked by the caller)
@@ -2415,7 +2379,7 @@ int launch_gemm_xres(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, 
     dim3 grid(wgs, tiles_x, batch), block(256);
     mh_plan_main(ctx, MACE_HIP_KF_Q8_GEMM_XRES, variant, grid, block, lds);
     MH_PROF_BEGIN(ctx);
-    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p, tab);
+    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p);
     MH_PROF_END(ctx);
     MH_LAUNCH_CHECK(ctx);
     return MACE_HIP_SUCCESS;
@@ -2455,17 +2419,17 @@ int launch_gemm_xres(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, 
 // blocks give twice the wavefronts, which measured faster (or equal) from one block per CU up to
 // sixteen (56x56x128 -> 128 at batch 64: 22.2 -> 19.6 us; 4096 x 512 x 1024: 14.3 -> 9.6 us).
 // The gather variant is built for 64-row blocks only (32-row blocks measured within +-5 % there).
-int launch_gemm_xres_any(mace_hip_ctx *ctx, GemmParams &p, const RequantTable &tab, bool out_u8,
+int launch_gemm_xres_any(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
                          int batch, int tx, bool xt) {
   const int64_t blocks64 = (int64_t)((p.XN + tx - 1) / tx) * ((p.YN + 63) / 64) * batch;
   const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
   const bool fy1 = !p.conv && blocks64 > cus && blocks64 < 16 * cus;
   if (tx == 64) {
-    if (fy1) return launch_gemm_xres<2, 1>(ctx, p, tab, out_u8, batch, xt);
-    return launch_gemm_xres<2, 2>(ctx, p, tab, out_u8, batch, xt);
+    if (fy1) return launch_gemm_xres<2, 1>(ctx, p, out_u8, batch, xt);
+    return launch_gemm_xres<2, 2>(ctx, p, out_u8, batch, xt);
   }
-  if (fy1) return launch_gemm_xres<4, 1>(ctx, p, tab, out_u8, batch, xt);
-  return launch_gemm_xres<4, 2>(ctx, p, tab, out_u8, batch, xt);
+  if (fy1) return launch_gemm_xres<4, 1>(ctx, p, out_u8, batch, xt);
+  return launch_gemm_xres<4, 2>(ctx, p, out_u8, batch, xt);
 }
 
 // the streaming kernel; the caller has checked its preconditions (see the kernel)
@@ -2773,10 +2737,8 @@ int Q8Call::small_problem(bool *done) {
       p.x_dword = p.x_bytewise && by_dwords(p.X, p.ldx, p.xbs, xt, p.XN);
       p.y_dword = p.y_bytewise && (cv ? (uintptr_t)p.Y % 4 == 0 && cv->cin % 4 == 0
                                       : by_dwords(p.Y, p.ldy, p.ybs, yt, p.YN));
-      RequantTable tab;
-      if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
       *done = true;
-      return launch_gemm_fused_small(ctx, p, tab, out_u8, xt, yt, (int)batch);
+      return launch_gemm_fused_small(ctx, p, out_u8, xt, yt, (int)batch);
     }
   }
   return MACE_HIP_SUCCESS;
@@ -2836,10 +2798,8 @@ int Q8Call::kmajor_in_place(bool *done) {
         !(ctx->kernel_mask & MH_MASK_NO_XRES)) {
       GemmParams p = kmajor_params();
       p.sum_y = true;
-      RequantTable tab;
-      if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
       *done = true;
-      return launch_gemm_xres_any(ctx, p, tab, out_u8, (int)batch, tx, true);
+      return launch_gemm_xres_any(ctx, p, out_u8, (int)batch, tx, true);
     }
     // The same operand layout in the tile-count range of the eight-wavefront 128 x 128 kernel (see
     // below): its transposing LDS reads take the operand as it lies, so the repack (2048^3: zeroing
@@ -2851,10 +2811,8 @@ int Q8Call::kmajor_in_place(bool *done) {
     // and is left out; with k-contiguous operands two rounds lose by 2 - 5 % and stay where they were).
     if (mid_xt) {
       GemmParams p = kmajor_params();
-      RequantTable tab;
-      if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
       *done = true;
-      return launch_gemm_mid(ctx, p, tab, out_u8, (int)batch, true);
+      return launch_gemm_mid(ctx, p, out_u8, (int)batch, true);
     }
     // A depth that is an odd multiple of 8 (24 input channels of a MobileNetV2 block, 40, 72 ...),
     // both operands k-contiguous at 8-byte aligned addresses, a long Y panel and an X tile that fits
@@ -2872,10 +2830,8 @@ int Q8Call::kmajor_in_place(bool *done) {
         GemmParams p = q8_params(xl, Lo, Ro, rows, cols, depth, (int)depth, out, out_u8, rq, lhs_offset,
                                  rhs_offset, ep.bias);
         p.sum_y = true;
-        RequantTable tab;
-        if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
         *done = true;
-        return launch_gemm_xres_any(ctx, p, tab, out_u8, (int)batch, tx8, false);
+        return launch_gemm_xres_any(ctx, p, out_u8, (int)batch, tx8, false);
       }
     }
     // A k-major Y operand (the ColMajor left-hand matrix of a transpose_a MatMul with a RowMajor
@@ -2898,10 +2854,8 @@ int Q8Call::kmajor_in_place(bool *done) {
         const Q8Operand Yo{yp, yn, (xl ? rhs_nb : lhs_nb) > 1 ? yn * depth : 0};
         GemmParams p = q8_params(xl, xl ? Xo : Yo, xl ? Yo : Xo, rows, cols, depth, (int)depth, out,
                                  out_u8, rq, lhs_offset, rhs_offset, ep.bias);
-        RequantTable tab;
-        if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
         *done = true;
-        return launch_gemm_mid(ctx, p, tab, out_u8, (int)batch, x_kmajor, true);
+        return launch_gemm_mid(ctx, p, out_u8, (int)batch, x_kmajor, true);
       }
     }
     // ... and where the 256 x 256 tiles are the choice: the ring kernel's k-major variant; the
@@ -2931,10 +2885,8 @@ int Q8Call::kmajor_in_place(bool *done) {
         MH_RETURN_IF_ERROR(launch_kmajor_sums(ctx, xp, xn, p.xbs, xn, depth, x_nb, sum_x));
       if (!p.sum_y)
         MH_RETURN_IF_ERROR(launch_panel_sums(ctx, yp, depth, p.ybs, yn, (int)depth, y_nb, sum_y_buf));
-      RequantTable tab;
-      if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
       *done = true;
-      return launch_gemm_big_xt(ctx, p, tab, out_u8, (int)batch, sum_x_in_kernel);
+      return launch_gemm_big_xt(ctx, p, out_u8, (int)batch, sum_x_in_kernel);
     }
   }
   return MACE_HIP_SUCCESS;
@@ -3231,8 +3183,6 @@ int Q8Call::general() {
   p.corrY = x_is_lhs ? sumR : sumL;
   p.cxbs = (x_is_lhs ? lhs_nb : rhs_nb) > 1 ? p.XN : 0;
   p.cybs = (x_is_lhs ? rhs_nb : lhs_nb) > 1 ? p.YN : 0;
-  RequantTable tab;
-  if (out_u8 && rq.table && !requant_by_mad(rq)) mh_requant_table_cached(ctx, rq, tab.t);
   p.sum_y = sum_y;
   if (cv) {
     q8_params_conv(&p, *cv);
@@ -3243,9 +3193,9 @@ int Q8Call::general() {
   }
   if (xres) {
     p.sum_y = true;
-    return launch_gemm_xres_any(ctx, p, tab, out_u8, (int)batch, route.tx, false);
+    return launch_gemm_xres_any(ctx, p, out_u8, (int)batch, route.tx, false);
   }
-  if (mid) return launch_gemm_mid(ctx, p, tab, out_u8, (int)batch);
+  if (mid) return launch_gemm_mid(ctx, p, out_u8, (int)batch);
   if (stream) {
     switch ((p.XN + 31) / 32) {
       case 1: return launch_gemm_stream<1, 1>(ctx, p, (int)batch);
@@ -3268,37 +3218,37 @@ int Q8Call::general() {
   // the DMA kernels address a tile's rows with 32-bit offsets from its first row
   const bool dma_ok = p.ldx < (1 << 24) && p.ldy < (1 << 24);
   if (p.K == 2 * SLAB && !p.conv && dma_ok) {
-    if (skinny) return launch_gemm_dma<1, 4, 2, 2, 3, 2>(ctx, p, tab, out_u8, (int)batch);
-    if (big || medium) return launch_gemm_dma<2, 2, 2, 2, 3, 3>(ctx, p, tab, out_u8, (int)batch);
+    if (skinny) return launch_gemm_dma<1, 4, 2, 2, 3, 2>(ctx, p, out_u8, (int)batch);
+    if (big || medium) return launch_gemm_dma<2, 2, 2, 2, 3, 3>(ctx, p, out_u8, (int)batch);
   }
   // 128-byte slabs (whole cache lines per row) where they measure faster: the 256 x 256 tile
   // (+5 % at 8192^3) and long-k 128 x 128 tiles; short k gains nothing from them
   if (p.K % 128 == 0 && p.K >= 256 && !p.conv && dma_ok) {
-    if (big && PX.flipped) return launch_gemm_big_xf(ctx, p, tab, out_u8, (int)batch);
-    if (big) return launch_gemm_dma<2, 2, 4, 4, 2, 1, 128>(ctx, p, tab, out_u8, (int)batch);
+    if (big && PX.flipped) return launch_gemm_big_xf(ctx, p, out_u8, (int)batch);
+    if (big) return launch_gemm_dma<2, 2, 4, 4, 2, 1, 128>(ctx, p, out_u8, (int)batch);
     // Between half a round and one round of 128 x 128 tiles every CU has one workgroup and every
     // SIMD one wavefront, with nothing to overlap its waits: eight wavefronts of 64 x 32 results
     // instead of four of 64 x 64 (2048^3: -6 %; with a quarter of the CUs busy it is slower)
     if (medium && p.K >= 1024 && tiles(128, 128) <= cu && 2 * tiles(128, 128) > cu)
-      return launch_gemm_dma<2, 4, 2, 1, 2, 1, 128>(ctx, p, tab, out_u8, (int)batch);
+      return launch_gemm_dma<2, 4, 2, 1, 2, 1, 128>(ctx, p, out_u8, (int)batch);
     if (medium && p.K >= 1024)
-      return launch_gemm_dma<2, 2, 2, 2, 2, 2, 128>(ctx, p, tab, out_u8, (int)batch);
+      return launch_gemm_dma<2, 2, 2, 2, 2, 2, 128>(ctx, p, out_u8, (int)batch);
   }
   MH_CHECK(ctx, !PX.flipped, "internal: shifted panel outside the 256 x 256 kernel");
   if (p.K % SLAB == 0 && p.K >= SLAB * 3 && dma_ok) {
-    if (big) return launch_gemm_dma<2, 2, 4, 4, 4, 1>(ctx, p, tab, out_u8, (int)batch);
-    if (skinny) return launch_gemm_dma<1, 4, 2, 2, 4, 2>(ctx, p, tab, out_u8, (int)batch);
-    if (medium) return launch_gemm_dma<2, 2, 2, 2, 4, 2>(ctx, p, tab, out_u8, (int)batch);
-    return launch_gemm_dma<2, 2, 1, 1, 4, 4>(ctx, p, tab, out_u8, (int)batch);
+    if (big) return launch_gemm_dma<2, 2, 4, 4, 4, 1>(ctx, p, out_u8, (int)batch);
+    if (skinny) return launch_gemm_dma<1, 4, 2, 2, 4, 2>(ctx, p, out_u8, (int)batch);
+    if (medium) return launch_gemm_dma<2, 2, 2, 2, 4, 2>(ctx, p, out_u8, (int)batch);
+    return launch_gemm_dma<2, 2, 1, 1, 4, 4>(ctx, p, out_u8, (int)batch);
   }
   // The 256 x 256 instantiation of the register-staged kernel is switched off: one launch of it
   // (XN = 144, YN = 200704, K = 64, both operands repacked to 64-byte rows, Y summed in the kernel,
   // uint8 result) ended in a GPU memory fault, and reading the kernel and its compiled code has
   // not shown the cause.  Until it is known, the shapes that would choose that tile (a short k
   // that the resident-tile and ring kernels do not take) go to the 128 x 128 one.
-  if (skinny) return launch_gemm<1, 4, 2, 2>(ctx, p, tab, out_u8, (int)batch);
-  if (big || medium) return launch_gemm<2, 2, 2, 2>(ctx, p, tab, out_u8, (int)batch);
-  return launch_gemm<2, 2, 1, 1>(ctx, p, tab, out_u8, (int)batch);
+  if (skinny) return launch_gemm<1, 4, 2, 2>(ctx, p, out_u8, (int)batch);
+  if (big || medium) return launch_gemm<2, 2, 2, 2>(ctx, p, out_u8, (int)batch);
+  return launch_gemm<2, 2, 1, 1>(ctx, p, out_u8, (int)batch);
 }
 
 int mh_q8_gemm(mace_hip_ctx *ctx, const uint8_t *lhs, int lhs_order, const uint8_t *rhs,

@@ -5,8 +5,8 @@
 // of a wavefront), and every case runs one launch with operands allocated at exactly their size.
 // Built with AddressSanitizer: an access outside an operand aborts the run.  int32 results are
 // compared with sums formed directly from the operands; uint8 launches must write every byte of
-// the result (the table look-up of the requantization reads LDS through a 32-bit LDS pointer and
-// has no host form, so their values are not compared here; the GPU parity tests do that).
+// the result (the requantization ends in GPU assembly and has no host form, so their values are not
+// compared here; the GPU parity tests do that).
 //
 // What this covers is indexing and arithmetic of the source: row clamps, ragged tiles, depth
 // tails, swizzles, store guards.  A transfer into LDS lands at once here, so the order of
@@ -151,30 +151,23 @@ uint32_t emu_perm(uint32_t hi, uint32_t lo, uint32_t sel) {
   }
   return r;
 }
-float emu_fmed3f(float a, float b, float c) { return std::max(std::min(a, b), std::min(std::max(a, b), c)); }
 uint32_t __float_as_uint(float f) { uint32_t u; memcpy(&u, &f, 4); return u; }
 float __fmaf_rn(float a, float b, float c) { return fmaf(a, b, c); }
 inline int emu_readfirstlane(int v) { return v; }
-const void *emu_kernarg();
 #define __builtin_amdgcn_mfma_i32_32x32x32_i8 emu_mfma
 #define __builtin_amdgcn_permlane32_swap emu_permlane32_swap
 #define __builtin_amdgcn_sad_u8 emu_sad_u8
 #define __builtin_amdgcn_sdot4 emu_sdot4
 #define __builtin_amdgcn_udot4 emu_udot4
 #define __builtin_amdgcn_perm emu_perm
-#define __builtin_amdgcn_fmed3f emu_fmed3f
 #define __builtin_amdgcn_readfirstlane emu_readfirstlane
 #define __builtin_amdgcn_sched_barrier(x) ((void)0)
 #define __builtin_amdgcn_s_barrier emu_s_barrier
-#define __builtin_amdgcn_kernarg_segment_ptr emu_kernarg
 
 // ---- what the kernels' text takes from common.h and from other parts of q8_gemm.hip --------------
 struct RequantFixed {
-  int32_t mult, shift, mask, half, blo, bhi, zp, table, n, lo;
-  float inv, off, top;
+  int32_t mult, shift, mask, half, blo, bhi, zp;
 };
-constexpr float MH_REQUANT_MAGIC = 1048576.0f;
-constexpr int MH_REQUANT_TABLE_MAX = 258;
 inline int32_t mh_requant_fixed(int32_t, const RequantFixed &) { return 1; }
 
 #include "requant.inc"
@@ -196,12 +189,6 @@ inline void dma_16B(mh_rsrc rs, uint32_t lane_off, uint32_t uniform_off, uint8_t
 constexpr int SLAB = 64;
 #include "kernels.inc"
 }  // namespace
-
-static struct KernArgs {
-  GemmParams p;
-  RequantTable t;
-} g_args;
-const void *emu_kernarg() { return &g_args; }
 
 // all workgroups of a grid, one after the other, on as many host threads as a workgroup has
 static void run_grid(dim3 grid, const std::function<void()> &body, int threads = 256) {
@@ -274,11 +261,9 @@ struct Problem {
     p.XN = xn; p.YN = yn; p.K = k;
     p.corrX = sumx; p.corrY = sumy;
     p.ldo = xn; p.obs = (int64_t)xn * yn;
-    p.rq = RequantFixed{1 << 30, 8, 255, 127, -128, 127, 128, 1, 255, 0, 1e-3f, MH_REQUANT_MAGIC + 128.0f,
-                        MH_REQUANT_MAGIC + 255.875f};
+    p.rq = RequantFixed{1 << 30, 8, 255, 127, -128, 127, 128};
     p.xcoef = -3; p.xadd = 11; p.xbias = bias;
     p.ycoef = 5; p.yadd = -7; p.ybias = nullptr;
-    for (int i = 0; i < MH_REQUANT_TABLE_MAX; ++i) g_args.t.t[i] = i * 1000 - 100000;
   }
   ~Problem() {
     delete[] X; delete[] Y; delete[] sumx; delete[] sumy; delete[] bias;
@@ -297,7 +282,6 @@ struct Problem {
       int32_t *out = new int32_t[(int64_t)xn * yn];
       for (int64_t i = 0; i < (int64_t)xn * yn; ++i) out[i] = 0x5EEDBEEF;
       p.out = out;
-      g_args.p = p;
       launch32(p);
       int64_t bad = 0;
       for (int y = 0; y < yn; ++y)
@@ -309,7 +293,6 @@ struct Problem {
       uint8_t *out = new uint8_t[(int64_t)xn * yn];
       memset(out, 0xEE, (int64_t)xn * yn);
       p.out = out;
-      g_args.p = p;
       launch8(p);
       int64_t untouched = 0;
       for (int64_t i = 0; i < (int64_t)xn * yn; ++i) untouched += out[i] == 0xEE;
@@ -336,11 +319,11 @@ static void ring_case(int xn, int yn, int k) {
            FX, FY, STAGES, KB, (int)SUMY, (int)XT, (int)XF, (int)SUMX);
   pr.check(what,
            [&](GemmParams &p) {
-             run_grid(grid, [&] { q8_gemm_dma_kernel<WX, WY, FX, FY, STAGES, int32_t, 1, SUMY, false, KB, XT, XF, SUMX>(p, g_args.t); },
+             run_grid(grid, [&] { q8_gemm_dma_kernel<WX, WY, FX, FY, STAGES, int32_t, 1, SUMY, false, KB, XT, XF, SUMX>(p); },
                       WX * WY * 64);
            },
            [&](GemmParams &p) {
-             run_grid(grid, [&] { q8_gemm_dma_kernel<WX, WY, FX, FY, STAGES, uint8_t, 1, SUMY, false, KB, XT, XF, SUMX>(p, g_args.t); },
+             run_grid(grid, [&] { q8_gemm_dma_kernel<WX, WY, FX, FY, STAGES, uint8_t, 1, SUMY, false, KB, XT, XF, SUMX>(p); },
                       WX * WY * 64);
            });
 }
@@ -356,8 +339,8 @@ static void mid_case(int xn, int yn, int k) {
   char what[64];
   snprintf(what, sizeof what, "q8_gemm_mid_kernel<STAGES=4,XT=%d,YT=%d>", (int)XT, (int)YT);
   pr.check(what,
-           [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_mid_kernel<int32_t, 4, XT, YT>(p, g_args.t); }, 512); },
-           [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_mid_kernel<uint8_t, 4, XT, YT>(p, g_args.t); }, 512); });
+           [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_mid_kernel<int32_t, 4, XT, YT>(p); }, 512); },
+           [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_mid_kernel<uint8_t, 4, XT, YT>(p); }, 512); });
 }
 
 template <int WX, int WY, int FX, int FY>
@@ -374,12 +357,12 @@ static void tiled_case(int xn, int yn, int k, bool sum_y) {
   snprintf(what, sizeof what, "q8_gemm_kernel<%d,%d,%d,%d,SUMY=%d>", WX, WY, FX, FY, (int)sum_y);
   if (sum_y)
     pr.check(what,
-             [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_kernel<WX, WY, FX, FY, int32_t, true>(p, g_args.t); }); },
-             [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_kernel<WX, WY, FX, FY, uint8_t, true>(p, g_args.t); }); });
+             [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_kernel<WX, WY, FX, FY, int32_t, true>(p); }); },
+             [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_kernel<WX, WY, FX, FY, uint8_t, true>(p); }); });
   else
     pr.check(what,
-             [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_kernel<WX, WY, FX, FY, int32_t, false>(p, g_args.t); }); },
-             [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_kernel<WX, WY, FX, FY, uint8_t, false>(p, g_args.t); }); });
+             [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_kernel<WX, WY, FX, FY, int32_t, false>(p); }); },
+             [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_kernel<WX, WY, FX, FY, uint8_t, false>(p); }); });
 }
 
 // the resident-tile kernel on operands as they lie (row pitch = k); TAIL: k % 64 != 0
@@ -392,10 +375,10 @@ static void xres_case(int xn, int yn, int k, int wgs) {
   snprintf(what, sizeof what, "q8_gemm_xres_kernel<FX=%d,FY=%d,G=64,TAIL=%d> grid %d", FX, FY, (int)TAIL, wgs);
   pr.check(what,
            [&](GemmParams &p) {
-             run_grid(grid, [&] { q8_gemm_xres_kernel<FX, FY, 64, int32_t, 2, false, false, TAIL>(p, g_args.t); });
+             run_grid(grid, [&] { q8_gemm_xres_kernel<FX, FY, 64, int32_t, 2, false, false, TAIL>(p); });
            },
            [&](GemmParams &p) {
-             run_grid(grid, [&] { q8_gemm_xres_kernel<FX, FY, 64, uint8_t, 2, false, false, TAIL>(p, g_args.t); });
+             run_grid(grid, [&] { q8_gemm_xres_kernel<FX, FY, 64, uint8_t, 2, false, false, TAIL>(p); });
            });
 }
 
@@ -418,8 +401,7 @@ static void mid_batched_case(int batch, int xn, int yn, int k) {
   p.sum_y = true;
   p.tiles_x = (xn + 127) / 128;
   p.tiles_y = (yn + 127) / 128;
-  g_args.p = p;
-  run_grid(dim3(p.tiles_x * p.tiles_y, 1, batch), [&] { q8_gemm_mid_kernel<int32_t, 4, false, false>(p, g_args.t); }, 512);
+  run_grid(dim3(p.tiles_x * p.tiles_y, 1, batch), [&] { q8_gemm_mid_kernel<int32_t, 4, false, false>(p); }, 512);
   int64_t bad = 0;
   for (int b = 0; b < batch; ++b)
     for (int y = 0; y < yn; ++y)
@@ -473,8 +455,7 @@ static void small_case(int xn, int yn, int k, const Conv *cv = nullptr) {
   p.X = X; p.ldx = ldx; p.Y = Y; p.ldy = ldy;
   p.XN = xn; p.YN = yn; p.K = k;
   p.ldo = xn; p.obs = (int64_t)xn * yn;
-  p.rq = RequantFixed{1 << 30, 8, 255, 127, -128, 127, 128, 1, 255, 0, 1e-3f, MH_REQUANT_MAGIC + 128.0f,
-                      MH_REQUANT_MAGIC + 255.875f};
+  p.rq = RequantFixed{1 << 30, 8, 255, 127, -128, 127, 128};
   p.xcoef = -3; p.xadd = 11; p.xbias = bias.data();
   p.ycoef = 5; p.yadd = -7; p.ybias = nullptr;
   p.sum_y = true;
@@ -496,15 +477,13 @@ static void small_case(int xn, int yn, int k, const Conv *cv = nullptr) {
     p.y_bytewise = !vec(YT, yn);
     p.y_dword = p.y_bytewise && dwords(YT, yn);
   }
-  for (int i = 0; i < MH_REQUANT_TABLE_MAX; ++i) g_args.t.t[i] = i * 1000 - 100000;
   const bool bw = p.x_bytewise || p.y_bytewise;
   const dim3 grid(p.tiles_x * p.tiles_y, 1, 1);
   {
     std::vector<int32_t> out((int64_t)xn * yn, 0x5EEDBEEF);
     p.out = out.data();
-    g_args.p = p;
-    if (bw) run_grid(grid, [&] { q8_gemm_fused_small_kernel<int32_t, XT, YT, true>(p, g_args.t); });
-    else run_grid(grid, [&] { q8_gemm_fused_small_kernel<int32_t, XT, YT, false>(p, g_args.t); });
+    if (bw) run_grid(grid, [&] { q8_gemm_fused_small_kernel<int32_t, XT, YT, true>(p); });
+    else run_grid(grid, [&] { q8_gemm_fused_small_kernel<int32_t, XT, YT, false>(p); });
     int64_t bad = 0;
     for (int y = 0; y < yn; ++y)
       for (int x = 0; x < xn; ++x) {
@@ -520,9 +499,8 @@ static void small_case(int xn, int yn, int k, const Conv *cv = nullptr) {
   {
     std::vector<uint8_t> out((int64_t)xn * yn, 0xEE);
     p.out = out.data();
-    g_args.p = p;
-    if (bw) run_grid(grid, [&] { q8_gemm_fused_small_kernel<uint8_t, XT, YT, true>(p, g_args.t); });
-    else run_grid(grid, [&] { q8_gemm_fused_small_kernel<uint8_t, XT, YT, false>(p, g_args.t); });
+    if (bw) run_grid(grid, [&] { q8_gemm_fused_small_kernel<uint8_t, XT, YT, true>(p); });
+    else run_grid(grid, [&] { q8_gemm_fused_small_kernel<uint8_t, XT, YT, false>(p); });
     int64_t untouched = 0;
     for (uint8_t v : out) untouched += v == 0xEE;
     EXPECT(untouched == 0, "fused_small<XT=%d,YT=%d,BW=%d> XN %d YN %d K %d: %lld uint8 results not written",

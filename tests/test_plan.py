@@ -391,6 +391,24 @@ def test_gemv_dispatch(ctx):
     assert gemv(ctx, 33, 1000, 4096).grid == (63, 3, 1)
 
 
+def test_output_scales_do_not_change_the_kernel(ctx):
+    """real multipliers of 1/2 and more (right shift 0) down to 2^-22 (2^-32 at zero point 0)
+    requantize in the same kernels"""
+    def plan(n, hw, cin, cout, k, stride, real, ozp):
+        ctx.call("mace_hip_conv2d_q8_nhwc", A, B, BIAS, n, hw, hw, cin, cout, k, k, stride, stride, k - 1, k - 1,
+                 0.02, 128, 0.01, 127, 0.0002, 0.0002 / real, ozp, 0, 255, O)
+        p = ctx.last_plan()
+        return p.kernel, p.launches, p.grid
+
+    for n, hw, cin, cout, k, stride, family in ((64, 224, 3, 32, 3, 2, "conv_short"), (64, 56, 32, 32, 3, 1, "conv_rows"),
+                                                (64, 112, 32, 64, 1, 1, "gemm_stream"), (64, 28, 256, 256, 1, 1, "xres"),
+                                                (1, 14, 256, 256, 3, 1, "conv_ksplit")):
+        usual = plan(n, hw, cin, cout, k, stride, 0.004, 0)
+        assert family in usual[0], usual
+        for real, ozp in ((0.999, 0), (0.5, 128), (0.3, 255), (2e-7, 128), (2.4e-10, 0)):
+            assert plan(n, hw, cin, cout, k, stride, real, ozp) == usual, (real, ozp)
+
+
 # ---- the tables themselves -------------------------------------------------------------------------
 
 def test_variant_tables_are_consistent():
