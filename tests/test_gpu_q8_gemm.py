@@ -341,6 +341,20 @@ def test_q8_gemm_repacked_operands(ctx, batch, rows, depth, cols, lb, rb, lo, ro
         ctx.call("mace_hip_ctx_set_kernel_mask", 0)
 
 
+# The 256 x 256 kernel on a right-hand matrix copied already shifted, in columns of any number: the copy
+# adds up its rows; with more than 4096 columns the left-hand matrix's own pass goes first and clears them.
+@pytest.mark.parametrize("batch,rows,depth,cols,aux", [
+    (2, 300, 1280, 8001, mh.AUX_PACK_TRANSPOSE | mh.AUX_PACK_SHIFTED | mh.AUX_PANEL_SUMS),
+    (4, 300, 1280, 4001, mh.AUX_PACK_TRANSPOSE | mh.AUX_PACK_SHIFTED | mh.AUX_ZERO)])
+def test_q8_gemm_shifted_panel_of_any_width(ctx, batch, rows, depth, cols, aux):
+    ctx.call("mace_hip_ctx_set_kernel_mask", mh.MASK_NO_MID)
+    try:
+        assert check_gemm(ctx, batch, rows, depth, cols, True, True, R, R, R) == ("ring_xf", "ring_xf")
+        assert ctx.last_plan().aux == aux, ctx.last_plan()
+    finally:
+        ctx.call("mace_hip_ctx_set_kernel_mask", 0)
+
+
 def test_q8_gemm_config1_matmul(ctx):
     """benchmark configuration 1: A [128x256], B [256x128], zero points 128/128/128, scales
     0.02/0.015/0.05 -> (1649267328, shift 7)."""
