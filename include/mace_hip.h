@@ -126,8 +126,8 @@ enum {
   MACE_HIP_KF_Q8_GEMV_MFMA,          /* q8_gemv_mfma_kernel: rows too wide for LDS                */
   MACE_HIP_KF_Q8_GEMV_ROWS,          /* q8_gemv_rows_kernel: vectors of one pass in LDS           */
   MACE_HIP_KF_Q8_GEMV_GENERAL,       /* q8_gemv_kernel: any width and alignment                   */
-  MACE_HIP_KF_F32_GEMM_VEC,          /* f32_gemm_vec_kernel: fp32 by bf16 MFMAs, see f32_gemm.hip */
-  MACE_HIP_KF_F32_GEMM_GENERAL,      /* f32_gemm_kernel: the same for any length and alignment    */
+  MACE_HIP_KF_F32_GEMM_VEC,          /* f32_gemm_vec_kernel, operands in aligned 16-byte pieces  */
+  MACE_HIP_KF_F32_GEMM_GENERAL,      /* the same or, for ragged depths, f32_gemm_kernel: others   */
   MACE_HIP_KF_F32_GEMM_FILL,         /* depths 0 to 2: multiply-adds, element by element          */
   MACE_HIP_KF_F32_GEMV_VEC,          /* f32_gemv_vec_kernel                                       */
   MACE_HIP_KF_F32_GEMV_GENERAL,      /* f32_gemv_kernel                                           */

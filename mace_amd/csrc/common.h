@@ -222,10 +222,13 @@ inline int gemv_rows(int nb, bool out_u8) { return log2i(nb) * 2 + (out_u8 ? 1 :
 inline int gemv_general(int nb, bool vec, bool out_u8) {
   return (log2i(nb) * 2 + (vec ? 1 : 0)) * 2 + (out_u8 ? 1 : 0);
 }
-inline int f32_gemm_vec(bool split, bool lk, bool rk) {
-  return (split ? 4 : 0) | (lk ? 2 : 0) | (rk ? 1 : 0);
+// tiles of 128 rows by four wavefronts, by eight, of 64 rows by four
+enum { F32_128 = 0, F32_SPLIT, F32_64, F32_FORMS };
+inline int f32_gemm_vec(int form, bool lk, bool rk) { return form * 4 + (lk ? 2 : 0) + (rk ? 1 : 0); }
+// guard: every load checked against the depth; without it the kernel is f32_gemm_vec_kernel
+inline int f32_gemm_general(bool guard, int form, bool lk, bool rk) {
+  return (guard ? 0 : F32_FORMS * 4) + f32_gemm_vec(form, lk, rk);
 }
-inline int f32_gemm_general(bool lk, bool rk) { return (lk ? 2 : 0) | (rk ? 1 : 0); }
 inline int f32_gemv_vec(int nb) { return log2i(nb); }
 }  // namespace mhv
 

@@ -401,9 +401,9 @@ template <bool LK, bool RK, int SPLIT, int TMT>
 __global__ __launch_bounds__(256 * SPLIT, SPLIT == 1 ? 3 : 1) void f32_gemm_vec_kernel(F32GemmParams p) {
   f32_tile<LK, RK, SPLIT, false, TMT>(p);
 }
-template <bool LK, bool RK, int SPLIT, int TMT, bool GUARD>
-__global__ __launch_bounds__(256 * SPLIT, SPLIT == 2 ? 1 : (GUARD && TMT == 128 ? 2 : 3)) void f32_gemm_kernel(F32GemmParams p) {
-  f32_tile<LK, RK, SPLIT, GUARD, TMT>(p);
+template <bool LK, bool RK, int SPLIT, int TMT>
+__global__ __launch_bounds__(256 * SPLIT, SPLIT == 1 ? 3 : 1) void f32_gemm_kernel(F32GemmParams p) {
+  f32_tile<LK, RK, SPLIT, true, TMT>(p);
 }
 
 // Depths of at most two: 0 (the reference's loop leaves sum = 0), and 1 and 2 by binary32 multiply-adds,
@@ -648,8 +648,11 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
   const bool split = tiles * batch <= cus;   // at most one tile per CU
   const bool lk = lhs_major == MACE_HIP_ROW_MAJOR;   // depth contiguous
   const bool rk = rhs_major == MACE_HIP_COL_MAJOR;
-  // 16-byte pieces: whole k tiles; an operand whose rows run along k may have any number of rows
-  // (a ragged last tile re-reads its last row), one that runs along m / n needs them in fours
+  // Depths in whole k tiles, and rows along depth in aligned 16-byte pieces: no load is checked.  (An
+  // operand that runs along m / n is read by 4-byte loads, so it may have any length and address.)
+  const bool whole = depth % TK == 0 && (!lk || (uintptr_t)lhs % 16 == 0) && (!rk || (uintptr_t)rhs % 16 == 0);
+  // The plan files calls whose operands are aligned 16-byte pieces in either direction under a family of
+  // their own, which they had when those loads were 16 bytes wide as well.
   const bool vec = depth % TK == 0 && (lk || rows % 4 == 0) && (rk || cols % 4 == 0) &&
                    rows >= 4 && cols >= 4 && ((uintptr_t)lhs % 16 == 0) &&
                    ((uintptr_t)rhs % 16 == 0);
@@ -678,13 +681,12 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
       mh_plan_aux(ctx, MACE_HIP_AUX_F32_KSPLIT);
     }
   }
-  if (vec) mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_VEC, mhv::f32_gemm_vec(split, lk, rk), grid,
+  const int form = split ? mhv::F32_SPLIT : (half ? mhv::F32_64 : mhv::F32_128);
+  if (vec) mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_VEC, mhv::f32_gemm_vec(form, lk, rk), grid,
                         split ? block2 : block, 0);
-  else mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_GENERAL, mhv::f32_gemm_general(lk, rk), grid,
+  else mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_GENERAL, mhv::f32_gemm_general(!whole, form, lk, rk), grid,
                     split ? block2 : block, 0);
   MH_PROF_BEGIN(ctx);
-  // depths in whole k tiles, and rows along depth in aligned 16-byte pieces
-  const bool whole = depth % TK == 0 && (!lk || (uintptr_t)lhs % 16 == 0) && (!rk || (uintptr_t)rhs % 16 == 0);
 #define MH_F32(KERNEL, ...) MH_KLAUNCH(ctx, (KERNEL<__VA_ARGS__>), grid, split ? block2 : block, 0, ctx->stream, p)
 #define MH_F32_LR(KERNEL, ...)                                                                  \
   do {                                                                                          \
@@ -693,15 +695,12 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
     else if (rk) MH_F32(KERNEL, false, true, __VA_ARGS__);                                      \
     else MH_F32(KERNEL, false, false, __VA_ARGS__);                                             \
   } while (0)
-  if (vec && split) MH_F32_LR(f32_gemm_vec_kernel, 2, 128);
-  else if (vec && half) MH_F32_LR(f32_gemm_vec_kernel, 1, 64);
-  else if (vec) MH_F32_LR(f32_gemm_vec_kernel, 1, 128);
-  else if (whole && split) MH_F32_LR(f32_gemm_kernel, 2, 128, false);
-  else if (whole && half) MH_F32_LR(f32_gemm_kernel, 1, 64, false);
-  else if (whole) MH_F32_LR(f32_gemm_kernel, 1, 128, false);
-  else if (split) MH_F32_LR(f32_gemm_kernel, 2, 128, true);
-  else if (half) MH_F32_LR(f32_gemm_kernel, 1, 64, true);
-  else MH_F32_LR(f32_gemm_kernel, 1, 128, true);
+  if (whole && split) MH_F32_LR(f32_gemm_vec_kernel, 2, 128);
+  else if (whole && half) MH_F32_LR(f32_gemm_vec_kernel, 1, 64);
+  else if (whole) MH_F32_LR(f32_gemm_vec_kernel, 1, 128);
+  else if (split) MH_F32_LR(f32_gemm_kernel, 2, 128);
+  else if (half) MH_F32_LR(f32_gemm_kernel, 1, 64);
+  else MH_F32_LR(f32_gemm_kernel, 1, 128);
 #undef MH_F32_LR
 #undef MH_F32
   MH_PROF_END(ctx);

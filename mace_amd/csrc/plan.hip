@@ -26,8 +26,8 @@ const int kVariantCount[MACE_HIP_KF_COUNT] = {
     4,                        // Q8_GEMV_MFMA
     8,                        // Q8_GEMV_ROWS
     16,                       // Q8_GEMV_GENERAL
-    8,                        // F32_GEMM_VEC
-    4,                        // F32_GEMM_GENERAL
+    mhv::F32_FORMS * 4,       // F32_GEMM_VEC
+    mhv::F32_FORMS * 8,       // F32_GEMM_GENERAL
     1,                        // F32_GEMM_FILL
     3,                        // F32_GEMV_VEC
     1,                        // F32_GEMV_GENERAL
@@ -181,11 +181,13 @@ int mace_hip_plan_describe(int family, int v, char *buf, size_t len) {
       snprintf(buf, len, "%s<NB=%d,VEC=%s,%s>", k, 1 << (v >> 2), tf(v & 2), out_name(v & 1));
       break;
     case MACE_HIP_KF_F32_GEMM_VEC:
-      snprintf(buf, len, "%s<LK=%s,RK=%s,SPLIT=%d>", k, tf(v & 2), tf(v & 1), (v & 4) ? 2 : 1);
+    case MACE_HIP_KF_F32_GEMM_GENERAL: {
+      const int form = v / 4 % mhv::F32_FORMS;
+      if (v >= mhv::F32_FORMS * 4) k = kFamilyName[MACE_HIP_KF_F32_GEMM_VEC];
+      snprintf(buf, len, "%s<LK=%s,RK=%s,SPLIT=%d%s>", k, tf(v & 2), tf(v & 1), form == mhv::F32_SPLIT ? 2 : 1,
+               form == mhv::F32_64 ? ",TM=64" : "");
       break;
-    case MACE_HIP_KF_F32_GEMM_GENERAL:
-      snprintf(buf, len, "%s<LK=%s,RK=%s>", k, tf(v & 2), tf(v & 1));
-      break;
+    }
     case MACE_HIP_KF_Q8_CONV_SHORT:
       snprintf(buf, len, "%s<FX=%d>", k, 1 << v);
       break;

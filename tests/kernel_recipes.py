@@ -136,6 +136,16 @@ def candidates():
                     for (lm, rm, om) in ORDERS:
                         yield {"kind": "f32gemm", "batch": b, "rows": m, "cols": n, "depth": k, "lm": lm,
                                "rm": rm, "om": om}, b * m * n * (k + 1) / 1e9
+    # more tiles than CUs: of 128 rows, of 64 rows, and with fewer columns than a 16-byte piece has
+    for (m, n) in ((2304, 2304), (2301, 2301), (2220, 2052), (2221, 2050), (33024, 3), (33044, 3)):
+        for k in (16, 19):
+            for (lm, rm, om) in ORDERS:
+                yield {"kind": "f32gemm", "batch": 1, "rows": m, "cols": n, "depth": k, "lm": lm, "rm": rm,
+                       "om": om}, m * n * (k + 1) / 1e9
+    for n in (2, 3):
+        for (lm, rm, om) in ORDERS:
+            yield {"kind": "f32gemm", "batch": 1, "rows": 31, "cols": n, "depth": 16, "lm": lm, "rm": rm,
+                   "om": om}, 31 * n * 17 / 1e9
     for H in (100, 1000):
         for W in (100, 101, 1024):
             for b in (1, 2, 5):
