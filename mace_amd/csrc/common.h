@@ -477,7 +477,13 @@ inline bool mh_q8_small_problem(const mace_hip_ctx *ctx, int64_t batch, int64_t 
 }
 
 // Into how many parts the fp32 GEMM deals a tile's k range (1: no split): only while at most half
-// the CUs would have a tile, at least four k tiles of 16 per part, at most 16 parts.
+// the CUs would have a tile, at least four k tiles of 16 per part, at most 16 parts.  Forced to 1, 2, 3, 4, 8 and
+// 16 parts, the choice is the best or within 3 % of it: 512^3 (8) 26.8 unsplit, 17.7; 1024^3 (4) 46.7, 28.2, with
+// 8 41.9; 128 x 4096 x 128 (16) 158, 23.7; 1536 x 2048 x 1024 (2) 85.4, 54.9; 300 x 200 x 300 (3) 19.5, 15.7, with
+// 8 13.2 us; above half the CUs every split loses (1280 x 1024 x 1664, 130 tiles, 47.2 and 52.7).
+// A k tile takes 0.6 us whatever else runs; the parts are written and read once more, 8 bytes per
+// output at about 4 TB/s.  Where that takes longer than the k tiles it saves the call stays whole
+// (1024 x 160 x 1568: 14.4 us, 21.7 in two parts).
 inline int mh_f32_ksplit(const mace_hip_ctx *ctx, int64_t batch, int64_t rows, int64_t cols,
                          int64_t depth) {
   const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
@@ -487,7 +493,9 @@ inline int mh_f32_ksplit(const mace_hip_ctx *ctx, int64_t batch, int64_t rows, i
   int64_t parts = cus / wgs;
   if (parts > nk / 4) parts = nk / 4;
   if (parts > 16) parts = 16;
-  return parts < 2 ? 1 : (int)parts;
+  if (parts < 2) return 1;
+  const double saved_us = 0.6 * nk * (parts - 1) / parts, moved_us = 8.0 * parts * batch * rows * cols / 4e6;
+  return saved_us < moved_us ? 1 : (int)parts;
 }
 // scratch of that split (0 without one); joined: a batch may also be run as one long row of columns
 inline size_t mh_f32_ksplit_bytes(const mace_hip_ctx *ctx, int64_t batch, int64_t rows, int64_t cols,

@@ -391,6 +391,17 @@ def test_gemv_dispatch(ctx):
     assert gemv(ctx, 33, 1000, 4096).grid == (63, 3, 1)
 
 
+def test_f32_split_and_tile_height_boundaries(ctx):
+    def plan(m, k, n):
+        ctx.call("mace_hip_gemm_f32", A, B, 1, m, n, k, 0, 0, 0, 1, 1, O)
+        return ctx.last_plan()
+
+    assert plan(1024, 160, 1568).grid == (104, 1, 1)        # ten k tiles against 6 MB of parts
+    assert plan(1536, 512, 1024).grid == (96, 2, 1)
+    assert plan(300, 200, 300).grid == (9, 3, 1)
+    assert plan(1280, 1024, 1664).grid == (130, 1, 1)       # more than half the CUs have a tile
+
+
 def test_output_scales_do_not_change_the_kernel(ctx):
     """real multipliers of 1/2 and more (right shift 0) down to 2^-22 (2^-32 at zero point 0)
     requantize in the same kernels"""
