@@ -81,8 +81,9 @@ __device__ inline float apply_act(float v, int act, float limit) {
 // with four, where the binary32 instruction rounds it to nearest: depths 1 and 2 go to f32_fill_kernel
 // for that.  (Rows with one entry other than zero keep it; where that entry is a power of two the product
 // is exact.)  In time, 4 x 1024^3 against transposed weights 86.0 -> 51.3 us, MobileNet's five pointwise layers
-// at batch 64 688 -> 318 us; the matrix cores are busy 35 - 45 % of it, the rest is each k tile's chain of
-// LDS reads, MFMAs, LDS writes and barrier (one to three workgroups per CU overlap).
+// at batch 64 688 -> 318 us.  The matrix cores are busy 42 - 51 % of 4 x 1024^3 and 12 - 35 % of the pointwise
+// layers; the rest is each k tile's chain of LDS reads, MFMAs, LDS writes and barrier (one to three workgroups
+// per CU overlap) and, at short depths, the first loads and the stores of every tile.
 //
 // Both operands are multiplied by 2^23 before the split and the sums by 2^-46 behind it, all exact: the
 // last bit of the smallest subnormal number then lies at 2^-126, so every part of every number is a
@@ -150,7 +151,8 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
   constexpr int FM = 2, FN = TN / 32 / WN;
   static_assert(TN * KC == NT && TMT * KC <= NT, "at most one unit of either operand per thread");
   // (PAD: where depth is contiguous 16 lanes write 16 / KC rows of all KC pieces, which a pitch of a
-  // whole 256 bytes would put into the same banks: 27 % of the cycles of 4 x 1024^3)
+  // whole 256 bytes would put into the same banks.  With it conflicts take 13 % of the cycles of 4 x 1024^3 where
+  // both operands lie so, 6 % where one does.)
   constexpr int PAD = 16 / KC, PA_ = TMT + PAD, PB_ = TN + PAD;
   __shared__ __align__(16) u4v sA[2][3][KC][PA_];
   __shared__ __align__(16) u4v sB[2][3][KC][PB_];
@@ -636,10 +638,13 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
     p.N = (int)(batch * cols);
     batch = 1;
   }
-  // Rows that leave the last 128-row tile at most half full: tiles of 64 rows (while there is at least
-  // one for every CU; below, the eight-wavefront form with 128 rows).
+  // Up to 192 rows that leave the last 128-row tile at most half full: tiles of 64 rows (while there is at
+  // least one for every CU; below, the eight-wavefront form with 128 rows).  A 64-row tile takes 1.2 to 1.4 times
+  // half the time of a 128-row one, so a quarter of the work has to be padding: 64 x 256 x 70000 42.0 -> 29.7 us,
+  // 192 x 512 x 40000 74.3 -> 66.5, but 320 x 256 x 20000 33.9 -> 38.0, 576 x 512 x 12000 54.8 -> 64.7.
   const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  const bool half = (p.M - 1) % TM < TM / 2 && ((p.M + 63) / 64) * ((p.N + TN - 1) / TN) * batch > cus;
+  const bool half = p.M <= TM + TM / 2 && (p.M - 1) % TM < TM / 2 &&
+                    ((p.M + 63) / 64) * ((p.N + TN - 1) / TN) * batch > cus;
   const int tm = half ? TM / 2 : TM;
   p.tiles_m = (p.M + tm - 1) / tm;
   const int64_t tiles = (int64_t)p.tiles_m * ((p.N + TN - 1) / TN);
@@ -657,8 +662,7 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
                    rows >= 4 && cols >= 4 && ((uintptr_t)lhs % 16 == 0) &&
                    ((uintptr_t)rhs % 16 == 0);
   // Few tiles and a long depth: the k tiles are dealt to several workgroups per tile, whose parts a
-  // second launch adds up in a fixed order.  (A tile's time is its k tiles at about 1 us each
-  // whatever else runs: 512^3, 16 tiles, took 43.7 us with 240 CUs idle.)
+  // second launch adds up in a fixed order (see mh_f32_ksplit).
   ArenaScope scope(ctx);
   auto bytes_of = [&](int n) { return sizeof(float) * (size_t)n * total + 256; };
   int parts = mh_f32_ksplit(ctx, batch, rows, p.N, depth);

@@ -18,9 +18,8 @@ typedef unsigned v2u __attribute__((ext_vector_type(2)));
 // does for [y < 0] (where x < 0 and y = 0 both give 0).  A floor of a floor is a floor, so all of
 // it is
 //   z + zp = floor((x m + C - [x < 0] 2^31) / 2^(31+s)),   C = 2^30 + 2^(30+s) + zp 2^(31+s),
-// a v_mad_i64_i32 (full rate here: 4.9 cycles per wavefront measured, a 32-bit add 4.6) whose high
-// dword, shifted right by s - 1 more, is the unclamped output.  v_ashr_pk_u8_i32 does that shift,
-// the clamp to 0..255 and the packing of two outputs at once.  Outputs that zp and the clamp keep
+// a v_mad_i64_i32 (2.2 ns per wavefront on a SIMD; a 32-bit add takes 1.1) whose high dword, shifted
+// right by s - 1 more, is the unclamped output.  v_ashr_pk_u8_i32 does that shift, the clamp to 0..255 and the packing of two outputs at once.  Outputs that zp and the clamp keep
 // from ever being a z below 1 (zp = 0: a quantized ReLU) need no sign term: 1.5 instructions per
 // output beside the correction terms' addition, 3.5 with it, 4.5 with a narrower clamp (the high
 // dword is clamped to lo 2^(s-1) .. hi 2^(s-1)), against 7.75 and an LDS read by the table, which

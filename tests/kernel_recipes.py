@@ -137,7 +137,7 @@ def candidates():
                         yield {"kind": "f32gemm", "batch": b, "rows": m, "cols": n, "depth": k, "lm": lm,
                                "rm": rm, "om": om}, b * m * n * (k + 1) / 1e9
     # more tiles than CUs: of 128 rows, of 64 rows, and with fewer columns than a 16-byte piece has
-    for (m, n) in ((2304, 2304), (2301, 2301), (2220, 2052), (2221, 2050), (33024, 3), (33044, 3)):
+    for (m, n) in ((2304, 2304), (2301, 2301), (188, 16400), (190, 16401), (33024, 3), (3, 33024)):
         for k in (16, 19):
             for (lm, rm, om) in ORDERS:
                 yield {"kind": "f32gemm", "batch": 1, "rows": m, "cols": n, "depth": k, "lm": lm, "rm": rm,

@@ -78,7 +78,7 @@ def test_few_tiles_and_a_long_depth(ctx):
 
 # (at most one tile per CU; more: 128-row tiles, 64-row tiles with idle loader threads; depths that are not
 # whole k tiles)
-OUTSIDE = [(140, 64, 133), (40, 50, 300), (2304, 32, 2200), (2304, 33, 2200), (2221, 48, 2050), (2221, 19, 2050)]
+OUTSIDE = [(140, 64, 133), (40, 50, 300), (2304, 32, 2200), (2304, 33, 2200), (190, 48, 16401), (190, 19, 16401)]
 
 
 @pytest.mark.parametrize("m,k,n", OUTSIDE)

@@ -400,6 +400,8 @@ def test_f32_split_and_tile_height_boundaries(ctx):
     assert plan(1536, 512, 1024).grid == (96, 2, 1)
     assert plan(300, 200, 300).grid == (9, 3, 1)
     assert plan(1280, 1024, 1664).grid == (130, 1, 1)       # more than half the CUs have a tile
+    for m, tall in ((64, False), (65, True), (128, True), (129, False), (192, False), (193, True), (320, True)):
+        assert ("TM=64" in plan(m, 256, 40000).kernel) != tall, m
 
 
 def test_output_scales_do_not_change_the_kernel(ctx):
