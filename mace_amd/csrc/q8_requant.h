@@ -117,7 +117,7 @@ __device__ __forceinline__ void requant_16_by_mad(const int32_t (&v)[16], const 
   if (m.no_sign) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) h[r] = (int32_t)(((int64_t)v[r] * m.mult + m.c) >> 32);
-    if (m.more) {
+    if (__builtin_expect(m.more, 0)) {
       if (m.plus_x) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) h[r] = __builtin_elementwise_add_sat(h[r], v[r]);
