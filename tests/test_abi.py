@@ -65,8 +65,8 @@ def test_fixed_point_requant_matches_oracle():
 
 
 def test_threshold_requant_matches_oracle_at_every_step():
-    """The kernels' uint8 stores locate the output step with a float estimate and one exact
-    threshold comparison.  Pin that form where it can go wrong: one below, at and one above
+    """The kernels' uint8 stores take one 64-bit multiply-add and a shift per output.  Pin that form
+    where it can go wrong: one below, at and one above
     every point where the oracle's output changes (found by bisection on the oracle, which is
     monotone for a positive multiplier), plus the int32 extremes and random accumulators."""
     import ctypes as C
@@ -110,11 +110,27 @@ def test_threshold_requant_matches_oracle_at_every_step():
                 used_table += rc
                 assert got == ref(acc), (acc, mult, shift, zp, lo, hi, rc)
     assert used_table > 0
-    # parameters outside the threshold form fall back to the plain arithmetic
+    # parameters outside that form fall back to the plain arithmetic
     for (mult, shift, zp) in ((-2 ** 31, 3, 10), (-5, 0, 0), (2 ** 30, 4, 40000), (2 ** 30, 4, -40000)):
         for acc in (-2 ** 31, -12345, 0, 999, 2 ** 31 - 1):
             rc, got = table(acc, mult, shift, zp, 0, 255)
             assert rc == 0 and got == orc.requant_fixed_u8(acc, mult, shift, zp, 0, 255)
+
+
+def test_which_parameters_requantize_by_multiply_add():
+    """any offset of a byte up to right shift 23, offset 0 at every shift; and at the edge of what fits the
+    largest accumulators still come out right"""
+    import ctypes as C
+    lib = mh.load()
+    out = C.c_uint8()
+    for shift in range(32):
+        for zp in (0, 1, 3, 127, 128, 255, -1, -128, -300, 700, 32767):
+            for mult in (1, 2 ** 30 - 1, 2 ** 30, 2 ** 31 - 1):
+                held = shift == 0 or 2 * abs(zp) + 1 <= 2 ** (32 - shift)
+                for acc in (-2 ** 31, -2 ** 31 + 1, -2 ** 30, -1, 0, 1, 2 ** 30, 2 ** 31 - 1):
+                    rc = lib.mace_hip_requant_table_u8(acc, mult, shift, zp, 0, 255, C.byref(out))
+                    assert (rc, out.value) == (int(held), orc.requant_fixed_u8(acc, mult, shift, zp, 0, 255)), \
+                        (acc, mult, shift, zp)
 
 
 def test_float_requant_matches_oracle():
