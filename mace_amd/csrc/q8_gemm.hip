@@ -2959,6 +2959,7 @@ int Q8Call::general() {
       j.rows = nb * n;
       j.blocks = (j.rows * (kp / 16) + REPACK_PIECES - 1) / REPACK_PIECES;
     } else {
+      // (the bound of an earlier launch, kept: what was refused stays refused)
       MH_CHECK(ctx, (kp / 64) <= 65535, "depth too large to repack");
       mh_plan_aux(ctx, MACE_HIP_AUX_PACK_TRANSPOSE);
       j.tiles_n = (int)((n + 127) / 128);
