@@ -1197,7 +1197,10 @@ extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
   // still skips it and reads past the input; here a padded 1x1 takes the im2col path.)
   const bool in_place = k_h == 1 && k_w == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 &&
                         pad_w == 0;
-  if (!in_place) {
+  // (An image without a pixel, all padding: the strip and depth-split kernels load what lies outside the image
+  // from the nearest pixel inside, and there is none.  The kernels below load a zero-point page or nothing.)
+  const bool has_pixels = in_h > 0 && in_w > 0;
+  if (!in_place && has_pixels) {
     bool taken = false;
     MH_RETURN_IF_ERROR(conv_short(ctx, input, filter, bias, n, in_h, in_w, cin, cout, k_h, k_w,
                                   stride_h, stride_w, pad_h >> 1, pad_w >> 1, out_h, out_w,
@@ -1210,7 +1213,7 @@ extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
                                  shift, out_zp, clamp_min, clamp_max, out, &taken));
     if (taken) return MACE_HIP_SUCCESS;
   }
-  {
+  if (has_pixels) {
     bool taken = false;
     MH_RETURN_IF_ERROR(conv_ksplit(ctx, input, filter, bias, n, in_h, in_w, cin, cout, k_h, k_w,
                                    stride_h, stride_w, pad_h >> 1, pad_w >> 1, out_h, out_w,

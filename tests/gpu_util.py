@@ -74,3 +74,10 @@ def kernel_mask(ctx, mask):
         yield
     finally:
         ctx.lib.mace_hip_ctx_set_kernel_mask(ctx.handle, 0)
+
+
+# (in_h, in_w, cin, cout, pad_h, pad_w): images without a pixel, all padding, of the shapes that the strip kernels and
+# the depth split take otherwise
+EMPTY_IMAGES = [(0, 8, 3, 8, 4, 4), (8, 0, 3, 8, 4, 4), (0, 200, 16, 16, 4, 4), (200, 0, 16, 16, 4, 4),
+                (0, 60, 32, 32, 40, 4), (0, 14, 128, 64, 6, 4), (14, 0, 128, 64, 4, 6), (0, 7, 512, 64, 5, 4),
+                (0, 0, 64, 40, 5, 5), (0, 20, 50, 24, 6, 4)]

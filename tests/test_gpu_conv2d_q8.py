@@ -12,7 +12,7 @@ import pytest
 
 from mace_amd import lib as mh
 from oracle import mace_oracle as orc
-from gpu_util import c_, ptr
+from gpu_util import EMPTY_IMAGES, c_, ptr
 
 pytestmark = pytest.mark.gpu
 GOLDEN = json.load(open(os.path.join(os.path.dirname(__file__), "golden", "reference_vectors.json")))
@@ -314,6 +314,24 @@ def test_conv2d_q8_strips_of_any_channel_count(ctx, n, cout, cin, hw, k, off, fa
     got = out.cpu().numpy()
     np.testing.assert_array_equal(got[16 + off:16 + off + want.size].reshape(want.shape), want)
     assert (got[:16 + off] == 0xA5).all() and (got[16 + off + want.size:] == 0xA5).all()
+
+
+@pytest.mark.parametrize("in_h,in_w,cin,cout,pad_h,pad_w", EMPTY_IMAGES)
+def test_conv2d_q8_images_without_a_pixel(ctx, in_h, in_w, cin, cout, pad_h, pad_w):
+    """all padding: every patch is the zero point"""
+    import torch
+    rng = np.random.default_rng(cin + cout)
+    f = rng.integers(0, 256, (cout, 3, 3, cin), dtype=np.uint8)
+    bias = rng.integers(-2 ** 15, 2 ** 15, cout).astype(np.int32)
+    want = orc.conv2d_q8_nhwc(np.empty((1, in_h, in_w, cin), np.uint8), f, bias, 1, in_h, in_w, cin, cout, 3, 3, (1, 1),
+                              (pad_h, pad_w), 0.02, 90, 0.01, 127, np.float32(0.02 * 0.01), 0.05, 10)
+    none, fd, bd = torch.empty(16, dtype=torch.uint8, device="cuda"), torch.from_numpy(f).cuda(), torch.from_numpy(bias).cuda()
+    out = torch.empty(want.size, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    ctx.call("mace_hip_conv2d_q8_nhwc", none.data_ptr(), fd.data_ptr(), bd.data_ptr(), 1, in_h, in_w, cin, cout, 3, 3, 1, 1,
+             pad_h, pad_w, 0.02, 90, 0.01, 127, float(np.float32(0.02 * 0.01)), 0.05, 10, 0, 255, out.data_ptr())
+    ctx.sync()
+    np.testing.assert_array_equal(out.cpu().numpy().reshape(want.shape), want)
 
 
 KSPLIT_CASES = [  # batch, cout, cin, in_h, in_w, k_h, k_w, padding, strides
