@@ -571,7 +571,11 @@ int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
                       int64_t k_w, int stride_h, int stride_w, int pad_top, int pad_left, int64_t out_h,
                       int64_t out_w, float input_scale, int32_t input_zp, float filter_scale, int32_t filter_zp,
                       float bias_scale, int32_t mult, int shift, int32_t out_zp, int clamp_min, int clamp_max,
-                      uint8_t *out, int fused, bool *taken);
+                      uint8_t *out, double other, bool *taken);
+// Estimates of what a gathered convolution takes otherwise, in us: the one-launch kernel (conv_planes.hip; piece: bytes it
+// loads at a time), the gathering or patch-matrix GEMM (q8_gemm.hip).
+double mh_q8_conv_small_us(const mace_hip_ctx *ctx, int64_t cout, int64_t columns, int64_t depth, int piece);
+double mh_q8_conv_gather_us(const mace_hip_ctx *ctx, int64_t cout, int64_t columns, int64_t depth, bool patch_matrix);
 int mh_q8_gemm(mace_hip_ctx *ctx, const uint8_t *lhs, int lhs_order, const uint8_t *rhs,
                int rhs_order, void *out, int out_order, bool out_u8, int64_t batch,
                int64_t rows, int64_t depth, int64_t cols, int lhs_batched, int rhs_batched,

@@ -1230,16 +1230,7 @@ extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
   const bool small_gather = !in_place && in_h * in_w * cin < (1ll << 31) &&
                             mh_q8_small_problem(ctx, 1, cout, columns, depth, small_vec, cin % 64 != 0) &&
                             !(ctx->kernel_mask & MH_MASK_NO_SMALL);
-  // Anything else goes through padded planes where those are faster.
-  if (!in_place) {
-    bool taken = false;
-    MH_RETURN_IF_ERROR(mh_q8_conv_planes(ctx, input, filter, bias, n, in_h, in_w, cin, cout, k_h, k_w, stride_h,
-                                         stride_w, pad_h >> 1, pad_w >> 1, out_h, out_w, input_scale, input_zp,
-                                         filter_scale, filter_zp, bias_scale, mult, shift, out_zp, clamp_min,
-                                         clamp_max, out, small_gather ? (small_vec ? 16 : (cin % 4 == 0 ? 4 : 1)) : 0, &taken));
-    if (taken) return MACE_HIP_SUCCESS;
-  }
-  // ... unless the patches make at most one round of 128 x 128 tiles with a long k: the gathering
+  // No gathering where the patches make at most one round of 128 x 128 tiles with a long k: the gathering
   // tiled kernel then leaves most CUs without a tile for its whole length, while the patch matrix
   // is small and the eight-wavefront GEMM kernel takes it (7x7x512 -> 512, 3 x 3, batch 64: 46.4 ->
   // 31.6 us; 7x7x1024 -> 1024: 86.7 -> 52.2; 14x14x256 -> 512 at stride 2: 28.4 -> 20.4; ties at 196
@@ -1253,7 +1244,25 @@ extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
                       (!im2col_one_round && !in_place && cin % 64 == 0 && depth >= 192 &&
                        ((uintptr_t)input % 16 == 0) && ((uintptr_t)filter % 16 == 0) &&
                        in_h * in_w * cin < (1ll << 31));
-  const int64_t kp = (int64_t)mh_align_up((size_t)(depth > 0 ? depth : 1), 64);
+  const int64_t kp = (int64_t)mh_align_up((size_t)(depth > 0 ? depth : 1), 64);   // row of a patch matrix
+  // All of these go through padded planes where that is faster.  (Up to nine taps of 64 channels stay with the kernel that
+  // keeps the filter in LDS: 56 x 56 x 64 -> 64 at batch 64 21.5 us, on planes 28.4.)
+  if (!in_place && (small_gather || cin % 64 != 0 || depth > 576)) {
+    bool taken = false;
+    // (a patch matrix of one tap, a 1 x 1 filter at a stride, is a fraction of the input, which the planes copy whole: 30 x
+    // 30 x 995 -> 818 at stride 2, batch 7, 21.0 us, on planes 32.9, but 28 x 28 x 523 -> 129 at 21 28.8 and 21.3)
+    const bool by_pieces = cin % 16 == 0 && (uintptr_t)input % 16 == 0;
+    const double other = small_gather ? mh_q8_conv_small_us(ctx, cout, columns, depth, small_vec ? 16 : (cin % 4 == 0 ? 4 : 1))
+                         : gather || (im2col_one_round && cin % 64 == 0 && by_pieces)
+                             ? mh_q8_conv_gather_us(ctx, cout, columns, depth, !gather)
+                         : k_h * k_w == 1 && stride_h * stride_w > 1 ? (by_pieces ? 13 + 0.3e-6 * columns * kp : 16.5 + 1.9e-6 * columns * kp)
+                                          : HUGE_VAL;
+    MH_RETURN_IF_ERROR(mh_q8_conv_planes(ctx, input, filter, bias, n, in_h, in_w, cin, cout, k_h, k_w, stride_h,
+                                         stride_w, pad_h >> 1, pad_w >> 1, out_h, out_w, input_scale, input_zp,
+                                         filter_scale, filter_zp, bias_scale, mult, shift, out_zp, clamp_min,
+                                         clamp_max, out, other, &taken));
+    if (taken) return MACE_HIP_SUCCESS;
+  }
   size_t need = sizeof(int32_t) * cout + 4096 +
                 conv_gemm_scratch(cout, depth, columns, !in_place || depth % 16 == 0);
   if (!in_place && !gather) need += (size_t)columns * kp + 4096;

@@ -1,6 +1,8 @@
 // Quantized Conv2D (NHWC) for any channel count, filter, stride and padding: the input copied once into padded
 // planes that the multiplying kernel stages in LDS as they lie.  (mace/ops/conv_2d.cc:201-412: Im2col and the
 // gemmlowp product it feeds; here no patch matrix exists.)
+#include <math.h>
+
 #include <algorithm>
 
 #include "common.h"
@@ -566,40 +568,59 @@ bool plane_fits(const PlaneShape &s) {
 }
 }  // namespace
 
-// Time that the one-launch GEMM kernel (q8_gemm_fused_small_kernel) would take, in us: its workgroups' depth, in
-// pieces of 16, 4 or 1 bytes, one after the other on a CU where there are more than CUs.  (3 x 3, model and measured:
-// 61 x 59 x 29 -> 80 at batch 12 39 and 34, 32 x 31 x 18 -> 42 at 41 15 and 14, 33 x 34 x 112 -> 214 at 22 30 and 32,
-// 20 x 22 x 35 -> 38 at 3 16 and 15, 112 x 112 x 24 -> 16 at 10 23 and 18, 36 x 36 x 20 -> 112 at 1 6.5 and 6.1.)
-static double fused_small_us(const mace_hip_ctx *ctx, int64_t cout, int64_t columns, int64_t depth, int piece) {
+// Time that the one-launch GEMM kernel (q8_gemm_fused_small_kernel) would take, in us: a workgroup's depth, in
+// pieces of 16, 4 or 1 bytes, and those of a CU's workgroups together, whose square sum it follows.  (Within 3 % in the
+// median of 300 drawn 3 x 3 layers, 8 % in nine of ten; model and measured: 61 x 59 x 29 -> 80 at batch 12 39 and 34, 33 x
+// 34 x 112 -> 214 at 22 31 and 32, 20 x 22 x 35 -> 38 at 3 16 and 15, 36 x 36 x 20 -> 112 at 1 5.8 and 6.1.)
+double mh_q8_conv_small_us(const mace_hip_ctx *ctx, int64_t cout, int64_t columns, int64_t depth, int piece) {
   const double cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  const double wgs = (double)((cout + 63) / 64) * (double)((columns + 63) / 64);
-  const double alone = piece == 16 ? 0.006 : (piece == 4 ? 0.01 : 0.035), packed = piece == 16 ? 0.0033 : (piece == 4 ? 0.007 : 0.022);
-  return 3.7 + std::max(alone * depth + 1, wgs / cu * (packed * depth + 1));
+  const double wgs = (double)((cout + 63) / 64) * (double)((columns + 63) / 64) / cu;
+  if (piece == 16) return 4.6 + hypot(0.0076 * depth - 0.27, wgs * (0.0034 * depth + 0.45));
+  if (piece == 4) return 2.0 + hypot(0.0137 * depth + 2.3, wgs * (0.002 * depth + 1.45));
+  return 5.6 + hypot(0.0315 * depth - 0.25, wgs * (0.0124 * depth + 0.89));
 }
 
-// *taken = false: not a call for it.  `fused`: bytes of the pieces in which the one-launch GEMM kernel
-// would run the call; 0: an im2col or a gathering GEMM would.
+// Time of the two launches, in us: their start, the bytes that the first moves, and what a CU's tiles cost each (the
+// hand-over, the stages' bytes) and one after the other (k steps).  By tile form and by whether a filter row is three k
+// steps; 32 x 256, which few calls take, as 64 x 256.  Within 5 % in the median of 1400 layers of all kinds, 13 % in nine
+// of ten.
+struct PlaneCost { double start, per_mb, per_tile, per_staged, per_step; };   // (staged: 100 KB)
+static double planes_us(int form, const ConvPlaneParams &p, const PlaneShape &s, int64_t staged, int64_t span, int64_t at_once) {
+  static const PlaneCost kThree[3] = {{6.8, 0.178, 1.76, 1.23, 0.111}, {7.8, 0.183, 0.565, 0.926, 0.060}, {8.3, 0.186, 0.313, 0.722, 0.038}};
+  static const PlaneCost kAny[3] = {{9.3, 0.121, 1.40, 1.77, 0.096}, {9.0, 0.15, 0.09, 1.24, 0.072}, {9.2, 0.36, 0.02, 1.0, 0.033}};
+  const PlaneCost &c = (p.spr == 3 && p.pieces == 2 ? kThree : kAny)[std::max(0, form - 1)];
+  const double moved = (double)s.n * s.in_h * s.in_w * s.cin + (double)p.plane_bytes * p.slabs * p.pieces;
+  return c.start + c.per_mb * moved / 1e6 + at_once * span * (c.per_tile + c.per_staged * staged / 1e5) +
+         c.per_step * span * p.slabs * p.steps;
+}
+
+// *taken = false: not a call for it.  `other`: an estimate of the time, in us, that the call takes otherwise (HUGE_VAL
+// where a patch matrix of several taps is written out: of 700 such layers none was faster than the planes).
 //
 // Two launches take 8.2 us at the least where a caller waits for none of them, one 4.  Against the kernels that
 // took these calls before (3 x 3, us): an im2col of odd channel counts 34 x 36 x 108 -> 28 at batch 52 146 -> 17.5,
 // 96 x 97 x 38 -> 21 at 7 65.6 -> 13.3, 7 x 9 x 797 -> 209 at 16 55.6 -> 17.8, 80 x 81 x 97 -> 35 of one image 24 -> 10;
 // of whole pieces 27 x 29 x 224 -> 24 at 37 29.7 -> 15.4, 14 x 14 x 256 -> 256 at 64 27 -> 19, 7 x 7 x 512 -> 512 at 64
-// 29 -> 24; a gathering GEMM on 128 channels 28 x 28 -> 128 at 64 21.3 -> 18.9; on 64 channels the resident-tile
-// kernel keeps its calls (56 x 56 -> 64 at 64 21.5, here 28.4).
+// 29 -> 24; a gathering GEMM on 128 channels 28 x 28 -> 128 at 64 21.3 -> 18.9.  A tile of 64 x 256 reads three fragments from LDS per two
+// products, the gathering GEMM's 256 x 256 eight per sixteen, so layers that fill its rounds stay there, and so do
+// strides that leave most of what the first launch copies unused: 56 x 56 x 512 -> 256 at stride 2, batch 64, 84 against
+// 132 here, 28 x 28 x 1024 -> 1024 at stride 2, 64, 143 against 203, 28 x 28 x 256 -> 256 at 64 46 against 52, 56 x 56 x
+// 128 -> 64 at stride 2, 64, 18.0 against 24.9; but 28 x 28 x 512 -> 256 at 32 49 against 43, 56 x 56 x 256 -> 256 at 8
+// 30 against 25.  Of 712 gathered layers 104 lost more than 3 % here (the worst 71 %) before both times were estimated,
+// 11 since (10 %).
 int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, const int32_t *bias,
                       int64_t n, int64_t in_h, int64_t in_w, int64_t cin, int64_t cout, int64_t k_h,
                       int64_t k_w, int stride_h, int stride_w, int pad_top, int pad_left, int64_t out_h,
                       int64_t out_w, float input_scale, int32_t input_zp, float filter_scale, int32_t filter_zp,
                       float bias_scale, int32_t mult, int shift, int32_t out_zp, int clamp_min, int clamp_max,
-                      uint8_t *out, int fused, bool *taken) {
+                      uint8_t *out, double other, bool *taken) {
   *taken = false;
   const PlaneShape s{n, in_h, in_w, cin, cout, k_h, k_w, stride_h, stride_w, pad_top, pad_left, out_h, out_w};
   if (!plane_fits(s) || filter_zp < 0 || filter_zp > 255 || (ctx->kernel_mask & MH_MASK_NO_CONV_SHORT))
     return MACE_HIP_SUCCESS;
   if (shift < 0 || shift > 31 || clamp_min < 0 || clamp_max > 255 || clamp_min > clamp_max)
     return MACE_HIP_SUCCESS;   // (the general path reports these)
-  const int64_t depth = k_h * k_w * cin, columns = n * out_h * out_w;
-  if (!fused && cin % 64 == 0 && depth <= 576) return MACE_HIP_SUCCESS;
+  const int64_t columns = n * out_h * out_w;
   ConvPlaneParams p{};
   if (!mh_make_requant(mult, shift, out_zp, clamp_min, clamp_max, &p.rq)) return MACE_HIP_SUCCESS;
   p.by_mad = requant_by_mad(p.rq);
@@ -628,13 +649,12 @@ int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
   }
   if (!plan.fits || plan.lds > ctx->lds_bytes || !mh_arena_can_hold(ctx, (size_t)plan.scratch + 8 * 256 + 4 * cout))
     return MACE_HIP_SUCCESS;
-  if (fused) {
-    const double moved = (double)n * in_h * in_w * cin + (double)p.plane_bytes * p.slabs * p.pieces;
-    const double rounds = (double)p.tiles_x * p.tiles_p / cu, steps = (double)p.slabs * p.steps;
-    const double us = 8.3 + moved / 3.5e6 + (form == mhv::PLANES_64x256 ? rounds * (1.2 + 0.1 * steps)
-                                                                        : rounds * (p.pieces == 1 ? 1.8 : 0.6 + 0.035 * steps));
-    if (fused_small_us(ctx, cout, columns, depth, fused) <= 1.1 * us) return MACE_HIP_SUCCESS;
-  }
+  const int64_t at_once = std::max<int64_t>(1, std::min<int64_t>(ctx->lds_bytes / std::max<int64_t>(1, plan.lds), 1024 / plan.threads));
+  // (workgroups of a channel tile: as many as fit at once)
+  const int64_t room = std::min<int64_t>(p.tiles_p, std::max<int64_t>(1, cu * at_once / p.tiles_x));
+  const int64_t staged = (p.keep ? 0 : (int64_t)p.slabs * p.steps * plan.xt * 32) + (int64_t)p.slabs * p.pieces * p.row_bytes;
+  if (planes_us(form, p, s, staged, (p.tiles_p + room - 1) / room, (room * p.tiles_x + cu - 1) / cu) >= 0.95 * other)
+    return MACE_HIP_SUCCESS;
   *taken = true;
 
   MH_RETURN_IF_ERROR(mh_arena_reserve(ctx, (size_t)plan.scratch + 8 * 256 + sizeof(int32_t) * cout));

@@ -2637,6 +2637,27 @@ static MhTile mh_q8_tile_choice(int64_t xn, int64_t yn, int64_t batch, int64_t c
   return MH_TILE_SMALL;
 }
 
+// What a convolution of whole 64-channel pieces takes here, launches before the GEMM included: with its patches
+// gathered, by the kernel and the tile shape that Q8Call chooses for it, or through a patch matrix by the eight-wavefront
+// kernel.  (Fitted to 712 layers of 0.2 to 400 G operations: within 2 % in the median, 10 % in nineteen of twenty.)
+double mh_q8_conv_gather_us(const mace_hip_ctx *ctx, int64_t cout, int64_t columns, int64_t depth, bool patch_matrix) {
+  const int64_t cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  const double k = depth / 1e3;
+  if (patch_matrix) return 11.5 + 2.95 * k + 0.3 * columns * k / 1e3;
+  if (columns >= 256 && 2 * (XRES_SC_BYTES + (size_t)(cout <= 64 ? 64 : 128) * depth) <=
+                            (ctx->lds_bytes > 0 ? (size_t)ctx->lds_bytes : 65536))
+    return std::max(17.0, 9 + 0.16 * columns * k / 1e3);
+  auto rounds = [&](int tx, int ty, int64_t slots) {
+    return (double)((((cout + tx - 1) / tx) * ((columns + ty - 1) / ty) + slots - 1) / slots);
+  };
+  switch (mh_q8_tile_choice(cout, columns, 1, cu)) {
+    case MH_TILE_BIG: return 4.5 + rounds(256, 256, cu) * (10.5 + 14 * k);
+    case MH_TILE_MEDIUM: return 7.5 + rounds(128, 128, cu) * (1.7 + 2.5 * k) + rounds(128, 128, 2 * cu) * 5.3 * k;
+    case MH_TILE_SKINNY: return 7.3 + rounds(64, 256, cu) * (0.35 + 4.9 * k) + rounds(64, 256, 2 * cu) * 4.4 * k;
+    default: return 4 + rounds(64, 64, cu) * (4 + 4.4 * k);
+  }
+}
+
 static bool mh_q8_stream_shape(int64_t depth, int64_t xn, int64_t yn) {
   return depth >= 16 && depth <= 64 && depth % 16 == 0 && xn >= 16 && xn <= 128 && xn % 16 == 0 &&
          yn >= 1024;
