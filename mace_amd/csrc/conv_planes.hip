@@ -615,6 +615,8 @@ int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
                       float bias_scale, int32_t mult, int shift, int32_t out_zp, int clamp_min, int clamp_max,
                       uint8_t *out, double other, bool *taken) {
   *taken = false;
+  // (the two launches' start alone, before a tile's geometry is worked out: calls of 4 - 6 us notice a tenth)
+  if (0.95 * other <= 7.5) return MACE_HIP_SUCCESS;
   const PlaneShape s{n, in_h, in_w, cin, cout, k_h, k_w, stride_h, stride_w, pad_top, pad_left, out_h, out_w};
   if (!plane_fits(s) || filter_zp < 0 || filter_zp > 255 || (ctx->kernel_mask & MH_MASK_NO_CONV_SHORT))
     return MACE_HIP_SUCCESS;
