@@ -1019,7 +1019,10 @@ __global__ __launch_bounds__(WX *WY * 64, OCC) void q8_gemm_dma_kernel(GemmParam
     // were fetched in the k step above), before going on: one barrier covers both.
     // Slabs up to kt+AHEAD-1 have been issued (past the end: repeats of the last slab, see
     // below), so exactly AHEAD-2 slabs newer than kt+1 may stay in flight.
-    wait_vmcnt<(AHEAD - 2) * (LX + LY)>();
+    // (REUSE: a read is done when its data is back, not when it was issued; small wavefront tiles flip their last
+    // fragments only behind the barrier, and another wavefront's transfer overtook the reads: seen with two
+    // 128 x 128 workgroups on a CU.  In the 4 x 4 tile nothing is left to wait for.)
+    wait_vmcnt<(AHEAD - 2) * (LX + LY), REUSE>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     int next = stage + 1;

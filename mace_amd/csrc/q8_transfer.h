@@ -29,11 +29,12 @@ __device__ inline void dma_16B(mh_rsrc rs, uint32_t lane_off, uint32_t uniform_o
                                            16, (int)lane_off, (int)uniform_off, 0, 0);
 }
 
-// s_waitcnt vmcnt(N) alone (expcnt / lgkmcnt fields left at "no wait")
-template <int N>
+// s_waitcnt vmcnt(N) alone (expcnt / lgkmcnt fields left at "no wait"), or with LDS for the wavefront's LDS
+// accesses too (lgkmcnt(0))
+template <int N, bool LDS = false>
 __device__ inline void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit field");
-  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+  __builtin_amdgcn_s_waitcnt((LDS ? 0x0070 : 0x0f70) | (N & 15) | ((N >> 4) << 14));
 }
 
 }  // namespace

@@ -188,7 +188,7 @@ inline uint32_t __umul24(uint32_t a, uint32_t b) { return (a & 0xffffff) * (b & 
 inline int __mul24(int a, int b) { return (int)((uint32_t)(a << 8 >> 8) * (uint32_t)(b << 8 >> 8)); }
 namespace mhv { enum { PLANES_FORMS = 4 }; }
 inline size_t mh_align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
-template <int N> inline void wait_vmcnt() {}
+template <int N, bool LDS = false> inline void wait_vmcnt() {}
 // global -> LDS transfer: lane l's 16 bytes land at lds_wave_base + 16 l
 inline void dma_16B(const uint8_t *g, uint8_t *lds_wave_base) {
   memcpy(lds_wave_base + 16 * (threadIdx.x & 63), g, 16);

@@ -1,7 +1,8 @@
-"""Distances between instructions that the compiler keeps for its own but not for inline assembly,
-checked in the machine code of the built library: a v_permlane32_swap must come at least two wait
+"""What only the machine code of the built library shows.  Distances between instructions that the compiler
+keeps for its own but not for inline assembly: a v_permlane32_swap must come at least two wait
 states after the vector instruction that writes one of its operands (an instruction in between counts
-one, s_nop N counts N + 1)."""
+one, s_nop N counts N + 1).  And waits that it does not place: where a transfer behind a barrier overwrites
+the LDS that was read before it, no read may be outstanding at the barrier."""
 import os
 import re
 import struct
@@ -66,6 +67,48 @@ def too_close(listing, wait=2):
                 written |= registers(operands[1])
             recent.append((text, written, 0))
     return swaps, bad
+
+
+# the ring kernel with slabs of 128 bytes: its transfers refill the stage of the slab being multiplied
+REFILLS = re.compile(r"q8_gemm_dma_kernelI(Li\d+E){5}[hi]Li\d+E(Lb[01]E){2}Li128E")
+
+
+def reads_at_barriers(listing):
+    """{kernel: [LDS reads outstanding at each of its barriers]} of the kernels that REFILLS names, in the order of the
+    listing; LDS reads return in order, lgkmcnt(N) leaves N"""
+    found, kernel, out = {}, None, 0
+    for line in listing.splitlines():
+        label = re.match(r"[0-9a-f]+ <(.*)>:", line)
+        if label:
+            kernel, out = label[1] if REFILLS.search(label[1]) else None, 0
+            continue
+        text = line.split("//")[0].strip()
+        if kernel is None:
+            continue
+        if text.startswith("ds_read"):
+            out += 1
+        elif text.startswith("s_waitcnt"):
+            left = re.search(r"lgkmcnt\((\d+)\)", text)
+            out = min(out, int(left[1])) if left else out
+        elif text.startswith("s_barrier"):
+            found.setdefault(kernel, []).append(out)
+    return found
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="needs ROCm's llvm-objdump")
+def test_no_lds_read_is_outstanding_where_its_stage_is_refilled(tmp_path):
+    name = "q8_gemm_dma_kernelILi2ELi2ELi2ELi2ELi2EhLi2ELb1ELb0ELi128E"
+    head, read, wait, barrier = "0000000000001000 <%s>:\n" % name, "\tds_read_b128 v[0:3], v4\n", \
+        "\ts_waitcnt vmcnt(0) lgkmcnt(%d)\n", "\ts_barrier\n"
+    assert reads_at_barriers(head + read + read + wait % 1 + barrier + wait % 0 + barrier) == {name: [1, 0]}
+    kernels = {}
+    for i, blob in enumerate(code_objects(mh.LIB_PATH)):
+        path = tmp_path / ("%d.co" % i)
+        path.write_bytes(blob)
+        kernels.update(reads_at_barriers(subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", str(path)], check=True,
+                                                        capture_output=True, text=True).stdout))
+    assert len(kernels) >= 20 and all(len(v) >= 3 for v in kernels.values()), kernels   # prologue, loop, epilogue
+    assert not any(n for v in kernels.values() for n in v), {k: v for k, v in kernels.items() if any(v)}
 
 
 def test_the_check_itself():
