@@ -202,8 +202,10 @@ int mace_hip_memcpy_d2h(mace_hip_ctx *ctx, void *dst_host, const void *src_dev, 
  * calls (GemmParam::should_cache_pack_ with Tensor::is_weight(), mace/ops/delegator/gemm.h:28-33,
  * mace/ops/arm/base/gemm.cc:560-576).  The counterpart here: once a device buffer is registered,
  * every uint8 GEMM / Conv2D call on this context whose lhs or rhs pointer equals device_ptr (and
- * fits in `bytes`) reuses the k-contiguous panel and the row sums derived from it on first use
- * instead of rebuilding them per call.  The caller must not change the buffer while it is
+ * fits in `bytes`) reuses the k-contiguous panel and the row sums (a convolution on padded planes: the
+ * filter in fragment order and its channels' sums) derived from it on first use
+ * instead of rebuilding them per call; a kernel that reads the buffer as it lies derives nothing.
+ * The caller must not change the buffer while it is
  * registered; register it again (or unregister it) after a change.  Unregistering frees what
  * was derived (after synchronizing the stream); so does destroying the context. */
 int mace_hip_weight_register(mace_hip_ctx *ctx, const void *device_ptr, size_t bytes);

@@ -27,23 +27,32 @@ struct mh_weight_panel {
   int32_t *sums;        // [nb][n], device memory owned by the cache
   bool flipped;         // the panel holds the bytes already shifted to int8 (one consumer only)
 };
+// ... and what the convolution on padded planes derives: the filter in fragment order, its channels' sums.
+struct mh_weight_planes {
+  int64_t cin, cout, k_h, k_w;
+  int64_t channels;     // packed: cout and zeros
+  uint8_t *packed;      // device memory owned by the cache, as the sums are
+  int32_t *sums;
+};
 struct mh_weight {
   const void *ptr;
   size_t bytes;
   std::vector<mh_weight_panel> panels;
+  std::vector<mh_weight_planes> planes;
 };
 
 // Frees what was derived from a weight -- or, while a captured graph may still read it (or on a
 // plan-only context, whose panels are not real memory), hands it to `retired` / forgets it.
 inline void mh_weight_drop_panels(mh_weight *w, bool real_memory, std::vector<void *> *retired) {
-  for (mh_weight_panel &c : w->panels) {
-    for (void *p : {(void *)c.panel, (void *)c.sums}) {
-      if (!p || !real_memory) continue;
-      if (retired) retired->push_back(p);
-      else (void)hipFree(p);
-    }
-  }
+  auto drop = [&](void *p) {
+    if (!p || !real_memory) return;
+    if (retired) retired->push_back(p);
+    else (void)hipFree(p);
+  };
+  for (mh_weight_panel &c : w->panels) { drop(c.panel); drop(c.sums); }
+  for (mh_weight_planes &c : w->planes) { drop(c.packed); drop(c.sums); }
   w->panels.clear();
+  w->planes.clear();
 }
 
 // A constant operand in HOST memory (mace_hip_host_weight_register): its device copy, which the
@@ -269,6 +278,13 @@ void *mh_arena_take(mace_hip_ctx *ctx, size_t bytes);   // 256-byte aligned, aft
 inline bool mh_arena_can_hold(const mace_hip_ctx *ctx, size_t bytes) {
   return ctx->arena_used + bytes + 16 * 256 <= ctx->arena_bytes ||
          !(ctx->no_alloc || ctx->capturing || ctx->arena_used != 0);
+}
+// The registration of an operand as a constant weight, if there is one that covers it.
+inline mh_weight *mh_find_weight(mace_hip_ctx *ctx, const void *src, size_t bytes) {
+  if (ctx->no_alloc) return nullptr;   // (the cache allocates on first use)
+  for (mh_weight &w : ctx->weights)
+    if (w.ptr == src && bytes <= w.bytes) return &w;
+  return nullptr;
 }
 inline size_t mh_align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 struct ArenaScope {

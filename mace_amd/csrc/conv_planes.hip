@@ -18,6 +18,8 @@ struct ConvPlaneParams {
   const int32_t *bias;
   uint8_t *planes, *packed;     // written by the first launch: padded input, filter in fragment order
   int32_t *psum, *cx;           // ... sums of its pixels' bytes, corrections by channel
+  int32_t *wsums;               // a registered filter's sums by channel: kept with `packed`; else null
+  bool kept;                    // ... both are there from an earlier call
   uint8_t *out;
   int n, in_h, in_w, cin, cout, k_h, k_w, sh, sw, pt, pl, out_h, out_w;
   int depth, columns, tiles_x, tiles_p, channels;   // channels: cout in whole tiles
@@ -121,6 +123,10 @@ __global__ __launch_bounds__(256) void q8_conv_planes_pack_kernel(ConvPlaneParam
 #pragma unroll
     for (int u = 0; u < PACK_PIXELS; ++u)
       if (g == 0 && px0 + u * slots < p.pixels) p.psum[px0 + u * slots] = sum[u];
+  } else if (p.kept) {
+    const int x = ((int)blockIdx.x - p.pixel_blocks) * 256 + (int)threadIdx.x;
+    if (x < p.channels)
+      p.cx[x] = (int32_t)((uint32_t)p.xcoef * (uint32_t)p.wsums[x] + (uint32_t)(p.bias && x < p.cout ? p.bias[x] : 0));
   } else {
     const int lane = threadIdx.x & 63;
     const int x = ((int)blockIdx.x - p.pixel_blocks) * 4 + (int)(threadIdx.x >> 6);
@@ -161,8 +167,10 @@ __global__ __launch_bounds__(256) void q8_conv_planes_pack_kernel(ConvPlaneParam
       }
     }
     for (int m = 32; m > 0; m >>= 1) sum += __shfl_xor(sum, m, 64);
-    if (lane == 0)
+    if (lane == 0) {
+      if (p.wsums) p.wsums[x] = sum;
       p.cx[x] = (int32_t)((uint32_t)p.xcoef * (uint32_t)sum + (uint32_t)(p.bias && real ? p.bias[x] : 0));
+    }
   }
 }
 
@@ -663,11 +671,45 @@ int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
   ArenaScope scope(ctx);
   const int32_t *bias_used = nullptr;
   MH_RETURN_IF_ERROR(mh_conv_bias(ctx, bias, cout, input_scale, filter_scale, bias_scale, &bias_used));
-  p.packed = (uint8_t *)mh_arena_take(ctx, (size_t)plan.packed_bytes);
+  // A registered filter is packed and summed once, into memory of its own.  (Not where that cannot be had, nor in a
+  // capture, which would fill it at a replay only: then as any other filter.)
+  mh_weight *weight = mh_find_weight(ctx, filter, (size_t)(cout * p.depth));
+  mh_weight_planes built{cin, cout, k_h, k_w, p.channels, nullptr, nullptr};
+  auto give_back = [&]() {
+    if (!ctx->plan_only) { (void)hipFree(built.packed); (void)hipFree(built.sums); }
+    built.packed = nullptr;
+  };
+  if (weight) {
+    for (const mh_weight_planes &c : weight->planes)
+      if (c.cin == cin && c.cout == cout && c.k_h == k_h && c.k_w == k_w && c.channels >= p.channels) {
+        p.kept = true;
+        p.packed = c.packed;
+        p.wsums = c.sums;
+      }
+    if (!p.kept && ctx->plan_only) {   // (addresses stand in for the two buffers)
+      built.packed = (uint8_t *)(uintptr_t)0x300000000ull;
+      built.sums = (int32_t *)(uintptr_t)0x300000000ull;
+    } else if (!p.kept && !ctx->capturing) {
+      if (hipMalloc((void **)&built.packed, (size_t)plan.packed_bytes) != hipSuccess ||
+          hipMalloc((void **)&built.sums, (size_t)p.channels * 4) != hipSuccess) {
+        (void)hipGetLastError();
+        give_back();
+      }
+    }
+    if (built.packed) {
+      p.packed = built.packed;
+      p.wsums = built.sums;
+    }
+  }
+  if (p.kept) plan.pack_blocks = p.pixel_blocks + (p.channels + 255) / 256;
+  if (!p.packed) p.packed = (uint8_t *)mh_arena_take(ctx, (size_t)plan.packed_bytes);
   p.psum = (int32_t *)mh_arena_take(ctx, (size_t)plan.psum_bytes);
   p.cx = (int32_t *)mh_arena_take(ctx, (size_t)plan.cx_bytes);
   p.planes = (uint8_t *)mh_arena_take(ctx, (size_t)plan.planes_bytes);
-  if (!p.packed || !p.psum || !p.cx || !p.planes) return mh_fail(ctx, MACE_HIP_RUNTIME_ERROR, "arena slice unavailable");
+  if (!p.packed || !p.psum || !p.cx || !p.planes) {
+    give_back();
+    return mh_fail(ctx, MACE_HIP_RUNTIME_ERROR, "arena slice unavailable");
+  }
   p.in = input; p.filter = filter; p.bias = bias_used; p.out = out;
   const uint32_t zl = (uint32_t)filter_zp - 128u, zr = (uint32_t)input_zp - 128u;
   p.xcoef = (int32_t)(0u - zr); p.ycoef = (int32_t)(0u - zl); p.yadd = (int32_t)((uint32_t)p.depth * zl * zr);
@@ -680,7 +722,7 @@ int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
     // workgroups of a channel tile: as many as fit at once
     const int64_t groups = std::min<int64_t>(p.tiles_p, std::max<int64_t>(1, fit / p.tiles_x));
     p.span = (int)(p.tiles_p / groups); p.span_more = (int)(p.tiles_p % groups);
-    mh_plan_aux(ctx, MACE_HIP_AUX_CONV_PLANES);
+    mh_plan_aux(ctx, MACE_HIP_AUX_CONV_PLANES | (p.kept ? MACE_HIP_AUX_WEIGHT_HIT : 0) | (built.packed ? MACE_HIP_AUX_WEIGHT_BUILD : 0));
     MH_KLAUNCH(ctx, q8_conv_planes_pack_kernel, dim3((unsigned)plan.pack_blocks), dim3(256), 0, ctx->stream, p);
     dim3 grid((unsigned)(groups * p.tiles_x)), block((unsigned)plan.threads);
     mh_plan_main(ctx, MACE_HIP_KF_Q8_CONV_PLANES, mhv::conv_planes(form, three), grid, block, (int)lds);
@@ -690,13 +732,22 @@ int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
     MH_LAUNCH_CHECK(ctx);
     return MACE_HIP_SUCCESS;
   };
+  int rc = MACE_HIP_SUCCESS;
 #define MH_PLANES(...)                                                                 \
-  return three ? launch(q8_conv_planes_kernel<__VA_ARGS__, 3, 4>) : launch(q8_conv_planes_kernel<__VA_ARGS__, 0, 4>)
+  rc = three ? launch(q8_conv_planes_kernel<__VA_ARGS__, 3, 4>) : launch(q8_conv_planes_kernel<__VA_ARGS__, 0, 4>)
   switch (form) {
-    case mhv::PLANES_64x256: MH_PLANES(2, 1, 1, 8, 1);
-    case mhv::PLANES_32x256: MH_PLANES(1, 2, 1, 4, 1);
-    case mhv::PLANES_32x128: MH_PLANES(1, 1, 1, 4, 1);
-    default: MH_PLANES(1, 1, 1, 1, 4);
+    case mhv::PLANES_64x256: MH_PLANES(2, 1, 1, 8, 1); break;
+    case mhv::PLANES_32x256: MH_PLANES(1, 2, 1, 4, 1); break;
+    case mhv::PLANES_32x128: MH_PLANES(1, 1, 1, 4, 1); break;
+    default: MH_PLANES(1, 1, 1, 1, 4); break;
   }
 #undef MH_PLANES
+  if (rc == MACE_HIP_SUCCESS && p.kept) ++ctx->weight_hits;
+  if (rc == MACE_HIP_SUCCESS && built.packed) {
+    weight->planes.push_back(built);
+    ++ctx->weight_builds;
+  } else if (built.packed) {
+    give_back();
+  }
+  return rc;
 }

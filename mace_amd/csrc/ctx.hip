@@ -228,7 +228,7 @@ int mace_hip_weight_register(mace_hip_ctx *ctx, const void *device_ptr, size_t b
       w.bytes = bytes;
       return MACE_HIP_SUCCESS;
     }
-  ctx->weights.push_back(mh_weight{device_ptr, bytes, {}});
+  ctx->weights.push_back(mh_weight{device_ptr, bytes, {}, {}});
   return MACE_HIP_SUCCESS;
 }
 

@@ -2797,10 +2797,7 @@ int Q8Call::prepare(bool *done) {
 
   // operands registered as constant weights keep their panel and sums in the context
   auto find_weight = [&](const uint8_t *src, size_t bytes) -> mh_weight * {
-    if (depth == 0 || ctx->no_alloc) return nullptr;   // the cache allocates on first use
-    for (mh_weight &w : ctx->weights)
-      if (w.ptr == (const void *)src && bytes <= w.bytes) return &w;
-    return nullptr;
+    return depth == 0 ? nullptr : mh_find_weight(ctx, src, bytes);
   };
   lhs_w = find_weight(lhs, (size_t)lhs_nb * rows * depth);
   rhs_w = (rhs_ld != 0 || cv) ? nullptr : find_weight(rhs, (size_t)rhs_nb * cols * depth);

@@ -88,6 +88,62 @@ def test_cached_weight_matches_uncached_and_oracle(ctx, rows, depth, cols, lo, r
     assert stats(ctx)[0] == b1                     # no longer cached: nothing new was built
 
 
+# n, in_h, in_w, cin, cout; tiles of 32 x 128, of 64 x 256, in parts of the depth, one plane only
+@pytest.mark.parametrize("n,h,w,cin,cout", [(8, 34, 36, 108, 28), (64, 14, 14, 256, 256), (1, 18, 18, 160, 160),
+                                            (24, 40, 41, 13, 70)])
+def test_registered_filter_on_padded_planes(ctx, n, h, w, cin, cout):
+    """packed on first use, reused by calls with another input, zero point and bias; refreshed by a registration; in a
+    capture before its first use it is packed with every replay"""
+    import torch
+    rng = np.random.default_rng(n + cin)
+    filters = [rng.integers(0, 256, (cout, 3, 3, cin), dtype=np.uint8) for _ in range(2)]
+    fd = torch.from_numpy(filters[0]).cuda()
+    out = torch.empty(n * h * w * cout, dtype=torch.uint8, device="cuda")
+
+    def call(f, seed, zp, capture=False):
+        r = np.random.default_rng(seed)
+        x = r.integers(0, 256, (n, h, w, cin), dtype=np.uint8)
+        bias = r.integers(-2 ** 15, 2 ** 15, cout).astype(np.int32)
+        xd, bd = torch.from_numpy(x).cuda(), torch.from_numpy(bias).cuda()
+        out.fill_(0xA5)
+        torch.cuda.synchronize()
+        args = (xd.data_ptr(), fd.data_ptr(), bd.data_ptr(), n, h, w, cin, cout, 3, 3, 1, 1, 2, 2, 0.02, zp, 0.01, 121,
+                float(np.float32(0.02 * 0.01)), 2.0, 10, 0, 255, out.data_ptr())
+        if capture:
+            ctx.call("mace_hip_graph_capture_begin")
+        ctx.call("mace_hip_conv2d_q8_nhwc", *args)
+        plan = ctx.last_plan()
+        if capture:
+            graph = C.c_void_p()
+            ctx.call("mace_hip_graph_capture_end", C.byref(graph))
+            for _ in range(3):
+                out.fill_(0xA5)
+                torch.cuda.synchronize()
+                ctx.call("mace_hip_graph_launch", graph)
+                ctx.sync()
+            ctx.call("mace_hip_graph_destroy", graph)
+        ctx.sync()
+        want = orc.conv2d_q8_nhwc(x, f, bias, n, h, w, cin, cout, 3, 3, (1, 1), (2, 2), 0.02, zp, 0.01, 121,
+                                  np.float32(0.02 * 0.01), 2.0, 10)
+        assert plan.family == mh.KF_Q8_CONV_PLANES
+        np.testing.assert_array_equal(out.cpu().numpy().reshape(want.shape), want)
+        return plan.aux & ~mh.AUX_CONV_PLANES
+
+    assert call(filters[0], 1, 90) == 0                       # (the arena has what a capture needs)
+    ctx.call("mace_hip_weight_register", fd.data_ptr(), fd.numel())
+    b0, h0 = stats(ctx)
+    assert call(filters[0], 2, 128, capture=True) == 0
+    assert [call(filters[0], s, z) for s, z in ((3, 90), (4, 128), (5, 200))] == [mh.AUX_WEIGHT_BUILD] + 2 * [mh.AUX_WEIGHT_HIT]
+    assert call(filters[0], 6, 17, capture=True) == mh.AUX_WEIGHT_HIT
+    assert stats(ctx) == (b0 + 1, h0 + 3)
+    fd.copy_(torch.from_numpy(filters[1]).cuda())
+    torch.cuda.synchronize()
+    ctx.call("mace_hip_weight_register", fd.data_ptr(), fd.numel())
+    assert [call(filters[1], s, 90) for s in (7, 8)] == [mh.AUX_WEIGHT_BUILD, mh.AUX_WEIGHT_HIT]
+    ctx.call("mace_hip_weight_unregister", fd.data_ptr())
+    assert call(filters[1], 9, 90) == 0
+
+
 def test_reregistration_refreshes_and_errors(ctx):
     import torch
     rng = np.random.default_rng(3)
