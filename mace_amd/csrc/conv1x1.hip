@@ -102,10 +102,31 @@ struct ConvShortParams {
   int pitch;    // LDS bytes per staged input row (a multiple of 4)
   int lead;     // offset of an input row's first byte inside its staged row (a multiple of 4)
   int gbase;    // lead - pad_left * cin: where output column 0's patches start
+  bool pieces;  // results in aligned 16-byte pieces
   uint32_t zp4; // the input zero point in all four bytes
   int32_t xcoef, ycoef, yadd;
   RequantFixed rq;
 };
+
+// 16 channels of a pixel, `left` of which exist.  pieces: every pixel is whole aligned pieces, which cost one comparison
+// (with the others' fifteen in line, layers of 16 to 96 channels on one image took 5 - 10 % more: 64 x 66 x 3 -> 16 at
+// stride 2 5.7 us for 5.2).  Else 16 bytes at any address, the piece with the last channels byte by byte.
+__device__ __forceinline__ void store_strip_piece(uint8_t *to, const v4i &o, int left, bool live, bool pieces) {
+  if (pieces) {
+    if (live && left > 0) *(v4i *)to = o;
+    return;
+  }
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(left));   // (its comparisons below are not kept over the loop)
+#endif
+  if (live && left >= 16) {
+    __builtin_memcpy(to, &o, 16);
+  } else if (live) {
+#pragma unroll
+    for (int e = 0; e < 15; ++e)
+      if (e < left) to[e] = (uint8_t)(((uint32_t)o[e / 4] >> (8 * (e % 4))) & 0xff);
+  }
+}
 
 // (Occupancy 3 in the launch bounds: with at most 170 registers the compiler keeps the MFMA results
 // in ordinary registers, which spares the epilogue a move per output.)
@@ -285,18 +306,7 @@ __global__ __launch_bounds__(256, 3) void q8_conv_short_kernel(ConvShortParams p
       const v2u s02 = __builtin_amdgcn_permlane32_swap(packed[0], packed[2], false, false);
       const v2u s13 = __builtin_amdgcn_permlane32_swap(packed[1], packed[3], false, false);
       const v4i o = {(int)s02.x, (int)s02.y, (int)s13.x, (int)s13.y};
-      // (16 bytes at any address; the piece with the pixel's last channels byte by byte)
-      int left = p.cout - i * 32 - 16 * h;
-#if defined(__HIP_DEVICE_COMPILE__)
-      asm volatile("" : "+v"(left));   // (its comparisons below are not kept over the loop)
-#endif
-      if (live && left >= 16) {
-        __builtin_memcpy(orow + i * 32, &o, 16);
-      } else if (live) {
-#pragma unroll
-        for (int e = 0; e < 15; ++e)
-          if (e < left) orow[i * 32 + e] = (uint8_t)(((uint32_t)o[e / 4] >> (8 * (e % 4))) & 0xff);
-      }
+      store_strip_piece(orow + i * 32, o, p.cout - i * 32 - 16 * h, live, p.pieces);
     }
     q += 128;
     ow += dr;
@@ -509,18 +519,7 @@ __global__ __launch_bounds__(256, 2) void q8_conv_rows_kernel(ConvShortParams p)
       const v2u s02 = __builtin_amdgcn_permlane32_swap(packed[0], packed[2], false, false);
       const v2u s13 = __builtin_amdgcn_permlane32_swap(packed[1], packed[3], false, false);
       const v4i o = {(int)s02.x, (int)s02.y, (int)s13.x, (int)s13.y};
-      // (16 bytes at any address; the piece with the pixel's last channels byte by byte)
-      int left = p.cout - i * 32 - 16 * h;
-#if defined(__HIP_DEVICE_COMPILE__)
-      asm volatile("" : "+v"(left));   // (its comparisons below are not kept over the loop)
-#endif
-      if (live && left >= 16) {
-        __builtin_memcpy(orow + i * 32, &o, 16);
-      } else if (live) {
-#pragma unroll
-        for (int e = 0; e < 15; ++e)
-          if (e < left) orow[i * 32 + e] = (uint8_t)(((uint32_t)o[e / 4] >> (8 * (e % 4))) & 0xff);
-      }
+      store_strip_piece(orow + i * 32, o, p.cout - i * 32 - 16 * h, live, p.pieces);
     }
   }
 }
@@ -909,7 +908,7 @@ int conv_short(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, c
   p.in_h = (int)in_h; p.in_w = (int)in_w; p.cin = (int)cin; p.cout = (int)cout; p.k_h = (int)k_h;
   p.sh = stride_h; p.sw = stride_w; p.pt = pad_top; p.out_h = (int)out_h; p.out_w = (int)out_w;
   p.depth = (int)depth; p.run = (int)(k_w * cin); p.strip = (int)strip; p.strips = (int)strips;
-  p.pitch = (int)pitch; p.lead = lead; p.gbase = gbase;
+  p.pitch = (int)pitch; p.lead = lead; p.gbase = gbase; p.pieces = pieces;
   p.zp4 = (uint32_t)(input_zp & 0xff) * 0x01010101u;
   p.xcoef = (int32_t)(0u - zr);
   p.ycoef = (int32_t)(0u - zl);
@@ -941,9 +940,13 @@ int conv_rows(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, co
   // (17 - 18 pieces against more than 64 output channels would hold 36 filter fragments and 64
   // accumulators per lane, one workgroup per CU: measured no faster than the one-launch kernel on
   // 56 x 56 x 32 -> 128 at batch 64, 42.2 against 41.2 us, and 34 % slower on 28 x 28; not built)
+  // (Pixels of odd channel counts, here and in the one-launch GEMM kernel, us: up to 32 channels faster here throughout;
+  // 67 x 67 x 16 -> 47 6.3 and 5.5, 78 x 78 x 16 -> 75 8.6 and 5.8, 15 of 70 x 71 x 16 -> 77 at stride 2 9.1 and 7.4, but 8
+  // of 56 x 57 x 16 -> 99 6.7 and 8.2, 36 of 48 x 48 x 32 -> 62 15.8 and 16.4.)
+  const bool pieces = cout % 16 == 0 && (uintptr_t)out % 16 == 0;   // results in aligned 16-byte pieces
   if (cin % 16 != 0 || depth <= 32 || (ks != 5 && ks != 9) || cout > 128 ||
       (ks == 9 && cout > 64) || (uintptr_t)input % 16 != 0 ||
-      columns < (cout % 16 != 0 || (uintptr_t)out % 16 != 0 ? 4096 : (cout <= 32 ? 256 : 1024)) ||
+      columns < (!pieces ? (cout <= 32 ? 4096 : (cout <= 64 ? 8192 : 20000)) : (cout <= 32 ? 256 : 1024)) ||
       (ctx->kernel_mask & MH_MASK_NO_CONV_SHORT))
     return MACE_HIP_SUCCESS;
   if (shift < 0 || shift > 31 || clamp_min < 0 || clamp_max > 255 || clamp_min > clamp_max)
@@ -989,7 +992,7 @@ int conv_rows(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, co
   p.in_h = (int)in_h; p.in_w = (int)in_w; p.cin = (int)cin; p.cout = (int)cout; p.k_h = (int)k_h;
   p.sh = stride_h; p.sw = stride_w; p.pt = pad_top; p.out_h = (int)out_h; p.out_w = (int)out_w;
   p.depth = (int)depth; p.run = (int)(k_w * cin); p.strip = (int)strip; p.strips = (int)strips;
-  p.pitch = (int)pitch; p.lead = lead; p.gbase = 0;
+  p.pitch = (int)pitch; p.lead = lead; p.gbase = 0; p.pieces = pieces;
   p.zp4 = (uint32_t)(input_zp & 0xff) * 0x01010101u;
   p.xcoef = (int32_t)(0u - zr);
   p.ycoef = (int32_t)(0u - zl);

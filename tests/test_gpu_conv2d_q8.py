@@ -290,7 +290,8 @@ def test_conv2d_q8_on_padded_planes(ctx, n, cout, cin, in_h, in_w, k_h, k_w, pad
 @pytest.mark.parametrize("n,cout,cin,hw,k,off,family", [
     (28, 20, 3, 72, 3, 0, mh.KF_Q8_CONV_SHORT), (9, 101, 3, 40, 3, 1, mh.KF_Q8_CONV_SHORT),
     (1, 7, 2, 33, 3, 3, mh.KF_Q8_CONV_SHORT), (3, 45, 16, 64, 3, 0, mh.KF_Q8_CONV_ROWS),
-    (6, 32, 32, 32, 3, 5, mh.KF_Q8_CONV_ROWS), (2, 127, 16, 60, 3, 2, mh.KF_Q8_CONV_ROWS)])
+    (6, 32, 32, 32, 3, 5, mh.KF_Q8_CONV_ROWS), (2, 127, 16, 60, 3, 2, mh.KF_Q8_GEMM_FUSED_SMALL),
+    (6, 127, 16, 60, 3, 2, mh.KF_Q8_CONV_ROWS)])
 def test_conv2d_q8_strips_of_any_channel_count(ctx, n, cout, cin, hw, k, off, family):
     """The strip kernels store rows of any length at any address; nothing beside the result is written."""
     import torch
