@@ -131,7 +131,7 @@ enum {
   MACE_HIP_KF_F32_GEMM_GENERAL,      /* the same or, for ragged depths, f32_gemm_kernel: others   */
   MACE_HIP_KF_F32_GEMM_FILL,         /* depths 0 to 2: multiply-adds, element by element          */
   MACE_HIP_KF_F32_GEMV_VEC,          /* f32_gemv_rows_kernel: four rows a wavefront               */
-  MACE_HIP_KF_F32_GEMV_GENERAL,      /* f32_gemv_kernel                                           */
+  MACE_HIP_KF_F32_GEMV_GENERAL,      /* f32_gemv_kernel, f32_gemv_floats_kernel: one              */
   MACE_HIP_KF_Q8_CONV_SHORT,         /* q8_conv_short_kernel: patches of at most 32 bytes        */
   MACE_HIP_KF_Q8_CONV_ROWS,          /* q8_conv_rows_kernel: several taps of 16-channel pieces   */
   MACE_HIP_KF_Q8_CONV_KSPLIT,        /* q8_conv_ksplit_kernel: few pixels, a wavefront per slice of the depth */

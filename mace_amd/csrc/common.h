@@ -249,7 +249,7 @@ inline int f32_gemm_general(bool guard, int form, bool lk, bool rk) {
 enum { F32_SLICES_FORMS = 3 };
 inline int f32_slices(int form, bool lk, bool rk) { return form * 4 + (lk ? 2 : 0) + (rk ? 1 : 0); }
 // vectors a pass: 1, 2, 3, 4, 6, 8, 12, 16 (one row a wavefront: the first four)
-enum { F32_GEMV_VECTORS = 8 };
+enum { F32_GEMV_VECTORS = 8, F32_GEMV_FLOATS = 4 };   // (FLOATS: f32_gemv_floats_kernel, in the general family)
 }  // namespace mhv
 
 // Brackets a kernel launch with the dominant-kernel stopwatch when profiling is enabled.

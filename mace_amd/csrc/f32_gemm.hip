@@ -9,7 +9,7 @@
 // loop, which the reference's own tolerance (1e-4 relative + 1e-2 absolute) covers.
 //
 // Gemv replaces delegator::Gemv for float (mace/ops/delegator/gemv.h:35-44,
-// mace/ops/ref/gemv.cc:46-81): one wavefront per output row, lane-strided loads.
+// mace/ops/ref/gemv.cc:46-81): rows in slices by 16-byte pieces, up to 16 vectors a pass, or one row a wavefront.
 #include <math.h>
 
 #include <type_traits>
@@ -821,6 +821,38 @@ __global__ __launch_bounds__(512, 4) void f32_gemv_rows_kernel(F32GemvParams p, 
   gemv_rows<NB, 4, 1>(p, batch, slice_bits, groups);
 }
 
+// One row a wavefront, float by float: coalesced 4-byte loads, which the address path takes at full width wherever a row
+// begins, where 16-byte loads at odd addresses cost it twice.  For widths that are not whole pieces and rows for about
+// a round of wavefronts (3323 x 2343 8.5 us by pieces, 6.9 here, 3712 x 1305 6.0 and 5.3, 8 x 119 x 1838 4.8 and 3.6).
+// (A last turn of masked loads instead of the loads left over: 10 - 20 % slower.)
+__global__ __launch_bounds__(256) void f32_gemv_floats_kernel(F32GemvParams p) {
+  const int lane = threadIdx.x & 63;
+  const int h = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (h >= p.H) return;
+  const int b = blockIdx.y;
+  const float *l = p.lhs + (int64_t)b * p.lbs + (int64_t)h * p.W;
+  const float *r = p.rhs + (int64_t)b * p.rbs;
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};   // (short chains: rounding as in the kernel by pieces)
+  int w = lane;
+  auto turn = [&](int at) __attribute__((always_inline)) {   // four loads of each operand in flight
+    float a[4], x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) { a[u] = l[w + 64 * u]; x[u] = r[w + 64 * u]; }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) s[at + u] = __builtin_fmaf(a[u], x[u], s[at + u]);
+    w += 256;
+  };
+  while (w + 192 < p.W) {
+    turn(0);
+    if (w + 192 < p.W) turn(4);
+  }
+  for (; w < p.W; w += 64) s[7] = __builtin_fmaf(l[w], r[w], s[7]);
+  float t = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+  if (lane == 0) p.out[(int64_t)b * p.H + h] = apply_act((p.bias ? p.bias[h] : 0.f) + t, p.act, p.limit);
+}
+
 }  // namespace
 
 // Tiles of 32 x 32 fn, their depth in wk slices.
@@ -1105,6 +1137,24 @@ int mace_hip_gemv_f32_act(mace_hip_ctx *ctx, const float *lhs, const float *rhs,
   // (three vectors as four with four rows: 3 x 4000 x 1000 6.0 us, 11.2 with loads that wait for one another)
   while (kVectors[form] < (vectors + passes - 1) / passes || (four && kVectors[form] == 3)) ++form;
   const int nb = kVectors[form];
+  // Widths that are not whole aligned pieces: float by float where that is faster.  (Drawn widths, time against the kernels
+  // by pieces: one vector a pass, 2400 to 6600 rows of 512 to 4096 floats, 44 MB at most, no more than two loads left over
+  // behind turns of 256: 52 calls, 0.81 - 1.01, median 0.96; with more left over 0.84 - 1.16, with more rows to 1.25, with
+  // 65 to 71 MB 1.09 - 1.11.  Four vectors a pass, too few rows for four a wavefront: 28 calls, 0.76 - 1.01, median 0.89;
+  // three vectors 0.79 - 1.23.)
+  const bool pieces = width % 4 == 0 && (uintptr_t)lhs % 16 == 0 && (uintptr_t)rhs % 16 == 0;
+  const int64_t all_rows = batch * height;
+  if (!pieces && width >= 512 &&
+      (vectors == 1 ? all_rows >= 2400 && all_rows < 6600 && width < 4096 && all_rows * width < 11000000 && width % 256 <= 128
+                    : !four && nb == 4 && all_rows < 6144 && width < 2700)) {
+    const dim3 grid((unsigned)((height + 3) / 4), (unsigned)batch), block(256);
+    mh_plan_main(ctx, MACE_HIP_KF_F32_GEMV_GENERAL, mhv::F32_GEMV_FLOATS, grid, block, 0);
+    MH_PROF_BEGIN(ctx);
+    MH_KLAUNCH(ctx, f32_gemv_floats_kernel, grid, block, 0, ctx->stream, p);
+    MH_PROF_END(ctx);
+    MH_LAUNCH_CHECK(ctx);
+    return MACE_HIP_SUCCESS;
+  }
   const int waves = slices > 4 ? slices : 4, bits = mhv::log2i(slices), groups = waves >> bits, rows = groups * (four ? 4 : 1);
   const dim3 grid((unsigned)((height + rows - 1) / rows), (unsigned)((batch + nb - 1) / nb)), block(64 * waves);
   if (four) mh_plan_main(ctx, MACE_HIP_KF_F32_GEMV_VEC, form - (nb > 3), grid, block, 0);

@@ -30,7 +30,7 @@ const int kVariantCount[MACE_HIP_KF_COUNT] = {
     mhv::F32_FORMS * 8,       // F32_GEMM_GENERAL
     1,                        // F32_GEMM_FILL
     mhv::F32_GEMV_VECTORS - 1,   // F32_GEMV_VEC (not three)
-    4,                           // F32_GEMV_GENERAL
+    mhv::F32_GEMV_FLOATS + 1,    // F32_GEMV_GENERAL
     3,                        // Q8_CONV_SHORT
     5,                        // Q8_CONV_ROWS (FX = 4 exists with KS = 5 only)
     2,                        // Q8_CONV_KSPLIT
@@ -217,6 +217,10 @@ int mace_hip_plan_describe(int family, int v, char *buf, size_t len) {
     case MACE_HIP_KF_F32_GEMV_VEC:
     case MACE_HIP_KF_F32_GEMV_GENERAL: {
       static const int vectors[mhv::F32_GEMV_VECTORS] = {1, 2, 3, 4, 6, 8, 12, 16};
+      if (family == MACE_HIP_KF_F32_GEMV_GENERAL && v == mhv::F32_GEMV_FLOATS) {
+        snprintf(buf, len, "f32_gemv_floats_kernel");
+        break;
+      }
       snprintf(buf, len, "%s<NB=%d>", k, vectors[family == MACE_HIP_KF_F32_GEMV_VEC && v >= 2 ? v + 1 : v]);
       break;
     }

@@ -285,6 +285,9 @@ GEMV_CASES += [(1, 5, 3, False, False), (2, 9, 1, False, True), (1, 64, 16383, F
                (3, 700, 2047, False, True), (5, 515, 4098, False, True), (6, 4099, 330, False, True),
                (9, 130, 1030, False, True), (12, 2830, 1025, False, True), (16, 2801, 7, False, True),
                (16, 11300, 70, False, True), (33, 600, 257, False, True), (3, 515, 333, True, True)]
+# float by float: turns of 256 in odd and even numbers, nothing to two loads left over, rows that leave wavefronts idle
+GEMV_CASES += [(1, 2401, 513, False, False), (1, 2403, 769, False, False), (1, 2402, 1125, False, False), (1, 2499, 3967, False, False),
+               (3, 811, 577, True, True), (4, 101, 514, False, True), (7, 33, 1023, False, True), (16, 130, 2699, False, True)]
 
 
 @pytest.mark.parametrize("batch,h,w,lb,rb", GEMV_CASES)
