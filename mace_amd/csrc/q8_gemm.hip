@@ -2456,7 +2456,7 @@ int launch_gemm_big_xf(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
   return MACE_HIP_SUCCESS;
 }
 
-// the one-launch kernel for small problems; the caller has checked its preconditions
+// a wavefront per slice of a tile's depth; the caller has checked its preconditions
 int launch_gemm_slices(mace_hip_ctx *ctx, GemmParams &p, bool out_u8, bool xt, bool yt, int wk, int batch) {
   const int64_t tiles = (int64_t)p.tiles_x * p.tiles_y, wt = 8 / wk;
   dim3 grid((unsigned)((tiles + wt - 1) / wt), 1, (unsigned)batch), block(512);
@@ -2481,6 +2481,7 @@ int launch_gemm_slices(mace_hip_ctx *ctx, GemmParams &p, bool out_u8, bool xt, b
   return MACE_HIP_SUCCESS;
 }
 
+// the one-launch kernel for small problems; the caller has checked its preconditions
 int launch_gemm_fused_small(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
                             bool xt, bool yt, int batch) {
   p.tiles_x = (p.XN + 63) / 64;
@@ -2712,8 +2713,8 @@ static void q8_params_conv(GemmParams *p, const Q8ConvGather &cv) {
 }
 
 // One uint8 GEMM call on its way to a kernel: the arguments of mh_q8_gemm, what prepare() derives
-// from them, and the three stages of the dispatch.  Every stage is host logic only (a plan-only
-// context runs it without a GPU): small_problem() and kmajor_in_place() each either launch the
+// from them, and the four stages of the dispatch.  Every stage is host logic only (a plan-only
+// context runs it without a GPU): slices(), small_problem() and kmajor_in_place() each either launch the
 // whole call as one kernel and set *done, or leave it to the next stage; general() repacks what
 // cannot be read in place, takes the panel sums the chosen kernel does not take itself, and
 // launches one of the tiled kernels.
@@ -2876,6 +2877,15 @@ int Q8Call::prepare(bool *done) {
 //   one-launch kernel: its workgroups' depth, in 16-byte pieces or less; operands read in place: 5 + 0.0035 K (0.006 K where
 //     K is not a multiple of 64);
 //   operands copied first: 11 + 0.0036 K and the results' bytes.
+// For long depths these are not close enough, and two more have to hold (with the operands' and results' MB):
+//   from eight k steps a wavefront on, both operands along the depth and not in whole dwords: 1.25 per step less 3 is below
+//     copies at 10 + 0.0028 K + 0.55 per MB copied (0.25 of results).  (6957 deep, 46 x 40 30.4 us by copies and 35.6, 5761
+//     deep, 224 x 73 27.7 and 42.1, but 4497 deep, 2688 x 32 29.2 and 24.3.)
+//   from 64 k steps on, more tiles than CUs: the busiest CU's tiles one after the other, 1.2 and 0.067 or 0.08 per k step
+//     each, are below copies at 10.8 + 0.0028 K + 0.29 per MB (0.13 of results), or 1.1 times what is said above in place;
+//     not for whole pieces that are not whole slabs, which the other kernels do slowly (576 x 7824 x 512 71).  (640 x 7936 x
+//     459 29 and 36.5, 1096 x 2624 x 576 21 and 26.)
+//   Of 1700 drawn calls that come here 21 are more than 3 % slower than the kernels that had them, where 40 of 2130 were.
 // Measured, before and slices: 634 x 393 x 256 (both transposed) 17.3 and 4.9, 394 x 336 x 51 12.9 and 3.9, 576 x 1715 x
 // 320 15.2 and 7.6, 320 x 1088 x 768 -> int32 12.9 and 6.0, 402 x 3584 x 73 16.0 and 9.1, 128 x 256 x 128 5.1 and 4.4, 1600
 // x 2988 x 224 21.3 and 16.4; against the rule 320 x 5777 x 1020 33 and 58, 2048^3 15.4 and 74.
@@ -2893,8 +2903,9 @@ int Q8Call::slices(bool *done) {
   const bool l4 = dwords(lhs, lhs_t ? rows : depth), r4 = dwords(rhs, rhs_t ? cols : depth);
   const bool ragged = (!lhs_t && !l4) || (!rhs_t && !r4);
   const int wk = tiles <= 450 ? 8 : 4;
+  const int64_t steps = (nk + wk - 1) / wk;   // of a wavefront
   const double step = ragged ? 0.17 : (l4 && r4 ? 0.065 : 0.09);
-  const double mine = 4 + std::max((ragged ? 0.75 : 0.3) * ((nk + wk - 1) / wk) + 0.3,
+  const double mine = 4 + std::max((ragged ? 0.75 : 0.3) * steps + 0.3,
                                    tiles / cu * ((wk == 8 ? 0.7 : 0.45) + (out_u8 ? 0 : 0.3) + step * nk));
   // (rows along the depth in place as prepare() says; k-major ones by the kernels that turn whole 16-byte pieces)
   auto pieces = [&](const uint8_t *at, bool t, int64_t n, bool direct) {
@@ -2905,16 +2916,25 @@ int Q8Call::slices(bool *done) {
   const bool halves = depth % 16 == 8 && depth <= 576 && (xl ? cols : rows) >= 256 && (uintptr_t)lhs % 8 == 0 &&
                       (uintptr_t)rhs % 8 == 0;
   const bool in_place = !lhs_t && !rhs_t && ((l16 && r16) || halves);
-  double other;
+  const double copied = ((double)lhs_nb * rows + (double)rhs_nb * cols) * depth / 1e6;
+  const double results = (double)batch * rows * cols * (out_u8 ? 1 : 4) / 1e6;
+  bool worse;
   if (mh_q8_small_problem(ctx, batch, rows, cols, depth, l16 && r16) && !mid_first_xt && !mid_first_kc && !mid_first_yt) {
     const double wgs = (double)batch * ((rows + 63) / 64) * ((cols + 63) / 64);
-    other = 4 + std::max((l16 && r16 ? 0.006 : 0.02) * depth, wgs / cu * ((l16 && r16 ? 0.0033 : 0.01) * depth + 0.6));
-  } else if (in_place || (l16 && r16 && depth % 128 == 0)) {
-    other = 5 + (depth % 64 == 0 ? 0.0035 : 0.006) * depth;
+    worse = mine >= 0.9 * (4 + std::max((l16 && r16 ? 0.006 : 0.02) * depth, wgs / cu * ((l16 && r16 ? 0.0033 : 0.01) * depth + 0.6)));
   } else {
-    other = 11 + 0.0036 * depth + (double)batch * rows * cols * (out_u8 ? 1 : 4) / 4e6;
+    const bool copies = !in_place && !(l16 && r16 && depth % 128 == 0);
+    const double other = copies ? 11 + 0.0036 * depth + 0.25 * results : 5 + (depth % 64 == 0 ? 0.0035 : 0.006) * depth;
+    worse = mine >= 0.9 * other;
+    if (ragged && !lhs_t && !rhs_t && steps >= 8) {
+      worse |= 1.3 + 1.25 * steps >= 10 + 0.0028 * depth + 0.55 * copied + 0.25 * results;
+    } else if (nk >= 64 && tiles > cu && (depth % 16 != 0 || depth % 64 == 0)) {
+      const int64_t wt = 8 / wk, groups = (tiles + wt - 1) / wt, busiest = wt * ((groups + (int64_t)cu - 1) / (int64_t)cu);
+      worse |= 1.5 + busiest * (1.2 + (l4 && r4 ? 0.067 : 0.08) * nk) >=
+               (copies ? 10.8 + 0.0028 * depth + 0.29 * copied + 0.13 * results : 1.1 * other);
+    }
   }
-  if (mine >= 0.9 * other) return MACE_HIP_SUCCESS;
+  if (worse) return MACE_HIP_SUCCESS;
 
   const bool xt = xl ? lhs_t : rhs_t, yt = xl ? rhs_t : lhs_t;
   const Q8Operand L{lhs, lhs_t ? rows : depth, lhs_nb > 1 ? rows * depth : 0};
