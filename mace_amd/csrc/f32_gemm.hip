@@ -873,14 +873,18 @@ static int f32_slices_form(const mace_hip_ctx *ctx, int64_t batch, int64_t rows,
   const double old = parts > 1 ? (whole ? 12 : 15) + 0.63 * ((nk + parts - 1) / parts) + 8.0 * parts * total / 4e6
                                : (whole ? 5.3 : 8.3) + 0.63 * nk;
   const int form = tiles <= 400 ? 0 : 1, wk = kF32Slices[form].wk;
-  const double one = 4.2 + std::max(0.75 * ((nk + wk - 1) / wk), tiles / cus * (whole ? 0.25 + 0.14 * nk : 0.6 + 0.17 * nk));
+  // (a second tile on a few CUs counts from long depths on: 62 x 2112 x 4552, 286 tiles, 34.7 us, 27.1 by 128 x 128 tiles)
+  const double share = nk > 64 && form == 0 && tiles > cus ? std::max(tiles / cus, 0.8 * ceil(tiles / cus)) : tiles / cus;
+  const double one = 4.2 + std::max(0.75 * ((nk + wk - 1) / wk), share * (whole ? 0.25 + 0.14 * nk : 0.6 + 0.17 * nk));
   if (nk >= 24 && tiles > cus) {
     const int64_t wide = batch * ((rows + 31) / 32) * ((cols + 63) / 64);
     // (one workgroup a CU: rounds of them, with their starts and ends)
     const double rounds = ceil(wide / cus), two = 1.2 + rounds * (3 + 1.5 * ((nk + 7) / 8));
     if (two < one) return two < 0.95 * old ? 2 : -1;
   }
-  return tiles <= 1200 && one < 0.9 * old ? form : -1;   // (more, in two slices: within 5 % of the tiles)
+  // (more, in two slices: within 5 % of the tiles; at one or two k steps a third workgroup on a CU is 20 - 30 % more:
+  // pointwise 12 x 13 x 17 -> 384 at batch 20, 1176 tiles, 11.4 us, 8.7 by tiles)
+  return tiles <= (nk <= 2 ? 4 * cus : 1200) && one < 0.9 * old ? form : -1;
 }
 
 int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t batch,
