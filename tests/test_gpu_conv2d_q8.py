@@ -335,6 +335,50 @@ def test_conv2d_q8_images_without_a_pixel(ctx, in_h, in_w, cin, cout, pad_h, pad
     np.testing.assert_array_equal(out.cpu().numpy().reshape(want.shape), want)
 
 
+def test_conv2d_q8_planes_where_scratch_cannot_grow():
+    """In a capture nothing may be allocated: a call whose padded planes do not fit in the scratch there is goes to a
+    kernel that needs none, with the same results from every replay."""
+    import ctypes as C
+    import torch
+    n, h, w, cin, cout = 12, 61, 59, 29, 80
+    rng = np.random.default_rng(9)
+    x = rng.integers(0, 256, (n, h, w, cin), dtype=np.uint8)
+    f = rng.integers(0, 256, (cout, 3, 3, cin), dtype=np.uint8)
+    bias = rng.integers(-2 ** 15, 2 ** 15, cout).astype(np.int32)
+    want = orc.conv2d_q8_nhwc(x, f, bias, n, h, w, cin, cout, 3, 3, (1, 1), (2, 2), 0.02, 120, 0.01, 131,
+                              np.float32(0.02 * 0.01), 0.4, 128, nthreads=16)
+    xd, fd, bd = (torch.from_numpy(a.reshape(-1)).cuda() for a in (x, f, bias))
+    out = torch.zeros(want.size, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    c = mh.Context(0)
+    try:
+        def call(images):
+            c.call("mace_hip_conv2d_q8_nhwc", xd.data_ptr(), fd.data_ptr(), bd.data_ptr(), images, h, w, cin, cout, 3, 3, 1, 1,
+                   2, 2, 0.02, 120, 0.01, 131, float(np.float32(0.02 * 0.01)), 0.4, 128, 0, 255, out.data_ptr())
+            return c.last_plan().family
+        call(1)                                       # (scratch for one image)
+        c.sync()
+        c.call("mace_hip_graph_capture_begin")
+        family = call(n)
+        graph = C.c_void_p()
+        c.call("mace_hip_graph_capture_end", C.byref(graph))
+        assert family == mh.KF_Q8_GEMM_FUSED_SMALL
+        for _ in range(3):
+            out.zero_()
+            torch.cuda.synchronize()
+            c.call("mace_hip_graph_launch", graph)
+            c.sync()
+            np.testing.assert_array_equal(out.cpu().numpy().reshape(want.shape), want)
+        c.call("mace_hip_graph_destroy", graph)
+        out.zero_()
+        torch.cuda.synchronize()
+        assert call(n) == mh.KF_Q8_CONV_PLANES
+        c.sync()
+        np.testing.assert_array_equal(out.cpu().numpy().reshape(want.shape), want)
+    finally:
+        c.close()
+
+
 KSPLIT_CASES = [  # batch, cout, cin, in_h, in_w, k_h, k_w, padding, strides
     (1, 512, 512, 7, 7, 3, 3, S, (1, 1)),       # the deep layers of a single image
     (1, 256, 256, 14, 14, 3, 3, S, (1, 1)),

@@ -113,6 +113,7 @@ def test_gemm_f32_k_split(ctx, batch, rows, cols, depth, lm, rm, om, lb, rb, ker
     L = rng.standard_normal(((batch if lb else 1), rows, depth)).astype(np.float32)
     Rr = rng.standard_normal(((batch if rb else 1), depth, cols)).astype(np.float32)
     l, r = as_major(L, lm), as_major(Rr, rm)
+    whole = gemm_host(ctx, l, r, batch, rows, cols, depth, lm, rm, om, lb, rb)   # by whatever kernel takes it
     with kernel_mask(ctx, mh.MASK_NO_F32_SLICES):
         got = gemm_host(ctx, l, r, batch, rows, cols, depth, lm, rm, om, lb, rb)
     plan = ctx.last_plan()
@@ -125,7 +126,9 @@ def test_gemm_f32_k_split(ctx, batch, rows, cols, depth, lm, rm, om, lb, rb, ker
     near(got, orc.gemm_f32(l, r, batch, rows, cols, depth, lm, rm, om, lb, rb))
     want = orc.gemm_f32(l, r, batch, rows, cols, depth, lm, rm, om, lb, rb, acc64=True)
     near(got, want)
+    near(whole, want)
     assert np.linalg.norm(got.astype(np.float64) - want) <= 1e-4 * np.linalg.norm(want)
+    assert np.linalg.norm(whole.astype(np.float64) - want) <= 1e-4 * np.linalg.norm(want)
 
 
 @pytest.mark.parametrize("mask", [mh.MASK_NO_F32_SLICES, 0])
@@ -238,6 +241,32 @@ def test_gemm_f32_config2(ctx, ta, tb):
                                            nthreads=16))
 
 
+# the three forms of the slices kernel: depths of a few steps and of many, a row and a column beyond whole tiles
+@pytest.mark.parametrize("form,batch,m,n,k", [("FN=1,WK=8", 1, 97, 129, 301), ("FN=1,WK=8", 2, 33, 64, 16), ("FN=1,WK=4", 1, 1001, 545, 71),
+                                              ("FN=2,WK=8", 1, 500, 621, 777)])
+@pytest.mark.parametrize("om", [R, Cm])
+@pytest.mark.parametrize("lm,rm", [(R, R), (R, Cm), (Cm, R), (Cm, Cm)])
+def test_gemm_f32_slices_write_the_result_alone(ctx, form, batch, m, n, k, lm, rm, om):
+    """either order of the result, every order of the operands, nothing beside the result written; the error of k
+    rounded products and sums is at most k 2^-24 of the products' sizes"""
+    import torch
+    rng = np.random.default_rng(m + n + k)
+    L, Rr = rng.standard_normal((batch, m, k)).astype(np.float32), rng.standard_normal((batch, k, n)).astype(np.float32)
+    l, r = (torch.from_numpy(np.ascontiguousarray(as_major(a, o))).cuda() for a, o in ((L, lm), (Rr, rm)))
+    size, edge = batch * m * n, 64
+    out = torch.full((size + 2 * edge,), -7.5, dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    ctx.call("mace_hip_gemm_f32", l.data_ptr(), r.data_ptr(), batch, m, n, k, lm, rm, om, 1, 1, out.data_ptr() + 4 * edge)
+    assert form in ctx.last_plan().kernel, ctx.last_plan()
+    ctx.sync()
+    out = out.cpu().numpy()
+    assert (out[:edge] == -7.5).all() and (out[edge + size:] == -7.5).all()
+    want, bound = np.matmul(L.astype(np.float64), Rr.astype(np.float64)), np.matmul(np.abs(L).astype(np.float64), np.abs(Rr))
+    got = out[edge:edge + size].reshape((batch, m, n) if om == R else (batch, n, m))
+    got = got if om == R else got.transpose(0, 2, 1)
+    assert np.all(np.abs(got - want) <= (k + 16) * 2.0 ** -24 * bound)
+
+
 def test_gemm_f32_config2_small(ctx):
     """the same at 4 x 512^3: at most one tile per compute unit, i.e. the eight-wavefront
     variant of the kernel, in all four transpose combinations."""
@@ -260,6 +289,9 @@ def test_gemm_f32_config2_small(ctx):
             want64 = orc.gemm_f32(A, B, b, n, n, n, lm, rm, R, acc64=True, nthreads=16)
             near(got, orc.gemm_f32(A, B, b, n, n, n, lm, rm, R, nthreads=16))
             near(got, want64)
+            ctx.call("mace_hip_gemm_f32_transpose", dA, dB, b, n, n, n, n, ta, tb, 0, 1, 1, p)   # by whatever kernel takes it
+            ctx.sync()
+            near(t.cpu().numpy(), want64)
             rel = np.linalg.norm(got.astype(np.float64) - want64) / np.linalg.norm(want64)
             assert rel <= 1e-4, rel
 
@@ -301,6 +333,28 @@ def test_gemv_f32_parity(ctx, batch, h, w, lb, rb):
         ctx.call("mace_hip_gemv_f32_host", ptr(L), ptr(x), ptr(bb), batch, h, w, int(lb),
                  int(rb), ptr(out))
         near(out, orc.gemv_f32(L, x, bb, batch, h, w, lb, rb))
+
+
+# one vector by pieces and float by float, slices of a row, several vectors with one and with four rows a wavefront
+@pytest.mark.parametrize("batch,h,w,off", [(1, 70, 3, 0), (1, 131, 4099, 1), (1, 2403, 517, 0), (1, 8197, 333, 2), (3, 301, 1023, 0),
+                                           (7, 33, 1023, 1), (5, 515, 258, 3), (16, 603, 129, 0)])
+def test_gemv_f32_writes_the_result_alone(ctx, batch, h, w, off):
+    """results at any multiple of four bytes, nothing beside them written"""
+    import torch
+    rng = np.random.default_rng(h + w)
+    L, x = rng.standard_normal((h, w)).astype(np.float32), rng.standard_normal((batch, w)).astype(np.float32)
+    bias = rng.standard_normal(h).astype(np.float32)
+    ld, xd, bd = (torch.from_numpy(a).cuda() for a in (L, x, bias))
+    edge = 64 + off
+    out = torch.full((batch * h + 2 * edge,), -7.5, dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    ctx.call("mace_hip_gemv_f32", ld.data_ptr(), xd.data_ptr(), bd.data_ptr(), batch, h, w, 0, 1, out.data_ptr() + 4 * edge)
+    ctx.sync()
+    out = out.cpu().numpy()
+    assert (out[:edge] == -7.5).all() and (out[edge + batch * h:] == -7.5).all()
+    want = x.astype(np.float64) @ L.astype(np.float64).T + bias
+    bound = np.abs(x).astype(np.float64) @ np.abs(L).astype(np.float64).T + np.abs(bias)
+    assert np.all(np.abs(out[edge:edge + batch * h].reshape(batch, h) - want) <= (w + 2) * 2.0 ** -24 * bound)
 
 
 def test_fully_connected_f32_goldens(ctx):
