@@ -1,4 +1,5 @@
-// Runs the SOURCE of the uint8 GEMM kernels of mace_amd/csrc/q8_gemm.hip on the CPU:
+// Runs the SOURCE of the uint8 GEMM kernels of mace_amd/csrc/q8_gemm.hip, of the convolution on padded planes and of
+// some fp32 kernels on the CPU:
 // kernel_emu_extract.py cuts their text out, this file supplies what the text needs from the GPU
 // (thread and block indices, LDS, barriers, and the wavefront-wide instructions -- MFMA, lane
 // shuffles, transfers into LDS, the transposing LDS read -- as collectives over the 64 host threads
@@ -203,6 +204,60 @@ constexpr int SLAB = 64;
 #include "kernels.inc"
 #include "conv_planes.inc"
 }  // namespace
+
+// ---- what the fp32 kernels' text needs ---------------------------------------------------------------
+namespace f32 {
+typedef float v16f __attribute__((ext_vector_type(16)));
+enum { MACE_HIP_ACT_NOOP, MACE_HIP_ACT_RELU, MACE_HIP_ACT_RELUX };
+inline float __uint_as_float(uint32_t u) { float f; memcpy(&f, &u, 4); return f; }
+inline float __shfl_xor(float v, int m, int n) { return __uint_as_float((uint32_t)::__shfl_xor((int)__float_as_uint(v), m, n)); }
+int g_any;
+inline int __syncthreads_or(int v) {
+  __syncthreads();
+  g_any = 0;
+  __syncthreads();
+  if (v) __atomic_store_n(&g_any, 1, __ATOMIC_RELAXED);
+  __syncthreads();
+  return g_any;
+}
+inline uint32_t emu_bf16(float f) {   // to nearest even
+  const uint32_t u = __float_as_uint(f);
+  if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 64;
+  return (u + 0x7fff + ((u >> 16) & 1)) >> 16;
+}
+inline uint32_t emu_bf16_pair(float x, float y) { return emu_bf16(x) | (emu_bf16(y) << 16); }
+// lane l supplies row l % 32 of each operand, depths [DEPTHS (l / 32), + DEPTHS); results as emu_mfma's
+template <int DEPTHS>
+inline v16f emu_mfma_f32(const float *a, const float *b, v16f c) {
+  static float sa[8][64][8], sb[8][64][8];
+  Wave &w = wave_of_thread();
+  const int l = lane_of_thread(), wave = threadIdx.x >> 6;
+  for (int k = 0; k < DEPTHS; ++k) { sa[wave][l][k] = a[k]; sb[wave][l][k] = b[k]; }
+  w.bar.arrive_and_wait();
+  for (int r = 0; r < 16; ++r) {
+    const int x = 8 * (r / 4) + 4 * (l / 32) + r % 4;
+    double s = c[r];
+    for (int h = 0; h < 2; ++h)
+      for (int k = 0; k < DEPTHS; ++k) s += (double)sa[wave][x + 32 * h][k] * sb[wave][(l & 31) + 32 * h][k];
+    c[r] = (float)s;
+  }
+  w.bar.arrive_and_wait();
+  return c;
+}
+template <typename V>
+inline v16f emu_mfma_bf16(V a, V b, v16f c, int, int, int) {
+  uint16_t ua[8], ub[8];
+  memcpy(ua, &a, 16);
+  memcpy(ub, &b, 16);
+  float fa[8], fb[8];
+  for (int k = 0; k < 8; ++k) { fa[k] = __uint_as_float((uint32_t)ua[k] << 16); fb[k] = __uint_as_float((uint32_t)ub[k] << 16); }
+  return emu_mfma_f32<8>(fa, fb, c);
+}
+inline v16f emu_mfma_2f32(float a, float b, v16f c, int, int, int) { return emu_mfma_f32<1>(&a, &b, c); }
+#define __builtin_amdgcn_mfma_f32_32x32x16_bf16 emu_mfma_bf16
+#define __builtin_amdgcn_mfma_f32_32x32x2f32 emu_mfma_2f32
+#include "f32.inc"
+}  // namespace f32
 
 // all workgroups of a grid, one after the other, on as many host threads as a workgroup has
 static void run_grid(dim3 grid, const std::function<void()> &body, int threads = 256) {
@@ -648,6 +703,16 @@ static void planes_case(int n, int in_h, int in_w, int cin, int cout, int k_h, i
       if (g_block.lds[i] != 0xA5) { EXPECT(false, "planes: LDS byte %lld of %lld written", (long long)i, (long long)plan.lds); break; }
     delete[] out;
   }
+  // a filter whose packed bytes and sums are kept: the first launch leaves the sums, a later one takes them
+  p.wsums = new int32_t[p.channels];
+  run_grid(dim3(plan.pack_blocks), [&] { q8_conv_planes_pack_kernel(p); });
+  std::vector<int32_t> cx(p.cx, p.cx + p.channels);
+  std::vector<uint8_t> packed(p.packed, p.packed + plan.packed_bytes);
+  memset(p.cx, 0x5A, p.channels * 4);
+  p.kept = true;
+  run_grid(dim3(p.pixel_blocks + (p.channels + 255) / 256), [&] { q8_conv_planes_pack_kernel(p); });
+  EXPECT(std::equal(cx.begin(), cx.end(), p.cx) && std::equal(packed.begin(), packed.end(), p.packed), "planes: a kept filter's corrections differ");
+  delete[] p.wsums;
   delete[] in;
   delete[] filter;
   delete[] bias;
@@ -655,6 +720,96 @@ static void planes_case(int n, int in_h, int in_w, int cin, int cout, int k_h, i
   delete[] p.packed;
   delete[] (uint8_t *)p.psum;
   delete[] (uint8_t *)p.cx;
+}
+
+// ---- fp32: results against binary64, to the sum of the products' sizes times their number --------------
+static float rnd_f32() { return ((int)rnd() * 256 + rnd() - 32768) / 8192.0f; }
+static void check_f32(const char *what, const float *got, const std::vector<double> &want, const std::vector<double> &size, int k) {
+  int64_t bad = 0;
+  for (size_t i = 0; i < want.size(); ++i)
+    bad += std::isfinite(want[i]) ? !(std::fabs(got[i] - want[i]) <= (k + 16) * std::ldexp(size[i], -24)) : std::isfinite(got[i]);
+  EXPECT(bad == 0, "%s k %d: %lld of %zu results differ", what, k, (long long)bad, want.size());
+}
+
+// the fp32 slices kernel: operands along the depth (LK, RK) or along their rows and columns, images side by side
+// (flat: columns of each), `inf`: one operand element that no sum can take
+template <bool LK, bool RK, int FN, int WK>
+static void f32_slices_case(int batch, int m, int n, int k, int flat = 0, bool inf = false) {
+  ++g_cases;
+  const int images = flat ? batch : 1, cols = flat ? flat * batch : n, gz = flat ? 1 : batch;
+  const int per = flat ? flat : n;   // columns of a right-hand matrix in memory
+  const int lb = flat ? 1 : batch;
+  float *A = new float[(int64_t)lb * m * k], *B = new float[(int64_t)batch * k * per], *out = new float[(int64_t)batch * m * per];
+  float *bias = new float[m];
+  for (int64_t i = 0; i < (int64_t)lb * m * k; ++i) A[i] = rnd_f32();
+  for (int64_t i = 0; i < (int64_t)batch * k * per; ++i) B[i] = rnd_f32();
+  for (int i = 0; i < m; ++i) bias[i] = rnd_f32();
+  if (inf) A[(int64_t)lb * m * k - 1] = INFINITY;
+  std::vector<double> want((int64_t)batch * m * per), size(want.size());
+  for (int b = 0; b < batch; ++b)
+    for (int i = 0; i < m; ++i)
+      for (int j = 0; j < per; ++j) {
+        double s = bias[i], t = std::fabs(bias[i]);
+        for (int c = 0; c < k; ++c) {
+          const int64_t ao = (int64_t)(flat ? 0 : b) * m * k + (LK ? (int64_t)i * k + c : (int64_t)c * m + i);
+          const int64_t bo = (int64_t)b * k * per + (RK ? (int64_t)j * k + c : (int64_t)c * per + j);
+          s += (double)A[ao] * B[bo];
+          t += std::fabs((double)A[ao] * B[bo]);
+        }
+        want[((int64_t)b * m + i) * per + j] = s;
+        size[((int64_t)b * m + i) * per + j] = t;
+      }
+  f32::F32GemmParams p{};
+  p.lhs = A; p.rhs = B; p.out = out;
+  p.lrs = LK ? k : 1; p.lcs = LK ? 1 : m;
+  p.rrs = RK ? 1 : per; p.rcs = RK ? k : 1;
+  p.ors = per; p.ocs = 1;
+  p.lbs = flat ? 0 : (int64_t)m * k; p.rbs = (int64_t)k * per; p.obs = (int64_t)m * per;
+  p.M = m; p.N = cols; p.K = k; p.flat = images > 1 ? flat : 0; p.bias_row = bias;
+  p.tiles_m = (m + 31) / 32;
+  const int tiles = p.tiles_m * ((cols + 32 * FN - 1) / (32 * FN)), wt = 8 / WK;
+  run_grid(dim3((tiles + wt - 1) / wt, 1, gz), [&] { f32::f32_gemm_slices_kernel<LK, RK, FN, WK>(p); }, 512);
+  char what[96];
+  snprintf(what, sizeof what, "f32_gemm_slices_kernel<%d,%d,%d,%d> batch %d m %d n %d", (int)LK, (int)RK, FN, WK, batch, m, n);
+  check_f32(what, out, want, size, k);
+  delete[] A; delete[] B; delete[] out; delete[] bias;
+}
+
+// the Gemv kernels: NB vectors a pass with one row a wavefront (R = 1) or four, rows in 2^bits slices; NB = 0: float by float
+template <int NB, int R>
+static void f32_gemv_case(int batch, int h, int w, bool lb, int bits) {
+  ++g_cases;
+  float *L = new float[(int64_t)(lb ? batch : 1) * h * w], *x = new float[(int64_t)batch * w], *bias = new float[h],
+        *out = new float[(int64_t)batch * h];
+  for (int64_t i = 0; i < (int64_t)(lb ? batch : 1) * h * w; ++i) L[i] = rnd_f32();
+  for (int64_t i = 0; i < (int64_t)batch * w; ++i) x[i] = rnd_f32();
+  for (int i = 0; i < h; ++i) bias[i] = rnd_f32();
+  std::vector<double> want((int64_t)batch * h), size(want.size());
+  for (int b = 0; b < batch; ++b)
+    for (int i = 0; i < h; ++i) {
+      double s = bias[i], t = std::fabs(bias[i]);
+      for (int c = 0; c < w; ++c) {
+        const double v = (double)L[((int64_t)(lb ? b : 0) * h + i) * w + c] * x[(int64_t)b * w + c];
+        s += v;
+        t += std::fabs(v);
+      }
+      want[(int64_t)b * h + i] = s;
+      size[(int64_t)b * h + i] = t;
+    }
+  f32::F32GemvParams p{L, x, bias, out, lb ? (int64_t)h * w : 0, w, h, w, f32::MACE_HIP_ACT_NOOP, 0.f};
+  char what[80];
+  snprintf(what, sizeof what, "f32_gemv<NB=%d,R=%d> %d x %d x %d in %d", NB, R, batch, h, w, 1 << bits);
+  if constexpr (NB == 0) {
+    run_grid(dim3((h + 3) / 4, batch), [&] { f32::f32_gemv_floats_kernel(p); });
+  } else {
+    const int waves = (1 << bits) > 4 ? 1 << bits : 4, groups = waves >> bits, rows = groups * R;
+    run_grid(dim3((h + rows - 1) / rows, (batch + NB - 1) / NB), [&] {
+      if constexpr (R == 1) f32::f32_gemv_kernel<NB>(p, batch, bits, groups);
+      else f32::f32_gemv_rows_kernel<NB>(p, batch, bits, groups);
+    }, 64 * waves);
+  }
+  check_f32(what, out, want, size, w);
+  delete[] L; delete[] x; delete[] bias; delete[] out;
 }
 
 template <int LPR>
@@ -678,13 +833,13 @@ static void sums_case(int n, int k) {
 }
 
 // PART (compile-time): 1 = everything but what follows, 2 = the ring and eight-wavefront kernels, 3 = the
-// convolution kernel on staged rows; the
-// test builds and runs the parts side by side.
+// uint8 slices kernel and the convolution on padded planes, 4 = the fp32 kernels and the planes' tile of eight
+// wavefronts; the test builds and runs the parts side by side.
 #ifndef PART
 #define PART 0
 #endif
 int main() {
-#if PART != 2 && PART != 3
+#if PART != 2 && PART != 3 && PART != 4
   // the repacks of k-contiguous rows and of k-major operands: any row length
   for (int k : {1, 3, 15, 16, 17, 24, 63, 64, 65, 100, 127}) pack_case(1, 37, k, k, false);
   for (int k : {4, 8, 24, 40, 60, 64, 68, 120}) pack_case(1, 301, 130 + k, k, true);
@@ -743,7 +898,7 @@ int main() {
   xres_case<2, 1, true>(24, 4000, 120, 40);
   xres_case<4, 2, true>(128, 256, 328, 1);
 #endif
-#if PART != 1 && PART != 3
+#if PART != 1 && PART != 3 && PART != 4
   // the ring kernel in the tile shapes, ring depths and slab widths the dispatch uses; ragged tiles
   ring_case<2, 2, 4, 4, 2, 128, false>(300, 260, 384);
   ring_case<2, 2, 4, 4, 2, 128, true>(256, 257, 256);
@@ -767,7 +922,7 @@ int main() {
   mid_batched_case(8, 200, 128, 128);    // 16 workgroups: dealt to the XCDs in spans of (batch, tile)
   mid_batched_case(3, 129, 130, 128);    // a workgroup count that is not a multiple of 8
 #endif
-#if PART != 1 && PART != 2
+#if PART != 1 && PART != 2 && PART != 4
   // the slices kernel in every layout: depths below a step, ragged and whole, operands that end inside a piece, fewer
   // rows than a tile, rows shorter than a piece
   slices_case<false, false, 8>(70, 33, 333);
@@ -791,6 +946,38 @@ int main() {
   planes_case<1, 1, 1, 1, 4>(1, 6, 9, 64, 64, 5, 2, 1, 3, 4, 0, 10, 4, 50000, 2, 1);
   planes_case<1, 1, 1, 4, 1>(2, 5, 6, 48, 31, 3, 3, 1, 1, 1, 1, 5, 6, 80000, 1, 1);
   planes_case<1, 1, 1, 1, 4, 3>(1, 4, 9, 200, 40, 3, 3, 1, 1, 1, 1, 4, 9, 150000, 2, 1);
+#endif
+#if PART == 0 || PART == 4
+  // the fp32 slices kernel in its three forms: depths of less than half a step, a step, a step and a bit, fewer steps than
+  // slices and more; the planes' tile of eight wavefronts; Gemv widths of less than a piece, a piece and a rest, whole
+  // and broken turns, rows that leave part of a wavefront's four, vectors that leave part of a pass
+  f32_slices_case<true, true, 1, 8>(1, 33, 31, 3);
+  f32_slices_case<true, false, 1, 8>(2, 1, 65, 15);
+  f32_slices_case<false, true, 1, 8>(1, 70, 1, 17);
+  f32_slices_case<false, false, 1, 8>(1, 40, 33, 200);
+  f32_slices_case<true, true, 1, 8>(1, 32, 32, 16, 0, true);
+  f32_slices_case<true, true, 1, 4>(1, 65, 33, 100);
+  f32_slices_case<false, false, 1, 4>(3, 31, 34, 41);
+  f32_slices_case<true, false, 1, 4>(3, 40, 0, 23, 49);
+  f32_slices_case<true, true, 2, 8>(1, 33, 65, 129);
+  f32_slices_case<true, false, 2, 8>(2, 64, 0, 50, 37);
+  f32_slices_case<false, true, 2, 8>(1, 5, 63, 301, 0, true);
+  f32_gemv_case<1, 1>(1, 5, 1, false, 0);
+  f32_gemv_case<1, 1>(1, 7, 255, false, 0);
+  f32_gemv_case<1, 1>(2, 3, 1027, true, 1);
+  f32_gemv_case<1, 1>(1, 2, 4097, false, 3);
+  f32_gemv_case<3, 1>(5, 6, 261, false, 2);
+  f32_gemv_case<4, 1>(7, 3, 1030, false, 0);
+  f32_gemv_case<1, 4>(1, 9, 3, false, 0);
+  f32_gemv_case<2, 4>(2, 17, 259, false, 0);
+  f32_gemv_case<4, 4>(6, 33, 516, false, 1);
+  f32_gemv_case<6, 4>(6, 6, 77, false, 2);
+  f32_gemv_case<16, 4>(17, 18, 2051, false, 3);
+  f32_gemv_case<0, 1>(1, 6, 513, false, 0);
+  f32_gemv_case<0, 1>(3, 3, 767, true, 0);
+  f32_gemv_case<0, 1>(2, 5, 1090, false, 0);
+  planes_case<2, 1, 1, 8, 1, 3>(2, 9, 20, 20, 70, 3, 3, 1, 1, 1, 1, 9, 20, 150000, 2, 1);
+  planes_case<2, 1, 1, 8, 1, 3>(5, 7, 9, 50, 33, 3, 3, 1, 1, 1, 1, 7, 9, 60000, 1, 2);
 #endif
   if (g_failures) {
     printf("kernel_emu: %d failures in %d cases\n", g_failures, g_cases);

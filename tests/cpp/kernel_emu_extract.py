@@ -1,4 +1,4 @@
-"""Cuts the source text of a few GPU kernels out of mace_amd/csrc/q8_gemm.hip for kernel_emu.cpp, which
+"""Cuts the source text of a few GPU kernels out of the .hip files in mace_amd/csrc for kernel_emu.cpp, which
 compiles them for the host (see there).  Usage: kernel_emu_extract.py <output directory>."""
 import os
 import sys
@@ -25,6 +25,13 @@ PIECES = [
     ("struct RepackJob {", "__global__ __launch_bounds__(256) void q8_zero_i32_kernel"),
     ("template <int LPR>\n__global__ __launch_bounds__(256) void q8_panel_sums_kernel",
      "int launch_panel_sums("),
+]
+# the fp32 slices kernel and the Gemv kernels
+F32_PIECES = [
+    ("struct F32GemmParams {", "// ---- the tile kernels: binary32 products"),
+    ("typedef float f4v __attribute__", "// A TMT x 128 tile of the result per workgroup."),
+    ("template <bool LK, bool RK, int FN, int WK>", "// Depths of at most two: 0"),
+    ("struct F32GemvParams {", "}  // namespace\n\n// Tiles of 32 x 32 fn"),
 ]
 # source lines that only make sense on the GPU, and what stands in for them on the host
 PATCHES = [
@@ -61,6 +68,16 @@ def main(out_dir):
             sys.exit("kernel_emu_extract: conv_planes.hip no longer has the line %r" % old)
         planes = planes.replace(old, new)
     open(os.path.join(out_dir, "conv_planes.inc"), "w").write(planes)
+    src = open(os.path.join(CSRC, "f32_gemm.hip")).read()
+    parts = []
+    for first, after in F32_PIECES:
+        if first not in src or after not in src[src.index(first):]:
+            sys.exit("kernel_emu_extract: f32_gemm.hip no longer has the piece that starts with %r" % first)
+        parts.append(src[src.index(first):src.index(after, src.index(first))])
+    body = "\n".join(parts)
+    if body.count("  return 0;\n#endif\n}") != 1:
+        sys.exit("kernel_emu_extract: f32_gemm.hip no longer has the host's bf16_pair")
+    open(os.path.join(out_dir, "f32.inc"), "w").write(body.replace("  return 0;\n#endif\n}", "  return emu_bf16_pair(x, y);\n#endif\n}"))
     rq = open(os.path.join(CSRC, "q8_requant.h")).read().replace('#include "common.h"', "")
     rq = rq.replace("#pragma once", "")
     open(os.path.join(out_dir, "requant.inc"), "w").write(rq)
