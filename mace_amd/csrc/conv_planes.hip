@@ -53,18 +53,6 @@ __device__ __forceinline__ int plane_div(int n, uint32_t magic) {
 __device__ __forceinline__ uint32_t low_bytes(int n) {
   return n >= 4 ? 0xffffffffu : (n <= 0 ? 0u : (1u << (8 * n)) - 1u);
 }
-// A piece of which less than 16 bytes are left in the operand was loaded `early` bytes before its place: moved
-// down to it, zeros behind.  (The last piece of the last pixel or filter row.)
-__device__ __forceinline__ v4i tail_of(const v4i &v, uint32_t early) {
-  const bool two = (early & 8) != 0, one = (early & 4) != 0;
-  const uint32_t a0 = (uint32_t)(two ? v.z : v.x), a1 = (uint32_t)(two ? v.w : v.y), a2 = two ? 0u : (uint32_t)v.z,
-                 a3 = two ? 0u : (uint32_t)v.w;
-  const uint32_t b0 = one ? a1 : a0, b1 = one ? a2 : a1, b2 = one ? a3 : a2, b3 = one ? 0u : a3;
-  const uint32_t by = early & 3;
-  return v4i{(int)__builtin_amdgcn_alignbyte(b1, b0, by), (int)__builtin_amdgcn_alignbyte(b2, b1, by),
-             (int)__builtin_amdgcn_alignbyte(b3, b2, by), (int)__builtin_amdgcn_alignbyte(0u, b3, by)};
-}
-
 // ---- first launch: planes and packed filter ------------------------------------------------------
 //
 // planes[16 channels][image, row, column][16]: the input shifted (x ^ 0x80), pixels of the padding as the
@@ -105,7 +93,7 @@ __global__ __launch_bounds__(256) void q8_conv_planes_pack_kernel(ConvPlaneParam
       uint8_t *to = p.planes + (uint32_t)pc * (uint32_t)p.plane_bytes;
 #pragma unroll
       for (int u = 0; u < PACK_PIXELS; ++u) {
-        if (base[u] + c > p.in_last) v[u] = tail_of(v[u], base[u] + c - p.in_last);
+        if (base[u] + c > p.in_last) v[u] = moved_down(v[u], base[u] + c - p.in_last);
         v4i w = v[u] ^ flip;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -155,7 +143,7 @@ __global__ __launch_bounds__(256) void q8_conv_planes_pack_kernel(ConvPlaneParam
       for (int u = 0; u < 4; ++u) {
         const int q = q0 + 64 * u;
         if (q < slots) {
-          if (off[u] > p.filter_last) v[u] = tail_of(v[u], off[u] - p.filter_last);
+          if (off[u] > p.filter_last) v[u] = moved_down(v[u], off[u] - p.filter_last);
           v4i w = v[u] ^ flip;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {

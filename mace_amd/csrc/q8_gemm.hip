@@ -114,16 +114,8 @@ __device__ inline void tile_and_batch_of_block(int tiles_x, int tiles_y, int *tx
   else tile_of_block(blockIdx.x, gridDim.x, tiles_x, tiles_y, tx, ty);
 }
 
-// A piece that was loaded `early` (below 16, else nothing of it exists) bytes before its place: moved down to it.
-__device__ inline v4i bytes_from(const v4i &v, uint32_t early) {
-  if (early >= 16) return v4i{0, 0, 0, 0};
-  const bool two = (early & 8) != 0, one = (early & 4) != 0;
-  const uint32_t a0 = (uint32_t)(two ? v.z : v.x), a1 = (uint32_t)(two ? v.w : v.y), a2 = two ? 0u : (uint32_t)v.z,
-                 a3 = two ? 0u : (uint32_t)v.w;
-  const uint32_t b0 = one ? a1 : a0, b1 = one ? a2 : a1, b2 = one ? a3 : a2, b3 = one ? 0u : a3, by = early & 3;
-  return v4i{(int)__builtin_amdgcn_alignbyte(b1, b0, by), (int)__builtin_amdgcn_alignbyte(b2, b1, by),
-             (int)__builtin_amdgcn_alignbyte(b3, b2, by), (int)__builtin_amdgcn_alignbyte(0u, b3, by)};
-}
+// A piece that was loaded `early` bytes before its place: moved down to it (from 16 on nothing of it exists).
+__device__ inline v4i bytes_from(const v4i &v, uint32_t early) { return early >= 16 ? v4i{0, 0, 0, 0} : moved_down(v, early); }
 
 // Sum of the 16 bytes of a fragment as read from memory (unsigned, before the flip), added to acc.
 // The sum of the shifted bytes the corrections need is this minus 128 per byte.  v_sad_u8 is an

@@ -201,6 +201,7 @@ inline void dma_16B(mh_rsrc rs, uint32_t lane_off, uint32_t uniform_off, uint8_t
   memcpy(lds_wave_base + 16 * (threadIdx.x & 63), rs.base + lane_off + uniform_off, 16);
 }
 constexpr int SLAB = 64;
+#include "pieces.inc"
 #include "kernels.inc"
 #include "conv_planes.inc"
 }  // namespace

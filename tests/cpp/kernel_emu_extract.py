@@ -8,7 +8,8 @@ CSRC = os.path.join(ROOT, "mace_amd", "csrc")
 
 # (first line of the piece, first line of what follows it)
 PIECES = [
-    ("constexpr int BK = 64;", "// Sum of the 16 bytes of a fragment as read"),
+    ("constexpr int BK = 64;", "// A piece that was loaded `early` bytes"),
+    ("__device__ inline v4i bytes_from", "// Sum of the 16 bytes of a fragment as read"),
     ("__device__ inline int sum16_u8", "// Epilogue shared by the GEMM kernels"),
     ("template <int WX, int WY, int FX, int FY, typename OutT, bool SUMY, bool PRESTAGED = false>",
      "// ---- small problems: everything in one launch"),
@@ -60,6 +61,9 @@ def main(out_dir):
             sys.exit("kernel_emu_extract: q8_gemm.hip no longer has the line %r" % old)
         body = body.replace(old, new)
     open(os.path.join(out_dir, "kernels.inc"), "w").write(body)
+    transfer = open(os.path.join(CSRC, "q8_transfer.h")).read()
+    open(os.path.join(out_dir, "pieces.inc"), "w").write(
+        transfer[transfer.index("__device__ __forceinline__ v4i moved_down"):transfer.index("// s_waitcnt vmcnt(N) alone")])
     planes = open(os.path.join(CSRC, "conv_planes.hip")).read()
     planes = planes[planes.index("struct ConvPlaneParams {"):planes.index("}  // namespace\n\n// Time that the one-launch")]
     for old, new in (("extern __shared__ __align__(16) uint8_t lds[];", "uint8_t *lds = emu_lds();"),
