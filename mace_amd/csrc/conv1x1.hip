@@ -1248,6 +1248,9 @@ extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
                        ((uintptr_t)input % 16 == 0) && ((uintptr_t)filter % 16 == 0) &&
                        in_h * in_w * cin < (1ll << 31));
   const int64_t kp = (int64_t)mh_align_up((size_t)(depth > 0 ? depth : 1), 64);   // row of a patch matrix
+  size_t need = sizeof(int32_t) * cout + 4096 +
+                conv_gemm_scratch(cout, depth, columns, !in_place || depth % 16 == 0);
+  if (!in_place && !gather) need += (size_t)columns * kp + 4096;
   // All of these go through padded planes where that is faster.  (Up to nine taps of 64 channels stay with the kernel that
   // keeps the filter in LDS: 56 x 56 x 64 -> 64 at batch 64 21.5 us, on planes 28.4.)
   if (!in_place && (small_gather || cin % 64 != 0 || depth > 576)) {
@@ -1255,7 +1258,9 @@ extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
     // (a patch matrix of one tap, a 1 x 1 filter at a stride, is a fraction of the input, which the planes copy whole: 30 x
     // 30 x 995 -> 818 at stride 2, batch 7, 21.0 us, on planes 32.9, but 28 x 28 x 523 -> 129 at 21 28.8 and 21.3)
     const bool by_pieces = cin % 16 == 0 && (uintptr_t)input % 16 == 0;
-    const double other = small_gather ? mh_q8_conv_small_us(ctx, cout, columns, depth, small_vec ? 16 : (cin % 4 == 0 ? 4 : 1))
+    // (whatever the times, where only the planes' scratch can be had)
+    const double other = !mh_arena_can_hold(ctx, need) ? HUGE_VAL
+                         : small_gather ? mh_q8_conv_small_us(ctx, cout, columns, depth, small_vec ? 16 : (cin % 4 == 0 ? 4 : 1))
                          : gather || (im2col_one_round && cin % 64 == 0 && by_pieces)
                              ? mh_q8_conv_gather_us(ctx, cout, columns, depth, !gather)
                          : k_h * k_w == 1 && stride_h * stride_w > 1 ? (by_pieces ? 13 + 0.3e-6 * columns * kp : 16.5 + 1.9e-6 * columns * kp)
@@ -1266,9 +1271,6 @@ extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
                                          clamp_max, out, other, &taken));
     if (taken) return MACE_HIP_SUCCESS;
   }
-  size_t need = sizeof(int32_t) * cout + 4096 +
-                conv_gemm_scratch(cout, depth, columns, !in_place || depth % 16 == 0);
-  if (!in_place && !gather) need += (size_t)columns * kp + 4096;
   MH_RETURN_IF_ERROR(mh_arena_reserve(ctx, need));
   ArenaScope scope(ctx);
   const uint8_t *rhs = input;

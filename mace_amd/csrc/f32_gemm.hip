@@ -873,8 +873,10 @@ static int f32_slices_form(const mace_hip_ctx *ctx, int64_t batch, int64_t rows,
   const double old = parts > 1 ? (whole ? 12 : 15) + 0.63 * ((nk + parts - 1) / parts) + 8.0 * parts * total / 4e6
                                : (whole ? 5.3 : 8.3) + 0.63 * nk;
   const int form = tiles <= 400 ? 0 : 1, wk = kF32Slices[form].wk;
-  // (a second tile on a few CUs counts from long depths on: 62 x 2112 x 4552, 286 tiles, 34.7 us, 27.1 by 128 x 128 tiles)
-  const double share = nk > 64 && form == 0 && tiles > cus ? std::max(tiles / cus, 0.8 * ceil(tiles / cus)) : tiles / cus;
+  // (a second tile on a few CUs counts from long depths on: 62 x 2112 x 4552, 286 tiles, 34.7 us, 27.1 by 128 x 128 tiles;
+  // not where the parts of those could not be had)
+  const bool held = parts <= 1 || mh_arena_can_hold(ctx, sizeof(float) * (size_t)parts * total + 256);
+  const double share = nk > 64 && form == 0 && tiles > cus && held ? std::max(tiles / cus, 0.8 * ceil(tiles / cus)) : tiles / cus;
   const double one = 4.2 + std::max(0.75 * ((nk + wk - 1) / wk), share * (whole ? 0.25 + 0.14 * nk : 0.6 + 0.17 * nk));
   if (nk >= 24 && tiles > cus) {
     const int64_t wide = batch * ((rows + 31) / 32) * ((cols + 63) / 64);

@@ -2918,9 +2918,12 @@ int Q8Call::slices(bool *done) {
     const bool copies = !in_place && !(l16 && r16 && depth % 128 == 0);
     const double other = copies ? 11 + 0.0036 * depth + 0.25 * results : 5 + (depth % 64 == 0 ? 0.0035 : 0.006) * depth;
     worse = mine >= 0.9 * other;
-    if (ragged && !lhs_t && !rhs_t && steps >= 8) {
+    // (not where the scratch for sums and panels cannot be had, as in a capture on a new context: slices need none)
+    const bool had = mh_arena_can_hold(ctx, ((size_t)lhs_nb * rows + (size_t)rhs_nb * cols) *
+                                                ((copies ? mh_align_up((size_t)depth, 128) : 0) + 8) + (1 << 16));
+    if (had && ragged && !lhs_t && !rhs_t && steps >= 8) {
       worse |= 1.3 + 1.25 * steps >= 10 + 0.0028 * depth + 0.55 * copied + 0.25 * results;
-    } else if (nk >= 64 && tiles > cu && (depth % 16 != 0 || depth % 64 == 0)) {
+    } else if (had && nk >= 64 && tiles > cu && (depth % 16 != 0 || depth % 64 == 0)) {
       const int64_t wt = 8 / wk, groups = (tiles + wt - 1) / wt, busiest = wt * ((groups + (int64_t)cu - 1) / (int64_t)cu);
       worse |= 1.5 + busiest * (1.2 + (l4 && r4 ? 0.067 : 0.08) * nk) >=
                (copies ? 10.8 + 0.0028 * depth + 0.29 * copied + 0.13 * results : 1.1 * other);

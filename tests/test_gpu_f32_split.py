@@ -197,6 +197,38 @@ def test_joined_images_captured_without_scratch():
         c.close()
 
 
+def test_long_depth_recorded_without_scratch():
+    """62 x 2112 x 4552: tiles in parts of the depth where the parts can be had, else the slices kernel"""
+    import ctypes as C
+    rng = np.random.default_rng(3)
+    a, b = rng.standard_normal((62, 2112)).astype(np.float32), rng.standard_normal((2112, 4552)).astype(np.float32)
+    want = np.matmul(a.astype(np.float64), b.astype(np.float64))
+    size = np.matmul(np.abs(a).astype(np.float64), np.abs(b).astype(np.float64))
+    c = mh.Context(0)
+    try:
+        d = Dev()
+        pa, pb = d.put(a), d.put(b)
+        t, po = d.empty(want.size, np.float32)
+        d.sync()
+        args = (pa, pb, 1, 62, 4552, 2112, 0, 0, 0, 1, 1, po)
+        g = C.c_void_p()
+        c.call("mace_hip_graph_capture_begin")
+        status, kernel = c.status("mace_hip_gemm_f32", *args), c.last_plan().kernel
+        c.call("mace_hip_graph_capture_end", C.byref(g))
+        assert status == mh.SUCCESS and "slices" in kernel
+        for _ in range(3):
+            for run_it in (lambda: c.call("mace_hip_graph_launch", g), lambda: c.call("mace_hip_gemm_f32", *args)):
+                t.zero_()
+                d.sync()
+                run_it()
+                c.sync()
+                close(t.cpu().numpy().reshape(want.shape), want, size, 2112)
+            assert "slices" not in c.last_plan().kernel
+        c.call("mace_hip_graph_destroy", g)
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("lm,rm,om", [(0, 0, 0), (0, 1, 1), (1, 0, 1), (1, 1, 0)])
 @pytest.mark.parametrize("k", [1, 2])
 @pytest.mark.parametrize("batch,m,n,lb", [(1, 300, 257, 1), (3, 70, 129, 1), (70, 1, 1001, 0), (3, 1001, 1, 1), (5, 1, 1, 1), (2, 64, 128, 1)])

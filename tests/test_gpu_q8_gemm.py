@@ -284,6 +284,43 @@ def test_q8_gemm_slices(ctx, batch, rows, depth, cols, lb, rb, wk, lo, ro, oo):
         assert "slices_kernel<" not in masked[0] + masked[1]
 
 
+# products that other kernels take where they have scratch, and the slices kernel where there is none
+@pytest.mark.parametrize("m,k,n,ta,tb", [(224, 5761, 73, 0, 1), (1096, 2624, 576, 1, 0), (640, 7936, 459, 0, 1)])
+def test_q8_gemm_recorded_without_scratch(m, k, n, ta, tb):
+    import ctypes as C
+    import torch
+    rng = np.random.default_rng(m)
+    a, b = rng.integers(0, 256, (m, k), dtype=np.uint8), rng.integers(0, 256, (k, n), dtype=np.uint8)
+    want = ((a.astype(np.float64) - 120) @ (b.astype(np.float64) - 131)).astype(np.int32)
+    ad, bd = (torch.from_numpy(np.ascontiguousarray(x.T if t else x)).cuda() for x, t in ((a, ta), (b, tb)))
+    out = torch.zeros((m, n), dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    c = mh.Context(0)
+    try:
+        args = (ad.data_ptr(), ta, bd.data_ptr(), tb, out.data_ptr(), 0, 1, m, k, n, 1, 1, -120, -131)
+        graph = C.c_void_p()
+        c.call("mace_hip_graph_capture_begin")
+        status = c.status("mace_hip_gemm_q8_i32", *args)
+        family = c.last_plan().family
+        c.call("mace_hip_graph_capture_end", C.byref(graph))
+        assert (status, family) == (mh.SUCCESS, mh.KF_Q8_GEMM_SLICES)
+        for _ in range(3):
+            out.zero_()
+            torch.cuda.synchronize()
+            c.call("mace_hip_graph_launch", graph)
+            c.sync()
+            np.testing.assert_array_equal(out.cpu().numpy(), want)
+            out.zero_()
+            torch.cuda.synchronize()
+            c.call("mace_hip_gemm_q8_i32", *args)      # outside the capture: with scratch
+            assert c.last_plan().family != mh.KF_Q8_GEMM_SLICES
+            c.sync()
+            np.testing.assert_array_equal(out.cpu().numpy(), want)
+        c.call("mace_hip_graph_destroy", graph)
+    finally:
+        c.close()
+
+
 # Shapes on the boundaries between the one-launch kernels under the normal dispatch: the
 # eight-wavefront kernel ahead of the one-launch and the resident-tile kernels (one round of
 # 128 x 128 tiles, k >= 512; k-contiguous against the one-launch kernel from k = 1024), the
