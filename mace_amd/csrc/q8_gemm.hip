@@ -1029,6 +1029,7 @@ __global__ __launch_bounds__(WX *WY * 64, OCC) void q8_gemm_dma_kernel(GemmParam
     k_step(std::true_type{}, a1, b1, a0, b0, next, std::integral_constant<int, 0>{}, dst, ks * KB);
     stage = next;
   }
+  wait_vmcnt<0>();   // the last transfers have landed: their stage's LDS is the epilogue's (the compiler waits for some only)
   if constexpr (SUMY) {
     // The sums are of the bytes as read: minus the fragments the last step fetched beyond the last
     // slab (still in b0, flipped), minus 128 per byte of this lane's half of every k step.

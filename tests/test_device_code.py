@@ -69,6 +69,42 @@ def too_close(listing, wait=2):
     return swaps, bad
 
 
+RING = re.compile(r"q8_gemm_dma_kernelI")
+
+
+def transfers_at_barriers(listing):
+    """{ring kernel: [memory operations outstanding at each of its barriers]}; vmcnt(N) leaves N"""
+    found, kernel, out = {}, None, 0
+    for line in listing.splitlines():
+        label = re.match(r"[0-9a-f]+ <(.*)>:", line)
+        if label:
+            kernel, out = label[1] if RING.search(label[1]) else None, 0
+            continue
+        text = line.split("//")[0].strip()
+        if kernel is None:
+            continue
+        if re.match(r"(buffer|global)_load", text):
+            out += 1
+        elif text.startswith("s_waitcnt"):
+            left = re.search(r"vmcnt\((\d+)\)", text)
+            out = min(out, int(left[1])) if left else out
+        elif text.startswith("s_barrier"):
+            found.setdefault(kernel, []).append(out)
+    return found
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="needs ROCm's llvm-objdump")
+def test_no_transfer_is_outstanding_where_the_epilogue_takes_its_lds(tmp_path):
+    kernels = {}
+    for i, blob in enumerate(code_objects(mh.LIB_PATH)):
+        path = tmp_path / ("%d.co" % i)
+        path.write_bytes(blob)
+        kernels.update(transfers_at_barriers(subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", str(path)], check=True,
+                                                            capture_output=True, text=True).stdout))
+    assert len(kernels) >= 50 and all(len(v) >= 3 for v in kernels.values()), kernels   # prologue, loop, epilogue
+    assert not any(n for v in kernels.values() for n in v[2:]), {k: v for k, v in kernels.items() if any(v[2:])}
+
+
 # the ring kernel with slabs of 128 bytes: its transfers refill the stage of the slab being multiplied
 REFILLS = re.compile(r"q8_gemm_dma_kernelI(Li\d+E){5}[hi]Li\d+E(Lb[01]E){2}Li128E")
 
