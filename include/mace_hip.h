@@ -139,6 +139,7 @@ enum {
   MACE_HIP_KF_Q8_CONV_PLANES,          /* q8_conv_planes_kernel: padded planes staged in LDS, any channel count */
   MACE_HIP_KF_F32_GEMM_SLICES,       /* f32_gemm_slices_kernel: few tiles, a wavefront per slice of the depth */
   MACE_HIP_KF_Q8_GEMM_SLICES,        /* q8_gemm_slices_kernel: few tiles, any layout, a wavefront per slice of the depth */
+  MACE_HIP_KF_Q8_CONV_STAGED,        /* q8_conv_staged_kernel: input rows staged and shifted in LDS, any channel count, one launch */
   MACE_HIP_KF_COUNT
 };
 /* auxiliary passes of a call (bits of mace_hip_plan.aux) */

@@ -121,7 +121,8 @@ struct mace_hip_ctx {
   std::vector<void *> retired;
 };
 constexpr int MH_MASK_NO_SMALL = 1, MH_MASK_NO_XRES = 2, MH_MASK_NO_MID = 4, MH_MASK_NO_XFLIP = 8,
-              MH_MASK_NO_CONV_SHORT = 16, MH_MASK_NO_F32_SLICES = 32, MH_MASK_NO_Q8_SLICES = 64;
+              MH_MASK_NO_CONV_SHORT = 16, MH_MASK_NO_F32_SLICES = 32, MH_MASK_NO_Q8_SLICES = 64,
+              MH_MASK_NO_CONV_STAGED = 128;
 
 int mh_fail(mace_hip_ctx *ctx, int code, const char *fmt, ...);
 
@@ -232,6 +233,11 @@ inline int conv_rows(int fx, int ks) { return log2i(fx) * 2 + (ks == 9 ? 1 : 0);
 enum { PLANES_64x256 = 0, PLANES_32x256, PLANES_32x128, PLANES_32x32, PLANES_FORMS };
 // three: three k steps of a filter row, on two planes (a filter three wide)
 inline int conv_planes(int form, bool three) { return form * 2 + (three ? 1 : 0); }
+// wavefronts that share a block of pixels: 1, 2, 4, 8 (the last two: 1, two workgroups per CU); whole: channels in
+// whole pieces
+inline int conv_staged(int fx, int wk, bool whole, bool two) {
+  return two ? 16 + (whole ? 1 : 0) : (log2i(wk) * 2 + (fx == 2 ? 1 : 0)) * 2 + (whole ? 1 : 0);
+}
 inline int conv_ksplit(int waves) { return waves == 16 ? 1 : 0; }
 inline int gemv_mfma(int nw, bool out_u8) { return (log2i(nw) - 2) * 2 + (out_u8 ? 1 : 0); }
 inline int gemv_rows(int nb, bool out_u8) { return log2i(nb) * 2 + (out_u8 ? 1 : 0); }
@@ -588,6 +594,17 @@ int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
                       int64_t out_w, float input_scale, int32_t input_zp, float filter_scale, int32_t filter_zp,
                       float bias_scale, int32_t mult, int shift, int32_t out_zp, int clamp_min, int clamp_max,
                       uint8_t *out, double other, bool *taken);
+// conv_staged.hip: a convolution in one launch, its input staged in LDS, and an estimate of its time in us (HUGE_VAL: not a
+// call for it).  *taken = false: parameters that the general path takes or reports.
+double mh_q8_conv_staged_us(const mace_hip_ctx *ctx, int64_t n, int64_t in_h, int64_t in_w, int64_t cin, int64_t cout,
+                            int64_t k_h, int64_t k_w, int stride_h, int stride_w, int pad_top, int pad_left,
+                            int64_t out_h, int64_t out_w);
+int mh_q8_conv_staged(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, const int32_t *bias,
+                      int64_t n, int64_t in_h, int64_t in_w, int64_t cin, int64_t cout, int64_t k_h,
+                      int64_t k_w, int stride_h, int stride_w, int pad_top, int pad_left, int64_t out_h,
+                      int64_t out_w, float input_scale, int32_t input_zp, float filter_scale, int32_t filter_zp,
+                      float bias_scale, int32_t mult, int shift, int32_t out_zp, int clamp_min, int clamp_max,
+                      uint8_t *out, bool *taken);
 // Estimates of what a gathered convolution takes otherwise, in us: the one-launch kernel (conv_planes.hip; piece: bytes it
 // loads at a time), the gathering or patch-matrix GEMM (q8_gemm.hip).
 double mh_q8_conv_small_us(const mace_hip_ctx *ctx, int64_t cout, int64_t columns, int64_t depth, int piece);

@@ -1251,25 +1251,50 @@ extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
   size_t need = sizeof(int32_t) * cout + 4096 +
                 conv_gemm_scratch(cout, depth, columns, !in_place || depth % 16 == 0);
   if (!in_place && !gather) need += (size_t)columns * kp + 4096;
-  // All of these go through padded planes where that is faster.  (Up to nine taps of 64 channels stay with the kernel that
-  // keeps the filter in LDS: 56 x 56 x 64 -> 64 at batch 64 21.5 us, on planes 28.4.)
-  if (!in_place && (small_gather || cin % 64 != 0 || depth > 576)) {
+  // All of these go through rows staged in LDS or through padded planes where one of those is faster.  (On planes not up to
+  // nine taps of 64 channels, whose filter the gathering kernel keeps in LDS: 56 x 56 x 64 -> 64 at batch 64 21 us, on
+  // planes 28, staged 18.4.  Nor a 1 x 1 filter in place, whose channels in other than pieces of 8 are copied into padded rows otherwise,
+  // staged where its tiles are too many for the slices kernel: 102 x 103 x 28 -> 48 at 12 19.7 us, staged 10.6, 61 x 63 x
+  // 21 -> 20 at 64 27.6 and 11.6, 111 x 109 x 20 -> 64 at 48 46.8 and 35.4.)
+  const bool unpacked = in_place && cin % 8 != 0 && ((cout + 31) / 32) * ((columns + 31) / 32) > 4096 &&
+                        !mh_q8_small_problem(ctx, 1, cout, columns, depth, false, false) &&
+                        !mh_find_weight(ctx, filter, (size_t)(cout * depth));
+  if (!in_place || unpacked) {
     bool taken = false;
     // (a patch matrix of one tap, a 1 x 1 filter at a stride, is a fraction of the input, which the planes copy whole: 30 x
     // 30 x 995 -> 818 at stride 2, batch 7, 21.0 us, on planes 32.9, but 28 x 28 x 523 -> 129 at 21 28.8 and 21.3)
     const bool by_pieces = cin % 16 == 0 && (uintptr_t)input % 16 == 0;
     // (whatever the times, where only the planes' scratch can be had)
-    const double other = !mh_arena_can_hold(ctx, need) ? HUGE_VAL
-                         : small_gather ? mh_q8_conv_small_us(ctx, cout, columns, depth, small_vec ? 16 : (cin % 4 == 0 ? 4 : 1))
-                         : gather || (im2col_one_round && cin % 64 == 0 && by_pieces)
-                             ? mh_q8_conv_gather_us(ctx, cout, columns, depth, !gather)
-                         : k_h * k_w == 1 && stride_h * stride_w > 1 ? (by_pieces ? 13 + 0.3e-6 * columns * kp : 16.5 + 1.9e-6 * columns * kp)
-                                          : HUGE_VAL;
-    MH_RETURN_IF_ERROR(mh_q8_conv_planes(ctx, input, filter, bias, n, in_h, in_w, cin, cout, k_h, k_w, stride_h,
-                                         stride_w, pad_h >> 1, pad_w >> 1, out_h, out_w, input_scale, input_zp,
-                                         filter_scale, filter_zp, bias_scale, mult, shift, out_zp, clamp_min,
-                                         clamp_max, out, other, &taken));
-    if (taken) return MACE_HIP_SUCCESS;
+    double other = !mh_arena_can_hold(ctx, need) ? HUGE_VAL
+                   : small_gather ? mh_q8_conv_small_us(ctx, cout, columns, depth, small_vec ? 16 : (cin % 4 == 0 ? 4 : 1))
+                   : unpacked ? 9 + 0.065e-3 * columns
+                   : gather || (im2col_one_round && cin % 64 == 0 && by_pieces)
+                       ? mh_q8_conv_gather_us(ctx, cout, columns, depth, !gather)
+                   : k_h * k_w == 1 && stride_h * stride_w > 1 ? (by_pieces ? 13 + 0.3e-6 * columns * kp : 16.5 + 1.9e-6 * columns * kp)
+                                    : HUGE_VAL;
+    // (6.2 us: the least that the staged kernel takes, before its tile's geometry is worked out)
+    const double staged = has_pixels && 0.95 * other > 6.2
+                              ? mh_q8_conv_staged_us(ctx, n, in_h, in_w, cin, cout, k_h, k_w, stride_h, stride_w,
+                                                     pad_h >> 1, pad_w >> 1, out_h, out_w) : HUGE_VAL;
+    // (the estimates for patches of whole pieces in one launch and for one tap at a stride run high: 96 x 98 x 48 -> 48 7.2 us,
+    // staged 7.5, 56 x 56 x 64 -> 256 at stride 2, batch 32, 9.7 and 11.3)
+    const bool high = (small_gather && small_vec) || (!in_place && k_h * k_w == 1);
+    const bool by_staged = staged < (high ? 0.82 : 0.95) * other;
+    if (by_staged) other = staged;
+    if (!in_place && (small_gather || cin % 64 != 0 || depth > 576)) {
+      MH_RETURN_IF_ERROR(mh_q8_conv_planes(ctx, input, filter, bias, n, in_h, in_w, cin, cout, k_h, k_w, stride_h,
+                                           stride_w, pad_h >> 1, pad_w >> 1, out_h, out_w, input_scale, input_zp,
+                                           filter_scale, filter_zp, bias_scale, mult, shift, out_zp, clamp_min,
+                                           clamp_max, out, other, &taken));
+      if (taken) return MACE_HIP_SUCCESS;
+    }
+    if (by_staged) {
+      MH_RETURN_IF_ERROR(mh_q8_conv_staged(ctx, input, filter, bias, n, in_h, in_w, cin, cout, k_h, k_w, stride_h,
+                                           stride_w, pad_h >> 1, pad_w >> 1, out_h, out_w, input_scale, input_zp,
+                                           filter_scale, filter_zp, bias_scale, mult, shift, out_zp, clamp_min,
+                                           clamp_max, out, &taken));
+      if (taken) return MACE_HIP_SUCCESS;
+    }
   }
   MH_RETURN_IF_ERROR(mh_arena_reserve(ctx, need));
   ArenaScope scope(ctx);

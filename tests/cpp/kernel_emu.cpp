@@ -153,6 +153,17 @@ uint32_t emu_perm(uint32_t hi, uint32_t lo, uint32_t sel) {
   }
   return r;
 }
+// v_mov_dpp within sixteen lanes: a permutation of four, eight or sixteen lanes mirrored
+int emu_update_dpp(int, int v, int ctrl, int, int, bool) {
+  Wave &w = wave_of_thread();
+  const int l = lane_of_thread();
+  w.w[l][0] = (uint32_t)v;
+  w.bar.arrive_and_wait();
+  const int from = ctrl == 0x140 ? l ^ 15 : (ctrl == 0x141 ? l ^ 7 : (l & ~3) + ((ctrl >> (2 * (l & 3))) & 3));
+  const int r = (int)w.w[from][0];
+  w.bar.arrive_and_wait();
+  return r;
+}
 uint32_t __float_as_uint(float f) { uint32_t u; memcpy(&u, &f, 4); return u; }
 float __fmaf_rn(float a, float b, float c) { return fmaf(a, b, c); }
 inline int emu_readfirstlane(int v) { return v; }
@@ -162,6 +173,8 @@ inline int emu_readfirstlane(int v) { return v; }
 #define __builtin_amdgcn_sdot4 emu_sdot4
 #define __builtin_amdgcn_udot4 emu_udot4
 #define __builtin_amdgcn_perm emu_perm
+#define __builtin_amdgcn_update_dpp emu_update_dpp
+#define __builtin_amdgcn_sched_group_barrier(...) ((void)0)
 #define __builtin_amdgcn_readfirstlane emu_readfirstlane
 #define __builtin_amdgcn_sched_barrier(x) ((void)0)
 #define __builtin_amdgcn_s_barrier emu_s_barrier
@@ -204,6 +217,7 @@ constexpr int SLAB = 64;
 #include "pieces.inc"
 #include "kernels.inc"
 #include "conv_planes.inc"
+#include "conv_staged.inc"
 }  // namespace
 
 // ---- what the fp32 kernels' text needs ---------------------------------------------------------------
@@ -833,14 +847,70 @@ static void sums_case(int n, int k) {
   delete[] sums;
 }
 
+// the convolution on staged rows: the tile that the host code chooses on a device of `cu` CUs with `lds` bytes
+// of LDS each, operands allocated at exactly their size, every byte of the accumulators compared
+template <int FX, int WK, bool WHOLE, bool TWO = false>
+static void staged_case(int n, int in_h, int in_w, int cin, int cout, int k_h, int k_w, int sh, int sw, int pt, int pl,
+                        int out_h, int out_w, int cu, int lds = 160 * 1024) {
+  ++g_cases;
+  const StagedShape s{n, in_h, in_w, cin, cout, k_h, k_w, sh, sw, pt, pl, out_h, out_w};
+  EXPECT(staged_fits(s), "staged: the shape does not fit");
+  const int64_t in_bytes = (int64_t)n * in_h * in_w * cin, depth = (int64_t)k_h * k_w * cin, columns = (int64_t)n * out_h * out_w;
+  uint8_t *in = new uint8_t[in_bytes], *filter = new uint8_t[cout * depth];
+  int32_t *bias = new int32_t[cout];
+  for (int64_t i = 0; i < in_bytes; ++i) in[i] = rnd();
+  for (int64_t i = 0; i < cout * depth; ++i) filter[i] = rnd();
+  for (int i = 0; i < cout; ++i) bias[i] = (int)rnd() * 91 - 9000;
+  const int zi = 77, zf = 140;
+  ConvStagedParams p{};
+  const StagedPlan plan = staged_plan(s, FX, cu, lds, &p);
+  EXPECT(plan.groups > 0 && plan.lds <= lds && plan.fx == FX && plan.wk == WK && (TWO == (FX == 2 && plan.two)) && (cin % 16 == 0) == WHOLE,
+         "staged: %lld tiles of %d pixels, FX %d WK %d, %lld bytes of LDS", (long long)plan.groups, p.tile_px, plan.fx, plan.wk,
+         (long long)plan.lds);
+  p.in = in; p.filter = filter; p.bias = bias;
+  p.xcoef = -(zi - 128); p.ycoef = -(zf - 128); p.yadd = (int)depth * (zi - 128) * (zf - 128);
+  p.zpf4 = (uint32_t)(zi ^ 0x80) * 0x01010101u;
+  for (int byte = 0; byte < 3; byte += 2) {
+    p.rq = RequantFixed{-1 - byte, 0, 0, 0, 0, 255, 0};
+    uint8_t *out = new uint8_t[columns * cout];
+    memset(g_block.lds, 0xA5, sizeof(g_block.lds));
+    p.out = out;
+    run_grid(dim3(plan.groups * p.tiles_x), [&] { q8_conv_staged_kernel<FX, WK, WHOLE, TWO>(p); }, 512);
+    int64_t bad = 0;
+    for (int64_t px = 0; px < columns; ++px) {
+      const int ow = px % out_w, oh = px / out_w % out_h, img = px / out_w / out_h;
+      for (int c = 0; c < cout; ++c) {
+        int64_t acc = bias[c];
+        for (int kh = 0; kh < k_h; ++kh)
+          for (int kw = 0; kw < k_w; ++kw) {
+            const int ih = oh * sh - pt + kh, iw = ow * sw - pl + kw;
+            if (ih < 0 || ih >= in_h || iw < 0 || iw >= in_w) continue;   // the zero point
+            for (int ch = 0; ch < cin; ++ch)
+              acc += ((int)in[(((int64_t)img * in_h + ih) * in_w + iw) * cin + ch] - zi) *
+                     ((int)filter[c * depth + (kh * k_w + kw) * cin + ch] - zf);
+          }
+        bad += out[px * cout + c] != (uint8_t)((int32_t)acc >> (8 * byte));
+      }
+    }
+    EXPECT(bad == 0, "staged<%d,%d,%d> n %d %dx%dx%d>%d k%dx%d s%dx%d tiles of %d pixels: byte %d of %lld results differs", FX, WK,
+           (int)WHOLE, n, in_h, in_w, cin, cout, k_h, k_w, sh, sw, p.tile_px, byte, (long long)bad);
+    for (int64_t i = plan.lds; i < (int64_t)sizeof(g_block.lds); ++i)
+      if (g_block.lds[i] != 0xA5) { EXPECT(false, "staged: LDS byte %lld of %lld written", (long long)i, (long long)plan.lds); break; }
+    delete[] out;
+  }
+  delete[] in;
+  delete[] filter;
+  delete[] bias;
+}
+
 // PART (compile-time): 1 = everything but what follows, 2 = the ring and eight-wavefront kernels, 3 = the
 // uint8 slices kernel and the convolution on padded planes, 4 = the fp32 kernels and the planes' tile of eight
-// wavefronts; the test builds and runs the parts side by side.
+// wavefronts, 5 = the convolution on staged rows; the test builds and runs the parts side by side.
 #ifndef PART
 #define PART 0
 #endif
 int main() {
-#if PART != 2 && PART != 3 && PART != 4
+#if PART != 2 && PART != 3 && PART != 4 && PART != 5
   // the repacks of k-contiguous rows and of k-major operands: any row length
   for (int k : {1, 3, 15, 16, 17, 24, 63, 64, 65, 100, 127}) pack_case(1, 37, k, k, false);
   for (int k : {4, 8, 24, 40, 60, 64, 68, 120}) pack_case(1, 301, 130 + k, k, true);
@@ -979,6 +1049,19 @@ int main() {
   f32_gemv_case<0, 1>(2, 5, 1090, false, 0);
   planes_case<2, 1, 1, 8, 1, 3>(2, 9, 20, 20, 70, 3, 3, 1, 1, 1, 1, 9, 20, 150000, 2, 1);
   planes_case<2, 1, 1, 8, 1, 3>(5, 7, 9, 50, 33, 3, 3, 1, 1, 1, 1, 7, 9, 60000, 1, 2);
+#endif
+#if PART == 0 || PART == 5
+  // the convolution on staged rows: every tile form, whole and broken pieces, tiles over rows and images, tiles of
+  // whole images, strides above and below the filter, padding on any side, patches that end inside a stage
+  staged_case<2, 8, true>(1, 4, 9, 16, 40, 3, 3, 1, 1, 1, 1, 4, 9, 4);
+  staged_case<1, 8, false>(2, 3, 4, 45, 31, 3, 3, 1, 1, 2, 2, 5, 6, 2);
+  staged_case<2, 4, false>(2, 7, 7, 35, 33, 3, 3, 1, 1, 1, 1, 7, 7, 1);
+  staged_case<1, 4, true>(1, 9, 8, 32, 5, 4, 2, 2, 1, 1, 1, 4, 18, 1);
+  staged_case<2, 2, true>(1, 13, 14, 64, 36, 1, 1, 1, 1, 0, 0, 13, 14, 1);
+  staged_case<1, 2, false>(1, 29, 9, 21, 20, 2, 3, 1, 2, 0, 1, 28, 5, 1);
+  staged_case<2, 1, false>(1, 19, 15, 3, 34, 5, 5, 1, 1, 2, 2, 19, 15, 1);
+  staged_case<2, 1, true, true>(1, 25, 22, 16, 34, 1, 1, 1, 1, 0, 0, 25, 22, 1);
+  staged_case<1, 1, true>(6, 16, 20, 16, 9, 3, 3, 2, 2, 0, 0, 7, 9, 1);
 #endif
   if (g_failures) {
     printf("kernel_emu: %d failures in %d cases\n", g_failures, g_cases);

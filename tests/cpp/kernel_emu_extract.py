@@ -72,6 +72,12 @@ def main(out_dir):
             sys.exit("kernel_emu_extract: conv_planes.hip no longer has the line %r" % old)
         planes = planes.replace(old, new)
     open(os.path.join(out_dir, "conv_planes.inc"), "w").write(planes)
+    staged = open(os.path.join(CSRC, "conv_staged.hip")).read()
+    staged = staged[staged.index("struct ConvStagedParams {"):staged.index("// Time that the staged kernel takes, in us")]
+    old = "extern __shared__ __align__(16) uint8_t lds[];"
+    if old not in staged:
+        sys.exit("kernel_emu_extract: conv_staged.hip no longer has the line %r" % old)
+    open(os.path.join(out_dir, "conv_staged.inc"), "w").write(staged.replace(old, "uint8_t *lds = emu_lds();"))
     src = open(os.path.join(CSRC, "f32_gemm.hip")).read()
     parts = []
     for first, after in F32_PIECES:

@@ -280,11 +280,66 @@ def test_conv2d_q8_on_padded_planes(ctx, n, cout, cin, in_h, in_w, k_h, k_w, pad
                                        (bias, np.float32(s_in * s_f), np.float32(float(s_in * s_f) * 2.0 ** 26), 128, 0, 255)):
         want = orc.conv2d_q8_nhwc(x, f, bb, n, in_h, in_w, cin, cout, k_h, k_w, st, (ph, pw), s_in,
                                   z_in, s_f, z_f, s_b, so, z_o, lo, hi, nthreads=16)
-        got = conv_host(ctx, x, f, bb, n, in_h, in_w, cin, cout, k_h, k_w, st, (ph, pw), s_in,
-                        z_in, s_f, z_f, s_b, so, z_o, lo, hi)
+        ctx.call("mace_hip_ctx_set_kernel_mask", mh.MASK_NO_CONV_STAGED)
+        try:
+            got = conv_host(ctx, x, f, bb, n, in_h, in_w, cin, cout, k_h, k_w, st, (ph, pw), s_in,
+                            z_in, s_f, z_f, s_b, so, z_o, lo, hi)
+        finally:
+            ctx.call("mace_hip_ctx_set_kernel_mask", 0)
         assert ctx.last_plan().kernel == "q8_conv_planes_kernel<%s,SPR=%d>" % (form, spr), ctx.last_plan()
         assert got.shape == (n, oh, ow, cout)
         np.testing.assert_array_equal(got, want)
+
+
+STAGED_CASES = [  # batch, cout, cin, in_h, in_w, k_h, k_w, padding, strides, offset of the result, kernel
+    (6, 100, 70, 64, 67, 3, 3, S, (1, 1), 3, "FX=1,WK=1,WHOLE=false,TWO=false"),    # ragged channels, tiles over images
+    (13, 200, 66, 40, 41, 5, 5, S, (2, 1), 0, "FX=1,WK=1,WHOLE=false,TWO=false"),   # strides that differ
+    (10, 20, 37, 130, 130, 3, 3, V, (1, 1), 1, "FX=1,WK=1,WHOLE=false,TWO=false"),  # two workgroups on a CU
+    (11, 31, 50, 41, 39, 3, 3, Fu, (1, 1), 0, "FX=1,WK=4,WHOLE=false,TWO=false"),   # padding of 2 on every side
+    (6, 33, 79, 45, 37, 2, 4, S, (1, 1), 0, "FX=1,WK=4,WHOLE=false,TWO=false"),
+    (7, 90, 31, 50, 52, 3, 3, S, (1, 1), 0, "FX=1,WK=2,WHOLE=false,TWO=false"),
+    (1, 17, 333, 9, 8, 3, 3, S, (1, 1), 5, "FX=1,WK=8,WHOLE=false,TWO=false"),      # a pixel a tile
+    (2, 65, 161, 7, 13, 3, 3, S, (2, 2), 0, "FX=1,WK=8,WHOLE=false,TWO=false"),
+    (20, 24, 23, 17, 19, 6, 6, S, (1, 1), 0, "FX=1,WK=8,WHOLE=false,TWO=false"),
+    (64, 21, 19, 61, 63, 1, 1, S, (1, 1), 0, "FX=1,WK=1,WHOLE=false,TWO=false"),    # one tap, copied otherwise
+    (64, 64, 64, 14, 15, 3, 3, S, (1, 1), 0, "FX=1,WK=4,WHOLE=true,TWO=false"),
+    (3, 130, 256, 14, 14, 3, 3, S, (1, 1), 7, "FX=1,WK=8,WHOLE=true,TWO=false"),
+    (64, 64, 64, 56, 56, 3, 3, S, (1, 1), 0, "FX=2,WK=1,WHOLE=true,TWO=true"),
+    (64, 127, 128, 28, 28, 3, 3, S, (1, 1), 0, "FX=2,WK=1,WHOLE=true,TWO=false"),
+    (32, 130, 512, 7, 7, 3, 3, S, (1, 1), 0, "FX=1,WK=8,WHOLE=true,TWO=false"),
+]
+
+
+@pytest.mark.parametrize("n,cout,cin,in_h,in_w,k_h,k_w,pad,st,off,form", STAGED_CASES)
+def test_conv2d_q8_on_staged_rows(ctx, n, cout, cin, in_h, in_w, k_h, k_w, pad, st, off, form):
+    """Rows staged in LDS: bit for bit against the oracle, the kernel asserted, nothing beside the result written; with a
+    bias, with one that is rescaled and a narrow clamp, without, and with parameters outside the multiply-add form."""
+    import torch
+    rng = np.random.default_rng(cout * 7 + cin + k_h * 3 + k_w + in_w)
+    x = rng.integers(0, 256, (n, in_h, in_w, cin), dtype=np.uint8)
+    f = rng.integers(0, 256, (cout, k_h, k_w, cin), dtype=np.uint8)
+    bias = rng.integers(-2 ** 15, 2 ** 15, cout).astype(np.int32)
+    z_in, z_f = int(rng.integers(110, 147)), int(rng.integers(110, 147))
+    s_in, s_f = np.float32(0.02), np.float32(0.01)
+    s_out = np.float32(max(6.0, 3 * 74.0 * 74.0 * np.sqrt(k_h * k_w * cin) * float(s_in * s_f)) / 255.0)
+    _, _, ph, pw = orc.calc_padding_and_output_size(in_h, in_w, k_h, k_w, st, pad)
+    xd, fd, bd = (torch.from_numpy(a.reshape(-1)).cuda() for a in (x, f, bias))
+    for (bb, s_b, so, z_o, lo, hi) in ((bias, np.float32(s_in * s_f), s_out, 0, 0, 255),
+                                       (bias, np.float32(2.5 * float(s_in * s_f)), s_out, 100, 100, 230),
+                                       (None, np.float32(0), s_out, 128, 0, 255),
+                                       (bias, np.float32(s_in * s_f), np.float32(float(s_in * s_f) * 2.0 ** 26), 128, 0, 255)):
+        want = orc.conv2d_q8_nhwc(x, f, bb, n, in_h, in_w, cin, cout, k_h, k_w, st, (ph, pw), s_in,
+                                  z_in, s_f, z_f, s_b, so, z_o, lo, hi, nthreads=16)
+        out = torch.full((want.size + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        ctx.call("mace_hip_conv2d_q8_nhwc", xd.data_ptr(), fd.data_ptr(), None if bb is None else bd.data_ptr(), n, in_h, in_w,
+                 cin, cout, k_h, k_w, st[0], st[1], ph, pw, float(s_in), z_in, float(s_f), z_f, float(s_b), float(so), z_o, lo,
+                 hi, out.data_ptr() + 16 + off)
+        ctx.sync()
+        assert ctx.last_plan().kernel == "q8_conv_staged_kernel<%s>" % form, ctx.last_plan()
+        got = out.cpu().numpy()
+        np.testing.assert_array_equal(got[16 + off:16 + off + want.size].reshape(want.shape), want)
+        assert (got[:16 + off] == 0xA5).all() and (got[16 + off + want.size:] == 0xA5).all()
 
 
 @pytest.mark.parametrize("n,cout,cin,hw,k,off,family", [
@@ -351,6 +406,7 @@ def test_conv2d_q8_planes_where_scratch_cannot_grow():
     out = torch.zeros(want.size, dtype=torch.uint8, device="cuda")
     torch.cuda.synchronize()
     c = mh.Context(0)
+    c.call("mace_hip_ctx_set_kernel_mask", mh.MASK_NO_CONV_STAGED)   # (which needs no scratch)
     try:
         def call(images):
             c.call("mace_hip_conv2d_q8_nhwc", xd.data_ptr(), fd.data_ptr(), bd.data_ptr(), images, h, w, cin, cout, 3, 3, 1, 1,

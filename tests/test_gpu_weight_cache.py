@@ -111,7 +111,11 @@ def test_registered_filter_on_padded_planes(ctx, n, h, w, cin, cout):
                 float(np.float32(0.02 * 0.01)), 2.0, 10, 0, 255, out.data_ptr())
         if capture:
             ctx.call("mace_hip_graph_capture_begin")
-        ctx.call("mace_hip_conv2d_q8_nhwc", *args)
+        ctx.call("mace_hip_ctx_set_kernel_mask", mh.MASK_NO_CONV_STAGED)
+        try:
+            ctx.call("mace_hip_conv2d_q8_nhwc", *args)
+        finally:
+            ctx.call("mace_hip_ctx_set_kernel_mask", 0)
         plan = ctx.last_plan()
         if capture:
             graph = C.c_void_p()

@@ -1,7 +1,7 @@
 """Indexing of GPU kernels checked on the CPU: tests/cpp/kernel_emu.cpp compiles the source text of the
 uint8 GEMM kernels -- the ring kernel (k-contiguous, k-major and pre-shifted X, sums handed in or
 taken in the kernel), the eight-wavefront kernel (every layout of both operands), the
-resident-tile kernel (whole groups and depth tails), the one-launch kernel (every layout, rows read
+resident-tile kernel (whole groups and depth tails), the convolutions on padded planes and on staged rows, the one-launch kernel (every layout, rows read
 in pieces, dwords or bytes, gathered convolutions), the register-staged tiled kernel, the row
 repacks and the row sums -- for the host, runs them under AddressSanitizer on operands of exactly
 their size (ragged tiles, rows that are not whole pieces, fewer rows than a tile) and compares the
@@ -14,7 +14,7 @@ import subprocess
 import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-PARTS = (1, 2, 3, 4)
+PARTS = (1, 2, 3, 4, 5)
 CLANG = "/opt/rocm/llvm/bin/clang++"      # vector types of the kernels' text need clang
 
 
