@@ -99,7 +99,9 @@ int mace_hip_graph_destroy(mace_hip_ctx *ctx, mace_hip_graph *graph);
  * the eight-wavefront 128 x 128 kernel and the in-place reading of k-major operands; bit 3: the
  * repack that writes a panel already shifted to int8; bit 4: the convolution kernels for patches
  * of at most 32 bytes, for 16-channel pieces, for slices of the depth and on padded planes; bit 5: the fp32
- * kernel for slices of the depth; bit 6: the uint8 GEMM kernel for those (off with bit 0 too).  0 restores normal dispatch. */
+ * kernel for slices of the depth; bit 6: the uint8 GEMM kernel for those (off with bit 0 too);
+ * bit 7: the convolution kernel that stages its input rows (off with bit 4 too); bit 8: the fp32 kernel that keeps the
+ * left-hand matrix in LDS.  0 restores normal dispatch. */
 int mace_hip_ctx_set_kernel_mask(mace_hip_ctx *ctx, int mask);
 /* ---- kernel plans (test and measurement hook; no counterpart in the reference) ----------------
  * Which kernel a compute call runs is chosen on the host from the shapes, layouts, alignments and
@@ -140,6 +142,7 @@ enum {
   MACE_HIP_KF_F32_GEMM_SLICES,       /* f32_gemm_slices_kernel: few tiles, a wavefront per slice of the depth */
   MACE_HIP_KF_Q8_GEMM_SLICES,        /* q8_gemm_slices_kernel: few tiles, any layout, a wavefront per slice of the depth */
   MACE_HIP_KF_Q8_CONV_STAGED,        /* q8_conv_staged_kernel: input rows staged and shifted in LDS, any channel count, one launch */
+  MACE_HIP_KF_F32_GEMM_PANEL,        /* f32_gemm_panel_kernel: few rows kept in LDS, columns streamed past them */
   MACE_HIP_KF_COUNT
 };
 /* auxiliary passes of a call (bits of mace_hip_plan.aux) */

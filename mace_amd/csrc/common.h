@@ -122,7 +122,7 @@ struct mace_hip_ctx {
 };
 constexpr int MH_MASK_NO_SMALL = 1, MH_MASK_NO_XRES = 2, MH_MASK_NO_MID = 4, MH_MASK_NO_XFLIP = 8,
               MH_MASK_NO_CONV_SHORT = 16, MH_MASK_NO_F32_SLICES = 32, MH_MASK_NO_Q8_SLICES = 64,
-              MH_MASK_NO_CONV_STAGED = 128;
+              MH_MASK_NO_CONV_STAGED = 128, MH_MASK_NO_F32_PANEL = 256;
 
 int mh_fail(mace_hip_ctx *ctx, int code, const char *fmt, ...);
 
@@ -254,6 +254,8 @@ inline int f32_gemm_general(bool guard, int form, bool lk, bool rk) {
 // forms of kF32Slices: blocks of 32 columns and slices 1, 8; 1, 4; 2, 8
 enum { F32_SLICES_FORMS = 3 };
 inline int f32_slices(int form, bool lk, bool rk) { return form * 4 + (lk ? 2 : 0) + (rk ? 1 : 0); }
+// blocks of 32 rows; k steps of loads on their way: 2 or 4; guard: depths that are not whole k steps
+inline int f32_panel(int mi, int ahead, bool guard) { return (mi == 2 ? 4 : 0) | (ahead == 4 ? 2 : 0) | (guard ? 1 : 0); }
 // vectors a pass: 1, 2, 3, 4, 6, 8, 12, 16 (one row a wavefront: the first four)
 enum { F32_GEMV_VECTORS = 8, F32_GEMV_FLOATS = 4 };   // (FLOATS: f32_gemv_floats_kernel, in the general family)
 }  // namespace mhv

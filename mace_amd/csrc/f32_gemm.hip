@@ -410,6 +410,203 @@ __global__ __launch_bounds__(256 * SPLIT, SPLIT == 1 ? 3 : 1) void f32_gemm_kern
   f32_tile<LK, RK, SPLIT, true, TMT>(p);
 }
 
+// ---- a left-hand matrix that stays in LDS, columns streamed past it ----------------------------------
+//
+// A convolution's filter against the pixels of a batch is few rows against very many columns: per 128 x 128 tile the k loop
+// is short, and every tile pays for its first loads, a barrier per 16 depths and its stores, in step with the others on its
+// CU.  Here a workgroup keeps the three parts of 32 MI rows, all depths, in LDS as fragments (split once), and each of its
+// eight wavefronts walks blocks of 32 columns by itself: eight 4-byte loads a k step, coalesced over 32 columns, straight
+// into the fragment's registers and split there, no barrier.  The loads run D k steps ahead, on into the next block, so that
+// a block's stores and the next one's loads overlap.  Products and their order are f32_tile's with four wavefronts: the same
+// bits.
+// What bounds it: the bytes up to about 128 depths (112 x 112 x 32 -> 64 at batch 64 4.9 TB/s, what a copy reaches), beyond
+// that the vector ALU and the matrix cores, which take turns within a wavefront.  Before (tiles) and now, batch 64, us:
+// 112 x 112 x 32 -> 64 75 and 62.6, 56 x 56 x 128 -> 128 64.5 and 49.3, 28 x 28 x 256 -> 256 59.5 and 48.5, 56 x 56 x 100 ->
+// 200 130 and 95, 56 x 56 x 24 -> 144 59 and 37, 28 x 28 x 333 -> 111 56 and 45; 981 drawn layers of more tiles than CUs 1.38
+// times in the geometric mean.  (128 rows, eight wavefronts a CU: level at best, 36 % slower at 24 -> 144; a load under the
+// epilogue's test for a bias per column made every block wait for all of its loads and stores: 78 us on 56 x 56 x 128.)
+template <int MI, int D, bool GUARD>
+__global__ __launch_bounds__(512, 4) void f32_gemm_panel_kernel(F32GemmParams p, int groups, int blocks) {
+  extern __shared__ __align__(16) u4v panel[];     // [k step][part][32 rows][lane]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, r32 = lane & 31;
+  const int nks = (p.K + 15) >> 4;
+  float *const s_bias = (float *)(panel + (size_t)nks * 3 * MI * 64);
+  // Workgroup w runs on XCD w % 8: every XCD gets a contiguous span of (span of columns, rows), so that the
+  // workgroups that read the same columns share an L2.
+  int wg = blockIdx.x;
+  {
+    const int per = (int)gridDim.x >> 3, more = (int)gridDim.x & 7, xcd = wg & 7;
+    wg = xcd * per + min(xcd, more) + (wg >> 3);
+  }
+  const int group = wg / p.tiles_m, m0 = (wg - group * p.tiles_m) * (32 * MI);
+  const int b0 = (int)((int64_t)blocks * group / groups), b1 = (int)((int64_t)blocks * (group + 1) / groups);
+  const float *const B = p.rhs;
+
+  // byte offset of this lane's column of a block in the operand and in the result (there its half's first row)
+  auto columns_of = [&](int block, uint32_t *in, uint32_t *out) __attribute__((always_inline)) {
+    const int n = min(block * 32 + r32, p.N - 1);
+    int64_t at = n, to = n;
+    if (p.flat) {
+      const int img = n / p.flat, in_img = n - img * p.flat;
+      at = img * p.rbs + in_img;
+      to = img * p.obs + in_img;
+    }
+    *in = (uint32_t)(at * 4);
+    *out = (uint32_t)((to + (int64_t)(4 * h) * p.ors) * 4);
+  };
+  const int64_t row_bytes = p.rrs * 4;
+  const uint32_t half_off = h ? (uint32_t)(8 * row_bytes) : 0u;
+  float x[D][8];
+  // (no load sits under a condition: see f32_tile)
+  auto load = [&](int set, int ks, uint32_t off) __attribute__((always_inline)) {
+    const char *row = (const char *)B + (int64_t)(16 * ks) * row_bytes;
+    if constexpr (!GUARD) off += half_off;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (GUARD) {   // depths past the last re-read it; cleared when they are split
+        const int left = p.K - 1 - (16 * ks + e);
+        x[set][e] = *(const float *)(row + (off + (h ? (uint32_t)max(min(8, left), 0) * (uint32_t)row_bytes : 0u)));
+        row += left > 0 ? row_bytes : 0;
+      } else {
+        x[set][e] = *(const float *)(row + off);
+        row += row_bytes;
+      }
+    }
+  };
+  int block = b0 + wave;
+  uint32_t in_off, out_off;
+  columns_of(min(block, blocks - 1), &in_off, &out_off);
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, min(d, nks - 1), in_off);
+
+  // the rows' three parts, once; rows past the last repeat it, depths past the last are zeros
+  for (int u = tid; u < nks * 2 * 32 * MI; u += 512) {
+    const int row = u % (32 * MI), piece = u / (32 * MI);
+    const float *at = p.lhs + (int64_t)min(m0 + row, p.M - 1) * p.lrs + (int64_t)(8 * piece) * p.lcs;
+    float v[8];
+    if (p.lcs == 1 && 8 * piece + 8 <= p.K) {
+      __builtin_memcpy(&v[0], at, 16);
+      __builtin_memcpy(&v[4], at + 4, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int left = p.K - 1 - 8 * piece;      // (below 0: a piece of zeros)
+        v[e] = at[(int64_t)min(e, left) * p.lcs];
+        v[e] = e <= left ? v[e] : 0.f;
+      }
+    }
+    u4v part[3];
+    split_8(v, part);
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      panel[(((piece >> 1) * 3 + q) * MI + (row >> 5)) * 64 + (piece & 1) * 32 + (row & 31)] = part[q];
+  }
+  if (tid < 32 * MI) s_bias[tid] = p.bias_row ? p.bias_row[min(m0 + tid, p.M - 1)] : 0.f;
+  __syncthreads();
+
+  const int padded = (nks + D - 1) / D * D;
+  if (block >= b1) return;
+  do {   // (loops that run once at the least: no copies of registers whose loads are on their way)
+    const int next = block + 8;
+    uint32_t next_in, next_out;
+    columns_of(next < b1 ? next : block, &next_in, &next_out);
+    v16f acc[MI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
+    int ks0 = 0;
+    do {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const int ks = ks0 + d;
+        u4v b[3];
+        if constexpr (GUARD) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (16 * ks + 8 * h + e >= p.K) x[d][e] = 0.f;
+        }
+        split_8(x[d], b);
+        const int ahead = ks + D;
+        load(d, ahead < padded ? min(ahead, nks - 1) : min(ahead - padded, nks - 1), ahead < padded ? in_off : next_in);
+        if (ks < nks) {
+          const u4v *a = panel + (size_t)ks * (3 * MI * 64) + lane;
+          u4v f[3][MI];
+#pragma unroll
+          for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int i = 0; i < MI; ++i) f[q][i] = a[(q * MI + i) * 64];
+          constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};   // smallest products first
+#pragma unroll
+          for (int t = 0; t < 6; ++t)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+              acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8v, f[PA[t]][i]),
+                                                              __builtin_bit_cast(b8v, b[PB[t]]), acc[i], 0, 0, 0);
+        }
+      }
+      ks0 += D;
+    } while (ks0 < padded);
+    float worst = 0.f;   // not finite if one of the sums is not
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        worst = __fmaf_rn(acc[i][r], 0.f, worst);
+        acc[i][r] = acc[i][r] * SUM_SCALE;
+      }
+    if (__builtin_amdgcn_ballot_w64(worst != 0.f) != 0) {   // (see f32_tile)
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
+      for (int k0 = 0; k0 < p.K; k0 += 8) {
+        float v[4], a[4][MI];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int64_t k = min(k0 + 2 * u + h, p.K - 1);
+          v[u] = *(const float *)((const char *)(B + k * p.rrs) + in_off);
+#pragma unroll
+          for (int i = 0; i < MI; ++i) a[u][i] = p.lhs[(int64_t)min(m0 + i * 32 + r32, p.M - 1) * p.lrs + k * p.lcs];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const bool in = k0 + 2 * u + h < p.K;
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+            acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? a[u][i] : 0.f, in ? v[u] : 0.f, acc[i], 0, 0, 0);
+        }
+      }
+    }
+    const int n = block * 32 + r32;
+    const bool whole = m0 + 32 * MI <= p.M && block * 32 + 32 <= p.N;
+    auto store = [&](auto act_tag) __attribute__((always_inline)) {
+      constexpr int ACT = decltype(act_tag)::value;
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f4v bias = *(const f4v *)&s_bias[i * 32 + 8 * q + 4 * h];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int m = m0 + i * 32 + 8 * q + e;          // (and 4 h)
+            float v = acc[i][4 * q + e];
+            if (p.bias_row) v = v + bias[e];
+            v = apply_act(v, ACT, p.limit);
+            if (whole || (m + 4 * h < p.M && n < p.N)) *(float *)((char *)(p.out + (int64_t)m * p.ors) + out_off) = v;
+          }
+        }
+    };
+    if (p.act == MACE_HIP_ACT_RELU) store(std::integral_constant<int, MACE_HIP_ACT_RELU>{});
+    else if (p.act == MACE_HIP_ACT_RELUX) store(std::integral_constant<int, MACE_HIP_ACT_RELUX>{});
+    else store(std::integral_constant<int, MACE_HIP_ACT_NOOP>{});
+    block = next;
+    in_off = next_in;
+    out_off = next_out;
+  } while (block < b1);
+}
+
 // ---- few tiles, or shallow ones: a wavefront per slice of a 32 x 32 FN tile's depth -----------------
 //
 // A call of few 128 x 128 tiles is the serial chain of one of them: its k tiles one after the other, two launches where
@@ -980,6 +1177,42 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
       MH_PROF_END(ctx);
       MH_LAUNCH_CHECK(ctx);
       return MACE_HIP_SUCCESS;
+    }
+  }
+  // More tiles than CUs, a right-hand matrix along its columns and rows whose parts fit in LDS: columns streamed past the
+  // rows.  Tiles of 32 rows where a wavefront would have fewer than about two blocks of 32 rows x 32 columns (80 x 82 x 32
+  // -> 70 at batch 6 8.0 us, in tiles of 64 11.1) and where those leave an eighth less padding; else of 64.  (Of one k step
+  // the 128-row tiles are up to 10 % faster: 54 x 53 x 16 -> 129 at 10 9.0 us and 9.9.)
+  if (!split && batch == 1 && !rk && out_major == MACE_HIP_ROW_MAJOR && !p.bias_col && depth > 16 && p.N >= 8ll * p.M &&
+      images * depth * cols < (1ll << 30) && total < (1ll << 30) && !(ctx->kernel_mask & MH_MASK_NO_F32_PANEL)) {
+    const int nks = (int)((depth + 15) / 16), blocks = (p.N + 31) / 32;
+    auto lds_of = [&](int mi) { return (size_t)nks * 3 * mi * 1024 + 128 * mi; };
+    const int64_t small = (p.M + 31) / 32, large = (p.M + 63) / 64;
+    const bool narrow = p.M <= 32 || blocks * small <= 24 * cus || 23 * small <= 40 * large;
+    const int mi = narrow || lds_of(2) > (size_t)ctx->lds_bytes ? 1 : 2;
+    const size_t lds = lds_of(mi);
+    if (lds <= (size_t)ctx->lds_bytes) {
+      p.tiles_m = (int)(mi == 1 ? small : large);
+      // (k steps of loads on their way; a block's end is padded to a multiple of them)
+      const int ahead = nks % 4 == 0 || nks >= 7 ? 4 : 2;
+      auto launch = [&](auto kernel) -> int {
+        MH_HIP(ctx, mh_allow_big_lds(ctx, (const void *)kernel, lds));
+        const int64_t fit = cus * mh_blocks_per_cu(ctx, (const void *)kernel, 512, lds);
+        const int groups = (int)std::max<int64_t>(1, std::min<int64_t>((blocks + 7) / 8, fit / p.tiles_m));
+        grid.x = (unsigned)(groups * p.tiles_m);
+        mh_plan_main(ctx, MACE_HIP_KF_F32_GEMM_PANEL, mhv::f32_panel(mi, ahead, !whole), grid, block2, (int)lds);
+        MH_PROF_BEGIN(ctx);
+        MH_KLAUNCH(ctx, kernel, grid, block2, lds, ctx->stream, p, groups, blocks);
+        MH_PROF_END(ctx);
+        MH_LAUNCH_CHECK(ctx);
+        return MACE_HIP_SUCCESS;
+      };
+#define MH_F32_PANEL(MI, D) return whole ? launch(f32_gemm_panel_kernel<MI, D, false>) : launch(f32_gemm_panel_kernel<MI, D, true>)
+      if (mi == 1 && ahead == 2) MH_F32_PANEL(1, 2);
+      if (mi == 1) MH_F32_PANEL(1, 4);
+      if (ahead == 2) MH_F32_PANEL(2, 2);
+      MH_F32_PANEL(2, 4);
+#undef MH_F32_PANEL
     }
   }
   // Few tiles and a long depth: the k tiles are dealt to several workgroups per tile, whose parts a

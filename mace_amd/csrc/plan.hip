@@ -39,6 +39,7 @@ const int kVariantCount[MACE_HIP_KF_COUNT] = {
     mhv::F32_SLICES_FORMS * 4,   // F32_GEMM_SLICES
     16,                       // Q8_GEMM_SLICES
     18,                       // Q8_CONV_STAGED
+    8,                        // F32_GEMM_PANEL
 };
 static_assert(mhv::RING_CONFIGS * 8 <= kMaxVariants, "coverage table too narrow");
 
@@ -50,7 +51,8 @@ const char *const kFamilyName[MACE_HIP_KF_COUNT] = {
     "f32_gemm_kernel", "f32_fill_kernel", "f32_gemv_rows_kernel", "f32_gemv_kernel",
     "q8_conv_short_kernel", "q8_conv_rows_kernel", "q8_conv_ksplit_kernel",
     "q8_conv_kslices_kernel", "q8_conv_planes_kernel", "f32_gemm_slices_kernel",
-    "q8_gemm_slices_kernel", "q8_conv_staged_kernel"};
+    "q8_gemm_slices_kernel", "q8_conv_staged_kernel",
+    "f32_gemm_panel_kernel"};
 
 // <WX, WY, FX, FY, STAGES, OCC, KB> of the ring kernel's tile configurations (mhv::RING_*)
 const int kRing[mhv::RING_CONFIGS][7] = {
@@ -208,6 +210,9 @@ int mace_hip_plan_describe(int family, int v, char *buf, size_t len) {
     case MACE_HIP_KF_Q8_CONV_STAGED:
       snprintf(buf, len, "%s<FX=%d,WK=%d,WHOLE=%s,TWO=%s>", k, v >= 16 || (v & 2) ? 2 : 1, v >= 16 ? 1 : 1 << (v >> 2),
                tf(v & 1), tf(v >= 16));
+      break;
+    case MACE_HIP_KF_F32_GEMM_PANEL:
+      snprintf(buf, len, "%s<MI=%d,D=%d,GUARD=%s>", k, (v & 4) ? 2 : 1, (v & 2) ? 4 : 2, tf(v & 1));
       break;
     case MACE_HIP_KF_F32_GEMM_SLICES: {
       static const char *const form[mhv::F32_SLICES_FORMS] = {"FN=1,WK=8", "FN=1,WK=4", "FN=2,WK=8"};

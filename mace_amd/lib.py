@@ -14,7 +14,8 @@ ROW_MAJOR, COL_MAJOR = 0, 1
 REQUANT_REF, REQUANT_NEON = 0, 1
 ACT_NOOP, ACT_RELU, ACT_RELUX = 0, 1, 2
 (MASK_NO_SMALL, MASK_NO_XRES, MASK_NO_MID, MASK_NO_XFLIP, MASK_NO_CONV_SHORT,
- MASK_NO_F32_SLICES, MASK_NO_Q8_SLICES, MASK_NO_CONV_STAGED) = (1 << i for i in range(8))
+ MASK_NO_F32_SLICES, MASK_NO_Q8_SLICES, MASK_NO_CONV_STAGED,
+ MASK_NO_F32_PANEL) = (1 << i for i in range(9))
 NOALLOC_SCRATCH_BYTES = 32 << 20
 
 _STATUS_NAMES = {0: "MACE_SUCCESS", 1: "MACE_INVALID_ARGS", 2: "MACE_OUT_OF_RESOURCES",
@@ -133,7 +134,8 @@ SIGNATURES = {
  KF_Q8_GEMV_MFMA_LDS, KF_Q8_GEMV_MFMA, KF_Q8_GEMV_ROWS, KF_Q8_GEMV_GENERAL, KF_F32_GEMM_VEC,
  KF_F32_GEMM_GENERAL, KF_F32_GEMM_FILL, KF_F32_GEMV_VEC, KF_F32_GEMV_GENERAL, KF_Q8_CONV_SHORT,
  KF_Q8_CONV_ROWS, KF_Q8_CONV_KSPLIT, KF_Q8_CONV_KSLICES, KF_Q8_CONV_PLANES,
- KF_F32_GEMM_SLICES, KF_Q8_GEMM_SLICES, KF_Q8_CONV_STAGED, KF_COUNT) = range(29)
+ KF_F32_GEMM_SLICES, KF_Q8_GEMM_SLICES, KF_Q8_CONV_STAGED,
+ KF_F32_GEMM_PANEL, KF_COUNT) = range(30)
 (AUX_PACK_ROWS, AUX_PACK_TRANSPOSE, AUX_PACK_SHIFTED, AUX_PANEL_SUMS, AUX_KMAJOR_SUMS, AUX_ZERO,
  AUX_IM2COL, AUX_BIAS_RESCALE, AUX_F32_PAD, AUX_FILL, AUX_WEIGHT_HIT, AUX_WEIGHT_BUILD,
  AUX_F32_KSPLIT, AUX_Q8_KSPLIT, AUX_CONV_PLANES) = (1 << i for i in range(15))

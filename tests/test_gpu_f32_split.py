@@ -330,3 +330,53 @@ def test_slices_over_images_with_bias_and_activation():
             close(t.cpu().numpy().reshape(raw.shape), np.clip(raw, 0, 1.25), size, cin)
     finally:
         c.close()
+
+
+# tiles of 32 and 64 rows, two and four k steps ahead; rows, columns and depths that end inside a tile, a block, a step
+PANEL_CASES = [("MI=1,D=2,GUARD=false", 37, 32, 30, 900), ("MI=1,D=4,GUARD=true", 37, 53, 30, 901), ("MI=2,D=2,GUARD=true", 33, 21, 64, 3001),
+               ("MI=2,D=4,GUARD=false", 64, 128, 120, 800), ("MI=2,D=4,GUARD=true", 60, 211, 61, 1999), ("MI=1,D=4,GUARD=true", 24, 403, 129, 1500),
+               ("MI=1,D=2,GUARD=true", 1, 17, 5, 33001), ("MI=1,D=2,GUARD=false", 700, 96, 90, 49)]
+
+
+@pytest.mark.parametrize("form,images,k,m,n", PANEL_CASES)
+def test_columns_streamed_past_rows_in_lds(form, images, k, m, n):
+    """the same bits as the tile kernel's, the result alone written, against binary64; images that are not finite"""
+    rng = np.random.default_rng(m + n + k)
+    x, f, bias = (rng.standard_normal(s).astype(np.float32) for s in ((images, k, n), (m, k), (m,)))
+    c = mh.Context(0)
+    try:
+        d = Dev()
+        pf, pb = d.put(f), d.put(bias)
+
+        def conv(x, act, mask):
+            px = d.put(x)
+            t, po = d.empty(images * m * n + 32, np.float32)
+            t.fill_(-7.0)
+            d.sync()
+            c.lib.mace_hip_ctx_set_kernel_mask(c.handle, mask)
+            c.call("mace_hip_conv1x1_f32_nchw", px, pf, pb, images, k, n, m, act, 3.0, po.value + 64)
+            c.sync()
+            got = t.cpu().numpy()
+            assert (got[:16] == -7.0).all() and (got[16 + images * m * n:] == -7.0).all()
+            return got[16:16 + images * m * n].reshape(images, m, n)
+        for act in (mh.ACT_NOOP, mh.ACT_RELUX):
+            got = conv(x, act, 0)
+            assert c.last_plan().kernel == "f32_gemm_panel_kernel<%s>" % form, c.last_plan()
+            tiles = conv(x, act, mh.MASK_NO_F32_PANEL)
+            assert "panel" not in c.last_plan().kernel and "slices" not in c.last_plan().kernel
+            assert np.array_equal(got, tiles)
+        got = conv(x, mh.ACT_NOOP, 0)
+        want = np.matmul(f.astype(np.float64), x.astype(np.float64)) + bias[:, None].astype(np.float64)
+        size = np.matmul(np.abs(f).astype(np.float64), np.abs(x).astype(np.float64)) + np.abs(bias)[:, None]
+        close(got, want, size, k)
+        x[0, k // 2, n // 3] = np.inf
+        x[-1, k // 3, n // 2] = np.nan
+        x[images // 2, :, n - 1] = 1e36           # (beyond the split)
+        got = conv(x, mh.ACT_NOOP, 0)
+        want = np.matmul(f.astype(np.float64), x.astype(np.float64)) + bias[:, None].astype(np.float64)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+        fin = np.isfinite(want)
+        size = np.matmul(np.abs(f).astype(np.float64), np.abs(np.where(np.isfinite(x), x, 0)).astype(np.float64)) + np.abs(bias)[:, None]
+        close(got[fin], want[fin], size[fin], k)
+    finally:
+        c.close()
