@@ -1189,9 +1189,13 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
     auto lds_of = [&](int mi) { return (size_t)nks * 3 * mi * 1024 + 128 * mi; };
     const int64_t small = (p.M + 31) / 32, large = (p.M + 63) / 64;
     const bool narrow = p.M <= 32 || blocks * small <= 24 * cus || 23 * small <= 40 * large;
-    const int mi = narrow || lds_of(2) > (size_t)ctx->lds_bytes ? 1 : 2;
+    // (Depths from 417 on leave room for 32 rows of more than that at a time: where loads are not checked only against
+    // 128-row tiles that are a fifth padding.  14 x 14 x 512 -> 512 at batch 64 52 us in tiles, 55 - 66 here; 13440 columns,
+    // 512 -> 258 50 and 35, 7020 columns, 456 -> 575 79 and 47.)
+    const bool deep = lds_of(2) > (size_t)ctx->lds_bytes;
+    const int mi = narrow || deep ? 1 : 2;
     const size_t lds = lds_of(mi);
-    if (lds <= (size_t)ctx->lds_bytes) {
+    if (lds <= (size_t)ctx->lds_bytes && (!deep || p.M <= 32 || !whole || 4 * TM * ((p.M + TM - 1) / TM) >= 5ll * p.M)) {
       p.tiles_m = (int)(mi == 1 ? small : large);
       // (k steps of loads on their way; a block's end is padded to a multiple of them)
       const int ahead = nks % 4 == 0 || nks >= 7 ? 4 : 2;
