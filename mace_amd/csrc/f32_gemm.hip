@@ -135,7 +135,10 @@ __device__ __forceinline__ void split_8(const float (&x)[8], u4v (&part)[3]) {
 // for launches of at most one tile per CU, where one wavefront per SIMD would leave every LDS wait
 // exposed.
 // GUARD: depths that are not whole k tiles of 16, or an operand that is contiguous along depth in
-// rows that are not aligned 16-byte pieces: single loads, each checked against the depth.
+// rows that are not aligned 16-byte pieces: the same loads at any address; a unit that the depth ends in is read early
+// and moved down to its place in the last k tile (SHORT, depths below 8: single loads, each checked).  With every load
+// checked by itself, us, before and now: 3000 x 1000 x 1200 75 and 55 (1008 deep 54), 3000 x 1001 x 1201 against transposed
+// weights 104 and 54, 5000 x 300 x 2000 96 and 52, 627 x 1603 x 832 39 and 29.
 //
 // A thread's unit is eight consecutive depths of one row: two 16-byte loads where depth is
 // contiguous, else eight 4-byte loads, each coalesced over the wavefront's 64 rows (so rows of any
@@ -144,7 +147,7 @@ __device__ __forceinline__ void split_8(const float (&x)[8], u4v (&part)[3]) {
 // and read consecutive 16-byte pieces.  Two LDS stages and two register sets: k tile t + 3 is
 // requested, and k tile t + 1 split and stored, while k tile t is multiplied (a load has two k tiles
 // of time to arrive), the split's instructions dealt out between the MFMAs.
-template <bool LK, bool RK, int SPLIT, bool GUARD, int TMT>
+template <bool LK, bool RK, int SPLIT, bool GUARD, int TMT, bool SHORT = false>
 __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
   constexpr int NT = 256 * SPLIT;
   constexpr int BKT = 16 * SPLIT;          // depths per k tile
@@ -188,20 +191,25 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
   // No load sits under a condition (the waits in front of their use then leave younger requests in
   // flight): units past the depth re-read its last eight, single elements past it the last one.
   auto load_unit = [&](auto contig, const float *at, int64_t step, int kk, float (&x)[8]) __attribute__((always_inline)) {
-    if constexpr (GUARD) {
+    if constexpr (SHORT) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = at[(int64_t)min(kk + e, kend - 1) * step];
-    } else {
-      kk = min(kk, kend - 8);
-      if constexpr (decltype(contig)::value) {
+      return;
+    }
+    kk = min(kk, kend - 8);
+    if constexpr (decltype(contig)::value) {
+      if constexpr (GUARD) {
+        __builtin_memcpy(&x[0], at + kk, 16);
+        __builtin_memcpy(&x[4], at + kk + 4, 16);
+      } else {
         const f4v v0 = *(const f4v *)(at + kk), v1 = *(const f4v *)(at + kk + 4);
 #pragma unroll
         for (int e = 0; e < 4; ++e) { x[e] = v0[e]; x[4 + e] = v1[e]; }
-      } else {
-        const float *q = at + (int64_t)kk * step;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) { x[e] = *q; q += step; }
       }
+    } else {
+      const float *q = at + (int64_t)kk * step;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) { x[e] = *q; q += step; }
     }
   };
   float xa[2][8], xb[2][8];
@@ -211,18 +219,28 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
     load_unit(std::integral_constant<bool, RK>{}, pb, p.rrs, kt0 + kt * BKT + bc * 8, xb[S]);
   };
   auto clear_past_depth = [&](auto set, int kt) __attribute__((always_inline)) {
-    if constexpr (GUARD) {   // what lies past the depth counts as zero
+    if constexpr (GUARD) {
       constexpr int S = decltype(set)::value;
+      if (kt0 + (kt + 1) * BKT <= kend) return;
+      // the last k tile: units that were read early move down to their place; what lies past the depth counts as zero
+      auto settle = [&](int kk, float (&x)[8]) __attribute__((always_inline)) {
+        if constexpr (!SHORT) {
+          const int early = max(kk - (kend - 8), 0);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        if (kt0 + kt * BKT + ac * 8 + e >= kend) xa[S][e] = 0.f;
-        if (kt0 + kt * BKT + bc * 8 + e >= kend) xb[S][e] = 0.f;
-      }
+          for (int by = 4; by > 0; by >>= 1)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = early & by ? (e + by < 8 ? x[e + by] : 0.f) : x[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = kk + e < kend ? x[e] : 0.f;
+      };
+      settle(kt0 + kt * BKT + ac * 8, xa[S]);
+      settle(kt0 + kt * BKT + bc * 8, xb[S]);
     }
   };
-  auto store_tile = [&](auto set, int kt, int buf) __attribute__((always_inline)) {
+  auto store_tile = [&](auto set, int kt, int buf, auto last) __attribute__((always_inline)) {
     constexpr int S = decltype(set)::value;
-    clear_past_depth(set, kt);
+    if constexpr (decltype(last)::value) clear_past_depth(set, kt);
     u4v part[3];
     split_8(xa[S], part);
     if (has_a) {
@@ -276,15 +294,15 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
   load_tile(set0, 0);
   load_tile(set1, 1);
   if (tid < TMT) s_bias[tid] = bias_m;
-  store_tile(set0, 0, 0);
+  store_tile(set0, 0, 0, std::true_type{});
   load_tile(set0, 2);
   __syncthreads();
   // k tile t: its fragments read, the MFMAs with the split of tile t + 1 between them, then the request
   // for tile t + 3 into the registers that the split has freed
-  auto step = [&](auto set, int kt) __attribute__((always_inline)) {
+  auto step = [&](auto set, int kt, auto last) __attribute__((always_inline)) {
     constexpr int S = decltype(set)::value;   // tile kt + 1's registers
     multiply(std::integral_constant<int, BKT / 16>{}, S ^ 1);
-    store_tile(set, kt + 1, S);
+    store_tile(set, kt + 1, S, last);
     constexpr int MFMAS = BKT / 16 * 6 * FM * FN;
 #pragma unroll
     for (int i = 0; i < MFMAS; ++i) {
@@ -297,11 +315,18 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
   // (eight wavefronts: half a k tile at the end of a depth that has one; a guarded one is filled up
   // with zeros instead)
   const int nfull = GUARD ? nk : (kend - kt0) / BKT;
-  for (int kt = 0; kt + 1 < nfull; kt += 2) {
-    step(set1, kt);
-    step(set0, kt + 1);
+  int kt = 0;
+  if constexpr (GUARD) {   // (the test for the last k tile apart: with it between a step's MFMAs and its split they would not mix)
+    for (; kt + 3 < nfull; kt += 2) {
+      step(set1, kt, std::false_type{});
+      step(set0, kt + 1, std::false_type{});
+    }
   }
-  if (nfull & 1) step(set1, nfull - 1);
+  for (; kt + 1 < nfull; kt += 2) {
+    step(set1, kt, std::bool_constant<GUARD>{});
+    step(set0, kt + 1, std::bool_constant<GUARD>{});
+  }
+  if (nfull & 1) step(set1, nfull - 1, std::bool_constant<GUARD>{});
   if (BKT == 32 && nfull < nk) multiply(std::integral_constant<int, 1>{}, nfull & 1);
 
   if constexpr (NACC == 2) {
@@ -405,9 +430,9 @@ template <bool LK, bool RK, int SPLIT, int TMT>
 __global__ __launch_bounds__(256 * SPLIT, SPLIT == 1 ? 3 : 1) void f32_gemm_vec_kernel(F32GemmParams p) {
   f32_tile<LK, RK, SPLIT, false, TMT>(p);
 }
-template <bool LK, bool RK, int SPLIT, int TMT>
+template <bool LK, bool RK, int SPLIT, int TMT, bool SHORT>
 __global__ __launch_bounds__(256 * SPLIT, SPLIT == 1 ? 3 : 1) void f32_gemm_kernel(F32GemmParams p) {
-  f32_tile<LK, RK, SPLIT, true, TMT>(p);
+  f32_tile<LK, RK, SPLIT, true, TMT, SHORT>(p);
 }
 
 // ---- a left-hand matrix that stays in LDS, columns streamed past it ----------------------------------
@@ -1260,9 +1285,12 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
   if (whole && split) MH_F32_LR(f32_gemm_vec_kernel, 2, 128);
   else if (whole && half) MH_F32_LR(f32_gemm_vec_kernel, 1, 64);
   else if (whole) MH_F32_LR(f32_gemm_vec_kernel, 1, 128);
-  else if (split) MH_F32_LR(f32_gemm_kernel, 2, 128);
-  else if (half) MH_F32_LR(f32_gemm_kernel, 1, 64);
-  else MH_F32_LR(f32_gemm_kernel, 1, 128);
+  else if (depth < 8 && split) MH_F32_LR(f32_gemm_kernel, 2, 128, true);
+  else if (depth < 8 && half) MH_F32_LR(f32_gemm_kernel, 1, 64, true);
+  else if (depth < 8) MH_F32_LR(f32_gemm_kernel, 1, 128, true);
+  else if (split) MH_F32_LR(f32_gemm_kernel, 2, 128, false);
+  else if (half) MH_F32_LR(f32_gemm_kernel, 1, 64, false);
+  else MH_F32_LR(f32_gemm_kernel, 1, 128, false);
 #undef MH_F32_LR
 #undef MH_F32
   MH_PROF_END(ctx);
