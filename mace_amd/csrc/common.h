@@ -122,7 +122,7 @@ struct mace_hip_ctx {
 };
 constexpr int MH_MASK_NO_SMALL = 1, MH_MASK_NO_XRES = 2, MH_MASK_NO_MID = 4, MH_MASK_NO_XFLIP = 8,
               MH_MASK_NO_CONV_SHORT = 16, MH_MASK_NO_F32_SLICES = 32, MH_MASK_NO_Q8_SLICES = 64,
-              MH_MASK_NO_CONV_STAGED = 128, MH_MASK_NO_F32_PANEL = 256;
+              MH_MASK_NO_CONV_STAGED = 128, MH_MASK_NO_F32_PANEL = 256, MH_MASK_NO_Q8_LOOSE = 512;
 
 int mh_fail(mace_hip_ctx *ctx, int code, const char *fmt, ...);
 
@@ -197,7 +197,9 @@ enum { XRES_PLAIN = 0, XRES_XT = 1, XRES_TAIL = 2, XRES_CONV = 3 };
 inline int xres(int mode, int fx, int fy, int group, bool out_u8) {
   return ((((mode * 2 + (fx == 4)) * 2 + (fy == 2)) * 2 + (group == 128)) * 2) + (out_u8 ? 1 : 0);
 }
-inline int mid(bool out_u8, bool xt, bool yt = false) { return (yt ? 4 : 0) | (xt ? 2 : 0) | (out_u8 ? 1 : 0); }
+inline int mid(bool out_u8, bool xt, bool yt = false, bool loose = false) {
+  return (loose ? 8 : 0) | (yt ? 4 : 0) | (xt ? 2 : 0) | (out_u8 ? 1 : 0);
+}
 inline int stream(int fx, int ks) { return (fx - 1) * 2 + (ks - 1); }
 // tile configurations of the ring kernel: <WX, WY, FX, FY, STAGES, OCC, KB>
 enum { RING_1422_3_2 = 0, RING_2222_3_3, RING_2244_2_1_128, RING_2421_2_1_128, RING_2222_2_2_128,

@@ -61,6 +61,9 @@ struct GemmParams {
   const uint8_t *cv_zero;   // >= 64 bytes holding the input zero point (padding positions)
   uint32_t cv_zp4;          // the input zero point in all four bytes (q8_gemm_fused_small_kernel)
   bool conv;
+  // q8_gemm_mid_kernel<LOOSE>: the depth (K: in whole slabs), bytes from X and Y to the operands' ends
+  int k_real;
+  int64_t x_left, y_left;
   // q8_gemm_fused_small_kernel: the operand's rows are not 16-byte pieces (odd depth or row
   // length, unaligned base) and are read byte by byte
   bool x_bytewise, y_bytewise;
@@ -1250,9 +1253,16 @@ __global__ __launch_bounds__(512, 4) void q8_gemm_slices_kernel(GemmParams p) {
 //   * YT: the same for the Y operand (Y(y, k) at Y[k * ldy + y]: the ColMajor left-hand matrix of a
 //     MatMul with transpose_a and a RowMajor result); the MFMA's two operands have the same register
 //     layout, so the Y half of a slab and its fragment reads mirror the X half's.
-// Requirements (checked by the host): K % 128 == 0, rows addressable with 32-bit offsets; XT / YT:
+//   * LOOSE: operands of any alignment, row length and depth from 16 on.  A piece cannot be transferred from any address,
+//     so a thread loads its four pieces of a slab into registers (16 bytes at any address), two slabs ahead of the one that
+//     it stores, which is two ahead of the one that is multiplied: a ring of three stages.  In the slabs that reach past
+//     the depth, or past the end of a k-major operand, pieces are read early and moved down to their place; what lies past
+//     the depth is 0x80, zero behind the shift.  That replaces a launch that copied both operands into padded panels and
+//     what the panels cost to write and to read again: 4 x 1001 x 1500 x 777 -> int32 25.6 -> 18.7 us, 768 x 1984 x 4352 29.2 ->
+//     17.9.
+// Requirements (checked by the host): K % 128 == 0, rows addressable with 32-bit offsets; XT / YT but LOOSE:
 // XN / YN a multiple of 16, 16-byte aligned base, the whole operand within 32-bit offsets.
-template <typename OutT, int STAGES, bool XT, bool YT = false>
+template <typename OutT, int STAGES, bool XT, bool YT = false, bool LOOSE = false>
 __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p) {
   constexpr int KB = 128, T = 128, NW = 8;
   constexpr int RPI = 1024 / KB, CPR = KB / 16;
@@ -1261,6 +1271,7 @@ __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p) {
   constexpr int AHEAD = STAGES - 1;
   static_assert(STAGES >= 3 && STAGES <= 4, "ring depth");
   static_assert(NL == 4, "one transfer per MFMA slot of the second k step");
+  static_assert(!LOOSE || STAGES == 3, "two slabs in LDS beside the one that is read");
 
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x;
@@ -1300,6 +1311,63 @@ __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p) {
                         : (YT && j >= NL / 2) ? (uint32_t)k0 * (uint32_t)p.ldy
                                               : (uint32_t)k0;
     dma_16B(j < NL / 2 ? rsx : rsy, off[j], uo, lds + stage * STAGE_BYTES + (j * NW + wave) * 1024);
+  };
+
+  // LOOSE: off[j] as above (k-contiguous: of the row, its chunk in kcol[j]); the last piece of a k-major operand, and how
+  // many slabs end before the depth and that piece
+  v4i st[2][NL];
+  int kcol[NL];
+  uint32_t lastx = 0, lasty = 0;
+  int sound = 0;
+  if constexpr (LOOSE) {
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const int r = (j * NW + wave) * RPI + lane / CPR;
+      const bool t = j < NL / 2 ? XT : YT;
+      kcol[j] = ((lane % CPR) ^ ((r >> 1) & 7)) * 16;
+      const uint32_t chunk = (uint32_t)((lane % CPR) ^ (r & 6)) * 16u;
+      if (j < NL / 2) off[j] = t ? (uint32_t)r * (uint32_t)p.ldx + chunk : (uint32_t)(min(x0 + r, p.XN - 1) - x0) * (uint32_t)p.ldx;
+      else off[j] = t ? (uint32_t)(r - T) * (uint32_t)p.ldy + chunk : (uint32_t)(min(y0 + r - T, p.YN - 1) - y0) * (uint32_t)p.ldy;
+    }
+    const int64_t xl = p.x_left - (Xt - p.X), yl = p.y_left - (Yt - p.Y);
+    lastx = (uint32_t)min(xl - 16, (int64_t)0x7fffffff);
+    lasty = (uint32_t)min(yl - 16, (int64_t)0x7fffffff);
+    sound = p.k_real / KB;
+    if constexpr (XT) sound = min(sound, (int)(max(lastx - 144.f, 0.f) / (128.f * p.ldx)) - 1);
+    if constexpr (YT) sound = min(sound, (int)(max(lasty - 144.f, 0.f) / (128.f * p.ldy)) - 1);
+  }
+  auto loose_load = [&](auto set, int j, int k0) __attribute__((always_inline)) {
+    constexpr int S = decltype(set)::value;
+    const uint8_t *base = j < NL / 2 ? Xt : Yt;
+    const bool t = j < NL / 2 ? XT : YT;
+    const uint32_t at = t ? min(off[j] + (uint32_t)k0 * (uint32_t)(j < NL / 2 ? p.ldx : p.ldy), j < NL / 2 ? lastx : lasty)
+                          : off[j] + (uint32_t)min(k0 + kcol[j], p.k_real - 16);
+    __builtin_memcpy(&st[S][j], base + at, 16);
+  };
+  auto loose_store = [&](auto set, int j, int stage, int k0) __attribute__((always_inline)) {
+    constexpr int S = decltype(set)::value;
+    if (k0 >= sound * KB) {
+      const bool t = j < NL / 2 ? XT : YT;
+      v4i v = st[S][j];
+      int past;   // bytes of depth that the piece lacks, 16 and more: all
+      if (t) {
+        const uint32_t at = off[j] + (uint32_t)k0 * (uint32_t)(j < NL / 2 ? p.ldx : p.ldy), last = j < NL / 2 ? lastx : lasty;
+        if (at > last) v = moved_down(v, min(at - last, 15u));
+        const int r = ((j * NW + wave) * RPI + lane / CPR) & (T - 1);
+        past = k0 + r < p.k_real ? 0 : 16;
+      } else {
+        past = max(k0 + kcol[j] - (p.k_real - 16), 0);
+        if (past > 0) v = moved_down(v, (uint32_t)min(past, 15));
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {   // (the last `past` bytes)
+        const int keep = 16 - past - 4 * e;
+        const uint32_t mask = keep >= 4 ? 0xffffffffu : (keep <= 0 ? 0u : (1u << (8 * keep)) - 1u);
+        v[e] = (int)(((uint32_t)v[e] & mask) | (0x80808080u & ~mask));
+      }
+      st[S][j] = v;
+    }
+    *(v4i *)(lds + stage * STAGE_BYTES + (j * NW + wave) * 1024 + lane * 16) = st[S][j];
   };
 
   v16i acc[2][2];
@@ -1379,7 +1447,7 @@ __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p) {
   // Fragments of the other set are summed where their step takes that operand's sums (first step X,
   // second step Y) and flipped once they have landed: the X ones two slots after their read, the Y
   // ones behind the last MFMA.
-  auto k_step = [&](auto cur_tag, auto dma_tag, int dstage, int dk0) {
+  auto k_step = [&](auto cur_tag, auto dma_tag, int dstage, int dk0, auto set, int lk0) {
     constexpr int CUR = decltype(cur_tag)::value, OTH = 1 - CUR;
     constexpr bool dma = decltype(dma_tag)::value;
 #pragma unroll
@@ -1395,7 +1463,12 @@ __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p) {
         if constexpr (OTH == 0) xs[m - 2] = sum16_u8(fa[OTH][m - 2], xs[m - 2]);
         fa[OTH][m - 2] ^= flip;
       }
-      if constexpr (dma) dma_one(m, dstage, dk0);
+      if constexpr (dma && LOOSE) {   // (stores count as LDS instructions in the waits for transposing reads: stricter)
+        loose_store(set, m, dstage, dk0);
+        loose_load(set, m, lk0);
+      } else if constexpr (dma) {
+        dma_one(m, dstage, dk0);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
@@ -1408,12 +1481,32 @@ __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p) {
 
   const int nslab = p.K / KB;
   // prologue: slabs 0 .. AHEAD-1 in flight (past the end: the last slab again, see below)
+  constexpr std::integral_constant<int, 0> set0{};
+  constexpr std::integral_constant<int, 1> set1{};
+  if constexpr (LOOSE) {
 #pragma unroll
-  for (int s = 0; s < AHEAD; ++s)
+    for (int j = 0; j < NL; ++j) loose_load(set0, j, 0);
 #pragma unroll
-    for (int j = 0; j < NL; ++j) dma_one(j, s, min(s, nslab - 1) * KB);
-  wait_vmcnt<(AHEAD - 1) * NL>();
-  __builtin_amdgcn_s_barrier();
+    for (int j = 0; j < NL; ++j) loose_load(set1, j, min(1, nslab - 1) * KB);
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      loose_store(set0, j, 0, 0);
+      loose_load(set0, j, min(2, nslab - 1) * KB);
+    }
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      loose_store(set1, j, 1, min(1, nslab - 1) * KB);
+      loose_load(set1, j, min(3, nslab - 1) * KB);
+    }
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s)
+#pragma unroll
+      for (int j = 0; j < NL; ++j) dma_one(j, s, min(s, nslab - 1) * KB);
+    wait_vmcnt<(AHEAD - 1) * NL>();
+    __builtin_amdgcn_s_barrier();
+  }
   asm volatile("" ::: "memory");
   point_reads_at(0);
 #pragma unroll
@@ -1435,18 +1528,33 @@ __global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel(GemmParams p) {
   // reads any more, which keeps the in-flight count constant; the fragments fetched beyond the last
   // slab are never multiplied, and their sums are taken out again below.
   int stage = 0;
-  for (int kt = 0; kt < nslab; ++kt) {
-    k_step(std::integral_constant<int, 0>{}, std::false_type{}, 0, 0);
-    wait_vmcnt<(AHEAD - 2) * NL>();
-    __builtin_amdgcn_s_barrier();
+  auto slab = [&](int kt, auto set) __attribute__((always_inline)) {
+    k_step(std::integral_constant<int, 0>{}, std::false_type{}, 0, 0, set, 0);
+    if constexpr (LOOSE) {   // slab kt + 1 is stored by everybody
+      __syncthreads();
+    } else {
+      wait_vmcnt<(AHEAD - 2) * NL>();
+      __builtin_amdgcn_s_barrier();
+    }
     asm volatile("" ::: "memory");
     int next = stage + 1;
     if (next == STAGES) next = 0;
     int dst = stage + AHEAD;
     if (dst >= STAGES) dst -= STAGES;
     point_reads_at(next);
-    k_step(std::integral_constant<int, 1>{}, std::true_type{}, dst, min(kt + AHEAD, nslab - 1) * KB);
+    k_step(std::integral_constant<int, 1>{}, std::true_type{}, dst, min(kt + AHEAD, nslab - 1) * KB, set,
+           min(kt + AHEAD + 2, nslab - 1) * KB);
     stage = next;
+  };
+  if constexpr (LOOSE) {
+    int kt = 0;
+    for (; kt + 1 < nslab; kt += 2) {
+      slab(kt, set0);
+      slab(kt + 1, set1);
+    }
+    if (kt < nslab) slab(kt, set0);
+  } else {
+    for (int kt = 0; kt < nslab; ++kt) slab(kt, set0);
   }
 #pragma unroll
   for (int m = 0; m < 2; ++m) xs[m] -= sum16_u8(fa[0][m] ^ flip, 0);
@@ -2354,6 +2462,29 @@ int launch_gemm_dma(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
 }
 
 // one round of 128 x 128 tiles; the caller has checked K % 128 == 0 and the 32-bit row offsets
+int launch_gemm_mid_loose(mace_hip_ctx *ctx, GemmParams &p, bool out_u8, int batch, bool xt, bool yt) {
+  constexpr int STAGES = 3;
+  p.tiles_x = (p.XN + 127) / 128;
+  p.tiles_y = (p.YN + 127) / 128;
+  const size_t lds = (size_t)STAGES * 256 * 128;
+  dim3 grid(p.tiles_x * p.tiles_y, 1, batch), block(512);
+  mh_plan_main(ctx, MACE_HIP_KF_Q8_GEMM_MID, mhv::mid(out_u8, xt, yt, true), grid, block, lds);
+  auto launch = [&](auto k) -> int {
+    MH_HIP(ctx, mh_allow_big_lds(ctx, (const void *)k, lds));
+    MH_PROF_BEGIN(ctx);
+    MH_KLAUNCH(ctx, k, grid, block, lds, ctx->stream, p);
+    MH_PROF_END(ctx);
+    MH_LAUNCH_CHECK(ctx);
+    return MACE_HIP_SUCCESS;
+  };
+#define MH_LOOSE(XT, YT) return out_u8 ? launch(q8_gemm_mid_kernel<uint8_t, STAGES, XT, YT, true>) : launch(q8_gemm_mid_kernel<int32_t, STAGES, XT, YT, true>)
+  if (xt && yt) MH_LOOSE(true, true);
+  if (xt) MH_LOOSE(true, false);
+  if (yt) MH_LOOSE(false, true);
+  MH_LOOSE(false, false);
+#undef MH_LOOSE
+}
+
 int launch_gemm_mid(mace_hip_ctx *ctx, GemmParams &p, bool out_u8, int batch,
                     bool xt = false, bool yt = false) {
   constexpr int STAGES = 4;
@@ -2740,6 +2871,7 @@ struct Q8Call {
   int slices(bool *done);
   int small_problem(bool *done);
   int kmajor_in_place(bool *done);
+  int loose(bool *done);
   int general();
 };
 
@@ -3510,6 +3642,45 @@ int Q8Call::general() {
   return launch_gemm<2, 2, 1, 1>(ctx, p, out_u8, (int)batch);
 }
 
+// Operands that general() would copy into padded panels, at most one round of 128 x 128 tiles: read as they lie where an
+// estimate of the time is below the copies' (us; slabs of 128 bytes of depth, MB of operands and of results).  Here a slab
+// takes 0.5, 0.1 more for every k-contiguous operand whose rows are not whole dwords (their 16-byte loads cost the
+// address path twice) and 0.075 for such rows of a k-major one; copied, the launches 11, 0.34 a slab and the bytes.  Within
+// 5 and 7 % in the middle half of 1550 drawn calls; of those it takes 4 % are more than 3 % slower than copied (the worst
+// 18 %).  Measured, copied and here: 4 x 1001 x 1500 x 777 -> int32 25.6 and 18.7, 768 x 1984 x 4352 29.2 and 17.9, 160 x 2336
+// x 3831 -> int32 33.3 and 20.9, 1800 x 400 x 1900 17.7 and 11.7; against the rule, rows of odd length on both sides, 700 x
+// 5001 x 901 30.4 and 38.6, 1500 x 1001 x 1401 15.3 and 15.7.
+int Q8Call::loose(bool *done) {
+  const bool xl = out_order == MACE_HIP_COL_MAJOR;
+  const int64_t xn = xl ? rows : cols, yn = xl ? cols : rows;
+  const int64_t tiles = ((xn + 127) / 128) * ((yn + 127) / 128) * batch, cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  if (cv || rhs_ld != 0 || lhs_w || rhs_w || (lhs_direct && rhs_direct) || depth < 256 || xn <= 64 || yn <= 64 ||
+      tiles > cu || (xn + 256) * (depth + 256) >= (1ll << 31) || (yn + 256) * (depth + 256) >= (1ll << 31) ||
+      (size_t)3 * 256 * 128 > (ctx->lds_bytes > 0 ? (size_t)ctx->lds_bytes : 65536) ||
+      (ctx->kernel_mask & (MH_MASK_NO_MID | MH_MASK_NO_Q8_LOOSE)))
+    return MACE_HIP_SUCCESS;
+  const bool lhs_t = lhs_order == MACE_HIP_COL_MAJOR, rhs_t = rhs_order == MACE_HIP_ROW_MAJOR;
+  auto odd = [](const uint8_t *at, int64_t pitch) { return (uintptr_t)at % 4 != 0 || pitch % 4 != 0 ? 1 : 0; };
+  const int l_odd = odd(lhs, lhs_t ? rows : depth), r_odd = odd(rhs, rhs_t ? cols : depth);
+  const double share = (double)tiles / cu, mb = (double)batch * depth * (rows + cols) / 1e6,
+               result = (double)batch * rows * cols * (out_u8 ? 1 : 4) / 1e6;
+  const double here = 8.1 + ((depth + 127) / 128) * (0.505 + 0.099 * ((lhs_t ? 0 : l_odd) + (rhs_t ? 0 : r_odd)) +
+                                                    0.075 * ((lhs_t ? l_odd : 0) + (rhs_t ? r_odd : 0)) + 0.087 * share) +
+                      0.007 * mb + 0.18 * result;
+  const double copied = 11.2 + depth / 1e3 * (2.67 + 0.75 * share) + 0.34 * mb + 0.245 * result + (tiles < 64 ? 0.5 : 0);
+  if (here >= 0.95 * copied) return MACE_HIP_SUCCESS;
+  const Q8Operand L{lhs, lhs_t ? rows : depth, lhs_nb > 1 ? rows * depth : 0};
+  const Q8Operand R{rhs, rhs_t ? cols : depth, rhs_nb > 1 ? cols * depth : 0};
+  GemmParams p = q8_params(xl, L, R, rows, cols, depth, (int)mh_align_up((size_t)depth, 128), out, out_u8, rq, lhs_offset,
+                           rhs_offset, ep.bias);
+  p.k_real = (int)depth;
+  const int64_t l_bytes = (int64_t)lhs_nb * rows * depth, r_bytes = (int64_t)rhs_nb * cols * depth;
+  p.x_left = xl ? l_bytes : r_bytes;
+  p.y_left = xl ? r_bytes : l_bytes;
+  *done = true;
+  return launch_gemm_mid_loose(ctx, p, out_u8, (int)batch, xl ? lhs_t : rhs_t, xl ? rhs_t : lhs_t);
+}
+
 int mh_q8_gemm(mace_hip_ctx *ctx, const uint8_t *lhs, int lhs_order, const uint8_t *rhs,
                int rhs_order, void *out, int out_order, bool out_u8, int64_t batch,
                int64_t rows, int64_t depth, int64_t cols, int lhs_batched, int rhs_batched,
@@ -3530,6 +3701,8 @@ int mh_q8_gemm(mace_hip_ctx *ctx, const uint8_t *lhs, int lhs_order, const uint8
   MH_RETURN_IF_ERROR(call.small_problem(&done));
   if (done) return MACE_HIP_SUCCESS;
   MH_RETURN_IF_ERROR(call.kmajor_in_place(&done));
+  if (done) return MACE_HIP_SUCCESS;
+  MH_RETURN_IF_ERROR(call.loose(&done));
   if (done) return MACE_HIP_SUCCESS;
   return call.general();
 }

@@ -15,7 +15,7 @@ REQUANT_REF, REQUANT_NEON = 0, 1
 ACT_NOOP, ACT_RELU, ACT_RELUX = 0, 1, 2
 (MASK_NO_SMALL, MASK_NO_XRES, MASK_NO_MID, MASK_NO_XFLIP, MASK_NO_CONV_SHORT,
  MASK_NO_F32_SLICES, MASK_NO_Q8_SLICES, MASK_NO_CONV_STAGED,
- MASK_NO_F32_PANEL) = (1 << i for i in range(9))
+ MASK_NO_F32_PANEL, MASK_NO_Q8_LOOSE) = (1 << i for i in range(10))
 NOALLOC_SCRATCH_BYTES = 32 << 20
 
 _STATUS_NAMES = {0: "MACE_SUCCESS", 1: "MACE_INVALID_ARGS", 2: "MACE_OUT_OF_RESOURCES",

@@ -427,6 +427,25 @@ static void mid_case(int xn, int yn, int k) {
            [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_mid_kernel<uint8_t, 4, XT, YT>(p); }, 512); });
 }
 
+// the eight-wavefront kernel on operands of any row length and depth
+template <bool XT, bool YT>
+static void loose_case(int xn, int yn, int k) {
+  Problem pr(xn, yn, k, XT ? xn : k, YT ? yn : k, XT, YT);
+  pr.p.tiles_x = (xn + 127) / 128;
+  pr.p.tiles_y = (yn + 127) / 128;
+  pr.p.sum_y = true;
+  pr.p.K = (k + 127) / 128 * 128;
+  pr.p.k_real = k;
+  pr.p.x_left = pr.xbytes;
+  pr.p.y_left = pr.ybytes;
+  const dim3 grid(pr.p.tiles_x * pr.p.tiles_y, 1, 1);
+  char what[64];
+  snprintf(what, sizeof what, "q8_gemm_mid_kernel<STAGES=3,XT=%d,YT=%d,LOOSE>", (int)XT, (int)YT);
+  pr.check(what,
+           [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_mid_kernel<int32_t, 3, XT, YT, true>(p); }, 512); },
+           [&](GemmParams &p) { run_grid(grid, [&] { q8_gemm_mid_kernel<uint8_t, 3, XT, YT, true>(p); }, 512); });
+}
+
 // the slices kernel: either operand k-contiguous or k-major, of any row length
 template <bool XT, bool YT, int WK>
 static void slices_case(int xn, int yn, int k) {
@@ -990,6 +1009,12 @@ int main() {
   mid_case<false, true>(129, 208, 512);
   mid_case<true, true>(272, 144, 512);
   mid_case<false, false>(128, 128, 128);
+  // ... on rows that are not whole pieces: a slab and a byte, the fewest slabs, short k-major rows, tiles of a few columns
+  loose_case<false, false>(130, 77, 257);
+  loose_case<true, false>(133, 66, 391);
+  loose_case<false, true>(65, 131, 263);
+  loose_case<true, true>(67, 129, 300);
+  loose_case<true, false>(7, 128, 640);
   mid_batched_case(8, 200, 128, 128);    // 16 workgroups: dealt to the XCDs in spans of (batch, tile)
   mid_batched_case(3, 129, 130, 128);    // a workgroup count that is not a multiple of 8
 #endif

@@ -19,7 +19,7 @@ PIECES = [
      "// ---- few tiles, any layout, any depth"),
     ("template <typename OutT, bool XT, bool YT, int WK>\n__global__ __launch_bounds__(512, 4) void q8_gemm_slices_kernel",
      "// ---- one round of 128 x 128 tiles"),
-    ("template <typename OutT, int STAGES, bool XT, bool YT = false>\n__global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel",
+    ("template <typename OutT, int STAGES, bool XT, bool YT = false, bool LOOSE = false>\n__global__ __launch_bounds__(512, 1) void q8_gemm_mid_kernel",
      "// ---- the kernel for an X panel that fits in LDS"),
     ("template <int FX, int FY, int G, typename OutT, int OCC, bool CONV = false, bool XT = false,",
      "// ---- the streaming kernel for a small X panel"),

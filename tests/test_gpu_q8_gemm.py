@@ -65,9 +65,10 @@ def path(request, ctx):
     one too; kernel-mask bit 0 leaves the second, bit 1 on top of it only
     the general path (repack, row sums, tiled kernel), so that all three stay covered."""
     # (both also without the kernels that deal the depth of a few 32 x 32 tiles to wavefronts, which
-    # take uint8 calls with two k-contiguous operands under the default dispatch)
-    mask = {"default": 0, "no_small_kernel": mh.MASK_NO_SMALL | mh.MASK_NO_CONV_SHORT,
-            "general_path": mh.MASK_NO_SMALL | mh.MASK_NO_XRES | mh.MASK_NO_CONV_SHORT}[request.param]
+    # take uint8 calls with two k-contiguous operands under the default dispatch, and without the one
+    # that reads rows of any length)
+    mask = {"default": 0, "no_small_kernel": mh.MASK_NO_SMALL | mh.MASK_NO_CONV_SHORT | mh.MASK_NO_Q8_LOOSE,
+            "general_path": mh.MASK_NO_SMALL | mh.MASK_NO_XRES | mh.MASK_NO_CONV_SHORT | mh.MASK_NO_Q8_LOOSE}[request.param]
     ctx.call("mace_hip_ctx_set_kernel_mask", mask)
     yield request.param
     ctx.call("mace_hip_ctx_set_kernel_mask", 0)
@@ -194,7 +195,7 @@ def test_q8_gemm_one_round_of_tiles(ctx, mid, batch, rows, depth, cols, lb, rb, 
     # (the one-launch kernel and the kernel that keeps one panel in LDS would take the shallower
     # shapes: switched off here)
     ctx.call("mace_hip_ctx_set_kernel_mask", mh.MASK_NO_SMALL | mh.MASK_NO_XRES | mh.MASK_NO_CONV_SHORT |
-             (0 if mid == "one_round_kernel" else mh.MASK_NO_MID))
+             mh.MASK_NO_Q8_LOOSE | (0 if mid == "one_round_kernel" else mh.MASK_NO_MID))
     try:
         tag32, tag8 = check_gemm(ctx, batch, rows, depth, cols, lb, rb, lo, ro, oo)
     finally:
@@ -397,9 +398,29 @@ REPACK_SHAPES = [
 @pytest.mark.parametrize("batch,rows,depth,cols,lb,rb", REPACK_SHAPES)
 @pytest.mark.parametrize("lo,ro,oo", [(R, R, R), (R, Cm, R), (Cm, R, R), (Cm, Cm, Cm), (R, R, Cm)])
 def test_q8_gemm_repacked_operands(ctx, batch, rows, depth, cols, lb, rb, lo, ro, oo):
+    ctx.call("mace_hip_ctx_set_kernel_mask", mh.MASK_NO_SMALL | mh.MASK_NO_Q8_LOOSE)
+    try:
+        check_gemm(ctx, batch, rows, depth, cols, lb, rb, lo, ro, oo)
+    finally:
+        ctx.call("mace_hip_ctx_set_kernel_mask", 0)
+
+
+# Operands read as they lie by the eight-wavefront kernel: depths of two slabs and a byte, of a byte less than whole slabs, of
+# whole pieces; the fewest rows and columns; k-major rows shorter than a tile; one operand shared or both per batch.
+LOOSE_SHAPES = [
+    (1, 300, 257, 129, True, True), (2, 131, 639, 127, True, True), (3, 97, 1100, 113, False, True),
+    (2, 200, 654, 333, True, False), (1, 129, 385, 77, True, True), (1, 65, 639, 66, True, True),
+    (1, 257, 511, 255, True, True), (5, 70, 393, 301, True, True), (1, 1281, 386, 1279, True, True),
+]
+
+
+@pytest.mark.parametrize("batch,rows,depth,cols,lb,rb", LOOSE_SHAPES)
+@pytest.mark.parametrize("lo,ro,oo", [(R, R, R), (R, Cm, R), (Cm, R, R), (Cm, Cm, Cm), (R, R, Cm)])
+def test_q8_gemm_loose_operands(ctx, batch, rows, depth, cols, lb, rb, lo, ro, oo):
     ctx.call("mace_hip_ctx_set_kernel_mask", mh.MASK_NO_SMALL)
     try:
         check_gemm(ctx, batch, rows, depth, cols, lb, rb, lo, ro, oo)
+        assert "LOOSE=true" in ctx.last_plan().kernel, ctx.last_plan()
     finally:
         ctx.call("mace_hip_ctx_set_kernel_mask", 0)
 
