@@ -378,7 +378,7 @@ int64_t staged_layout(const StagedShape &s, int fx, int64_t tile_px, ConvStagedP
   const int64_t rows = (rows_out - 1) * s.sh + s.k_h + imgs * std::max<int64_t>(0, s.k_h - s.sh);
   const int64_t pixels = rows * p->cw;
   p->pitch = (int)mh_align_up((size_t)(pixels * 16), 128) + 16;
-  const int64_t at_filter = (int64_t)mh_align_up((size_t)(p->pitch * p->pieces), 16);
+  const int64_t at_filter = (int64_t)mh_align_up((size_t)p->pitch * p->pieces, 16);
   const int64_t at_offs = at_filter + 2 * 2 * STAGED_KS * staged_filter_pitch(fx);
   const int64_t operands = at_offs + (int64_t)p->stages * 2 * STAGED_KS * 4;
   // (the parts' sums take the place of the operands)
@@ -438,6 +438,7 @@ StagedPlan staged_plan(const StagedShape &s, int fx, int64_t cu, int64_t lds_byt
     r.two = found;
   }
   for (int64_t rounds = 2; !found && rounds <= 64 && rounds * per <= columns; ++rounds) found = try_tile(rounds * per, lds_bytes);
+  if (r.groups * p->tiles_x * p->tiles_x >= (1ll << 32)) r.groups = 0;   // (m_tiles)
   // (one image: every row is its own, whatever the divisor)
   p->m_cw = staged_magic((uint32_t)cw); p->m_vh = s.n > 1 ? staged_magic((uint32_t)vh) : 1;
   p->m_ow = staged_magic((uint32_t)s.out_w); p->m_oh = s.n > 1 ? staged_magic((uint32_t)s.out_h) : 1;
@@ -476,7 +477,6 @@ StagedPlan staged_best(const StagedShape &s, int64_t cu, int64_t lds_bytes, Conv
       *p = p2;
     }
   }
-  if (best.groups * p->tiles_x >= (1ll << 31)) *us = HUGE_VAL;
   return best;
 }
 }  // namespace
