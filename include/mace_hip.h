@@ -101,7 +101,8 @@ int mace_hip_graph_destroy(mace_hip_ctx *ctx, mace_hip_graph *graph);
  * of at most 32 bytes, for 16-channel pieces, for slices of the depth and on padded planes; bit 5: the fp32
  * kernel for slices of the depth; bit 6: the uint8 GEMM kernel for those (off with bit 0 too);
  * bit 7: the convolution kernel that stages its input rows (off with bit 4 too); bit 8: the fp32 kernel that keeps the
- * left-hand matrix in LDS; bit 9: the eight-wavefront kernel on operands of any alignment.  0 restores normal dispatch. */
+ * left-hand matrix in LDS; bit 9: the eight-wavefront kernel on operands of any alignment (off with bit 4 too).  0 restores
+ * normal dispatch. */
 int mace_hip_ctx_set_kernel_mask(mace_hip_ctx *ctx, int mask);
 /* ---- kernel plans (test and measurement hook; no counterpart in the reference) ----------------
  * Which kernel a compute call runs is chosen on the host from the shapes, layouts, alignments and

@@ -3657,7 +3657,7 @@ int Q8Call::loose(bool *done) {
   if (cv || rhs_ld != 0 || lhs_w || rhs_w || (lhs_direct && rhs_direct) || depth < 256 || xn <= 64 || yn <= 64 ||
       tiles > cu || (xn + 256) * (depth + 256) >= (1ll << 31) || (yn + 256) * (depth + 256) >= (1ll << 31) ||
       (size_t)3 * 256 * 128 > (ctx->lds_bytes > 0 ? (size_t)ctx->lds_bytes : 65536) ||
-      (ctx->kernel_mask & (MH_MASK_NO_MID | MH_MASK_NO_Q8_LOOSE)))
+      (ctx->kernel_mask & (MH_MASK_NO_MID | MH_MASK_NO_CONV_SHORT | MH_MASK_NO_Q8_LOOSE)))
     return MACE_HIP_SUCCESS;
   const bool lhs_t = lhs_order == MACE_HIP_COL_MAJOR, rhs_t = rhs_order == MACE_HIP_ROW_MAJOR;
   auto odd = [](const uint8_t *at, int64_t pitch) { return (uintptr_t)at % 4 != 0 || pitch % 4 != 0 ? 1 : 0; };
