@@ -249,7 +249,8 @@ inline int gemv_general(int nb, bool vec, bool out_u8) {
 // tiles of 128 rows by four wavefronts, by eight, of 64 rows by four
 enum { F32_128 = 0, F32_SPLIT, F32_64, F32_FORMS };
 inline int f32_gemm_vec(int form, bool lk, bool rk) { return form * 4 + (lk ? 2 : 0) + (rk ? 1 : 0); }
-// guard: every load checked against the depth; without it the kernel is f32_gemm_vec_kernel
+// guard: depths that are not whole k tiles, or operands along depth that are not aligned 16-byte pieces; without it the
+// kernel is f32_gemm_vec_kernel
 inline int f32_gemm_general(bool guard, int form, bool lk, bool rk) {
   return (guard ? 0 : F32_FORMS * 4) + f32_gemm_vec(form, lk, rk);
 }

@@ -136,9 +136,11 @@ __device__ __forceinline__ void split_8(const float (&x)[8], u4v (&part)[3]) {
 // exposed.
 // GUARD: depths that are not whole k tiles of 16, or an operand that is contiguous along depth in
 // rows that are not aligned 16-byte pieces: the same loads at any address; a unit that the depth ends in is read early
-// and moved down to its place in the last k tile (SHORT, depths below 8: single loads, each checked).  With every load
-// checked by itself, us, before and now: 3000 x 1000 x 1200 75 and 55 (1008 deep 54), 3000 x 1001 x 1201 against transposed
-// weights 104 and 54, 5000 x 300 x 2000 96 and 52, 627 x 1603 x 832 39 and 29.
+// and moved down to its place in the last k tile (depths below 8, one k tile: single loads, each checked).  With every load
+// checked by itself, us, before and now: 3000 x 1000 x 1200 75 and 55 - 60 (1008 deep 54), 3000 x 1001 x 1201 against
+// transposed weights 104 and 54 - 58, 5000 x 300 x 2000 96 and 52 - 55, 627 x 1603 x 832 39 and 29.  Behind the last k tile
+// nothing is split, stored or requested, and depths below 8 load no other: 1288 x 9 x 1554 10.9 -> 8.2, 1252 x 5 x 800
+// 8.9 -> 7.1, 3615 x 20 x 490 against transposed weights 10.0 -> 9.4 (depths 3 to 7 against those 9.4 -> 9.7).
 //
 // A thread's unit is eight consecutive depths of one row: two 16-byte loads where depth is
 // contiguous, else eight 4-byte loads, each coalesced over the wavefront's 64 rows (so rows of any
@@ -147,7 +149,7 @@ __device__ __forceinline__ void split_8(const float (&x)[8], u4v (&part)[3]) {
 // and read consecutive 16-byte pieces.  Two LDS stages and two register sets: k tile t + 3 is
 // requested, and k tile t + 1 split and stored, while k tile t is multiplied (a load has two k tiles
 // of time to arrive), the split's instructions dealt out between the MFMAs.
-template <bool LK, bool RK, int SPLIT, bool GUARD, int TMT, bool SHORT = false>
+template <bool LK, bool RK, int SPLIT, bool GUARD, int TMT>
 __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
   constexpr int NT = 256 * SPLIT;
   constexpr int BKT = 16 * SPLIT;          // depths per k tile
@@ -191,11 +193,6 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
   // No load sits under a condition (the waits in front of their use then leave younger requests in
   // flight): units past the depth re-read its last eight, single elements past it the last one.
   auto load_unit = [&](auto contig, const float *at, int64_t step, int kk, float (&x)[8]) __attribute__((always_inline)) {
-    if constexpr (SHORT) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = at[(int64_t)min(kk + e, kend - 1) * step];
-      return;
-    }
     kk = min(kk, kend - 8);
     if constexpr (decltype(contig)::value) {
       if constexpr (GUARD) {
@@ -218,19 +215,24 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
     load_unit(std::integral_constant<bool, LK>{}, pa, p.lcs, kt0 + kt * BKT + ac * 8, xa[S]);
     load_unit(std::integral_constant<bool, RK>{}, pb, p.rrs, kt0 + kt * BKT + bc * 8, xb[S]);
   };
+  // depths below 8: the one k tile there is, what lies past the depth as zeros
+  auto load_shallow = [&](auto contig, const float *at, int64_t step, int kk, float (&x)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = at[min(kk + e, kend - 1) * (decltype(contig)::value ? 1 : step)];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = kk + e < kend ? x[e] : 0.f;
+  };
   auto clear_past_depth = [&](auto set, int kt) __attribute__((always_inline)) {
     if constexpr (GUARD) {
       constexpr int S = decltype(set)::value;
       if (kt0 + (kt + 1) * BKT <= kend) return;
       // the last k tile: units that were read early move down to their place; what lies past the depth counts as zero
       auto settle = [&](int kk, float (&x)[8]) __attribute__((always_inline)) {
-        if constexpr (!SHORT) {
-          const int early = max(kk - (kend - 8), 0);
+        const int early = max(kk - (kend - 8), 0);
 #pragma unroll
-          for (int by = 4; by > 0; by >>= 1)
+        for (int by = 4; by > 0; by >>= 1)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = early & by ? (e + by < 8 ? x[e + by] : 0.f) : x[e];
-        }
+          for (int e = 0; e < 8; ++e) x[e] = early & by ? (e + by < 8 ? x[e + by] : 0.f) : x[e];
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = kk + e < kend ? x[e] : 0.f;
       };
@@ -291,17 +293,19 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
   constexpr std::integral_constant<int, 0> set0{};
   constexpr std::integral_constant<int, 1> set1{};
   const float bias_m = p.bias_row ? p.bias_row[min(m0 + tid % TMT, p.M - 1)] : 0.f;
-  load_tile(set0, 0);
-  load_tile(set1, 1);
-  if (tid < TMT) s_bias[tid] = bias_m;
-  store_tile(set0, 0, 0, std::true_type{});
-  load_tile(set0, 2);
-  __syncthreads();
+  // (eight wavefronts: half a k tile at the end of a depth that has one; a guarded one is filled up
+  // with zeros instead)
+  const int nfull = GUARD ? nk : (kend - kt0) / BKT;
   // k tile t: its fragments read, the MFMAs with the split of tile t + 1 between them, then the request
   // for tile t + 3 into the registers that the split has freed
   auto step = [&](auto set, int kt, auto last) __attribute__((always_inline)) {
     constexpr int S = decltype(set)::value;   // tile kt + 1's registers
     multiply(std::integral_constant<int, BKT / 16>{}, S ^ 1);
+    if constexpr (decltype(last)::value) {   // (of the last three k tiles: there is nothing to request any more)
+      if (kt + 1 < nfull) store_tile(set, kt + 1, S, last);
+      __syncthreads();
+      return;
+    }
     store_tile(set, kt + 1, S, last);
     constexpr int MFMAS = BKT / 16 * 6 * FM * FN;
 #pragma unroll
@@ -312,22 +316,37 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
     load_tile(set, kt + 3);
     __syncthreads();
   };
-  // (eight wavefronts: half a k tile at the end of a depth that has one; a guarded one is filled up
-  // with zeros instead)
-  const int nfull = GUARD ? nk : (kend - kt0) / BKT;
-  int kt = 0;
-  if constexpr (GUARD) {   // (the test for the last k tile apart: with it between a step's MFMAs and its split they would not mix)
-    for (; kt + 3 < nfull; kt += 2) {
+  if (GUARD && p.K < 8) {   // (one k tile.  Apart: loads under a condition would make the usual ones wait for all of theirs)
+    load_shallow(std::integral_constant<bool, LK>{}, pa, p.lcs, ac * 8, xa[0]);
+    load_shallow(std::integral_constant<bool, RK>{}, pb, p.rrs, bc * 8, xb[0]);
+    if (tid < TMT) s_bias[tid] = bias_m;
+    store_tile(set0, 0, 0, std::false_type{});
+    __syncthreads();
+  } else {
+    load_tile(set0, 0);
+    load_tile(set1, 1);
+    if (tid < TMT) s_bias[tid] = bias_m;
+    store_tile(set0, 0, 0, std::true_type{});
+    load_tile(set0, 2);
+    __syncthreads();
+    int kt = 0;
+    for (; kt + (GUARD ? 3 : 1) < nfull; kt += 2) {
       step(set1, kt, std::false_type{});
       step(set0, kt + 1, std::false_type{});
     }
+    if constexpr (GUARD) {
+      for (; kt + 1 < nfull; kt += 2) {
+        step(set1, kt, std::true_type{});
+        step(set0, kt + 1, std::true_type{});
+      }
+    }
   }
-  for (; kt + 1 < nfull; kt += 2) {
-    step(set1, kt, std::bool_constant<GUARD>{});
-    step(set0, kt + 1, std::bool_constant<GUARD>{});
+  if constexpr (GUARD) {
+    if (nfull & 1) multiply(std::integral_constant<int, BKT / 16>{}, 0);
+  } else {
+    if (nfull & 1) step(set1, nfull - 1, std::false_type{});
+    if (BKT == 32 && nfull < nk) multiply(std::integral_constant<int, 1>{}, nfull & 1);
   }
-  if (nfull & 1) step(set1, nfull - 1, std::bool_constant<GUARD>{});
-  if (BKT == 32 && nfull < nk) multiply(std::integral_constant<int, 1>{}, nfull & 1);
 
   if constexpr (NACC == 2) {
 #pragma unroll
@@ -350,16 +369,22 @@ __device__ __forceinline__ void f32_tile(const F32GemmParams &p) {
     for (int t = 0; t < FM * FN; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[0][t][r] = 0.f;
-    load_tile(set0, first);
+    const bool shallow = GUARD && p.K < 8;   // (one k tile)
+    if (shallow) {
+      load_shallow(std::integral_constant<bool, LK>{}, pa, p.lcs, ac * 8, xa[0]);
+      load_shallow(std::integral_constant<bool, RK>{}, pb, p.rrs, bc * 8, xb[0]);
+    } else {
+      load_tile(set0, first);
+    }
     for (int kt = first; kt < nk; ++kt) {
-      clear_past_depth(set0, kt);
+      if (!shallow) clear_past_depth(set0, kt);
       __syncthreads();   // (nobody reads the k tile before any more)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         if (has_a) fa[e * PA_] = xa[0][e];
         fb[e * PB_] = xb[0][e];
       }
-      load_tile(set0, kt + 1);
+      if (!shallow) load_tile(set0, kt + 1);
       __syncthreads();
       const int depth = min(BKT, kend - kt0 - kt * BKT);
       for (int k = lane >> 5; k < depth + (lane >> 5); k += 2) {
@@ -430,9 +455,9 @@ template <bool LK, bool RK, int SPLIT, int TMT>
 __global__ __launch_bounds__(256 * SPLIT, SPLIT == 1 ? 3 : 1) void f32_gemm_vec_kernel(F32GemmParams p) {
   f32_tile<LK, RK, SPLIT, false, TMT>(p);
 }
-template <bool LK, bool RK, int SPLIT, int TMT, bool SHORT>
+template <bool LK, bool RK, int SPLIT, int TMT>
 __global__ __launch_bounds__(256 * SPLIT, SPLIT == 1 ? 3 : 1) void f32_gemm_kernel(F32GemmParams p) {
-  f32_tile<LK, RK, SPLIT, true, TMT, SHORT>(p);
+  f32_tile<LK, RK, SPLIT, true, TMT>(p);
 }
 
 // ---- a left-hand matrix that stays in LDS, columns streamed past it ----------------------------------
@@ -1285,12 +1310,9 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
   if (whole && split) MH_F32_LR(f32_gemm_vec_kernel, 2, 128);
   else if (whole && half) MH_F32_LR(f32_gemm_vec_kernel, 1, 64);
   else if (whole) MH_F32_LR(f32_gemm_vec_kernel, 1, 128);
-  else if (depth < 8 && split) MH_F32_LR(f32_gemm_kernel, 2, 128, true);
-  else if (depth < 8 && half) MH_F32_LR(f32_gemm_kernel, 1, 64, true);
-  else if (depth < 8) MH_F32_LR(f32_gemm_kernel, 1, 128, true);
-  else if (split) MH_F32_LR(f32_gemm_kernel, 2, 128, false);
-  else if (half) MH_F32_LR(f32_gemm_kernel, 1, 64, false);
-  else MH_F32_LR(f32_gemm_kernel, 1, 128, false);
+  else if (split) MH_F32_LR(f32_gemm_kernel, 2, 128);
+  else if (half) MH_F32_LR(f32_gemm_kernel, 1, 64);
+  else MH_F32_LR(f32_gemm_kernel, 1, 128);
 #undef MH_F32_LR
 #undef MH_F32
   MH_PROF_END(ctx);

@@ -380,3 +380,58 @@ def test_columns_streamed_past_rows_in_lds(form, images, k, m, n):
         close(got[fin], want[fin], size[fin], k)
     finally:
         c.close()
+
+
+# more tiles than CUs, of 128 and of 64 rows, and few tiles by eight wavefronts
+GUARDED_TILES = [("SPLIT=1>", 2301, 2301), ("SPLIT=1,TM=64>", 190, 16401), ("SPLIT=2>", 300, 200)]
+
+
+@pytest.mark.parametrize("form,m,n", GUARDED_TILES)
+@pytest.mark.parametrize("k,off", [(3, 0), (7, 0), (8, 0), (9, 0), (15, 0), (49, 0), (63, 0), (65, 0), (1001, 0), (48, 1), (64, 3)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_tiles_of_guarded_depths(form, m, n, k, off, ta, tb):
+    """Depths that are not whole k tiles, and operands that are not 16-byte pieces, in every layout: against binary64, the
+    result alone written, and the same bits as the kernels without a check give for the depth filled up with zeros; then with
+    an infinity, a NaN and numbers beyond the split in a few rows."""
+    if off and ta and not tb:
+        pytest.skip("no operand along the depth: any address is whole")
+    rng = np.random.default_rng(m + 8 * k + off)
+    a, b, bias = (rng.standard_normal(s).astype(np.float32) for s in ((m, k), (k, n), (n,)))
+    c = mh.Context(0)
+    try:
+        c.lib.mace_hip_ctx_set_kernel_mask(c.handle, mh.MASK_NO_F32_SLICES | mh.MASK_NO_F32_PANEL)
+        d = Dev()
+        pbias = d.put(bias)
+
+        def matmul(a, b, off):
+            kk = a.shape[1]
+            l, r = (d.put(np.concatenate([np.zeros(off, np.float32), x.reshape(-1)]))
+                    for x in (np.ascontiguousarray(a.T if ta else a), np.ascontiguousarray(b.T if tb else b)))
+            t, po = d.empty(m * n + 32, np.float32)
+            t.fill_(-7.0)
+            d.sync()
+            c.call("mace_hip_matmul_f32", l.value + 4 * off, r.value + 4 * off, pbias, 1, *((kk, m) if ta else (m, kk)),
+                   *((n, kk) if tb else (kk, n)), int(ta), int(tb), 1, 1, po.value + 64)
+            c.sync()
+            got = t.cpu().numpy()
+            assert (got[:16] == -7.0).all() and (got[16 + m * n:] == -7.0).all()
+            return got[16:16 + m * n].reshape(m, n), c.last_plan().kernel
+        got, kernel = matmul(a, b, off)
+        assert kernel.startswith("f32_gemm_kernel<") and kernel.endswith(form), kernel
+        size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64) + np.abs(bias)
+        close(got, a.astype(np.float64) @ b.astype(np.float64) + bias, size, k)
+        more = -k % 16
+        filled, kernel = matmul(np.pad(a, ((0, 0), (0, more))), np.pad(b, ((0, more), (0, 0))), 0)
+        assert kernel.startswith("f32_gemm_vec_kernel<") and kernel.endswith(form), kernel
+        assert np.array_equal(got, filled)
+        if k > 65:
+            return
+        a[m // 2, k - 1], a[m // 3, 0], a[m - 1] = np.inf, np.nan, 1e36
+        got, _ = matmul(a, b, off)
+        want = a.astype(np.float64) @ b.astype(np.float64) + bias
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+        fin = np.isfinite(want)
+        size = np.abs(np.where(np.isfinite(a), a, 0)).astype(np.float64) @ np.abs(b).astype(np.float64) + np.abs(bias)
+        close(got[fin], want[fin], size[fin], k)
+    finally:
+        c.close()
