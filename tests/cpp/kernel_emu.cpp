@@ -269,6 +269,16 @@ inline v16f emu_mfma_bf16(V a, V b, v16f c, int, int, int) {
   return emu_mfma_f32<8>(fa, fb, c);
 }
 inline v16f emu_mfma_2f32(float a, float b, v16f c, int, int, int) { return emu_mfma_f32<1>(&a, &b, c); }
+inline uint64_t emu_ballot(bool v) {
+  Wave &w = wave_of_thread();
+  w.w[lane_of_thread()][0] = v;
+  w.bar.arrive_and_wait();
+  uint64_t r = 0;
+  for (int l = 0; l < 64; ++l) r |= (uint64_t)(w.w[l][0] != 0) << l;
+  w.bar.arrive_and_wait();
+  return r;
+}
+#define __builtin_amdgcn_ballot_w64 emu_ballot
 #define __builtin_amdgcn_mfma_f32_32x32x16_bf16 emu_mfma_bf16
 #define __builtin_amdgcn_mfma_f32_32x32x2f32 emu_mfma_2f32
 #include "f32.inc"
@@ -809,6 +819,93 @@ static void f32_slices_case(int batch, int m, int n, int k, int flat = 0, bool i
   delete[] A; delete[] B; delete[] out; delete[] bias;
 }
 
+// A right-hand matrix of images side by side (flat: columns of each) or one: operands of exactly their size, `off` floats
+// behind a multiple of 16 bytes, and what a sum of each result and of its products' sizes is
+struct F32Problem {
+  int m, n, k, flat, images, off;
+  bool lk, rk;
+  float *a0, *b0, *bias, *out;
+  std::vector<double> want, size;
+  f32::F32GemmParams p{};
+  F32Problem(int images_, int m_, int n_, int k_, bool lk_, bool rk_, int off_, bool inf)
+      : m(m_), n(n_), k(k_), flat(images_ > 1 ? n_ : 0), images(images_), off(off_), lk(lk_), rk(rk_) {
+    const int64_t as = (int64_t)m * k, bs = (int64_t)images * k * n;
+    a0 = new float[as + off]; b0 = new float[bs + off]; bias = new float[m]; out = new float[(int64_t)images * m * n];
+    for (int64_t i = 0; i < as + off; ++i) a0[i] = rnd_f32();
+    for (int64_t i = 0; i < bs + off; ++i) b0[i] = rnd_f32();
+    for (int i = 0; i < m; ++i) bias[i] = rnd_f32();
+    float *const a = a0 + off, *const b = b0 + off;
+    if (inf) a[as - 1] = INFINITY;
+    want.resize((int64_t)images * m * n);
+    size.resize(want.size());
+    for (int g = 0; g < images; ++g)
+      for (int i = 0; i < m; ++i)
+        for (int j = 0; j < n; ++j) {
+          double s = bias[i], t = std::fabs(bias[i]);
+          for (int c = 0; c < k; ++c) {
+            const double v = (double)a[lk ? (int64_t)i * k + c : (int64_t)c * m + i] *
+                             b[(int64_t)g * k * n + (rk ? (int64_t)j * k + c : (int64_t)c * n + j)];
+            s += v;
+            t += std::fabs(v);
+          }
+          want[((int64_t)g * m + i) * n + j] = s;
+          size[((int64_t)g * m + i) * n + j] = t;
+        }
+    p.lhs = a; p.rhs = b; p.out = out;
+    p.lrs = lk ? k : 1; p.lcs = lk ? 1 : m;
+    p.rrs = rk ? 1 : n; p.rcs = rk ? k : 1;
+    p.ors = n; p.ocs = 1;
+    p.rbs = (int64_t)k * n; p.obs = (int64_t)m * n;
+    p.M = m; p.N = images * n; p.K = k; p.flat = flat; p.bias_row = bias;
+  }
+  ~F32Problem() { delete[] a0; delete[] b0; delete[] bias; delete[] out; }
+};
+
+// the tile kernels: TMT x 128 tiles by four wavefronts (SPLIT = 1) or eight, loads checked (GUARD) or not; `parts` above 0:
+// k tiles of 16 of a part of the depth, whose sums are added up here
+template <bool LK, bool RK, int SPLIT, bool GUARD, int TMT>
+static void f32_tile_case(int images, int m, int n, int k, int off = 0, int parts = 0, bool inf = false) {
+  ++g_cases;
+  F32Problem pr(images, m, n, k, LK, RK, off, inf);
+  f32::F32GemmParams &p = pr.p;
+  p.tiles_m = (m + TMT - 1) / TMT;
+  const int ny = parts ? ((k + 15) / 16 + parts - 1) / parts : 1;
+  const int64_t total = (int64_t)images * m * n;
+  float *part = new float[parts ? ny * total : 1];
+  if (parts) { p.part = part; p.kt_split = parts; p.part_stride = total; }
+  run_grid(dim3(p.tiles_m * ((p.N + 127) / 128), ny), [&] {
+    if constexpr (GUARD) f32::f32_gemm_kernel<LK, RK, SPLIT, TMT>(p);
+    else f32::f32_gemm_vec_kernel<LK, RK, SPLIT, TMT>(p);
+  }, 256 * SPLIT);
+  if (parts)
+    for (int64_t i = 0; i < total; ++i) {
+      pr.out[i] = pr.bias[i / n % m];
+      for (int q = 0; q < ny; ++q) pr.out[i] += part[q * total + i];
+    }
+  char what[112];
+  snprintf(what, sizeof what, "f32_tile<%d,%d,SPLIT=%d,GUARD=%d,TM=%d> images %d m %d n %d off %d parts %d", (int)LK, (int)RK, SPLIT, (int)GUARD,
+           TMT, images, m, n, off, parts);
+  check_f32(what, pr.out, pr.want, pr.size, k);
+  delete[] part;
+}
+
+// the panel kernel: 32 MI rows in LDS, D k steps of loads ahead, `groups` spans of columns
+template <int MI, int D, bool GUARD>
+static void f32_panel_case(int images, int m, int n, int k, int groups, bool lk = true, bool inf = false) {
+  ++g_cases;
+  F32Problem pr(images, m, n, k, lk, false, 0, inf);
+  f32::F32GemmParams &p = pr.p;
+  p.tiles_m = (m + 32 * MI - 1) / (32 * MI);
+  const int64_t lds = (int64_t)((k + 15) / 16) * 3 * MI * 1024 + 128 * MI;
+  memset(g_block.lds, 0xA5, sizeof(g_block.lds));
+  run_grid(dim3(groups * p.tiles_m), [&] { f32::f32_gemm_panel_kernel<MI, D, GUARD>(p, groups, (p.N + 31) / 32); }, 512);
+  char what[96];
+  snprintf(what, sizeof what, "f32_gemm_panel_kernel<%d,%d,%d> images %d m %d n %d groups %d", MI, D, (int)GUARD, images, m, n, groups);
+  check_f32(what, pr.out, pr.want, pr.size, k);
+  for (int64_t i = lds; i < (int64_t)sizeof(g_block.lds); ++i)
+    if (g_block.lds[i] != 0xA5) { EXPECT(false, "%s: LDS byte %lld of %lld written", what, (long long)i, (long long)lds); break; }
+}
+
 // the Gemv kernels: NB vectors a pass with one row a wavefront (R = 1) or four, rows in 2^bits slices; NB = 0: float by float
 template <int NB, int R>
 static void f32_gemv_case(int batch, int h, int w, bool lb, int bits) {
@@ -924,7 +1021,7 @@ static void staged_case(int n, int in_h, int in_w, int cin, int cout, int k_h, i
 
 // PART (compile-time): 1 = everything but what follows, 2 = the ring and eight-wavefront kernels, 3 = the
 // uint8 slices kernel and the convolution on padded planes, 4 = the fp32 kernels and the planes' tile of eight
-// wavefronts, 5 = the convolution on staged rows; the test builds and runs the parts side by side.
+// wavefronts, 5 = the convolution on staged rows and the fp32 panel kernel; the test builds and runs the parts side by side.
 #ifndef PART
 #define PART 0
 #endif
@@ -1058,6 +1155,32 @@ int main() {
   f32_slices_case<true, true, 2, 8>(1, 33, 65, 129);
   f32_slices_case<true, false, 2, 8>(2, 64, 0, 50, 37);
   f32_slices_case<false, true, 2, 8>(1, 5, 63, 301, 0, true);
+  // the tiles with checked loads in every layout and form: depths below a piece, a piece, a piece and a bit, a k tile and
+  // a bit, several; operands at any address; parts that end inside a k tile and with less than a piece; an infinity
+  f32_tile_case<true, true, 1, true, 128>(1, 130, 3, 3);
+  f32_tile_case<true, false, 1, true, 128>(2, 3, 70, 7);
+  f32_tile_case<false, true, 1, true, 128>(1, 33, 129, 8);
+  f32_tile_case<false, false, 1, true, 128>(1, 129, 5, 9);
+  f32_tile_case<true, true, 1, true, 64>(1, 65, 130, 15);
+  f32_tile_case<true, false, 1, true, 64>(3, 7, 50, 49);
+  f32_tile_case<false, true, 1, true, 64>(1, 64, 33, 7);
+  f32_tile_case<false, false, 1, true, 64>(1, 5, 131, 65);
+  f32_tile_case<true, true, 2, true, 128>(1, 40, 129, 63);
+  f32_tile_case<true, false, 2, true, 128>(2, 131, 20, 5);
+  f32_tile_case<false, true, 2, true, 128>(1, 3, 33, 41);
+  f32_tile_case<false, false, 2, true, 128>(1, 35, 1, 100);
+  f32_tile_case<true, true, 1, true, 128>(1, 9, 17, 48, 1);
+  f32_tile_case<true, true, 1, true, 64>(1, 3, 2, 83, 3);
+  f32_tile_case<true, true, 2, true, 128>(1, 9, 17, 96, 2);
+  f32_tile_case<true, false, 2, true, 128>(1, 34, 40, 70, 0, 2);
+  f32_tile_case<true, true, 2, true, 128>(1, 33, 41, 85, 1, 3);
+  f32_tile_case<true, true, 1, true, 128>(1, 33, 34, 6, 0, 0, true);
+  f32_tile_case<false, true, 2, true, 128>(1, 33, 34, 43, 0, 0, true);
+  // ... and with loads that need no check
+  f32_tile_case<true, true, 1, false, 128>(1, 130, 131, 48);
+  f32_tile_case<true, false, 1, false, 64>(2, 33, 70, 16);
+  f32_tile_case<false, true, 2, false, 128>(1, 40, 33, 48);
+  f32_tile_case<false, false, 2, false, 128>(1, 7, 9, 64, 0, 2);
   f32_gemv_case<1, 1>(1, 5, 1, false, 0);
   f32_gemv_case<1, 1>(1, 7, 255, false, 0);
   f32_gemv_case<1, 1>(2, 3, 1027, true, 1);
@@ -1087,6 +1210,19 @@ int main() {
   staged_case<2, 1, false>(1, 19, 15, 3, 34, 5, 5, 1, 1, 2, 2, 19, 15, 1);
   staged_case<2, 1, true, true>(1, 25, 22, 16, 34, 1, 1, 1, 1, 0, 0, 25, 22, 1);
   staged_case<1, 1, true>(6, 16, 20, 16, 9, 3, 3, 2, 2, 0, 0, 7, 9, 1);
+  // the fp32 panel kernel in its forms: rows and columns that end inside a block, one row, images of other than whole
+  // blocks, more wavefronts than blocks and blocks for a second turn, depths of a step and a bit, a step less one, whole
+  // ones, padded to the steps ahead; rows along the depth or not; an infinity
+  f32_panel_case<1, 2, true>(1, 1, 33, 17, 1);
+  f32_panel_case<1, 2, false>(3, 31, 50, 32, 2);
+  f32_panel_case<1, 4, true>(2, 33, 49, 33, 1, false);
+  f32_panel_case<1, 4, false>(1, 32, 300, 64, 1);
+  f32_panel_case<2, 2, true>(5, 65, 7, 31, 1);
+  f32_panel_case<2, 2, false>(1, 64, 64, 48, 1, false);
+  f32_panel_case<2, 4, true>(2, 40, 33, 113, 2);
+  f32_panel_case<2, 4, false>(1, 5, 290, 80, 1);
+  f32_panel_case<1, 2, true>(2, 30, 40, 21, 1, true, true);
+  f32_panel_case<2, 4, true>(1, 70, 37, 59, 1, false, true);
 #endif
   if (g_failures) {
     printf("kernel_emu: %d failures in %d cases\n", g_failures, g_cases);

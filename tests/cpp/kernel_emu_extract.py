@@ -27,10 +27,10 @@ PIECES = [
     ("template <int LPR>\n__global__ __launch_bounds__(256) void q8_panel_sums_kernel",
      "int launch_panel_sums("),
 ]
-# the fp32 slices kernel and the Gemv kernels
+# the fp32 tile, panel and slices kernels and the Gemv kernels
 F32_PIECES = [
-    ("struct F32GemmParams {", "// ---- the tile kernels: binary32 products"),
-    ("typedef float f4v __attribute__", "// A TMT x 128 tile of the result per workgroup."),
+    ("constexpr int TM = 128, TN = 128, TK = 16;", "// ---- the tile kernels: binary32 products"),
+    ("typedef float f4v __attribute__", "// ---- few tiles, or shallow ones: a wavefront per slice"),
     ("template <bool LK, bool RK, int FN, int WK>", "// Depths of at most two: 0"),
     ("struct F32GemvParams {", "}  // namespace\n\n// Tiles of 32 x 32 fn"),
 ]
@@ -87,7 +87,13 @@ def main(out_dir):
     body = "\n".join(parts)
     if body.count("  return 0;\n#endif\n}") != 1:
         sys.exit("kernel_emu_extract: f32_gemm.hip no longer has the host's bf16_pair")
-    open(os.path.join(out_dir, "f32.inc"), "w").write(body.replace("  return 0;\n#endif\n}", "  return emu_bf16_pair(x, y);\n#endif\n}"))
+    body = body.replace("  return 0;\n#endif\n}", "  return emu_bf16_pair(x, y);\n#endif\n}")
+    for old, new in (('asm("" : "+v"(t), "+s"(first));', ""),
+                     ("extern __shared__ __align__(16) u4v panel[];", "u4v *const panel = (u4v *)emu_lds();")):
+        if old not in body:
+            sys.exit("kernel_emu_extract: f32_gemm.hip no longer has the line %r" % old)
+        body = body.replace(old, new)
+    open(os.path.join(out_dir, "f32.inc"), "w").write(body)
     rq = open(os.path.join(CSRC, "q8_requant.h")).read().replace('#include "common.h"', "")
     rq = rq.replace("#pragma once", "")
     open(os.path.join(out_dir, "requant.inc"), "w").write(rq)
