@@ -590,6 +590,7 @@ int mh_q8_gemm_depth_split(mace_hip_ctx *ctx, const uint8_t *lhs, const uint8_t 
                            int32_t mult, int shift, int32_t out_zp, int clamp_min, int clamp_max,
                            bool *taken);
 // conv1x1.hip: the bias as the kernels add it (conv_2d.cc's GetBiasData), rescaled into the arena where it has to be.
+bool mh_conv_bias_rescaled(const int32_t *bias, float input_scale, float filter_scale, float bias_scale);
 int mh_conv_bias(mace_hip_ctx *ctx, const int32_t *bias, int64_t cout, float input_scale,
                  float filter_scale, float bias_scale, const int32_t **used);
 // conv_planes.hip: a convolution on padded planes.  *taken = false: not a call for it.

@@ -813,13 +813,16 @@ inline int64_t floor_div(int64_t a, int64_t b) { return a >= 0 ? a / b : -((-a +
 // into an arena slice where its scale is not input_scale * filter_scale
 }  // namespace
 
+bool mh_conv_bias_rescaled(const int32_t *bias, float input_scale, float filter_scale, float bias_scale) {
+  volatile float prod = input_scale * filter_scale;
+  volatile float diff = prod - bias_scale;
+  return bias != nullptr && fabs((double)diff) > 1e-6;
+}
 int mh_conv_bias(mace_hip_ctx *ctx, const int32_t *bias, int64_t cout, float input_scale,
               float filter_scale, float bias_scale, const int32_t **used) {
   volatile float prod = input_scale * filter_scale;
-  volatile float diff = prod - bias_scale;
-  const bool adjust = bias != nullptr && fabs((double)diff) > 1e-6;
   *used = bias;   // a null bias adds nothing, like the zero vector
-  if (adjust) {
+  if (mh_conv_bias_rescaled(bias, input_scale, filter_scale, bias_scale)) {
     int32_t *scaled = (int32_t *)mh_arena_take(ctx, sizeof(int32_t) * cout);
     if (!scaled) return mh_fail(ctx, MACE_HIP_RUNTIME_ERROR, "arena slice unavailable");
     volatile float adjust_scale = bias_scale / prod;

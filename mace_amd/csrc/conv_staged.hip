@@ -513,7 +513,8 @@ int mh_q8_conv_staged(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
   p.by_mad = requant_by_mad(p.rq);
   if (p.by_mad) p.rqm = requant_mad(p.rq);
   *taken = true;
-  MH_RETURN_IF_ERROR(mh_arena_reserve(ctx, sizeof(int32_t) * cout + 4096));
+  if (mh_conv_bias_rescaled(bias, input_scale, filter_scale, bias_scale))   // (the only scratch)
+    MH_RETURN_IF_ERROR(mh_arena_reserve(ctx, sizeof(int32_t) * cout + 4096));
   ArenaScope scope(ctx);
   MH_RETURN_IF_ERROR(mh_conv_bias(ctx, bias, cout, input_scale, filter_scale, bias_scale, &p.bias));
   p.in = input; p.filter = filter; p.out = out;

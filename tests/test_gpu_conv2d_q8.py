@@ -435,6 +435,52 @@ def test_conv2d_q8_planes_where_scratch_cannot_grow():
         c.close()
 
 
+def test_conv2d_q8_on_staged_rows_without_scratch():
+    """A new context holds no scratch, and a capture may not allocate any: the kernel on staged rows needs none unless the
+    bias is rescaled, which is then refused as before; the same results from every replay, and with scratch."""
+    import ctypes as C
+    import torch
+    n, h, w, cin, cout = 12, 61, 59, 29, 80
+    rng = np.random.default_rng(9)
+    x = rng.integers(0, 256, (n, h, w, cin), dtype=np.uint8)
+    f = rng.integers(0, 256, (cout, 3, 3, cin), dtype=np.uint8)
+    bias = rng.integers(-2 ** 15, 2 ** 15, cout).astype(np.int32)
+    same, other = np.float32(0.02 * 0.01), np.float32(0.03 * 0.01)
+    want = [orc.conv2d_q8_nhwc(x, f, bias, n, h, w, cin, cout, 3, 3, (1, 1), (2, 2), 0.02, 120, 0.01, 131, s, 0.4, 128,
+                               nthreads=16) for s in (same, other)]
+    xd, fd, bd = (torch.from_numpy(a.reshape(-1)).cuda() for a in (x, f, bias))
+    out = torch.zeros(want[0].size, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    c = mh.Context(0)
+    try:
+        def call(scale):
+            return c.status("mace_hip_conv2d_q8_nhwc", xd.data_ptr(), fd.data_ptr(), bd.data_ptr(), n, h, w, cin, cout, 3, 3, 1, 1,
+                            2, 2, 0.02, 120, 0.01, 131, float(scale), 0.4, 128, 0, 255, out.data_ptr())
+
+        def check(want):
+            c.sync()
+            assert c.last_plan().family == mh.KF_Q8_CONV_STAGED, c.last_plan()
+            np.testing.assert_array_equal(out.cpu().numpy().reshape(want.shape), want)
+            out.zero_()
+            torch.cuda.synchronize()
+        c.call("mace_hip_graph_capture_begin")
+        status = call(same)
+        refused = call(other)
+        graph = C.c_void_p()
+        c.call("mace_hip_graph_capture_end", C.byref(graph))
+        assert (status, refused) == (mh.SUCCESS, mh.INVALID_ARGS)
+        assert call(same) == mh.SUCCESS
+        check(want[0])
+        for _ in range(3):
+            c.call("mace_hip_graph_launch", graph)
+            check(want[0])
+            assert call(other) == mh.SUCCESS     # (scratch from here on, between the replays)
+            check(want[1])
+        c.call("mace_hip_graph_destroy", graph)
+    finally:
+        c.close()
+
+
 KSPLIT_CASES = [  # batch, cout, cin, in_h, in_w, k_h, k_w, padding, strides
     (1, 512, 512, 7, 7, 3, 3, S, (1, 1)),       # the deep layers of a single image
     (1, 256, 256, 14, 14, 3, 3, S, (1, 1)),
