@@ -3643,13 +3643,19 @@ int Q8Call::general() {
 }
 
 // Operands that general() would copy into padded panels, at most one round of 128 x 128 tiles: read as they lie where an
-// estimate of the time is below the copies' (us; slabs of 128 bytes of depth, MB of operands and of results).  Here a slab
-// takes 0.5, 0.1 more for every k-contiguous operand whose rows are not whole dwords (their 16-byte loads cost the
-// address path twice) and 0.075 for such rows of a k-major one; copied, the launches 11, 0.34 a slab and the bytes.  Within
-// 5 and 7 % in the middle half of 1550 drawn calls; of those it takes 4 % are more than 3 % slower than copied (the worst
-// 18 %).  Measured, copied and here: 4 x 1001 x 1500 x 777 -> int32 25.6 and 18.7, 768 x 1984 x 4352 29.2 and 17.9, 160 x 2336
-// x 3831 -> int32 33.3 and 20.9, 1800 x 400 x 1900 17.7 and 11.7; against the rule, rows of odd length on both sides, 700 x
-// 5001 x 901 30.4 and 38.6, 1500 x 1001 x 1401 15.3 and 15.7.
+// estimate of the time is below the copies' (us; slabs of 128 bytes of depth, MB of operands and of results, a shared operand
+// once).  Here a slab takes 0.5; 0.08, or 0.23 with two, more for k-contiguous operands whose rows are not whole dwords
+// (their 16-byte loads cost the address path twice), 0.07 for such k-major ones.  Copied, by the kernel that runs then:
+//   the eight-wavefront kernel: the launches 10.7, 0.37 a slab, the bytes copied;
+//   the kernel with a resident tile, which has a panel's bytes per workgroup to load first: slower at every one of 580 drawn
+//     calls, 1.38 times in the median;
+//   64 x 64 tiles, few of them: 3.2 per 1000 deep, with one operand alone copied 4.2.
+// The estimates' spread is taken off: 7 %, 11 % with two k-contiguous operands in other than dwords, 17 % where one operand
+// is copied for 64 x 64 tiles.  Of 6000 drawn calls 3046 are read here, 1.26 times faster in the geometric mean, 24 of them
+// more than 3 % slower, the worst 10 % (with one estimate for all of them 257 of 4145 and 38 %).  Measured, copied and here: 4 x 1001 x
+// 1500 x 777 -> int32 25.6 and 18.7, 768 x 1984 x 4352 29.2 and 17.9, 160 x 2336 x 3831 -> int32 33.3 and 20.9, 1800 x 400 x
+// 1900 17.7 and 11.7; not taken: 700 x 5001 x 901 30.4 and 38.6, 192 x 6848 x 2774 33.2 and 39.0, 201 x 6144 x 6327 32.0
+// and 40.0.
 int Q8Call::loose(bool *done) {
   const bool xl = out_order == MACE_HIP_COL_MAJOR;
   const int64_t xn = xl ? rows : cols, yn = xl ? cols : rows;
@@ -3662,13 +3668,27 @@ int Q8Call::loose(bool *done) {
   const bool lhs_t = lhs_order == MACE_HIP_COL_MAJOR, rhs_t = rhs_order == MACE_HIP_ROW_MAJOR;
   auto odd = [](const uint8_t *at, int64_t pitch) { return (uintptr_t)at % 4 != 0 || pitch % 4 != 0 ? 1 : 0; };
   const int l_odd = odd(lhs, lhs_t ? rows : depth), r_odd = odd(rhs, rhs_t ? cols : depth);
-  const double share = (double)tiles / cu, mb = (double)batch * depth * (rows + cols) / 1e6,
+  const int along = (lhs_t ? 0 : l_odd) + (rhs_t ? 0 : r_odd), across = (lhs_t ? l_odd : 0) + (rhs_t ? r_odd : 0);
+  const double share = (double)tiles / cu, l_mb = (double)lhs_nb * rows * depth / 1e6, r_mb = (double)rhs_nb * cols * depth / 1e6,
                result = (double)batch * rows * cols * (out_u8 ? 1 : 4) / 1e6;
-  const double here = 8.1 + ((depth + 127) / 128) * (0.505 + 0.099 * ((lhs_t ? 0 : l_odd) + (rhs_t ? 0 : r_odd)) +
-                                                    0.075 * ((lhs_t ? l_odd : 0) + (rhs_t ? r_odd : 0)) + 0.087 * share) +
-                      0.007 * mb + 0.18 * result;
-  const double copied = 11.2 + depth / 1e3 * (2.67 + 0.75 * share) + 0.34 * mb + 0.245 * result + (tiles < 64 ? 0.5 : 0);
-  if (here >= 0.95 * copied) return MACE_HIP_SUCCESS;
+  const double here = 8.4 + ((depth + 127) / 128) * (0.505 + (along == 2 ? 0.227 : 0.084 * along) + 0.077 * across + 0.183 * share) +
+                      0.182 * result;
+  // (the copies' row pitch and the kernel that it leads to, as general() has them)
+  const bool one = lhs_direct != rhs_direct && depth % 64 == 0, quarter = 4 * tiles >= cu;
+  const int64_t pitch = one ? depth
+                            : (depth > 512 && quarter ? (int64_t)mh_align_up((size_t)depth, 128)
+                                                      : (lhs_direct != rhs_direct ? depth : (int64_t)mh_align_up((size_t)depth, 64)));
+  const bool mid = pitch % 128 == 0 && pitch >= 512 && (quarter || pitch >= 2048);
+  const bool resident = !mid && pitch % 64 == 0 && yn >= 256 && 2 * (XRES_SC_BYTES + 128 * (size_t)pitch) <= (size_t)ctx->lds_bytes;
+  if (!resident) {
+    const double moved = one ? (lhs_direct ? r_mb : l_mb) : l_mb + r_mb;
+    const double copied = mid ? 10.7 + depth / 1e3 * (2.9 + 1.22 * share) + 0.34 * moved + 0.276 * result
+                          : one ? 10.2 + 4.18e-3 * depth + 0.53 * moved + 0.71 * result
+                                : 9.9 + 3.17e-3 * mh_align_up((size_t)depth, 64) + 0.55 * moved + 0.36 * result;
+    // (with the kernels for small problems switched off those come here too, at sizes below the estimates' range)
+    const bool small_too = ctx->kernel_mask & (MH_MASK_NO_SMALL | MH_MASK_NO_Q8_SLICES);
+    if (here >= (small_too ? 1.1 : !mid && one ? 0.83 : along == 2 ? 0.89 : 0.93) * copied) return MACE_HIP_SUCCESS;
+  }
   const Q8Operand L{lhs, lhs_t ? rows : depth, lhs_nb > 1 ? rows * depth : 0};
   const Q8Operand R{rhs, rhs_t ? cols : depth, rhs_nb > 1 ? cols * depth : 0};
   GemmParams p = q8_params(xl, L, R, rows, cols, depth, (int)mh_align_up((size_t)depth, 128), out, out_u8, rq, lhs_offset,
