@@ -601,10 +601,11 @@ int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
                       float bias_scale, int32_t mult, int shift, int32_t out_zp, int clamp_min, int clamp_max,
                       uint8_t *out, double other, bool *taken);
 // conv_staged.hip: a convolution in one launch, its input staged in LDS, and an estimate of its time in us (HUGE_VAL: not a
-// call for it).  *taken = false: parameters that the general path takes or reports.
+// call for it; *of_planes: the part of the planes' estimate that it has to be below).  *taken = false: parameters that the
+// general path takes or reports.
 double mh_q8_conv_staged_us(const mace_hip_ctx *ctx, int64_t n, int64_t in_h, int64_t in_w, int64_t cin, int64_t cout,
                             int64_t k_h, int64_t k_w, int stride_h, int stride_w, int pad_top, int pad_left,
-                            int64_t out_h, int64_t out_w);
+                            int64_t out_h, int64_t out_w, double *of_planes);
 int mh_q8_conv_staged(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *filter, const int32_t *bias,
                       int64_t n, int64_t in_h, int64_t in_w, int64_t cin, int64_t cout, int64_t k_h,
                       int64_t k_w, int stride_h, int stride_w, int pad_top, int pad_left, int64_t out_h,

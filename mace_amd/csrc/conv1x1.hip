@@ -1166,6 +1166,16 @@ inline size_t conv_gemm_scratch(int64_t cout, int64_t depth, int64_t columns, bo
   return need;
 }
 
+// What a 1 x 1 filter in place takes on rows that are copied into padded ones first, in us: the two launches, input and
+// result, and the padded rows, which every tile of 64 or 128 channels reads.  Within 6 % in the middle half of 3000 drawn
+// layers, 3 to 1020 channels.  (Measured, copied and staged: 64 x 62 x 105 -> 112 at batch 48 35.9 and 31.6 us, 77 x 77 x
+// 5 -> 80 at 20 17.8 and 19.4.)
+inline double mh_q8_conv_padded_rows_us(int64_t cin, int64_t cout, int64_t columns) {
+  const double m = columns / 1e6, rows = m * ((cin + 63) / 64 * 64);
+  return cout <= 64 ? 8.9 + 0.59 * m * cin + 0.49 * m * cout + 0.64 * rows
+                    : 8.7 + 0.55 * m * cin + 0.33 * m * cout + (0.42 + 0.27 * ((cout + 127) / 128)) * rows;
+}
+
 }  // namespace
 
 extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
@@ -1270,20 +1280,27 @@ extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
     // (whatever the times, where only the planes' scratch can be had)
     double other = !mh_arena_can_hold(ctx, need) ? HUGE_VAL
                    : small_gather ? mh_q8_conv_small_us(ctx, cout, columns, depth, small_vec ? 16 : (cin % 4 == 0 ? 4 : 1))
-                   : unpacked ? 9 + 0.065e-3 * columns
+                   : unpacked ? mh_q8_conv_padded_rows_us(cin, cout, columns)
                    : gather || (im2col_one_round && cin % 64 == 0 && by_pieces)
                        ? mh_q8_conv_gather_us(ctx, cout, columns, depth, !gather)
                    : k_h * k_w == 1 && stride_h * stride_w > 1 ? (by_pieces ? 13 + 0.3e-6 * columns * kp : 16.5 + 1.9e-6 * columns * kp)
                                     : HUGE_VAL;
-    // (6.2 us: the least that the staged kernel takes, before its tile's geometry is worked out)
-    const double staged = has_pixels && 0.95 * other > 6.2
+    // The staged kernel where its estimate, with the spread of both taken off, is the lower one: 7 % (18 % for one tap at a
+    // stride, whose other estimates run high: 56 x 56 x 64 -> 256 at stride 2, batch 32, 9.7 us, staged 11.3), against the
+    // planes 6 %.  Of 7000 drawn layers that could be staged 4800 are, 1.155
+    // times faster in the geometric mean, 107 more than 3 % slower, three of them more than 10 % (5242, 351 and 87 where 5 %
+    // were taken off one estimate); of 3000 1 x 1 ones in place 2525, 1.44 times faster, 35 more than 3 % slower.  (With the
+    // one-launch kernel switched off calls come here that are smaller than those.)
+    double of_planes;
+    // (7 us: the least that the staged kernel takes, before its tile's geometry is worked out)
+    const double staged = has_pixels && 0.95 * other > 7
                               ? mh_q8_conv_staged_us(ctx, n, in_h, in_w, cin, cout, k_h, k_w, stride_h, stride_w,
-                                                     pad_h >> 1, pad_w >> 1, out_h, out_w) : HUGE_VAL;
-    // (the estimates for patches of whole pieces in one launch and for one tap at a stride run high: 96 x 98 x 48 -> 48 7.2 us,
-    // staged 7.5, 56 x 56 x 64 -> 256 at stride 2, batch 32, 9.7 and 11.3)
-    const bool high = (small_gather && small_vec) || (!in_place && k_h * k_w == 1);
-    const bool by_staged = staged < (high ? 0.82 : 0.95) * other;
-    if (by_staged) other = staged;
+                                                     pad_h >> 1, pad_w >> 1, out_h, out_w, &of_planes) : HUGE_VAL;
+    const bool smaller = ctx->kernel_mask & MH_MASK_NO_SMALL;
+    const bool by_staged = staged < (smaller ? 1.1 : !in_place && k_h * k_w == 1 ? 0.82 : 0.93) * other;
+    // (mh_q8_conv_planes takes a call whose estimate is below 0.95 of the other)
+    if (by_staged && smaller) other = staged / (0.95 * 1.1);
+    else if (by_staged) other = staged / (0.95 * of_planes);
     if (!in_place && (small_gather || cin % 64 != 0 || depth > 576)) {
       MH_RETURN_IF_ERROR(mh_q8_conv_planes(ctx, input, filter, bias, n, in_h, in_w, cin, cout, k_h, k_w, stride_h,
                                            stride_w, pad_h >> 1, pad_w >> 1, out_h, out_w, input_scale, input_zp,

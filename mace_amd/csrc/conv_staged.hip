@@ -458,36 +458,40 @@ StagedPlan staged_plan(const StagedShape &s, int fx, int64_t cu, int64_t lds_byt
   p->in_last = (uint32_t)(s.n * s.in_h * s.in_w * s.cin - 16); p->filter_last = (uint32_t)(s.cout * depth - 16);
   return r;
 }
-// Time that the staged kernel takes, in us: its start, and for every tile of a CU the staging (a load's latency and the
-// pieces' arithmetic, more of it for broken pieces), a stage's hand-over, the MFMAs of two wavefronts on a SIMD, and the
-// epilogue; of tiles that share a CU the second takes 0.7 of the first, of others a
-// little more (56 x 56 x 192 -> 128, 5 x 5, at 4 34 us, on planes 25).  Within 3 % in the median of 500 drawn layers, 9 %
-// in nine of ten.
-double staged_us(const StagedPlan &r, const ConvStagedParams &p, int64_t cu, int64_t lds_bytes) {
+// Time that the staged kernel takes, in us: its start, for every tile of a CU the staging (a load's latency and the pieces'
+// arithmetic, more of it for broken pieces), a stage's hand-over, the MFMAs of two wavefronts on a SIMD, the taps' sums
+// where a filter row is not three, and the epilogue, and the bytes; of tiles that share a CU the second takes a part of the
+// first, of others a little more.  Within 2.5 % in the middle half of 7000 drawn layers, -9 and +7 % in nine of ten.
+// width: for the choice between widths of a tile alone, fitted to both of them on 500 layers.  (The other fit saw the width
+// that this one chooses, and has two rounds of narrow tiles too low: 28 x 28 x 128 -> 128 at batch 64 by 32 channels.)
+double staged_us(const StagedPlan &r, const ConvStagedParams &p, int64_t cu, int64_t lds_bytes, bool width) {
   const int slots = 512 >> p.lanes_log2, more = p.cin % 16 != 0 ? 1 : 0;
   const int64_t pixels = (p.pitch - 16) / 16, rounds = (r.groups * p.tiles_x + cu - 1) / cu;
   const double steps = (double)((pixels + slots * STAGED_PIXELS - 1) / (slots * STAGED_PIXELS)) *
                        ((p.pieces + (1 << p.lanes_log2) - 1) >> p.lanes_log2);
   const double mfma = p.stages * (STAGED_KS / r.wk) * r.fx * 2 * 2 * 32 / 2400.0;
-  const double tile = 2.4 + steps * (0.78 + 0.49 * more) + p.stages * (0.2 + 0.19 * more) + 1.94 * mfma +
-                      1.56 * (r.fx - 1) + (r.wk > 1 ? 0.22 : 0.0);
   const bool share = (r.fx == 1 || r.two) && 2 * r.lds <= lds_bytes;
-  return 2.8 + tile * (1 + (rounds - 1) * (share ? 0.7 : 1.15));
+  if (width) {
+    const double tile = 2.4 + steps * (0.78 + 0.49 * more) + p.stages * (0.2 + 0.19 * more) + 1.94 * mfma +
+                        1.56 * (r.fx - 1) + (r.wk > 1 ? 0.22 : 0.0);
+    return 2.8 + tile * (1 + (rounds - 1) * (share ? 0.7 : 1.15));
+  }
+  const double tile = 3.45 + steps * (1.29 + 0.17 * more) + p.stages * (0.228 + 0.083 * more) + 1.48 * mfma + 1.77 * (r.fx - 1) +
+                      (r.wk > 1 ? 0.19 + 0.32 * (r.fx - 1) : 0.0) + (p.k_w == 3 ? 0.0 : 0.026 * p.taps);
+  return 1.9 + tile * (1 + (rounds - 1) * (share ? 0.54 : 1.17)) + 0.206e-6 * p.columns * p.cout + 0.112e-6 * p.in_last;
 }
 // The better of the two widths of a tile, and its time.  (A tile of 64 channels costs 1.6 us more than one of 32.)
 StagedPlan staged_best(const StagedShape &s, int64_t cu, int64_t lds_bytes, ConvStagedParams *p, double *us) {
   StagedPlan best = staged_plan(s, 1, cu, lds_bytes, p);
-  *us = best.groups ? staged_us(best, *p, cu, lds_bytes) : HUGE_VAL;
   if (s.cout > 32) {
     ConvStagedParams p2{};
     const StagedPlan two = staged_plan(s, 2, cu, lds_bytes, &p2);
-    const double us2 = two.groups ? staged_us(two, p2, cu, lds_bytes) : HUGE_VAL;
-    if (us2 < *us) {
+    if (two.groups && (!best.groups || staged_us(two, p2, cu, lds_bytes, true) < staged_us(best, *p, cu, lds_bytes, true))) {
       best = two;
-      *us = us2;
       *p = p2;
     }
   }
+  *us = best.groups ? staged_us(best, *p, cu, lds_bytes, false) : HUGE_VAL;
   return best;
 }
 }  // namespace
@@ -495,13 +499,18 @@ StagedPlan staged_best(const StagedShape &s, int64_t cu, int64_t lds_bytes, Conv
 // HUGE_VAL: not a call for it.
 double mh_q8_conv_staged_us(const mace_hip_ctx *ctx, int64_t n, int64_t in_h, int64_t in_w, int64_t cin, int64_t cout,
                             int64_t k_h, int64_t k_w, int stride_h, int stride_w, int pad_top, int pad_left,
-                            int64_t out_h, int64_t out_w) {
+                            int64_t out_h, int64_t out_w, double *of_planes) {
+  *of_planes = 0.94;
   if (ctx->kernel_mask & (MH_MASK_NO_CONV_STAGED | MH_MASK_NO_CONV_SHORT)) return HUGE_VAL;
   const StagedShape s{n, in_h, in_w, cin, cout, k_h, k_w, stride_h, stride_w, pad_top, pad_left, out_h, out_w};
   if (!staged_fits(s)) return HUGE_VAL;
   ConvStagedParams p{};
   double us;
-  staged_best(s, ctx->cu_count > 0 ? ctx->cu_count : 256, ctx->lds_bytes, &p, &us);
+  const int64_t cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  const StagedPlan plan = staged_best(s, cu, ctx->lds_bytes, &p, &us);
+  // (64 channels whose depth wavefronts share, or few workgroups: the planes' estimate runs lower there)
+  if (plan.fx == 2 && plan.wk > 1) *of_planes = 1.05;
+  else if (2 * plan.groups * p.tiles_x < cu) *of_planes = 0.98;
   return us;
 }
 
