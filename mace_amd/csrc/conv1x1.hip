@@ -1287,8 +1287,8 @@ extern "C" int mace_hip_conv2d_q8_nhwc(mace_hip_ctx *ctx, const uint8_t *input,
                                     : HUGE_VAL;
     // The staged kernel where its estimate, with the spread of both taken off, is the lower one: 7 % (18 % for one tap at a
     // stride, whose other estimates run high: 56 x 56 x 64 -> 256 at stride 2, batch 32, 9.7 us, staged 11.3), against the
-    // planes 6 %.  Of 7000 drawn layers that could be staged 4800 are, 1.155
-    // times faster in the geometric mean, 107 more than 3 % slower, three of them more than 10 % (5242, 351 and 87 where 5 %
+    // planes 6 %.  Of 7000 drawn layers that could be staged 4838 are, 1.154
+    // times faster in the geometric mean, 109 more than 3 % slower, four of them more than 10 % (5242, 351 and 87 where 5 %
     // were taken off one estimate); of 3000 1 x 1 ones in place 2525, 1.44 times faster, 35 more than 3 % slower.  (With the
     // one-launch kernel switched off calls come here that are smaller than those.)
     double of_planes;

@@ -508,8 +508,9 @@ double mh_q8_conv_staged_us(const mace_hip_ctx *ctx, int64_t n, int64_t in_h, in
   double us;
   const int64_t cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
   const StagedPlan plan = staged_best(s, cu, ctx->lds_bytes, &p, &us);
-  // (64 channels whose depth wavefronts share, or few workgroups: the planes' estimate runs lower there)
-  if (plan.fx == 2 && plan.wk > 1) *of_planes = 1.05;
+  // (closer for tiles of 64 channels, whose estimate runs high, more so where wavefronts share the depth, and for few
+  // workgroups: 56 x 56 x 128 -> 128 at batch 16 21.4 us on planes, 17.8 staged and 20.1 by the estimate)
+  if (plan.fx == 2) *of_planes = plan.wk > 1 ? 1.05 : 0.98;
   else if (2 * plan.groups * p.tiles_x < cu) *of_planes = 0.98;
   return us;
 }
