@@ -651,8 +651,10 @@ int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
   // (workgroups of a channel tile: as many as fit at once)
   const int64_t room = std::min<int64_t>(p.tiles_p, std::max<int64_t>(1, cu * at_once / p.tiles_x));
   const int64_t staged = (p.keep ? 0 : (int64_t)p.slabs * p.steps * plan.xt * 32) + (int64_t)p.slabs * p.pieces * p.row_bytes;
-  if (planes_us(form, p, s, staged, (p.tiles_p + room - 1) / room, (room * p.tiles_x + cu - 1) / cu) >= 0.95 * other)
-    return MACE_HIP_SUCCESS;
+  // (packing the filter is 1 us a MB of it, which a registered one costs once: 7 x 7 x 512 -> 512 at batch 64 24.6 and 22.1)
+  mh_weight *weight = mh_find_weight(ctx, filter, (size_t)(cout * p.depth));
+  const double us = planes_us(form, p, s, staged, (p.tiles_p + room - 1) / room, (room * p.tiles_x + cu - 1) / cu);
+  if (us - (weight ? 1e-6 * cout * p.depth : 0.0) >= 0.95 * other) return MACE_HIP_SUCCESS;
   *taken = true;
 
   MH_RETURN_IF_ERROR(mh_arena_reserve(ctx, (size_t)plan.scratch + 8 * 256 + sizeof(int32_t) * cout));
@@ -661,7 +663,6 @@ int mh_q8_conv_planes(mace_hip_ctx *ctx, const uint8_t *input, const uint8_t *fi
   MH_RETURN_IF_ERROR(mh_conv_bias(ctx, bias, cout, input_scale, filter_scale, bias_scale, &bias_used));
   // A registered filter is packed and summed once, into memory of its own.  (Not where that cannot be had, nor in a
   // capture, which would fill it at a replay only: then as any other filter.)
-  mh_weight *weight = mh_find_weight(ctx, filter, (size_t)(cout * p.depth));
   mh_weight_planes built{cin, cout, k_h, k_w, p.channels, nullptr, nullptr};
   auto give_back = [&]() {
     if (!ctx->plan_only) { (void)hipFree(built.packed); (void)hipFree(built.sums); }
