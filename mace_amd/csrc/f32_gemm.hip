@@ -1245,7 +1245,12 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
     const bool deep = lds_of(2) > (size_t)ctx->lds_bytes;
     const int mi = narrow || deep ? 1 : 2;
     const size_t lds = lds_of(mi);
-    if (lds <= (size_t)ctx->lds_bytes && (!deep || p.M <= 32 || !whole || 4 * TM * ((p.M + TM - 1) / TM) >= 5ll * p.M)) {
+    // Depths that are not whole k steps cost every step here (loads are checked and cleared), the tiles only the last one: not
+    // two tiles of 32 rows, each of which reads the columns, against one of 64 rows.  1 x 1 layers, tiles and here: 840 x 137 ->
+    // 40 at batch 48 16.3 us and 20.8, 1640 x 201 -> 64 at 54 32.2 and 38.9.  Of 397 drawn such layers 241 are more than 3 %
+    // slower here, of 2053 others 56 (224 x 457 -> 576 at 48 52.9 and 71.7), of 1050 in whole k steps one.
+    const bool twice = !whole && mi == 1 && p.M > 32 && p.M <= 64;
+    if (lds <= (size_t)ctx->lds_bytes && !twice && (!deep || p.M <= 32 || !whole || 4 * TM * ((p.M + TM - 1) / TM) >= 5ll * p.M)) {
       p.tiles_m = (int)(mi == 1 ? small : large);
       // (k steps of loads on their way; a block's end is padded to a multiple of them)
       const int ahead = nks % 4 == 0 || nks >= 7 ? 4 : 2;
