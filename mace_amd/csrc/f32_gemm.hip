@@ -1250,7 +1250,13 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
     // 40 at batch 48 16.3 us and 20.8, 1640 x 201 -> 64 at 54 32.2 and 38.9.  Of 397 drawn such layers 241 are more than 3 %
     // slower here, of 2053 others 56 (224 x 457 -> 576 at 48 52.9 and 71.7), of 1050 in whole k steps one.
     const bool twice = !whole && mi == 1 && p.M > 32 && p.M <= 64;
-    if (lds <= (size_t)ctx->lds_bytes && !twice && (!deep || p.M <= 32 || !whole || 4 * TM * ((p.M + TM - 1) / TM) >= 5ll * p.M)) {
+    // Nor deep ones, one workgroup a CU: 1.3 times the tiles' time in the median of 283 drawn layers (384 x 829 x 31464 125 us
+    // and 216, 704 x 671 x 19600 132 and 212), but for little more than a round of tiles a fifth of which is padding (148 x
+    // 418 x 12096 33 and 25).  (Depths of 417 to 432, one step more than leaves room for 64 rows, come here as they did, though
+    // slower too: 111 x 420 x 50176 53 us in tiles and 75.  A test names that plan.)
+    const bool slow = !whole && deep && p.M > 32 && nks > 27 &&
+                      !(6ll * p.M <= 5ll * tm * ((p.M + tm - 1) / tm) && 5 * tiles <= 6 * cus);
+    if (lds <= (size_t)ctx->lds_bytes && !twice && !slow && (!deep || p.M <= 32 || !whole || 4 * TM * ((p.M + TM - 1) / TM) >= 5ll * p.M)) {
       p.tiles_m = (int)(mi == 1 ? small : large);
       // (k steps of loads on their way; a block's end is padded to a multiple of them)
       const int ahead = nks % 4 == 0 || nks >= 7 ? 4 : 2;
