@@ -92,7 +92,7 @@ __global__ __launch_bounds__(512, FX == 1 || TWO ? 4 : 2) void q8_conv_staged_ke
   const int group = staged_div(wg, p.m_tiles), x0 = (wg - group * p.tiles_x) * (32 * FX);
   const int px0 = group * p.tile_px, px1 = min(px0 + p.tile_px, p.columns) - 1;
 
-  // ---- the filter: thread (channel of 32, piece of 16), two stages of pieces on their way in registers
+  // ---- the filter: thread (channel of 32, piece of 16), the next stage's pieces on their way in registers
   const int fj = tid & 15, fc = tid >> 4;
   uint32_t frow[FX];
 #pragma unroll

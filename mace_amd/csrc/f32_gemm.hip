@@ -1108,10 +1108,13 @@ constexpr F32SlicesForm kF32Slices[mhv::F32_SLICES_FORMS] = {{1, 8}, {1, 4}, {2,
 // Which form of the slices kernel a call takes whose 128 x 128 tiles are at most one per CU; -1: none, the tiles are
 // faster.  Both times are estimated, in us: a k step takes a wavefront 0.75 (1.5 with two blocks), a CU's
 // wavefronts together 0.14 - 0.17 each and 0.25 - 0.6 a tile beside them; a 128 x 128 tile 0.63 per 16 depths behind
-// 5.3 (8.3 where loads are checked), in parts 12 and the parts' traffic.  Measured, tiles then slices: 16 x 17 x 384 ->
+// 5.3, in parts 12 and the parts' traffic, 3 more at depths in other than whole steps.  Measured, tiles then slices: 16 x 17 x 384 ->
 // 320 pointwise 14.3 and 5.8, 34 x 35 x 112 -> 91 9.7 and 4.2, 21 x 20 x 20 -> 576 at batch 5 8.9 and 6.8; 1904 x 39 x
 // 298 9.8 and 6.0, 653 x 1266 x 35 19.9 and 11.4, 883 x 2132 x 512 39.6 and 30.4 (one block 44); against the rule 20 x
 // 21 x 20 -> 160 at 20 9.1 and 9.5, 70 x 3456 x 679 22 and 30, 4 x 1024^3 53 and 107.
+// Of 2100 drawn calls of such depths (17 to 8192) 1837 go here, in 0.58 of the tiles' time in the geometric mean, 38 of them
+// more than 3 % slower (196 x 2913 x 273 against transposed weights 35.3 us, in tiles 22.4); without the 3 in parts 16 slower
+// ones, but 49 left to the tiles that are faster here, from 10; without either 133.
 static int f32_slices_form(const mace_hip_ctx *ctx, int64_t batch, int64_t rows, int64_t cols, int64_t depth,
                            int64_t total, bool whole) {
   const double cus = ctx->cu_count > 0 ? ctx->cu_count : 256;

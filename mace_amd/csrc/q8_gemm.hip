@@ -2461,7 +2461,8 @@ int launch_gemm_dma(mace_hip_ctx *ctx, GemmParams &p, bool out_u8,
   return MACE_HIP_SUCCESS;
 }
 
-// one round of 128 x 128 tiles; the caller has checked K % 128 == 0 and the 32-bit row offsets
+// at most one round of 128 x 128 tiles; the caller has set k_real, x_left and y_left, K to whole slabs, and checked the
+// 32-bit offsets
 int launch_gemm_mid_loose(mace_hip_ctx *ctx, GemmParams &p, bool out_u8, int batch, bool xt, bool yt) {
   constexpr int STAGES = 3;
   p.tiles_x = (p.XN + 127) / 128;
@@ -2485,6 +2486,7 @@ int launch_gemm_mid_loose(mace_hip_ctx *ctx, GemmParams &p, bool out_u8, int bat
 #undef MH_LOOSE
 }
 
+// one round of 128 x 128 tiles; the caller has checked K % 128 == 0 and the 32-bit row offsets
 int launch_gemm_mid(mace_hip_ctx *ctx, GemmParams &p, bool out_u8, int batch,
                     bool xt = false, bool yt = false) {
   constexpr int STAGES = 4;
