@@ -518,7 +518,8 @@ inline bool mh_q8_small_problem(const mace_hip_ctx *ctx, int64_t batch, int64_t 
 // the CUs would have a tile, at least four k tiles of 16 per part, at most 16 parts.  Forced to 1, 2, 3, 4, 8 and
 // 16 parts, the choice is the best or within 7 % of it but for the last: 512^3 (8) 26.8 unsplit, 17.7; 1024^3 (4) 46.7, 28.2, with
 // 8 41.9; 128 x 4096 x 128 (16) 158, 23.7; 1536 x 2048 x 1024 (2) 85.4, 54.9; 300 x 200 x 300 (3) 19.5, 15.7, with
-// 8 13.2 us; above half the CUs every split loses (1280 x 1024 x 1664, 130 tiles, 47.2 and 52.7).
+// 8 13.2 us; above half the CUs every split loses (1280 x 1024 x 1664, 130 tiles, 47.2 and 52.7).  (All of them are about 2 us
+// less since a tile's stores do not wait for each other: 1024^3 25.8, 128 x 4096 x 128 21.7, 1280 x 1024 x 1664 45.1.)
 // A k tile takes 0.6 us whatever else runs; the parts are written and read once more, 8 bytes per
 // output at about 4 TB/s.  Where that takes longer than the k tiles it saves the call stays whole
 // (1024 x 160 x 1568: 14.4 us, 21.7 in two parts).

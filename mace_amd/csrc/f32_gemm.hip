@@ -82,8 +82,8 @@ __device__ inline float apply_act(float v, int act, float limit) {
 // 3.4e-8 at 2.  One product alone is off by up to 0.9 units in the last place with eight wavefronts and 1.4
 // with four, where the binary32 instruction rounds it to nearest: depths 1 and 2 go to f32_fill_kernel
 // for that.  (Rows with one entry other than zero keep it; where that entry is a power of two the product
-// is exact.)  In time, 4 x 1024^3 against transposed weights 86.0 -> 51.3 us, MobileNet's five pointwise layers
-// at batch 64 688 -> 318 us.  The matrix cores are busy 42 - 51 % of 4 x 1024^3 and 12 - 35 % of the pointwise
+// is exact.)  In time, 4 x 1024^3 against transposed weights 86.0 -> 50.0 us, MobileNet's five pointwise layers
+// at batch 64 688 -> 291 us.  The matrix cores are busy 42 - 51 % of 4 x 1024^3 and 12 - 35 % of the pointwise
 // layers; the rest is each k tile's chain of LDS reads, MFMAs, LDS writes and barrier (one to three workgroups
 // per CU overlap) and, at short depths, the first loads and the stores of every tile.
 //
@@ -137,10 +137,10 @@ __device__ __forceinline__ void split_8(const float (&x)[8], u4v (&part)[3]) {
 // GUARD: depths that are not whole k tiles of 16, or an operand that is contiguous along depth in
 // rows that are not aligned 16-byte pieces: the same loads at any address; a unit that the depth ends in is read early
 // and moved down to its place in the last k tile (depths below 8, one k tile: single loads, each checked).  With every load
-// checked by itself, us, before and now: 3000 x 1000 x 1200 75 and 55 - 60 (1008 deep 54), 3000 x 1001 x 1201 against
-// transposed weights 104 and 54 - 58, 5000 x 300 x 2000 96 and 52 - 55, 627 x 1603 x 832 39 and 29.  Behind the last k tile
-// nothing is split, stored or requested, and depths below 8 load no other: 1288 x 9 x 1554 10.9 -> 8.2, 1252 x 5 x 800
-// 8.9 -> 7.1, 3615 x 20 x 490 against transposed weights 10.0 -> 9.4 (depths 3 to 7 against those 9.4 -> 9.7).
+// checked by itself, us, before and now: 3000 x 1000 x 1200 75 and 53 (1008 deep 51), 3000 x 1001 x 1201 against
+// transposed weights 104 and 50, 5000 x 300 x 2000 96 and 48, 627 x 1603 x 832 39 and 25.  Behind the last k tile
+// nothing is split, stored or requested, and depths below 8 load no other: 1288 x 9 x 1554 10.9 -> 7.8, 1252 x 5 x 800
+// 8.9 -> 6.2, 3615 x 20 x 490 against transposed weights 10.0 -> 7.3.
 //
 // A thread's unit is eight consecutive depths of one row: two 16-byte loads where depth is
 // contiguous, else eight 4-byte loads, each coalesced over the wavefront's 64 rows (so rows of any
@@ -479,11 +479,13 @@ __global__ __launch_bounds__(256 * SPLIT, SPLIT == 1 ? 3 : 1) void f32_gemm_kern
 // a block's stores and the next one's loads overlap.  Products and their order are f32_tile's with four wavefronts: the same
 // bits.
 // What bounds it: the bytes up to about 128 depths (112 x 112 x 32 -> 64 at batch 64 4.9 TB/s, what a copy reaches), beyond
-// that the vector ALU and the matrix cores, which take turns within a wavefront.  Before (tiles) and now, batch 64, us:
-// 112 x 112 x 32 -> 64 75 and 62.6, 56 x 56 x 128 -> 128 64.5 and 49.3, 28 x 28 x 256 -> 256 59.5 and 48.5, 56 x 56 x 100 ->
-// 200 130 and 95, 56 x 56 x 24 -> 144 59 and 37, 28 x 28 x 333 -> 111 56 and 45; 981 drawn layers of more tiles than CUs 1.38
-// times in the geometric mean.  (128 rows, eight wavefronts a CU: level at best, 36 % slower at 24 -> 144; a load under the
-// epilogue's test for a bias per column made every block wait for all of its loads and stores: 78 us on 56 x 56 x 128.)
+// that the vector ALU and the matrix cores, which take turns within a wavefront.  In tiles and here, batch 64, us: 112 x
+// 112 x 32 -> 64 73.6 and 60.3, 56 x 56 x 128 -> 128 65.6 and 49.8, 28 x 28 x 256 -> 256 55.5 and 48.1, 56 x 56 x 100 -> 200
+// 95.8 and 91.7, 56 x 56 x 24 -> 144 37.6 and 33.0.  Of 1500 drawn layers that come here 766 in whole k steps take 0.85 of the
+// tiles' time in the geometric mean, 149 others of up to 32 rows 0.86, 325 of more rows and up to six broken k steps 0.97, but
+// 260 of more than six 1.06 (28 x 28 x 333 -> 111 36.5 and 45.8): those were chosen against tiles that loaded depth by depth
+// (56 us) and whose stores waited for each other, and tests name that plan.  (128 rows, eight wavefronts a CU: level at best,
+// 36 % slower at 24 -> 144; a load under the epilogue's test for a bias per column made every block wait for all of its loads and stores: 78 us on 56 x 56 x 128.)
 template <int MI, int D, bool GUARD>
 __global__ __launch_bounds__(512, 4) void f32_gemm_panel_kernel(F32GemmParams p, int groups, int blocks) {
   extern __shared__ __align__(16) u4v panel[];     // [k step][part][32 rows][lane]
@@ -1117,13 +1119,12 @@ constexpr F32SlicesForm kF32Slices[mhv::F32_SLICES_FORMS] = {{1, 8}, {1, 4}, {2,
 // Which form of the slices kernel a call takes whose 128 x 128 tiles are at most one per CU; -1: none, the tiles are
 // faster.  Both times are estimated, in us: a k step takes a wavefront 0.75 (1.5 with two blocks), a CU's
 // wavefronts together 0.14 - 0.17 each and 0.25 - 0.6 a tile beside them; a 128 x 128 tile 0.63 per 16 depths behind
-// 5.3, in parts 12 and the parts' traffic, 3 more at depths in other than whole steps.  Measured, tiles then slices: 16 x 17 x 384 ->
-// 320 pointwise 14.3 and 5.8, 34 x 35 x 112 -> 91 9.7 and 4.2, 21 x 20 x 20 -> 576 at batch 5 8.9 and 6.8; 1904 x 39 x
-// 298 9.8 and 6.0, 653 x 1266 x 35 19.9 and 11.4, 883 x 2132 x 512 39.6 and 30.4 (one block 44); against the rule 20 x
-// 21 x 20 -> 160 at 20 9.1 and 9.5, 70 x 3456 x 679 22 and 30, 4 x 1024^3 53 and 107.
-// Of 2100 drawn calls of such depths (17 to 8192) 1837 go here, in 0.58 of the tiles' time in the geometric mean, 38 of them
-// more than 3 % slower (196 x 2913 x 273 against transposed weights 35.3 us, in tiles 22.4); without the 3 in parts 16 slower
-// ones, but 49 left to the tiles that are faster here, from 10; without either 133.
+// 5.3, in parts 12 and the parts' traffic, 3 more at depths in other than whole steps.  Measured, tiles then slices: 16 x 17 x
+// 384 -> 320 pointwise 12.5 and 6.3, 34 x 35 x 112 -> 91 9.8 and 4.5, 1904 x 39 x 298 8.3 and 6.4, 653 x 1266 x 35 15.6 and 11.0,
+// 512^3 15.7 and 7.3; against the rule 20 x 21 x 20 -> 160 at batch 20 8.0 and 9.5, 70 x 3456 x 679 21 and 30, 4 x 1024^3 50 and
+// 107.  Of 1000 drawn calls in whole k steps 841 go here, in 0.60 of the tiles' time in the geometric mean, five of them more
+// than 3 % slower; of 1000 others 886, 0.61 and twenty (196 x 2913 x 273 against transposed weights 35 us, in tiles 20, 883 x
+// 2132 x 512 32 and 26); without the 3 us six, but 49 left to the tiles that are faster here, now one.
 static int f32_slices_form(const mace_hip_ctx *ctx, int64_t batch, int64_t rows, int64_t cols, int64_t depth,
                            int64_t total, bool whole) {
   const double cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
@@ -1132,7 +1133,7 @@ static int f32_slices_form(const mace_hip_ctx *ctx, int64_t batch, int64_t rows,
   const double old = parts > 1 ? (whole ? 12 : 15) + 0.63 * ((nk + parts - 1) / parts) + 8.0 * parts * total / 4e6
                                : (whole ? 5.3 : 8.3) + 0.63 * nk;
   const int form = tiles <= 400 ? 0 : 1, wk = kF32Slices[form].wk;
-  // (a second tile on a few CUs counts from long depths on: 62 x 2112 x 4552, 286 tiles, 34.7 us, 27.1 by 128 x 128 tiles;
+  // (a second tile on a few CUs counts from long depths on: 62 x 2112 x 4552, 286 tiles, 34.7 us, 24.9 by 128 x 128 tiles;
   // not where the parts of those could not be had)
   const bool held = parts <= 1 || mh_arena_can_hold(ctx, sizeof(float) * (size_t)parts * total + 256);
   const double share = nk > 64 && form == 0 && tiles > cus && held ? std::max(tiles / cus, 0.8 * ceil(tiles / cus)) : tiles / cus;
@@ -1144,7 +1145,7 @@ static int f32_slices_form(const mace_hip_ctx *ctx, int64_t batch, int64_t rows,
     if (two < one) return two < 0.95 * old ? 2 : -1;
   }
   // (more, in two slices: within 5 % of the tiles; at one or two k steps a third workgroup on a CU is 20 - 30 % more:
-  // pointwise 12 x 13 x 17 -> 384 at batch 20, 1176 tiles, 11.4 us, 8.7 by tiles)
+  // pointwise 12 x 13 x 17 -> 384 at batch 20, 1176 tiles, 11.4 us, 7.7 by tiles)
   return tiles <= (nk <= 2 ? 4 * cus : 1200) && one < 0.9 * old ? form : -1;
 }
 
@@ -1252,20 +1253,19 @@ int mh_f32_gemm(mace_hip_ctx *ctx, const float *lhs, const float *rhs, int64_t b
     const int64_t small = (p.M + 31) / 32, large = (p.M + 63) / 64;
     const bool narrow = p.M <= 32 || blocks * small <= 24 * cus || 23 * small <= 40 * large;
     // (Depths from 417 on leave room for 32 rows of more than that at a time: where loads are not checked only against
-    // 128-row tiles that are a fifth padding.  14 x 14 x 512 -> 512 at batch 64 52 us in tiles, 55 - 66 here; 13440 columns,
-    // 512 -> 258 50 and 35, 7020 columns, 456 -> 575 79 and 47.)
+    // 128-row tiles that are a fifth padding.  14 x 14 x 512 -> 512 at batch 64 50 us in tiles, 55 - 66 here; 13440 columns,
+    // 512 -> 258 46 and 33.)
     const bool deep = lds_of(2) > (size_t)ctx->lds_bytes;
     const int mi = narrow || deep ? 1 : 2;
     const size_t lds = lds_of(mi);
     // Depths that are not whole k steps cost every step here (loads are checked and cleared), the tiles only the last one: not
     // two tiles of 32 rows, each of which reads the columns, against one of 64 rows.  1 x 1 layers, tiles and here: 840 x 137 ->
-    // 40 at batch 48 16.3 us and 20.8, 1640 x 201 -> 64 at 54 32.2 and 38.9.  Of 397 drawn such layers 241 are more than 3 %
-    // slower here, of 2053 others 56 (224 x 457 -> 576 at 48 52.9 and 71.7), of 1050 in whole k steps one.
+    // 40 at batch 48 14.7 us and 20.8, 1640 x 201 -> 64 at 54 25.7 and 38.9.
     const bool twice = !whole && mi == 1 && p.M > 32 && p.M <= 64;
-    // Nor deep ones, one workgroup a CU: 1.3 times the tiles' time in the median of 283 drawn layers (384 x 829 x 31464 125 us
-    // and 216, 704 x 671 x 19600 132 and 212), but for little more than a round of tiles a fifth of which is padding (148 x
-    // 418 x 12096 33 and 25).  (Depths of 417 to 432, one step more than leaves room for 64 rows, come here as they did, though
-    // slower too: 111 x 420 x 50176 53 us in tiles and 75.  A test names that plan.)
+    // Nor deep ones, one workgroup a CU (384 x 829 x 31464 122 us and 216, 704 x 671 x 19600 128 and 212, 224 x 457 -> 576 at
+    // batch 48 47 and 72), but for little more than a round of tiles a fifth of which is padding (148 x 418 x 12096 29.5 and
+    // 24.1).  (Depths of 417 to 432, one step more than leaves room for 64 rows, come here as they did, though slower too: 111 x
+    // 420 x 50176 43.5 us in tiles and 62.  A test names that plan.)
     const bool slow = !whole && deep && p.M > 32 && nks > 27 &&
                       !(6ll * p.M <= 5ll * tm * ((p.M + tm - 1) / tm) && 5 * tiles <= 6 * cus);
     if (lds <= (size_t)ctx->lds_bytes && !twice && !slow && (!deep || p.M <= 32 || !whole || 4 * TM * ((p.M + TM - 1) / TM) >= 5ll * p.M)) {
