@@ -485,7 +485,8 @@ __global__ __launch_bounds__(256 * SPLIT, SPLIT == 1 ? 3 : 1) void f32_gemm_kern
 // tiles' time in the geometric mean, 149 others of up to 32 rows 0.86, 325 of more rows and up to six broken k steps 0.97, but
 // 260 of more than six 1.06 (28 x 28 x 333 -> 111 36.5 and 45.8): those were chosen against tiles that loaded depth by depth
 // (56 us) and whose stores waited for each other, and tests name that plan.  (128 rows, eight wavefronts a CU: level at best,
-// 36 % slower at 24 -> 144; a load under the epilogue's test for a bias per column made every block wait for all of its loads and stores: 78 us on 56 x 56 x 128.)
+// 36 % slower at 24 -> 144; a load under the epilogue's test for a bias per column made every block wait for all of its loads
+// and stores: 78 us on 56 x 56 x 128.)
 template <int MI, int D, bool GUARD>
 __global__ __launch_bounds__(512, 4) void f32_gemm_panel_kernel(F32GemmParams p, int groups, int blocks) {
   extern __shared__ __align__(16) u4v panel[];     // [k step][part][32 rows][lane]
